@@ -386,7 +386,7 @@ class Solver:
     # ---- state ----
     def download(self):
         n = self.n
-        pos, vel, acc, box = np.zeros((n, 3)), np.zeros((n, 3)), np.zeros((n, 3)), np.zeros((self.nrep, 3))
+        pos, vel, acc, box = np.empty((n, 3)), np.empty((n, 3)), np.empty((n, 3)), np.empty((self.nrep, 3))
         _check(lib().sm_download_state(self.h, _dp(pos), _dp(vel), _dp(acc), _dp(box)))
         return pos, vel, acc, self._one(box)
 
@@ -433,7 +433,7 @@ class Solver:
 
     def compute_forces(self):
         n = self.n
-        fp, fc = np.zeros((n, 3)), np.zeros((n, 3))
+        fp, fc = np.empty((n, 3)), np.empty((n, 3))
         _check(lib().sm_compute_forces(self.h, _dp(fp), _dp(fc)))
         return fp, fc
 

@@ -5,6 +5,7 @@
 #include "sm_adjoint.hpp"
 #include "sm_errors.hpp"
 #include "sm_internal.hpp"
+#include "sm_transfer.hpp"
 
 #include <hip/hip_runtime.h>
 
@@ -178,6 +179,12 @@ struct sm_ctx {
     int sort_bits = 0;
     DevRep *reps = nullptr;
     DevGlobal *glob = nullptr;
+    HostLink link;             // results on their way to the host
+    // The boxes as last read or set, 3 per replica, and the box moves launched since: a box
+    // lies within moves * |delta_lxy| of them, so most runs need no read-back to know that the
+    // cell table is large enough.
+    std::vector<double> boxL, deltaL;
+    long long moves_since = 0;
     float *fconstF = nullptr;   // pair table: padded FP32 force rows, then the reach tables
     double *uconstD = nullptr;
     double *fconstD = nullptr;   // FP64 force rows (the force kernel's pair-count hook)
@@ -252,6 +259,7 @@ struct sm_ctx {
     {
         if (st) (void)hipStreamSynchronize(st);
         drop_graph();
+        link.destroy();
         for (auto &r : recs) { (void)hipEventDestroy(r.a); (void)hipEventDestroy(r.b); }
         for (auto e : pool) (void)hipEventDestroy(e);
         dfree(beads); dfree(sbeads); dfree(beads_alt); dfree(vel); dfree(acc); dfree(fpair); dfree(fscratch);
@@ -340,17 +348,49 @@ struct sm_ctx {
         return g;
     }
 
-    void check_flags()
+    void check_flags() { check_bits(link.fetch(st, glob, nullptr, 0, nullptr)); }
+    static void check_bits(int flags)
     {
-        const DevGlobal g = read_glob();
-        if (g.flags & FLAG_BAD_POSITION)
+        if (flags & FLAG_BAD_POSITION)
             throw ApiError(SM_ERR_STATE, "a particle position left the box or became non-finite");
-        if (g.flags & FLAG_SORT_TIMEOUT)
+        if (flags & FLAG_SORT_TIMEOUT)
             throw ApiError(SM_ERR_STATE, "cell-key sort look-back timed out");
-        if (g.flags & FLAG_SORT_COUNT)
+        if (flags & FLAG_SORT_COUNT)
             throw ApiError(SM_ERR_STATE, "incremental cell sort: inconsistent mover count");
-        if (g.flags & FLAG_CELL_OVERFLOW)
+        if (flags & FLAG_CELL_OVERFLOW)
             throw ApiError(SM_ERR_STATE, "an accepted box move would exceed the cell table or make fewer than 3 cells per axis");
+    }
+    // `count` doubles of results to the host, and the state checked
+    void fetch(const double *src, size_t count, double *dst) { check_bits(link.fetch(st, glob, src, count, dst)); }
+
+    // the device's boxes were set back to an earlier state's: read them when next needed
+    void forget_boxes() { moves_since = 1ll << 40; }
+
+    // the current box lengths (boxL), read back if box moves were launched since
+    void know_boxes()
+    {
+        if (moves_since == 0) return;
+        link.fetch_boxes(st, glob, reps, nrep, boxL.data());
+        moves_since = 0;
+    }
+
+    // cells that replica r needs for every box that `moves` MC moves from boxL can reach;
+    // kUnbounded when the moves could take the box anywhere (the device then refuses the
+    // accepted move that outgrows the table)
+    static constexpr long long kUnbounded = (long long)9e18;
+    long long cells_needed(int r, long long moves) const
+    {
+        const double dL = deltaL[r], *L = &boxL[3 * (size_t)r];
+        const double grow = (double)moves * std::fabs(dL);
+        double Lmax[3], Lmin[2];
+        for (int d = 0; d < 2; d++) {
+            Lmax[d] = L[d] + grow;
+            Lmin[d] = std::max(L[d] - grow, 1e-300);
+        }
+        Lmax[2] = (moves > 0 && dL != 0) ? L[2] * (L[0] * L[1]) / (Lmin[0] * Lmin[1]) : L[2];
+        double need = 1.0;   // a product that may pass 2^63 while the bound is loose
+        for (int d = 0; d < 3; d++) need *= std::floor(Lmax[d] / P.cutoff) + 1.0;
+        return need < 9e18 ? (long long)need : kUnbounded;
     }
 
     // Dense cell table sized for every box the next `moves` MC moves can reach, in every
@@ -358,34 +398,30 @@ struct sm_ctx {
     // recomputed each step, so only the table is reallocated).
     void ensure_capacity(long long moves)
     {
-        std::vector<DevRep> hr = read_reps();
-        bool relayout = capacity == 0;
-        const double rc = P.cutoff;
-        for (int r = 0; r < nrep; r++) {
-            const double dL = hr[r].delta_lxy;
-            const double grow = (double)moves * std::fabs(dL);
-            double Lmax[3], Lmin[2];
-            for (int d = 0; d < 2; d++) {
-                Lmax[d] = hr[r].L[d] + grow;
-                Lmin[d] = std::max(hr[r].L[d] - grow, 1e-300);
-            }
-            Lmax[2] = (moves > 0 && dL != 0) ? hr[r].L[2] * (hr[r].L[0] * hr[r].L[1]) / (Lmin[0] * Lmin[1]) : hr[r].L[2];
-            long long need = 1;
-            for (int d = 0; d < 3; d++) need *= (long long)(Lmax[d] / rc) + 1;
-            if (need > rh[r].capacity) {
-                rh[r].capacity = need + need / 8;
-                relayout = true;
-            }
-        }
+        auto grows = [&](int r) {
+            const long long need = cells_needed(r, moves);
+            return need > rh[r].capacity && need != kUnbounded;
+        };
+        bool relayout = false;
+        for (int r = 0; r < nrep && !relayout; r++) relayout = cells_needed(r, moves_since + moves) > rh[r].capacity;
         if (!relayout) return;
+        know_boxes();
+        relayout = false;
+        for (int r = 0; r < nrep && !relayout; r++) relayout = grows(r);
+        if (!relayout) return;
+        std::vector<DevRep> hr = read_reps();
         long long base = 0;
         for (int r = 0; r < nrep; r++) {
+            if (grows(r)) {
+                const long long need = cells_needed(r, moves);
+                rh[r].capacity = need + need / 8;
+            }
             rh[r].cellbase = base;
-            base += rh[r].capacity;
+            if (rh[r].capacity > 0xFFFFFFFFll || (base += rh[r].capacity) > 0xFFFFFFFFll)
+                unsupported("cell tables of all replicas exceed 2^32 cells");
             hr[r].cellbase = rh[r].cellbase;
             hr[r].capacity = rh[r].capacity;
         }
-        if (base > 0xFFFFFFFFll) unsupported("cell tables of all replicas exceed 2^32 cells");
         drop_graph();
         dfree(cstart);
         dfree(cend);
@@ -525,6 +561,7 @@ struct sm_ctx {
     }
     void mc_decide()
     {
+        moves_since++;
         timed(K_MC, [&] {
             launch_mc_decide(st, P, reps, glob, du_dev());
             launch_rescale(st, n, beads, reps);
@@ -624,6 +661,7 @@ struct sm_ctx {
             HIPCHK(hipGraphInstantiate(&gexec[p], graph[p], nullptr, nullptr, 0));
         }
         sort_parity = p;   // capture only recorded the toggles
+        if (any_mc) moves_since++;
         // the block advances from step s - 1
         launch_set_step(st, glob, s - 1);
         HIPCHK(hipGraphLaunch(gexec[p], st));
@@ -895,6 +933,8 @@ sm_ctx *create(const sm_system *s, int nrep)
             R.sigma_fixed = q.sigma_temperature > 0 ? 1 : 0;
             R.delta_lxy = q.delta_lxy;
             R.tension = q.tension;
+            c->boxL.insert(c->boxL.end(), q.box, q.box + 3);
+            c->deltaL.push_back(q.delta_lxy);
             if (q.delta_lxy != 0) c->any_mc = true;
         }
         const int nT = s[0].n_types;
@@ -1013,19 +1053,6 @@ sm_ctx *create(const sm_system *s, int nrep)
     return c;
 }
 
-template <class T>
-void download_f4(sm_ctx *c, const float4 *src, T *dst)
-{
-    std::vector<float4> h(c->n);
-    HIPCHK(hipMemcpyAsync(h.data(), src, sizeof(float4) * c->n, hipMemcpyDeviceToHost, c->st));
-    HIPCHK(hipStreamSynchronize(c->st));
-    for (int i = 0; i < c->n; i++) {
-        dst[3 * (size_t)i] = h[i].x;
-        dst[3 * (size_t)i + 1] = h[i].y;
-        dst[3 * (size_t)i + 2] = h[i].z;
-    }
-}
-
 }  // namespace
 
 // ---------------------------------------------------------------------------------------
@@ -1080,8 +1107,7 @@ int sm_sync(sm_ctx *c)
 {
     return guarded([&] {
         if (!c) invalid("null context");
-        HIPCHK(hipStreamSynchronize(c->st));
-        c->check_flags();
+        c->check_flags();   // waits for the stream
     });
 }
 
@@ -1089,24 +1115,16 @@ int sm_download_state(sm_ctx *c, double *pos, double *vel, double *acc, double *
 {
     return guarded([&] {
         if (!c) invalid("null context");
-        const int n = c->n;
-        if (pos) {
-            std::vector<Bead> hb(n);
-            HIPCHK(hipMemcpyAsync(hb.data(), c->beads, sizeof(Bead) * n, hipMemcpyDeviceToHost, c->st));
-            HIPCHK(hipStreamSynchronize(c->st));
-            for (int i = 0; i < n; i++) {
-                pos[3 * (size_t)i] = hb[i].x;
-                pos[3 * (size_t)i + 1] = hb[i].y;
-                pos[3 * (size_t)i + 2] = hb[i].z;
-            }
-        }
-        if (vel) download_f4(c, c->vel, vel);
-        if (acc) download_f4(c, c->acc, acc);
-        std::vector<DevRep> hr = c->read_reps();
-        if (box)
-            for (int r = 0; r < c->nrep; r++)
-                for (int d = 0; d < 3; d++) box[3 * r + d] = hr[r].L[d];
-        c->check_flags();
+        // positions, velocities and accelerations in one pass; the boxes and flags with them
+        const PackSrc src{c->beads, c->vel, c->acc};
+        int flags;
+        if (pos || vel || acc)
+            flags = c->link.fetch_beads(c->st, c->n, src, pos, vel, acc, c->glob, c->reps, c->nrep, c->boxL.data());
+        else
+            flags = c->link.fetch_boxes(c->st, c->glob, c->reps, c->nrep, c->boxL.data());
+        c->moves_since = 0;
+        if (box) std::copy(c->boxL.begin(), c->boxL.end(), box);
+        c->check_bits(flags);
     });
 }
 
@@ -1115,34 +1133,26 @@ int sm_upload_state(sm_ctx *c, const double *pos, const double *vel, const doubl
     return guarded([&] {
         if (!c) invalid("null context");
         const int n = c->n;
-        std::vector<DevRep> hr = c->read_reps();
+        std::vector<double> L(c->boxL.size());
         if (box) {
-            for (int r = 0; r < c->nrep; r++)
-                for (int d = 0; d < 3; d++) {
-                    const double L = box[3 * r + d];
-                    if (!(L > 0)) invalid("box lengths must be positive");
-                    const int nc = (int)(L / c->P.cutoff);
-                    if (nc < 3) unsupported("fewer than 3 cells along an axis");
-                    hr[r].L[d] = L;
-                    hr[r].nc[d] = nc;
-                    hr[r].cs[d] = L / nc;
-                }
+            std::copy(box, box + L.size(), L.begin());
+            for (const double l : L) {
+                if (!(l > 0)) invalid("box lengths must be positive");
+                if ((int)(l / c->P.cutoff) < 3) unsupported("fewer than 3 cells along an axis");
+            }
+        } else if (pos) {
+            c->know_boxes();
+            L = c->boxL;
         }
         if (pos) {
-            std::vector<Bead> hb(n);
-            HIPCHK(hipMemcpyAsync(hb.data(), c->beads, sizeof(Bead) * n, hipMemcpyDeviceToHost, c->st));
-            HIPCHK(hipStreamSynchronize(c->st));
-            for (int i = 0; i < n; i++) {
-                const DevRep &R = hr[hb[i].rep];
-                for (int d = 0; d < 3; d++) {
-                    const double p = pos[3 * (size_t)i + d];
-                    if (!(p >= 0 && p <= R.L[d])) invalid("particle " + std::to_string(i) + " position is out of bounds");
-                }
-                hb[i].x = pos[3 * (size_t)i];
-                hb[i].y = pos[3 * (size_t)i + 1];
-                hb[i].z = pos[3 * (size_t)i + 2];
-            }
-            HIPCHK(hipMemcpyAsync(c->beads, hb.data(), sizeof(Bead) * n, hipMemcpyHostToDevice, c->st));
+            for (int r = 0; r < c->nrep; r++)
+                for (int i = c->rh[r].first; i < c->rh[r].first + c->rh[r].count; i++)
+                    for (int d = 0; d < 3; d++) {
+                        const double p = pos[3 * (size_t)i + d];
+                        if (!(p >= 0 && p <= L[3 * (size_t)r + d]))
+                            invalid("particle " + std::to_string(i) + " position is out of bounds");
+                    }
+            c->link.send_positions(c->st, n, pos, c->beads);
         }
         auto up3 = [&](float4 *dst, const double *src) {
             std::vector<float4> h(n);
@@ -1153,8 +1163,19 @@ int sm_upload_state(sm_ctx *c, const double *pos, const double *vel, const doubl
         };
         if (vel) up3(c->vel, vel);
         if (acc) up3(c->acc, acc);
-        c->write_reps(hr);
-        c->ensure_capacity(0);
+        if (box) {
+            std::vector<DevRep> hr = c->read_reps();
+            for (int r = 0; r < c->nrep; r++)
+                for (int d = 0; d < 3; d++) {
+                    hr[r].L[d] = L[3 * (size_t)r + d];
+                    hr[r].nc[d] = (int)(hr[r].L[d] / c->P.cutoff);
+                    hr[r].cs[d] = hr[r].L[d] / hr[r].nc[d];
+                }
+            c->write_reps(hr);
+            c->boxL = L;
+            c->moves_since = 0;
+            c->ensure_capacity(0);
+        }
     });
 }
 
@@ -1211,11 +1232,7 @@ int sm_step_finish(sm_ctx *c, int64_t step, double *measure)
         const bool mc = c->mc_step(step);
         c->step_finish(measure != nullptr, mc);
         c->check_launch();
-        if (measure) {
-            HIPCHK(hipMemcpyAsync(measure, c->meas_dev(), 3 * sizeof(double) * c->nrep, hipMemcpyDeviceToHost, c->st));
-            HIPCHK(hipStreamSynchronize(c->st));
-            c->check_flags();
-        }
+        if (measure) c->fetch(c->meas_dev(), 3 * (size_t)c->nrep, measure);
     });
 }
 
@@ -1268,9 +1285,7 @@ int sm_measure(sm_ctx *c, double *out)
         c->build(0, kStepKeep);
         c->measure_device();
         c->check_launch();
-        HIPCHK(hipMemcpyAsync(out, c->meas_dev(), 3 * sizeof(double) * c->nrep, hipMemcpyDeviceToHost, c->st));
-        HIPCHK(hipStreamSynchronize(c->st));
-        c->check_flags();
+        c->fetch(c->meas_dev(), 3 * (size_t)c->nrep, out);
     });
 }
 
@@ -1377,9 +1392,12 @@ int sm_compute_forces(sm_ctx *c, double *pair_out, double *chain_out)
         c->pair_force();
         c->bonded(KICK_NONE, c->fscratch);
         c->check_launch();
-        if (pair_out) download_f4(c, c->fpair, pair_out);
-        if (chain_out) download_f4(c, c->fscratch, chain_out);
-        c->check_flags();
+        if (pair_out || chain_out) {
+            c->check_bits(c->link.fetch_beads(c->st, c->n, PackSrc{nullptr, c->fpair, c->fscratch}, nullptr, pair_out,
+                                              chain_out, c->glob, c->reps, c->nrep, nullptr));
+        } else {
+            c->check_flags();
+        }
     });
 }
 
@@ -1482,13 +1500,12 @@ int sm_potential_delta(sm_ctx *c, const double *scale, double *du_pair, double *
         }
         c->check_launch();
         std::vector<double> h(2 * (size_t)c->nrep);
-        HIPCHK(hipMemcpyAsync(h.data(), c->du_dev(), sizeof(double) * h.size(), hipMemcpyDeviceToHost, c->st));
-        HIPCHK(hipStreamSynchronize(c->st));
+        const int flags = c->link.fetch(c->st, c->glob, c->du_dev(), h.size(), h.data());
         for (int r = 0; r < c->nrep; r++) {
             if (du_pair) du_pair[r] = h[2 * r];
             if (du_chain) du_chain[r] = h[2 * r + 1];
         }
-        c->check_flags();
+        c->check_bits(flags);
     });
 }
 
@@ -1581,6 +1598,7 @@ int sm_autotune(sm_ctx *c, int32_t steps, double *best_ms_per_step)
                 copy(g0, c->glob, sizeof(DevGlobal));
             };
             auto restore = [&] {
+                c->forget_boxes();
                 copy(c->beads, b0, sizeof(Bead) * n); copy(c->vel, v0, sizeof(float4) * n);
                 copy(c->acc, a0, sizeof(float4) * n); copy(c->reps, r0, sizeof(DevRep) * c->nrep);
                 copy(c->glob, g0, sizeof(DevGlobal));
@@ -1810,6 +1828,7 @@ struct StateCopy {
     }
     void load(sm_ctx *c) const
     {
+        c->forget_boxes();
         HIPCHK(hipMemcpyAsync(c->beads, beads, sizeof(Bead) * c->n, hipMemcpyDeviceToDevice, c->st));
         HIPCHK(hipMemcpyAsync(c->vel, vel, sizeof(float4) * c->n, hipMemcpyDeviceToDevice, c->st));
         HIPCHK(hipMemcpyAsync(c->acc, acc, sizeof(float4) * c->n, hipMemcpyDeviceToDevice, c->st));
@@ -1876,11 +1895,10 @@ int sm_param_derivative(sm_ctx *c, int32_t type_a, int32_t type_b, double *out)
             }
         c->check_launch();
         std::vector<double> h((size_t)5 * R);
-        HIPCHK(hipMemcpyAsync(h.data(), w, sizeof(double) * h.size(), hipMemcpyDeviceToHost, c->st));
-        HIPCHK(hipStreamSynchronize(c->st));
+        const int flags = c->link.fetch(c->st, c->glob, w, h.size(), h.data());
         for (int r = 0; r < R; r++)
             for (int p = 0; p < 4; p++) out[4 * (size_t)r + p] = (p >= 2 && c->nchains == 0) ? 0.0 : h[5 * r + p];
-        c->check_flags();
+        c->check_bits(flags);
     });
 }
 
@@ -1936,8 +1954,7 @@ int sm_adjoint(sm_ctx *c, int32_t type_a, int32_t type_b, int32_t nsteps, int32_
             for (int s = 1; s <= S; s++) {
                 c->step_first(s);
                 c->step_finish(true, c->mc_step(s));
-                HIPCHK(hipMemcpyAsync(m.data(), c->meas_dev(), sizeof(double) * m.size(), hipMemcpyDeviceToHost, st));
-                HIPCHK(hipStreamSynchronize(st));
+                c->link.fetch(st, c->glob, c->meas_dev(), m.size(), m.data());
                 for (int r = 0; r < R; r++) Jsum[r] += m[3 * r] + m[3 * r + 1];
                 if (s % k == 0 && s / k < ncp) cps[s / k].save(c);
             }

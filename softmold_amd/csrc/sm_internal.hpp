@@ -215,6 +215,20 @@ void launch_mc_propose(hipStream_t st, int nrep, DevRep *reps, const DevGlobal *
 // du[r*2 + 0] = dU_pair, du[r*2 + 1] = dU_chain of replica r
 void launch_mc_decide(hipStream_t st, const Params &P, DevRep *reps, DevGlobal *glob, const double *du);
 void launch_rescale(hipStream_t st, int n, Bead *beads, const DevRep *reps);
+// Result packing (sm_transfer.hpp), into pinned host memory.  launch_post: head[0] = the state
+// flags as a 64-bit integer, head[1 ..] = src[0 .. count).  launch_pack: `count` beads from
+// `first` on, the positions as doubles, then each float4 array's x, y, z as floats (a NULL
+// source is left out); where head is given, the flags and the nrep boxes go to it.
+struct PackSrc {
+    const Bead *beads;
+    const float4 *a, *b;
+};
+constexpr size_t kPackBytes = 3 * (sizeof(double) + 2 * sizeof(float));   // per bead, all sources
+void launch_post(hipStream_t st, const double *src, size_t count, const DevGlobal *glob, double *head);
+void launch_pack(hipStream_t st, int first, int count, const PackSrc &src, double *out, const DevRep *reps, int nrep,
+                 const DevGlobal *glob, double *head);
+// beads[first ..].x, y, z = pos (pinned host memory, 3 per bead)
+void launch_set_positions(hipStream_t st, int first, int count, const double *pos, Bead *beads);
 // fill kernel (graph-capturable replacement for hipMemsetAsync)
 void launch_fill_u32(hipStream_t st, uint32_t *p, size_t count, uint32_t value);
 void launch_set_step(hipStream_t st, DevGlobal *glob, long long step);

@@ -6,6 +6,8 @@
 // thermostat and MC state through Bead::rep.
 #include "sm_sort_dev.hpp"
 
+#include <algorithm>
+
 namespace smdev {
 
 namespace {
@@ -845,6 +847,40 @@ __global__ __launch_bounds__(kBlock) void k_fill_u32(uint32_t *__restrict__ p, s
     if (i < count) p[i] = value;
 }
 
+// Results written straight to pinned host memory: consecutive lanes write consecutive words,
+// so a bead's three components come from neighbouring lanes (the loads hit the caches).
+__global__ __launch_bounds__(kBlock) void k_post(const double *__restrict__ src, size_t count,
+                                                 const DevGlobal *__restrict__ glob, double *__restrict__ head)
+{
+    const size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x;
+    if (i == 0) *reinterpret_cast<long long *>(head) = glob->flags;
+    if (i < count) head[1 + i] = src[i];
+}
+
+__global__ __launch_bounds__(kBlock) void k_pack(int first, int count, PackSrc src, double *__restrict__ out,
+                                                 const DevRep *__restrict__ reps, int nrep,
+                                                 const DevGlobal *__restrict__ glob, double *__restrict__ head)
+{
+    if (head && blockIdx.x == 0) {
+        if (threadIdx.x == 0) *reinterpret_cast<long long *>(head) = glob->flags;
+        for (int i = threadIdx.x; i < 3 * nrep; i += kBlock) head[1 + i] = reps[i / 3].L[i % 3];
+    }
+    const int e = blockIdx.x * kBlock + threadIdx.x;
+    if (e >= 3 * count) return;
+    const int i = first + e / 3, c = e % 3;
+    float *f = reinterpret_cast<float *>(out + (src.beads ? 3 * (size_t)count : 0));
+    if (src.beads) out[e] = (&src.beads[i].x)[c];
+    if (src.a) f[e] = (&src.a[i].x)[c];
+    if (src.b) f[(src.a ? 3 * (size_t)count : 0) + e] = (&src.b[i].x)[c];
+}
+
+__global__ __launch_bounds__(kBlock) void k_set_positions(int first, int count, const double *__restrict__ pos,
+                                                          Bead *__restrict__ beads)
+{
+    const int e = blockIdx.x * kBlock + threadIdx.x;
+    if (e < 3 * count) (&beads[first + e / 3].x)[e % 3] = pos[e];
+}
+
 inline int blocks(long long n) { return (int)((n + kBlock - 1) / kBlock); }
 
 }  // namespace
@@ -965,6 +1001,23 @@ void launch_mc_decide(hipStream_t st, const Params &P, DevRep *reps, DevGlobal *
 void launch_rescale(hipStream_t st, int n, Bead *beads, const DevRep *reps)
 {
     hipLaunchKernelGGL(k_rescale, dim3(blocks(n)), dim3(kBlock), 0, st, n, beads, reps);
+}
+
+void launch_post(hipStream_t st, const double *src, size_t count, const DevGlobal *glob, double *head)
+{
+    hipLaunchKernelGGL(k_post, dim3(std::max(1, blocks((long long)count))), dim3(kBlock), 0, st, src, count, glob, head);
+}
+
+void launch_pack(hipStream_t st, int first, int count, const PackSrc &src, double *out, const DevRep *reps, int nrep,
+                 const DevGlobal *glob, double *head)
+{
+    hipLaunchKernelGGL(k_pack, dim3(std::max(1, blocks(3ll * count))), dim3(kBlock), 0, st, first, count, src, out, reps,
+                       nrep, glob, head);
+}
+
+void launch_set_positions(hipStream_t st, int first, int count, const double *pos, Bead *beads)
+{
+    hipLaunchKernelGGL(k_set_positions, dim3(blocks(3ll * count)), dim3(kBlock), 0, st, first, count, pos, beads);
 }
 
 void launch_set_step(hipStream_t st, DevGlobal *glob, long long step)

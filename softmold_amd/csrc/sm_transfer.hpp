@@ -1,0 +1,213 @@
+// Device-to-host results of a context: a kernel packs what the caller asked for straight into
+// pinned host memory, and the host unpacks it into the caller's buffers.
+//
+// What bounds it: a small result costs its round trips, a large one the caller's fresh pages.
+// One pack kernel and one event take 13 us on an MI355X where every pageable copy takes 25 us
+// (a download was five of them); at 3M beads the 144 MB cross the bus in 3 ms, but one thread
+// fills the 216 MB of doubles in 46 ms, eight in 10 ms.  Large states therefore go in chunks
+// through two pinned buffers while up to kWorkers threads unpack the chunk before.
+#pragma once
+#include "sm_errors.hpp"
+#include "sm_internal.hpp"
+
+#include <algorithm>
+#include <atomic>
+#include <cstring>
+#include <system_error>
+#include <thread>
+#include <vector>
+
+namespace smdev {
+
+class HostLink {
+public:
+    static constexpr int kChunk = 65536;          // beads a pinned buffer holds
+    static constexpr int kThreadBeads = 65536;    // fewer beads are unpacked by the caller alone
+    static constexpr int kWorkers = 8;
+
+    void destroy()
+    {
+        for (void *&p : buf_) {
+            if (p) (void)hipHostFree(p);
+            p = nullptr;
+        }
+        for (hipEvent_t &e : ev_) {
+            if (e) (void)hipEventDestroy(e);
+            e = nullptr;
+        }
+        if (head_) (void)hipHostFree(head_);
+        head_ = nullptr;
+    }
+
+    // `count` doubles from device memory with the context's state flags: returns the flags
+    int fetch(hipStream_t st, const DevGlobal *glob, const double *src, size_t count, double *dst)
+    {
+        head(count);
+        launch_post(st, src, count, glob, head_);
+        check(hipGetLastError(), "post");
+        finish(st, 0);
+        if (count) std::memcpy(dst, head_ + 1, count * sizeof(double));
+        return flags();
+    }
+
+    // The box lengths of every replica and the state flags.
+    int fetch_boxes(hipStream_t st, const DevGlobal *glob, const DevRep *reps, int nrep, double *box)
+    {
+        head(3 * (size_t)nrep);
+        launch_pack(st, 0, 0, PackSrc{nullptr, nullptr, nullptr}, nullptr, reps, nrep, glob, head_);
+        check(hipGetLastError(), "pack");
+        finish(st, 0);
+        std::memcpy(box, head_ + 1, 3 * sizeof(double) * (size_t)nrep);
+        return flags();
+    }
+
+    // n beads' positions and up to two float4 arrays as n x 3 doubles (a NULL destination
+    // skips its source), the boxes if box, and the state flags.
+    int fetch_beads(hipStream_t st, int n, const PackSrc &src, double *pos, double *a, double *b,
+                    const DevGlobal *glob, const DevRep *reps, int nrep, double *box)
+    {
+        const PackSrc s{pos ? src.beads : nullptr, a ? src.a : nullptr, b ? src.b : nullptr};
+        const int chunks = (n + kChunk - 1) / kChunk;
+        head(3 * (size_t)nrep);
+        buffers(std::min(n, kChunk), chunks > 1 ? 2 : 1);
+        auto launch = [&](int c) {
+            const int first = c * kChunk, count = std::min(kChunk, n - first);
+            launch_pack(st, first, count, s, static_cast<double *>(buf_[c & 1]), reps, c == 0 ? nrep : 0, glob,
+                        c == 0 ? head_ : nullptr);
+            check(hipGetLastError(), "pack");
+            check(hipEventRecord(ev_[c & 1], st), "event");
+        };
+        auto wait = [&](int c) { check(hipEventSynchronize(ev_[c & 1]), "event"); };
+        // beads [count i / parts, count (i + 1) / parts) of chunk c into the caller's arrays
+        auto unpack = [&](int c, int i, int parts) {
+            const int first = c * kChunk, count = std::min(kChunk, n - first);
+            const size_t e0 = 3 * ((size_t)count * i / parts), e1 = 3 * ((size_t)count * (i + 1) / parts);
+            const double *p = static_cast<const double *>(buf_[c & 1]);
+            const float *f = reinterpret_cast<const float *>(p + (s.beads ? 3 * (size_t)count : 0));
+            const size_t o = 3 * (size_t)first;
+            if (s.beads) std::memcpy(pos + o + e0, p + e0, (e1 - e0) * sizeof(double));
+            if (s.a)
+                for (size_t e = e0; e < e1; e++) a[o + e] = f[e];
+            if (s.a) f += 3 * (size_t)count;
+            if (s.b)
+                for (size_t e = e0; e < e1; e++) b[o + e] = f[e];
+        };
+        const int want = n < kThreadBeads ? 1 : std::max(1, std::min(kWorkers, (int)std::thread::hardware_concurrency() / 2));
+        std::atomic<int> ready{0}, done{0};
+        std::atomic<bool> quit{false};
+        std::vector<std::thread> team;
+        struct Join {
+            std::vector<std::thread> &t;
+            std::atomic<bool> &quit;
+            ~Join()
+            {
+                quit.store(true);
+                for (auto &x : t) x.join();
+            }
+        };
+        int parts = 1;
+        {
+            Join join{team, quit};
+            launch(0);
+            std::atomic<int> size{0};   // parts, once every worker that could be started was
+            auto work = [&](int i) {
+                while (size.load(std::memory_order_acquire) == 0)
+                    if (quit.load()) return;
+                    else std::this_thread::yield();
+                const int parts = size.load();
+                for (int c = 0; c < chunks; c++) {
+                    while (ready.load(std::memory_order_acquire) <= c)
+                        if (quit.load()) return;
+                        else std::this_thread::yield();
+                    unpack(c, i, parts);
+                    done.fetch_add(1, std::memory_order_release);
+                }
+            };
+            try {
+                team.reserve(want);
+                for (int i = 1; i < want; i++) team.emplace_back(work, i);
+            } catch (const std::system_error &) {   // fewer threads then
+            }
+            parts = 1 + (int)team.size();
+            size.store(parts, std::memory_order_release);
+            if (chunks > 1) launch(1);
+            for (int c = 0; c < chunks; c++) {
+                wait(c);
+                ready.store(c + 1, std::memory_order_release);
+                unpack(c, 0, parts);
+                while (done.load(std::memory_order_acquire) < (c + 1) * (parts - 1)) std::this_thread::yield();
+                if (c + 2 < chunks) launch(c + 2);
+            }
+        }
+        if (box) std::memcpy(box, head_ + 1, 3 * sizeof(double) * (size_t)nrep);
+        return flags();
+    }
+
+    // beads[i].x, y, z = pos[3 i ..] for n beads; the caller's array is free again on return
+    void send_positions(hipStream_t st, int n, const double *pos, Bead *beads)
+    {
+        events();
+        const int chunks = (n + kChunk - 1) / kChunk;
+        buffers(std::min(n, kChunk), chunks > 1 ? 2 : 1);
+        for (int c = 0; c < chunks; c++) {
+            const int first = c * kChunk, count = std::min(kChunk, n - first);
+            check(hipEventSynchronize(ev_[c & 1]), "event");   // the buffer's last kernel is done
+            std::memcpy(buf_[c & 1], pos + 3 * (size_t)first, 3 * sizeof(double) * (size_t)count);
+            launch_set_positions(st, first, count, static_cast<const double *>(buf_[c & 1]), beads);
+            check(hipGetLastError(), "unpack");
+            check(hipEventRecord(ev_[c & 1], st), "event");
+        }
+    }
+
+private:
+    void *buf_[2] = {nullptr, nullptr};
+    size_t beads_[2] = {0, 0};
+    double *head_ = nullptr;      // flags, then up to head_count_ doubles
+    size_t head_count_ = 0;
+    hipEvent_t ev_[2] = {nullptr, nullptr};
+
+    static void check(hipError_t e, const char *what)
+    {
+        if (e != hipSuccess)
+            throw smapi::ApiError(SM_ERR_HIP, std::string(hipGetErrorName(e)) + " in a " + what + " of a result transfer");
+    }
+    void events()
+    {
+        for (hipEvent_t &e : ev_)
+            if (!e) check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "event");
+    }
+    void head(size_t count)
+    {
+        events();
+        if (head_ && count <= head_count_) return;
+        if (head_) (void)hipHostFree(head_);
+        head_ = nullptr;
+        head_count_ = 0;
+        check(hipHostMalloc(reinterpret_cast<void **>(&head_), (count + 1) * sizeof(double), hipHostMallocDefault), "buffer");
+        head_count_ = count;
+    }
+    void buffers(int beads, int want)
+    {
+        for (int i = 0; i < want; i++) {
+            if (buf_[i] && (size_t)beads <= beads_[i]) continue;
+            if (buf_[i]) (void)hipHostFree(buf_[i]);
+            buf_[i] = nullptr;
+            beads_[i] = 0;
+            check(hipHostMalloc(&buf_[i], (size_t)std::max(beads, 1) * kPackBytes, hipHostMallocDefault), "buffer");
+            beads_[i] = (size_t)beads;
+        }
+    }
+    void finish(hipStream_t st, int e)
+    {
+        check(hipEventRecord(ev_[e], st), "event");
+        check(hipEventSynchronize(ev_[e]), "event");
+    }
+    int flags() const
+    {
+        long long f;
+        std::memcpy(&f, head_, sizeof f);
+        return (int)f;
+    }
+};
+
+}  // namespace smdev
