@@ -84,9 +84,6 @@ struct Params {
     // the two-body tables' (a, b) and (b, a) rows differ somewhere: the pair kernels then
     // take each pair's row from the particle the reference's traversal makes first
     int asym;
-    // one system in a grid of fewer than 64 cell layers along z (a flat bilayer): how the pair
-    // kernels deal their chunks over the XCDs
-    int flat;
 };
 
 // Counter-RNG stream tags (word 3 of the Philox counter).
@@ -178,7 +175,7 @@ enum : int { KICK_STEP = 0, KICK_INIT = 1, KICK_NONE = 2 };
 // bonded + Langevin + second half kick of `step`, then Verlet::first, keys and digit
 // histograms of step + 1 (positions written to beads_out; the device step becomes step + 1)
 void launch_kick_first(hipStream_t st, const Params &P, const Bead *beads, Bead *beads_out, const int2 *chain,
-                       const double4 *cconst, const GenTables &gen, const float4 *fpair, float4 *vel,
+                       const double4 *cconst, const GenTables &gen, const float4 *fpair, float4 *vel, float4 *acc,
                        const DevRep *reps, DevGlobal *glob, long long step, uint32_t *key, uint32_t *idx,
                        uint32_t *ghist, int passes, const MoveBook &book,
                        const WinBook &wb = WinBook{nullptr, nullptr, nullptr, nullptr});
