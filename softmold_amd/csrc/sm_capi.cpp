@@ -614,7 +614,7 @@ struct sm_ctx {
         hist_pending = true;
         const int passes = sort_passes(sort_bits);
         timed(K_KICK_FIRST, [&] {
-            launch_kick_first(st, P, beads, beads_alt, chainPerBead, cconstD, gen(), fpair, vel, acc, reps, glob, s,
+            launch_kick_first(st, P, beads, beads_alt, chainPerBead, cconstD, gen(), fpair, vel, reps, glob, s,
                               key_out(), idx_out(), gh, passes, move_book(), win_keys());
         });
         std::swap(beads, beads_alt);

@@ -425,7 +425,10 @@ __global__ __launch_bounds__(kBlock) void k_bonded_kick(int n, const Bead *__res
 // the cell keys of step + 1, in one pass over the beads: the same arithmetic as
 // k_bonded_kick followed by k_first.  The drifted positions go to beads_out, since other
 // beads' bonded forces still read this step's positions; the step counter is taken as an
-// argument (no thread reads the device counter, which thread 0 advances to step + 1).
+// argument (no thread reads the device counter, which thread 0 advances to step + 1).  The
+// acceleration goes into both kicks from its registers and is not stored: a run ends in
+// k_bonded_kick, which stores it for the next Verlet::first (3M beads: 81 -> 77 us of HBM
+// traffic, 128 instead of 144 bytes a bead).
 // ONE: a single-replica context, whose replica constants are read from reps[0] without
 // waiting for the bead's replica index
 // WIN: keys for a window sort (wb)
@@ -435,7 +438,7 @@ __global__ __launch_bounds__(kBlock) void k_kick_first(int n, const Bead *__rest
                                                        const int2 *__restrict__ chain,
                                                        const double4 *__restrict__ cconst, GenTables gen,
                                                        const float4 *__restrict__ fpair, float4 *__restrict__ vel,
-                                                       float4 *__restrict__ acc, const DevRep *__restrict__ reps,
+                                                       const DevRep *__restrict__ reps,
                                                        DevGlobal *__restrict__ glob, float halfdt, double dt,
                                                        long long step, uint32_t *__restrict__ key,
                                                        uint32_t *__restrict__ idx, uint32_t *__restrict__ ghist,
@@ -460,7 +463,6 @@ __global__ __launch_bounds__(kBlock) void k_kick_first(int n, const Bead *__rest
         const double3 fc = bonded_force(i, n, b, beads, chain, cconst, gen, R.L[0], R.L[1], R.L[2]);
         float4 v = vel[i];
         const float4 a = total_accel(i, R, fc, fpair[i], v, step, TAG_LANGEVIN);
-        acc[i] = a;
         if (b.type != 0) {
             half_kick(v, a, halfdt);   // Verlet::second of this step
             half_kick(v, a, halfdt);   // Verlet::first of the next
@@ -920,22 +922,22 @@ void launch_bonded_kick(hipStream_t st, const Params &P, const Bead *beads, cons
 }
 
 void launch_kick_first(hipStream_t st, const Params &P, const Bead *beads, Bead *beads_out, const int2 *chain,
-                       const double4 *cconst, const GenTables &gen, const float4 *fpair, float4 *vel, float4 *acc,
+                       const double4 *cconst, const GenTables &gen, const float4 *fpair, float4 *vel,
                        const DevRep *reps, DevGlobal *glob, long long step, uint32_t *key, uint32_t *idx,
                        uint32_t *ghist, int passes, const MoveBook &book, const WinBook &wb)
 {
     const float halfdt = (float)(P.dt * 0.5);
     if (P.nrep == 1 && wb.desc)
         hipLaunchKernelGGL((k_kick_first<true, true>), dim3(blocks(P.n)), dim3(kBlock), 0, st, P.n, beads, beads_out,
-                           chain, cconst, gen, fpair, vel, acc, reps, glob, halfdt, P.dt, step, key, idx, ghist,
+                           chain, cconst, gen, fpair, vel, reps, glob, halfdt, P.dt, step, key, idx, ghist,
                            passes, book, wb);
     else if (P.nrep == 1)
         hipLaunchKernelGGL((k_kick_first<true, false>), dim3(blocks(P.n)), dim3(kBlock), 0, st, P.n, beads,
-                           beads_out, chain, cconst, gen, fpair, vel, acc, reps, glob, halfdt, P.dt, step, key, idx,
+                           beads_out, chain, cconst, gen, fpair, vel, reps, glob, halfdt, P.dt, step, key, idx,
                            ghist, passes, book, wb);
     else
         hipLaunchKernelGGL((k_kick_first<false, false>), dim3(blocks(P.n)), dim3(kBlock), 0, st, P.n, beads,
-                           beads_out, chain, cconst, gen, fpair, vel, acc, reps, glob, halfdt, P.dt, step, key, idx,
+                           beads_out, chain, cconst, gen, fpair, vel, reps, glob, halfdt, P.dt, step, key, idx,
                            ghist, passes, book, wb);
 }
 
