@@ -811,6 +811,7 @@ sm_ctx *create(const sm_system *s, int nrep)
         c->P.nT = s[0].n_types;
         c->P.cutoff = s[0].cutoff;
         c->P.dt = s[0].dt;
+        c->P.flat = nrep == 1 && s[0].box[2] / s[0].cutoff < 64.0 ? 1 : 0;
         HIPCHK(hipStreamCreate(&c->st));
         // the device's fixed scratch for the entry points that allocate nothing, looked up
         // once per device while it is current
@@ -1042,8 +1043,10 @@ sm_ctx *create(const sm_system *s, int nrep)
         }
         // sorted slots per wave in the pair kernel: short chunks keep small systems filling
         // the chip, longer ones cut the per-cell overhead of large ones (measured on the
-        // 15k, 240k and 3M-bead systems; every chunk gives the same forces)
-        c->chunk = n >= 50000 ? 8 : 2;
+        // 15k, 240k and 3M-bead systems; every chunk gives the same forces); from half a
+        // million beads on 16 slots (3M vesicle 995 -> 950 us, 3M bilayer 1028 -> 1000, the
+        // 64-vesicle sweep 848 -> 813; at 360k beads even, at 240k 96.6 -> 103.4)
+        c->chunk = n >= 500000 ? 16 : (n >= 50000 ? 8 : 2);
         c->ensure_capacity(0);
         HIPCHK(hipStreamSynchronize(st));
     } catch (...) {

@@ -84,6 +84,9 @@ struct Params {
     // the two-body tables' (a, b) and (b, a) rows differ somewhere: the pair kernels then
     // take each pair's row from the particle the reference's traversal makes first
     int asym;
+    // one system in a grid of fewer than 64 cell layers along z (a flat bilayer): how the pair
+    // kernels deal their chunks over the XCDs
+    int flat;
 };
 
 // Counter-RNG stream tags (word 3 of the Philox counter).

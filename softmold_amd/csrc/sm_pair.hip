@@ -86,23 +86,19 @@ __device__ inline void wave_lds_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Workgroups are dispatched round-robin over the 8 XCDs.  G == 0: each XCD gets one
-// contiguous range of the sorted particles (shared stencil cells stay in one L2); G > 0:
-// the XCDs take turns at groups of G consecutive chunks (the last partial round of groups
-// in order), which balances systems whose work is uneven along the sort order -- the
-// half-shell energy gathers over a flat bilayer ran 19 % faster, while the force over a
-// vesicle ran 5 % slower.
-template <int G>
-__device__ inline int xcd_block(int b, int nblocks)
+// Workgroups are dispatched round-robin over the 8 XCDs.  turn == 0: each XCD gets one
+// contiguous range of the sorted particles (shared stencil cells stay in one L2); turn > 0:
+// the XCDs take turns at groups of 2^turn consecutive chunks (the last partial round of
+// groups in order), which balances systems whose work is uneven along the sort order.
+__device__ inline int xcd_block(int b, int nblocks, int turn)
 {
-    if (G == 0) {
-        const int x = b & 7, q = nblocks >> 3, r = nblocks & 7;
-        return x * q + min(x, r) + (b >> 3);
-    }
-    const int full = (nblocks / (8 * G)) * (8 * G);
-    if (b >= full) return b;
     const int x = b & 7, k = b >> 3;
-    return ((k / (G > 0 ? G : 1)) * 8 + x) * G + (k % (G > 0 ? G : 1));
+    if (turn == 0) {
+        const int q = nblocks >> 3, r = nblocks & 7;
+        return x * q + min(x, r) + k;
+    }
+    if (b >= ((nblocks >> (3 + turn)) << (3 + turn))) return b;
+    return ((((k >> turn) << 3) + x) << turn) + (k & ((1 << turn) - 1));
 }
 
 // r^2 rounded as the reference computes it, (x*x + y*y) + z*z with every product and sum
@@ -350,7 +346,7 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
     int n, int nT, int chunk, int nblocks, double cut2, float cut2pre, const Bead *__restrict__ sb,
     const uint32_t *__restrict__ skey, const uint32_t *__restrict__ sidx, const int *__restrict__ cstart,
     const int *__restrict__ cend, const DevRep *__restrict__ reps, const float *__restrict__ tab,
-    const double *__restrict__ uconst, Out out)
+    const double *__restrict__ uconst, int turn, Out out)
 {
     // the one-phase force of a box-move step with the FP64 U(old) - U(scaled) of each pair
     // the home particle owns, in the same traversal (the box move's dU at the positions the
@@ -398,7 +394,7 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
     const int lane = threadIdx.x & (kWave - 1);
     // wave index, wave-uniform (the compiler then keeps the chunk's cell setup scalar)
     const int wave = kWaves == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
-    const long long a0 = ((long long)xcd_block<kE ? 64 : 0>(blockIdx.x, nblocks) * kWaves + wave) * chunk;
+    const long long a0 = ((long long)xcd_block(blockIdx.x, nblocks, turn) * kWaves + wave) * chunk;
     const int a = (int)min(a0, (long long)n);
     const int aend = min(a + chunk, n);
     // the first window's keys (this slot's and the one before), loaded before the constant
@@ -865,8 +861,16 @@ void launch_cells(hipStream_t st, const Params &P, int chunk, const Bead *sbeads
     // the two-phase kernel's FP32 screening radius (the culled modes take theirs per
     // candidate type from the constant tables, in the kernel)
     const float cut2pre = (float)(cut2 + slack);
+    // The sort order runs along z slowest, so an XCD's contiguous eighth of it is a slab of
+    // layers.  The force over one flat system (fewer than 64 layers) takes turns in groups
+    // of 128 chunks: its slabs hold the membrane's surface or its middle, and the uneven
+    // XCDs cost 5-16 % (3M bilayer 1072 -> 1000 us with 16 slots a chunk, 300k bilayer 128 ->
+    // 119); over a vesicle the ranges are even and turns cost 1-2 % (240k: 96.6 -> 98.0 us).
+    // The half-shell energy gathers gain on both in groups of 64.
+    const bool energy = MODE == M_U || MODE == M_DU;
+    const int turn = energy ? 6 : (P.flat ? 7 : 0);
     hipLaunchKernelGGL((k_cells<MODE, ASYM, ONE>), dim3(nb), dim3(kWaves * kWave), 0, st, P.n, P.nT, chunk, nb, cut2, cut2pre,
-                       sbeads, skey, sidx, cstart, cend, reps, fconst, uconst, out);
+                       sbeads, skey, sidx, cstart, cend, reps, fconst, uconst, turn, out);
 }
 
 }  // namespace
