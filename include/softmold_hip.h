@@ -181,10 +181,12 @@ int sm_potential_delta(sm_ctx *ctx, const double *scale, double *du_pair, double
  * "graph" = 1 to replay sm_run's aligned 8-step blocks as one captured hipGraph;
  * "sort_mode" = 1 to re-sort the cell keys incrementally -- the beads whose cell changed
  * are sorted and merged into the previous order (the default from a million beads up) --
- * 0 to sort every key each build, or 2 (single-replica contexts of at most 524288 beads,
- * their default) to sort every key within a window of cells around the previous build's
- * occupied cells: two 9-bit passes when every key lies in it, else the cell indices' 8-bit
- * passes, decided on the device.  All give the same order, so none changes a result.
+ * 0 to order every bead by key each build, or 2 (single-replica contexts of at most 524288
+ * beads, their default) to do so within a window of cells around the previous build's
+ * occupied cells: counted per cell when every key lies in it, else sorted by the cell
+ * indices' 8-bit passes, decided on the device.  0 and 2 count per cell without a window
+ * where the whole cell table holds at most 2^18 cells and there are at most 524288 beads.
+ * All give the same order, so none changes a result.
  * "mc_fused" = 1 (default) to take a box-move step's pair dU in the traversal of
  * that step's pair force, 0 in a gather of its own after the kick (sm_potential_delta
  * follows the same knob); the two sum the same FP64 terms in different orders.

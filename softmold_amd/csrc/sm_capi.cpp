@@ -166,14 +166,30 @@ struct sm_ctx {
     int *mcount = nullptr;
     int kcur = 0, scur = 0;
     bool order_valid = false;
-    // Window sort (sort_mode 2, when win_ok: a single replica of at most 256 sort tiles; it
-    // runs while the keys have 17 to 24 bits, the every-key sort otherwise): wdesc + 8p is
-    // the window of the sort with scratch parity p, which the previous sort's reorder
-    // derived on the device; (k2, v2) is the fallback's third buffer pair and then holds the
-    // sorted cell indices; win_last: the last sort was a window sort.
-    bool win_ok = false, win_last = false;
-    uint32_t *k2 = nullptr, *v2 = nullptr, *wdesc = nullptr;
+    // Counting builds (sm_internal.hpp).  Window: sort_mode 2, when win_ok (a single replica of
+    // at most 256 sort tiles), while the keys have 17 to 24 bits; wdesc + 8p is the window of
+    // the build with scratch parity p, which the previous build's reorder derived on the device.
+    // Dense: otherwise, sort_mode 0 or 2 with at most kCountBeads beads, while the cell table
+    // holds at most kWinCells cells.  counts and start: the cells' beads and first slots; k2
+    // then holds the sorted cell indices and v0 the bead indices ((k2, v2) is also the window
+    // fallback's third buffer pair).  cnt_last: the last build was a counting build, win_last:
+    // by a window.
+    bool win_ok = false, win_last = false, cnt_last = false;
+    uint32_t *k2 = nullptr, *v2 = nullptr, *wdesc = nullptr, *counts = nullptr, *start = nullptr;
     bool win_now() const { return sort_mode == 2 && win_ok && sort_bits >= 17 && sort_bits <= 24; }
+    bool dense_now() const
+    {
+        return !win_now() && sort_mode != 1 && counts && capacity <= kWinCells && n <= kCountBeads;
+    }
+    bool count_now() const { return dense_now() || win_now(); }
+    void alloc_counts()
+    {
+        if (counts) return;
+        counts = dalloc<uint32_t>(kWinCells);
+        start = dalloc<uint32_t>(kStartWords);
+        if (!k2) k2 = dalloc<uint32_t>(n);
+        HIPCHK(hipMemsetAsync(counts, 0, sizeof(uint32_t) * kWinCells, st));
+    }
     int *cstart = nullptr, *cend = nullptr;
     long long capacity = 0;   // cells in the dense table, all replicas
     int sort_bits = 0;
@@ -230,22 +246,24 @@ struct sm_ctx {
     double prof_ms[K_NCLASS] = {};
     long long prof_cnt[K_NCLASS] = {};
 
-    const uint32_t *skey() const { return sort_mode == 1 ? sk[scur] : (win_last ? k2 : (sorted_sel ? k1 : k0)); }
-    const uint32_t *sidx() const { return sort_mode == 1 ? sv[scur] : (win_last ? v0 : (sorted_sel ? v1 : v0)); }
+    const uint32_t *skey() const { return sort_mode == 1 ? sk[scur] : (cnt_last ? k2 : (sorted_sel ? k1 : k0)); }
+    const uint32_t *sidx() const { return sort_mode == 1 ? sv[scur] : (cnt_last ? v0 : (sorted_sel ? v1 : v0)); }
     // the key kernel's outputs and bookkeeping for the next sort
     uint32_t *key_out() const { return sort_mode == 1 ? kidx[kcur] : k0; }
-    // the window sort's first pass takes the bead indices from the keys' positions
-    uint32_t *idx_out() const { return sort_mode == 1 || win_now() ? nullptr : v0; }
-    WinBook win_keys() const
+    // bead indices for the every-key sort, arrival numbers for a counting build
+    uint32_t *idx_out() const { return sort_mode == 1 ? nullptr : v0; }
+    WinBook win_keys(int p) const
     {
-        if (!win_now()) return WinBook{nullptr, nullptr, nullptr, nullptr};
-        return win_book(hist[sort_parity], n, wdesc + 8 * sort_parity);
+        if (!count_now()) return WinBook{};
+        const bool win = win_now();
+        return win_book(hist[p], n, win ? wdesc + 8 * p : nullptr, counts, win ? 0u : (uint32_t)capacity);
     }
     // a key kernel ran without its sort: zero what it added to the sort's scratch
     void restart_hist(uint32_t *gh)
     {
         launch_fill_u32(st, gh, sort_hist_words(), 0u);
-        if (win_now()) launch_fill_u32(st, win_scratch(gh, n), kWinKeyWords, 0u);
+        launch_fill_u32(st, win_scratch(gh, n), kWinKeyWords, 0u);
+        if (counts) launch_fill_u32(st, counts, kWinCells, 0u);
     }
     MoveBook move_book() const
     {
@@ -264,7 +282,7 @@ struct sm_ctx {
         for (auto e : pool) (void)hipEventDestroy(e);
         dfree(beads); dfree(sbeads); dfree(beads_alt); dfree(vel); dfree(acc); dfree(fpair); dfree(fscratch);
         dfree(k0); dfree(v0); dfree(k1); dfree(v1); dfree(hist[0]); dfree(hist[1]); dfree(cstart); dfree(cend);
-        dfree(k2); dfree(v2); dfree(wdesc);
+        dfree(k2); dfree(v2); dfree(wdesc); dfree(counts); dfree(start);
         for (int p = 0; p < 2; p++) { dfree(kidx[p]); dfree(sk[p]); dfree(sv[p]); }
         dfree(mbefore); dfree(cnt_b); dfree(cnt_i); dfree(cnt_s); dfree(mflags); dfree(mcount);
         dfree(reps); dfree(glob); dfree(fconstF); dfree(uconstD); dfree(fconstD); dfree(chainPerBead); dfree(chainList);
@@ -434,6 +452,7 @@ struct sm_ctx {
         int bits = 1;
         while ((1ll << bits) < base) bits++;
         sort_bits = bits;
+        if (win_ok || (capacity <= kWinCells && n <= kCountBeads)) alloc_counts();
     }
 
     // keys (optionally after Verlet::first) with the next sort's digit histograms, sort,
@@ -448,7 +467,7 @@ struct sm_ctx {
         timed(K_FIRST, [&] {
             if (for_sort)
                 launch_first(st, P, beads, vel, acc, reps, glob, key_out(), idx_out(), integrate, step_set, gh, passes,
-                             move_book(), win_keys());
+                             move_book(), win_keys(sort_parity));
             else   // keys only (no sort follows): into the mover buffer, which no sort state holds
                 launch_first(st, P, beads, vel, acc, reps, glob, k0, nullptr, integrate, step_set, nullptr, passes,
                              MoveBook{nullptr, nullptr});
@@ -457,7 +476,8 @@ struct sm_ctx {
     void sort_and_reorder()
     {
         const int p = sort_parity;
-        const bool win = win_now();
+        const bool count = count_now();
+        const WinBook wb = win_keys(p);
         if (sort_mode == 1) {
             timed(K_SORT, [&] {
                 SortBuffers sb{k0, v0, k1, v1, {hist[0], hist[1]}, &glob->flags, n, 0};
@@ -468,10 +488,10 @@ struct sm_ctx {
             scur = 1 - scur;
             kcur = 1 - kcur;
             order_valid = true;
-        } else if (win) {
+        } else if (count) {
             timed(K_SORT, [&] {
                 SortBuffers sb{k0, v0, k1, v1, {hist[0], hist[1]}, &glob->flags, n, 0};
-                sort_window(st, sb, k2, v2, p, wdesc + 8 * p, reps);
+                count_build(st, sb, k2, v2, p, wb, start, reps);
             });
             order_valid = false;
         } else {
@@ -481,11 +501,12 @@ struct sm_ctx {
             });
             order_valid = false;
         }
-        win_last = win;
+        win_last = count && wb.desc;
+        cnt_last = count;
         timed(K_REORDER, [&] {
-            if (win)
-                launch_reorder_win(st, n, k0, v0, beads, sbeads, cstart, cend, hist[1 - p], hist_words,
-                                   win_book(hist[p], n, wdesc + 8 * p), k2, wdesc + 8 * (1 - p), reps);
+            if (count)
+                launch_reorder_count(st, n, k0, v0, k1, v1, k2, start, beads, sbeads, cstart, cend, hist[1 - p],
+                                     hist_words, wb, wdesc ? wdesc + 8 * (1 - p) : nullptr, reps);
             else
                 launch_reorder(st, n, skey(), sidx(), beads, sbeads, cstart, cend, hist[1 - p], hist_words);
         });
@@ -615,7 +636,7 @@ struct sm_ctx {
         const int passes = sort_passes(sort_bits);
         timed(K_KICK_FIRST, [&] {
             launch_kick_first(st, P, beads, beads_alt, chainPerBead, cconstD, gen(), fpair, vel, reps, glob, s,
-                              key_out(), idx_out(), gh, passes, move_book(), win_keys());
+                              key_out(), idx_out(), gh, passes, move_book(), win_keys(sort_parity));
         });
         std::swap(beads, beads_alt);
     }
@@ -984,7 +1005,7 @@ sm_ctx *create(const sm_system *s, int nrep)
         c->cnt_s = dalloc<uint32_t>(move_tiles(n));
         c->mflags = dalloc<unsigned long long>(((size_t)n + 63) / 64);
         c->mcount = dalloc<int>(1);
-        c->hist_words = sort_scratch_words(n, 4) + (c->win_ok ? sortw_words(n) : 0);
+        c->hist_words = sort_scratch_words(n, 4) + sortw_words(n, c->win_ok);
         for (int p = 0; p < 2; p++) {
             c->hist[p] = dalloc<uint32_t>(c->hist_words);
             HIPCHK(hipMemsetAsync(c->hist[p], 0, sizeof(uint32_t) * c->hist_words, c->st));
@@ -1557,7 +1578,7 @@ int sm_tune_get(sm_ctx *c, const char *knob, int32_t *value)
                 const int lp = 1 - c->sort_parity;
                 uint32_t wx = 0, flag = 0;
                 HIPCHK(hipMemcpyAsync(&wx, c->wdesc + 8 * lp + 3, sizeof(uint32_t), hipMemcpyDeviceToHost, c->st));
-                HIPCHK(hipMemcpyAsync(&flag, win_book(c->hist[lp], c->n, nullptr).flag, sizeof(uint32_t),
+                HIPCHK(hipMemcpyAsync(&flag, win_book(c->hist[lp], c->n, nullptr, nullptr, 0u).flag, sizeof(uint32_t),
                                       hipMemcpyDeviceToHost, c->st));
                 HIPCHK(hipStreamSynchronize(c->st));
                 *value = (wx != 0 && flag == 0) ? 1 : 0;

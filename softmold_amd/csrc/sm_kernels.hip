@@ -139,22 +139,22 @@ __global__ __launch_bounds__(kBlock) void k_first(int n, Bead *__restrict__ bead
     __shared__ uint32_t hs[1024];
     uint32_t (*h)[256] = reinterpret_cast<uint32_t (*)[256]>(hs);
     const int i = blockIdx.x * kBlock + threadIdx.x;
-    const bool win = wb.desc != nullptr;
+    const bool win = wb.counts != nullptr;
     WinDesc w{};
-    if (win) w = load_win(wb.desc);
+    if (win && wb.desc) w = load_win(wb.desc);
     if (i == 0 && step_set >= -1) glob->step = step_set >= 0 ? step_set : glob->step + 1;   // no other reader here
     if (ghist) {
         if (win)
-            for (int j = 0; j < 4; j++) hs[threadIdx.x + 256 * j] = 0u;
+            hs[threadIdx.x] = 0u;
         else
             for (int p = 0; p < passes; p++) h[p][threadIdx.x] = 0u;
         __syncthreads();
     }
-    uint32_t k = 0u;
+    uint32_t k = 0u, rank = (uint32_t)i;
     int cx = 0, cy = 0, cz = 0;
     if (i < n) k = first_one(i, beads, vel, acc, reps, glob, halfdt, dt, integrate, cx, cy, cz);
     if (ghist && win) {
-        k = win_key_end(wb, w, hs, k, cx, cy, cz, i < n);
+        k = win_key_end(wb, w, hs, k, cx, cy, cz, i < n, rank);
     } else if (ghist) {
         // the sort's digit histograms while the key is in a register (all lanes: ballots)
         const bool counted = note_move(book, i, k, i < n);
@@ -165,7 +165,7 @@ __global__ __launch_bounds__(kBlock) void k_first(int n, Bead *__restrict__ bead
     }
     if (i < n) {
         key[i] = k;
-        if (idx) idx[i] = (uint32_t)i;
+        if (idx) idx[i] = rank;
     }
 }
 
@@ -189,26 +189,35 @@ __global__ __launch_bounds__(kBlock) void k_reorder(int n, const uint32_t *__res
     if (s == n - 1 || knext != k) cend[k] = s + 1;
 }
 
-// k_reorder after a window sort: the sorted keys are window keys (the window path) or cell
-// indices (the fallback); either way equal keys are equal cells.  The cell indices go to
-// skf for the pair kernels.  Block 0 also sets the next sort's window: this sort's after
-// the window path; after the fallback, the occupied cell range the fallback measured,
-// widened by one cell on each side and clipped to the grid, or none (wx = 0) when that
-// holds more than 2^18 cells.
-__global__ __launch_bounds__(kBlock) void k_reorder_win(int n, const uint32_t *__restrict__ skey,
-                                                        const uint32_t *__restrict__ sidx,
-                                                        const Bead *__restrict__ beads, Bead *__restrict__ sbeads,
-                                                        int *__restrict__ cstart, int *__restrict__ cend,
-                                                        uint32_t *__restrict__ clear, size_t clear_words, WinBook wb,
-                                                        uint32_t *__restrict__ skf, uint32_t *__restrict__ desc_next,
-                                                        const DevRep *__restrict__ reps)
+// The reorder of a counting build (see launch_reorder_count).  On the window or dense path a
+// bead's slot is its run's first slot plus the run's beads of lower index: a run is a cell's
+// dozen beads, read by every one of its threads from the caches.  Block 0 also sets the next
+// build's window: this build's after the window path; after the fallback, the occupied cell
+// range the fallback measured, widened by one cell on each side and clipped to the grid, or
+// none (wx = 0) when that holds more than kWinCells cells.
+__global__ __launch_bounds__(kBlock) void k_reorder_count(int n, const uint32_t *__restrict__ k0,
+                                                          uint32_t *__restrict__ v0, const uint32_t *__restrict__ k1,
+                                                          const uint32_t *__restrict__ v1, uint32_t *__restrict__ k2,
+                                                          const uint32_t *__restrict__ start,
+                                                          const Bead *__restrict__ beads, Bead *__restrict__ sbeads,
+                                                          int *__restrict__ cstart, int *__restrict__ cend,
+                                                          uint32_t *__restrict__ clear, size_t clear_words, WinBook wb,
+                                                          uint32_t *__restrict__ desc_next,
+                                                          const DevRep *__restrict__ reps)
 {
-    const int nx = reps[0].nc[0], ny = reps[0].nc[1], nz = reps[0].nc[2];
     const int s = blockIdx.x * kBlock + threadIdx.x;
     for (size_t w = (size_t)s; w < clear_words; w += (size_t)gridDim.x * kBlock) clear[w] = 0u;
-    const WinDesc w = load_win(wb.desc);
-    const bool fallback = w.wx == 0u || *wb.flag != 0u;
-    if (blockIdx.x == 0 && threadIdx.x < kWave) {
+    const bool dense = wb.cells != 0u;
+    WinDesc w{};
+    bool fallback = false;
+    int nx = 1, ny = 1;
+    if (!dense) {
+        nx = reps[0].nc[0];
+        ny = reps[0].nc[1];
+        w = load_win(wb.desc);
+        fallback = w.wx == 0u || *wb.flag != 0u;
+    }
+    if (!dense && blockIdx.x == 0 && threadIdx.x < kWave) {
         const int t = threadIdx.x;
         uint32_t v = 0u;
         if (fallback && t < 6)
@@ -221,7 +230,7 @@ __global__ __launch_bounds__(kBlock) void k_reorder_win(int n, const uint32_t *_
             if (fallback) {
                 for (int j = 0; j < 6; j++) d[j] = 0u;
                 if (f[0] != 0u) {
-                    const int ncell[3] = {nx, ny, nz};
+                    const int ncell[3] = {nx, ny, reps[0].nc[2]};
                     unsigned long long cells = 1ull;
                     for (int a = 0; a < 3; a++) {
                         const int lo = max((int)(kBoxEnc - f[3 + a]) - 1, 0);
@@ -230,7 +239,7 @@ __global__ __launch_bounds__(kBlock) void k_reorder_win(int n, const uint32_t *_
                         d[3 + a] = (uint32_t)(hi - lo + 1);
                         cells *= (unsigned long long)(hi - lo + 1);
                     }
-                    if (cells > (1ull << 18))
+                    if (cells > (unsigned long long)kWinCells)
                         for (int j = 0; j < 6; j++) d[j] = 0u;
                 }
             }
@@ -238,17 +247,32 @@ __global__ __launch_bounds__(kBlock) void k_reorder_win(int n, const uint32_t *_
         }
     }
     if (s >= n) return;
-    const uint32_t k = skey[s], kprev = skey[s > 0 ? s - 1 : 0], knext = skey[s < n - 1 ? s + 1 : s];
-    sbeads[s] = beads[sidx[s]];
-    uint32_t full = k;
-    if (!fallback) {
-        const uint32_t wk = k & ~kWinTag;
+    if (fallback) {   // (k0, v0) is sorted
+        const uint32_t k = k0[s], kprev = k0[s > 0 ? s - 1 : 0], knext = k0[s < n - 1 ? s + 1 : s];
+        sbeads[s] = beads[v0[s]];
+        k2[s] = k;
+        if (s == 0 || kprev != k) cstart[k] = s;
+        if (s == n - 1 || knext != k) cend[k] = s + 1;
+        return;
+    }
+    const uint32_t wk = min(k1[s], (uint32_t)kWinCells - 1u), i = min(v1[s], (uint32_t)n - 1u);
+    const Bead b = beads[i];
+    const uint32_t c0 = min(start[wk], (uint32_t)n - 1u), c1 = min(start[wk + 1], (uint32_t)n);
+    uint32_t pos = c0;
+    for (uint32_t j = c0; j < c1; j++) pos += v1[j] < i ? 1u : 0u;
+    pos = min(pos, (uint32_t)n - 1u);   // in bounds also for counts that are not this build's
+    uint32_t full = wk;
+    if (!dense) {
         const uint32_t q = wk / w.wx, x = wk - q * w.wx, z = q / w.wy, y = q - z * w.wy;
         full = ((z + w.z0) * (uint32_t)ny + (y + w.y0)) * (uint32_t)nx + (x + w.x0);
     }
-    skf[s] = full;
-    if (s == 0 || kprev != k) cstart[full] = s;
-    if (s == n - 1 || knext != k) cend[full] = s + 1;
+    sbeads[pos] = b;
+    v0[pos] = i;
+    k2[pos] = full;
+    if (pos == c0) {
+        cstart[full] = (int)c0;
+        cend[full] = (int)c1;
+    }
 }
 
 // ---------------------------------------------------------------------------------------
@@ -431,7 +455,7 @@ __global__ __launch_bounds__(kBlock) void k_bonded_kick(int n, const Bead *__res
 // traffic, 128 instead of 144 bytes a bead).
 // ONE: a single-replica context, whose replica constants are read from reps[0] without
 // waiting for the bead's replica index
-// WIN: keys for a window sort (wb)
+// WIN: keys and arrival numbers for a counting build (wb)
 template <bool ONE, bool WIN>
 __global__ __launch_bounds__(kBlock) void k_kick_first(int n, const Bead *__restrict__ beads,
                                                        Bead *__restrict__ beads_out,
@@ -444,18 +468,18 @@ __global__ __launch_bounds__(kBlock) void k_kick_first(int n, const Bead *__rest
                                                        uint32_t *__restrict__ idx, uint32_t *__restrict__ ghist,
                                                        int passes, MoveBook book, WinBook wb)
 {
-    __shared__ uint32_t hs[1024];
+    __shared__ uint32_t hs[WIN ? kBlock : 1024];
     uint32_t (*h)[256] = reinterpret_cast<uint32_t (*)[256]>(hs);
     const int i = blockIdx.x * kBlock + threadIdx.x;
     WinDesc w{};
-    if (WIN) w = load_win(wb.desc);
+    if (WIN && wb.desc) w = load_win(wb.desc);
     if (i == 0) glob->step = step + 1;
     if (WIN)
-        for (int j = 0; j < 4; j++) hs[threadIdx.x + 256 * j] = 0u;
+        hs[threadIdx.x] = 0u;
     else
         for (int p = 0; p < passes; p++) h[p][threadIdx.x] = 0u;
     __syncthreads();
-    uint32_t k = 0u;
+    uint32_t k = 0u, rank = (uint32_t)i;
     int cx = 0, cy = 0, cz = 0;
     if (i < n) {
         Bead b = beads[i];
@@ -473,7 +497,7 @@ __global__ __launch_bounds__(kBlock) void k_kick_first(int n, const Bead *__rest
         k = bead_key(b, R, glob, cx, cy, cz);
     }
     if (WIN) {
-        k = win_key_end(wb, w, hs, k, cx, cy, cz, i < n);
+        k = win_key_end(wb, w, hs, k, cx, cy, cz, i < n, rank);
     } else {
         const bool counted = note_move(book, i, k, i < n);
         hist_add(h, k, counted, passes);
@@ -483,7 +507,7 @@ __global__ __launch_bounds__(kBlock) void k_kick_first(int n, const Bead *__rest
     }
     if (i < n) {
         key[i] = k;
-        if (idx) idx[i] = (uint32_t)i;
+        if (idx) idx[i] = rank;
     }
 }
 
@@ -905,12 +929,13 @@ void launch_reorder(hipStream_t st, int n, const uint32_t *skey, const uint32_t 
                        clear, clear_words);
 }
 
-void launch_reorder_win(hipStream_t st, int n, const uint32_t *skey, const uint32_t *sidx, const Bead *beads,
-                        Bead *sbeads, int *cstart, int *cend, uint32_t *clear, size_t clear_words,
-                        const WinBook &wb, uint32_t *skey_full, uint32_t *desc_next, const DevRep *reps)
+void launch_reorder_count(hipStream_t st, int n, const uint32_t *k0, uint32_t *v0, const uint32_t *k1,
+                          const uint32_t *v1, uint32_t *k2, const uint32_t *start, const Bead *beads, Bead *sbeads,
+                          int *cstart, int *cend, uint32_t *clear, size_t clear_words, const WinBook &wb,
+                          uint32_t *desc_next, const DevRep *reps)
 {
-    hipLaunchKernelGGL(k_reorder_win, dim3(blocks(n)), dim3(kBlock), 0, st, n, skey, sidx, beads, sbeads, cstart,
-                       cend, clear, clear_words, wb, skey_full, desc_next, reps);
+    hipLaunchKernelGGL(k_reorder_count, dim3(blocks(n)), dim3(kBlock), 0, st, n, k0, v0, k1, v1, k2, start, beads,
+                       sbeads, cstart, cend, clear, clear_words, wb, desc_next, reps);
 }
 
 void launch_bonded_kick(hipStream_t st, const Params &P, const Bead *beads, const int2 *chain,
@@ -927,7 +952,11 @@ void launch_kick_first(hipStream_t st, const Params &P, const Bead *beads, Bead 
                        uint32_t *ghist, int passes, const MoveBook &book, const WinBook &wb)
 {
     const float halfdt = (float)(P.dt * 0.5);
-    if (P.nrep == 1 && wb.desc)
+    if (P.nrep > 1 && wb.counts)
+        hipLaunchKernelGGL((k_kick_first<false, true>), dim3(blocks(P.n)), dim3(kBlock), 0, st, P.n, beads, beads_out,
+                           chain, cconst, gen, fpair, vel, reps, glob, halfdt, P.dt, step, key, idx, ghist, passes,
+                           book, wb);
+    else if (wb.counts)
         hipLaunchKernelGGL((k_kick_first<true, true>), dim3(blocks(P.n)), dim3(kBlock), 0, st, P.n, beads, beads_out,
                            chain, cconst, gen, fpair, vel, reps, glob, halfdt, P.dt, step, key, idx, ghist,
                            passes, book, wb);

@@ -28,14 +28,16 @@
 // mover by a search among the previous slots (inside its cell's previous run when that
 // cell was occupied).
 //
-// Window sort (sort_mode 2, one replica): the key kernel stores each key whose cell lies in
-// the sort's window -- the occupied cell range of the last build that had to measure it,
-// widened by one cell, at most 2^18 cells -- as its index in the window's (z, y, x) order,
-// which orders keys as the cell index does, and counts its two window digits.  Two launches
-// then sort 9 + 9 (or 9 + 8) bits.  If a key fell outside the window (or there is none),
-// the same launches sort the cell indices in three 8-bit passes and measure the occupied
-// range for the next window.  A vesicle of 240k beads in a 200^3-cell grid has 23-bit keys
-// but a 17-bit window: 31.8 against 36.6 us per sort.
+// Counting builds: where the cells of a build fit 2^18 counters -- the whole table (dense), or
+// a window around the previous build's occupied cells (sort_mode 2, one replica) -- the key
+// kernel counts the beads of each cell while the keys are in registers.  k_scan_cells turns the
+// counts into first slots, k_place puts each bead into its cell's run by its arrival number,
+// and the reorder puts each run into index order, so the order is the stable sort's without a
+// sort.  A vesicle of 240k beads in a 200^3-cell grid has 23-bit keys but a 50^3-cell window:
+// 36 us of radix passes and reorder became 19 us (scan and place 10.6, reorder 8.6, and 2 us
+// more in the key kernel); 15k beads 20 -> 13 us, 1.5k beads 14 -> 12 us.
+// If a key fell outside the window (or there is none), the same launches sort the cell indices
+// in three 8-bit passes and measure the occupied range for the next window.
 #include <algorithm>
 
 #include "sm_sort_dev.hpp"
@@ -450,42 +452,21 @@ __global__ __launch_bounds__(kThreads) void k_merge(int n, const int *__restrict
 
 
 // ---------------------------------------------------------------------------------------
-// The window sort (sort_mode 2) in two launches.  The window path runs one 9-bit pass in
-// each over the window keys.  The fallback sorts the cell indices in three 8-bit passes:
-// the first launch converts any window keys back to cell indices and counts their digits
-// (when the sort had a window), then runs two passes with a grid-wide barrier before each
-// (a launch has at most kWinMaxTiles workgroups, so all of them are resident together); the
-// second launch runs the third.  Each launch reads which path to take from the device.
+// The counting builds, and the window build's fallback: three 8-bit passes over the cell
+// indices.  Its first launch converts any window keys back to cell indices and counts their
+// digits, then runs two passes with a grid-wide barrier before each (a launch has at most
+// kWinMaxTiles workgroups that stay, so all of them are resident together); the second launch
+// runs the third.  Each launch reads which path to take from the device.
 // ---------------------------------------------------------------------------------------
-constexpr int kWDig = 512;
-
 template <int kRounds>
 struct WLds {
-    // per (round, wave, digit): count, then tile-local offset; a thread owning two adjacent
-    // digits reads and writes both as one word
-    union {
-        uint16_t h[kRounds][kWavesPerBlock][kWDig];
-        uint32_t w[kRounds][kWavesPerBlock][kWDig / 2];
-    } wc;
-    uint32_t dpos[kWDig];                          // per digit: output position of the tile's first item
-    uint32_t h[3][256];                            // fallback: digit counts of a tile's cell indices
-    uint32_t bb[kWavesPerBlock][6];                // fallback: occupied cell range of each wave's keys
+    uint32_t wc[kRounds][kWavesPerBlock][256];   // per (round, wave, digit): count, then tile-local offset
+    uint32_t dpos[256];                          // per digit: output position of the tile's first item
+    uint32_t h[3][256];                          // digit counts of a tile's cell indices
+    uint32_t bb[kWavesPerBlock][6];              // occupied cell range of each wave's keys
     uint32_t scan[kWavesPerBlock];
     uint32_t tile;
 };
-
-template <int kBits>
-__device__ inline unsigned long long match_bits(uint32_t d, bool valid)
-{
-    unsigned long long peers = __ballot(valid);
-#pragma unroll
-    for (int b = 0; b < kBits; b++) {
-        const bool bit = (d >> b) & 1u;
-        const unsigned long long m = __ballot(bit);
-        peers &= bit ? m : ~m;
-    }
-    return peers;
-}
 
 // Sum of the counts of digit d over the tiles before `tile` (decoupled look-back over
 // windows of kLook tiles, bounded like the every-key sort's).
@@ -497,7 +478,7 @@ __device__ inline uint32_t look_back(const uint32_t *status, int tile, int d, in
         uint32_t v[kLook];
 #pragma unroll
         for (int w = 0; w < kLook; w++)
-            v[w] = pt - w >= 0 ? __hip_atomic_load(status + (size_t)(pt - w) * kWDig + d, __ATOMIC_RELAXED,
+            v[w] = pt - w >= 0 ? __hip_atomic_load(status + (size_t)(pt - w) * 256 + d, __ATOMIC_RELAXED,
                                                    __HIP_MEMORY_SCOPE_AGENT)
                                : kFlagIncl;
         int used = 0;
@@ -524,90 +505,24 @@ __device__ inline uint32_t look_back(const uint32_t *status, int tile, int d, in
     return prefix;
 }
 
-// Sum of the counts of digits d0 and d1 over the tiles before `tile`: the two look-backs of
-// a thread walk together, so the loads of both are in flight at once.
-__device__ inline void look_back2(const uint32_t *status, int tile, int d0, int d1, uint32_t &p0, uint32_t &p1,
-                                  int *errflag)
-{
-    p0 = 0u;
-    p1 = 0u;
-    int pt0 = tile - 1, pt1 = tile - 1, spins = 0;
-    while (pt0 >= 0 || pt1 >= 0) {
-        uint32_t v0[kLook], v1[kLook];
-#pragma unroll
-        for (int w = 0; w < kLook; w++) {
-            v0[w] = pt0 - w >= 0 ? __hip_atomic_load(status + (size_t)(pt0 - w) * kWDig + d0, __ATOMIC_RELAXED,
-                                                     __HIP_MEMORY_SCOPE_AGENT)
-                                 : kFlagIncl;
-            v1[w] = pt1 - w >= 0 ? __hip_atomic_load(status + (size_t)(pt1 - w) * kWDig + d1, __ATOMIC_RELAXED,
-                                                     __HIP_MEMORY_SCOPE_AGENT)
-                                 : kFlagIncl;
-        }
-        bool wait = false;
-        if (pt0 >= 0) {
-            int used = 0;
-            bool done = false;
-#pragma unroll
-            for (int w = 0; w < kLook; w++) {
-                if (done || used < w) continue;
-                const uint32_t f = v0[w] & ~kCountMask;
-                if (f == 0u) continue;
-                p0 += v0[w] & kCountMask;
-                used = w + 1;
-                done = f == kFlagIncl;
-            }
-            pt0 = done ? -1 : pt0 - used;
-            wait = wait || (!done && used < kLook);
-        }
-        if (pt1 >= 0) {
-            int used = 0;
-            bool done = false;
-#pragma unroll
-            for (int w = 0; w < kLook; w++) {
-                if (done || used < w) continue;
-                const uint32_t f = v1[w] & ~kCountMask;
-                if (f == 0u) continue;
-                p1 += v1[w] & kCountMask;
-                used = w + 1;
-                done = f == kFlagIncl;
-            }
-            pt1 = done ? -1 : pt1 - used;
-            wait = wait || (!done && used < kLook);
-        }
-        if (wait) {
-            if (++spins >= kSpinLimit) {
-                atomicOr(errflag, FLAG_SORT_TIMEOUT);
-                break;
-            }
-            __builtin_amdgcn_s_sleep(1);
-        }
-    }
-}
-
-// One stable pass over the kBits-bit digit at `shift` of tile `tile`, whose items take
-// digit bases from the per-thread histogram sums g (the thread's kPer digits, over every
-// copy).  kIota: the first pass, whose values are the keys' positions (bead indices), not
-// loaded from vin.
-template <int kRounds, int kBits, bool kIota = false>
-__device__ void wpass(WLds<kRounds> &L, int n, int shift, int tile, const uint32_t (&g)[(1 << kBits) / kThreads],
+// One stable pass over the 8-bit digit at `shift` of tile `tile`, whose items take digit bases
+// from the thread's histogram sum g.  iota: the first pass, whose values are the keys'
+// positions (bead indices), not loaded from vin.
+template <int kRounds>
+__device__ void wpass(WLds<kRounds> &L, int n, int shift, int tile, uint32_t g, bool iota,
                       const uint32_t *__restrict__ kin, const uint32_t *__restrict__ vin, uint32_t *__restrict__ kout,
                       uint32_t *__restrict__ vout, uint32_t *__restrict__ status, int *__restrict__ errflag)
 {
-    constexpr int kDig = 1 << kBits, kPer = kDig / kThreads;   // thread t owns digits t*kPer .. t*kPer+kPer-1
     const int t = threadIdx.x, wave = t / kWave, lane = t & (kWave - 1);
     const int base = tile * kThreads * kRounds;
-    // every round's loads in flight before the LDS work
     uint32_t kr[kRounds], vr[kRounds], dr[kRounds], rk[kRounds];
 #pragma unroll
     for (int r = 0; r < kRounds; r++) {
         const int i = min(base + r * kThreads + t, n - 1);
         kr[r] = kin[i];
-        vr[r] = kIota ? (uint32_t)i : vin[i];
+        vr[r] = iota ? (uint32_t)i : vin[i];
     }
-    uint32_t gs = 0u;
-#pragma unroll
-    for (int j = 0; j < kPer; j++) gs += g[j];
-    uint32_t x = gs;
+    uint32_t x = g;
 #pragma unroll
     for (int o = 1; o < kWave; o <<= 1) {
         const uint32_t y = __shfl_up(x, o);
@@ -617,79 +532,45 @@ __device__ void wpass(WLds<kRounds> &L, int n, int shift, int tile, const uint32
 #pragma unroll
     for (int r = 0; r < kRounds; r++)
 #pragma unroll
-        for (int w = 0; w < kWavesPerBlock; w++) {
-            if (kPer == 2)
-                L.wc.w[r][w][t] = 0u;
-            else
-                L.wc.h[r][w][t] = 0;
-        }
+        for (int w = 0; w < kWavesPerBlock; w++) L.wc[r][w][t] = 0u;
     __syncthreads();
     uint32_t wpre = 0;
     for (int w = 0; w < wave; w++) wpre += L.scan[w];
-    uint32_t dbase[kPer];
-    dbase[0] = wpre + x - gs;
-#pragma unroll
-    for (int j = 1; j < kPer; j++) dbase[j] = dbase[j - 1] + g[j - 1];
+    const uint32_t dbase = wpre + x - g;
     const unsigned long long lt = lanes_below();
 #pragma unroll
     for (int r = 0; r < kRounds; r++) {
         const bool valid = base + r * kThreads + t < n;
-        dr[r] = valid ? (kr[r] >> shift) & (uint32_t)(kDig - 1) : (uint32_t)kDig;   // kDig: no item
-        const unsigned long long peers = match_bits<kBits>(dr[r] & (uint32_t)(kDig - 1), valid);
+        dr[r] = valid ? (kr[r] >> shift) & 255u : 256u;   // 256: no item
+        const unsigned long long peers = match_digit(dr[r] & 255u, valid);
         rk[r] = (uint32_t)__popcll(peers & lt);
-        if (valid && rk[r] == 0u) L.wc.h[r][wave][dr[r]] = (uint16_t)__popcll(peers);
+        if (valid && rk[r] == 0u) L.wc[r][wave][dr[r]] = (uint32_t)__popcll(peers);
     }
     __syncthreads();
 
-    // per digit: the counts read together, tile-local offsets written, the tile's count
-    // published for later tiles
-    uint32_t mine[kPer];
-    {
-        uint32_t cnt[kRounds][kWavesPerBlock];
+    // tile-local offsets written, the tile's count published for later tiles
+    uint32_t mine = 0;
 #pragma unroll
-        for (int r = 0; r < kRounds; r++)
+    for (int r = 0; r < kRounds; r++)
 #pragma unroll
-            for (int w = 0; w < kWavesPerBlock; w++) cnt[r][w] = kPer == 2 ? L.wc.w[r][w][t] : L.wc.h[r][w][t];
-        uint32_t off0 = 0, off1 = 0;
-#pragma unroll
-        for (int r = 0; r < kRounds; r++)
-#pragma unroll
-            for (int w = 0; w < kWavesPerBlock; w++) {
-                if (kPer == 2) {
-                    L.wc.w[r][w][t] = off0 | (off1 << 16);
-                    off0 += cnt[r][w] & 0xFFFFu;
-                    off1 += cnt[r][w] >> 16;
-                } else {
-                    L.wc.h[r][w][t] = (uint16_t)off0;
-                    off0 += cnt[r][w];
-                }
-            }
-        mine[0] = off0;
-        if (kPer == 2) mine[kPer - 1] = off1;
-    }
-#pragma unroll
-    for (int j = 0; j < kPer; j++)
-        __hip_atomic_store(status + (size_t)tile * kWDig + t * kPer + j, (tile == 0 ? kFlagIncl : kFlagAgg) | mine[j],
-                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    uint32_t prefix[kPer];
-    if (kPer == 2)
-        look_back2(status, tile, t * kPer, t * kPer + kPer - 1, prefix[0], prefix[kPer - 1], errflag);
-    else
-        prefix[0] = look_back(status, tile, t, errflag);
-#pragma unroll
-    for (int j = 0; j < kPer; j++) {
-        const int d = t * kPer + j;
-        if (tile > 0)
-            __hip_atomic_store(status + (size_t)tile * kWDig + d, kFlagIncl | (prefix[j] + mine[j]),
-                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        L.dpos[d] = dbase[j] + prefix[j];
-    }
+        for (int w = 0; w < kWavesPerBlock; w++) {
+            const uint32_t c = L.wc[r][w][t];
+            L.wc[r][w][t] = mine;
+            mine += c;
+        }
+    __hip_atomic_store(status + (size_t)tile * 256 + t, (tile == 0 ? kFlagIncl : kFlagAgg) | mine, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+    const uint32_t prefix = look_back(status, tile, t, errflag);
+    if (tile > 0)
+        __hip_atomic_store(status + (size_t)tile * 256 + t, kFlagIncl | (prefix + mine), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+    L.dpos[t] = dbase + prefix;
     __syncthreads();
 
 #pragma unroll
     for (int r = 0; r < kRounds; r++) {
-        if (dr[r] < (uint32_t)kDig) {
-            uint32_t p = L.dpos[dr[r]] + L.wc.h[r][wave][dr[r]] + rk[r];
+        if (dr[r] < 256u) {
+            uint32_t p = L.dpos[dr[r]] + L.wc[r][wave][dr[r]] + rk[r];
             p = p < (uint32_t)n ? p : (uint32_t)(n - 1);   // only reachable after a timeout
             kout[p] = kr[r];
             vout[p] = vr[r];
@@ -697,29 +578,13 @@ __device__ void wpass(WLds<kRounds> &L, int n, int shift, int tile, const uint32
     }
 }
 
-// A tile id from a counter, issued from vector registers (for a uniform address the
-// compiler would aggregate the atomic over the wave and wait for its result at once) and
-// shared through LDS at the next barrier.
-__device__ inline uint32_t draw_tile(uint32_t *tilectr)
+// the sum of this thread's digit over the histogram copies
+__device__ inline uint32_t hist_sum(const uint32_t *__restrict__ ghist)
 {
-    typedef __attribute__((address_space(1))) uint32_t global_u32;
-    global_u32 *ctr = (global_u32 *)tilectr;
-    asm volatile("" : "+v"(ctr));
-    uint32_t id = 0u;
-    if (threadIdx.x == 0) id = __hip_atomic_fetch_add(ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return id;
-}
-
-template <int kPer>
-__device__ inline void hist_sums(const uint32_t *__restrict__ ghist, uint32_t (&g)[kPer])
-{
-    const int t = threadIdx.x;
+    uint32_t g = 0u;
 #pragma unroll
-    for (int j = 0; j < kPer; j++) {
-        g[j] = 0u;
-#pragma unroll
-        for (int c = 0; c < kHistCopies; c++) g[j] += ghist[(size_t)c * 1024 + t * kPer + j];
-    }
+    for (int c = 0; c < kHistCopies; c++) g += ghist[(size_t)c * 1024 + threadIdx.x];
+    return g;
 }
 
 // Every workgroup of the launch arrives at *ctr before any goes on; its stores before are
@@ -743,53 +608,110 @@ __device__ inline void grid_sync(uint32_t *ctr, uint32_t count, int *errflag)
     __threadfence();
 }
 
+// First slots of scan tile t's kCoarseCells cells from their counts, which it clears for the
+// next key kernel.  The beads before the tile are the coarse counts of the tiles before it, so
+// no tile waits for another; eight cells a thread, in two 16-byte loads.  3 us at 125k cells.
+__device__ inline void scan_cells(int t, const WinBook &wb, uint32_t *__restrict__ start, uint32_t *lds)
+{
+    static_assert(kCoarseCells == 8 * kThreads && kCoarse <= kThreads, "eight cells and at most one tile a thread");
+    const int j = threadIdx.x, lane = j & (kWave - 1), wave = j / kWave;
+    uint4 *c = reinterpret_cast<uint4 *>(wb.counts + (size_t)t * kCoarseCells) + 2 * j;
+    const uint4 a = c[0], b = c[1];
+    uint32_t before = 0u;
+    if (j < kCoarse && j < t)
+        for (int k = 0; k < kCoarseCopies; k++) before += wb.coarse[k * kCoarse + j];
+    c[0] = c[1] = make_uint4(0u, 0u, 0u, 0u);
+    const uint32_t mine = a.x + a.y + a.z + a.w + b.x + b.y + b.z + b.w;
+    uint32_t x = mine;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+        const uint32_t y = __shfl_up(x, o);
+        if (lane >= o) x += y;
+    }
+#pragma unroll
+    for (int o = kWave / 2; o > 0; o >>= 1) before += __shfl_xor(before, o);
+    if (lane == kWave - 1) {
+        lds[wave] = x;
+        lds[kWavesPerBlock + wave] = before;
+    }
+    __syncthreads();
+    uint32_t p = x - mine;
+    for (int w = 0; w < kWavesPerBlock; w++) p += (w < wave ? lds[w] : 0u) + lds[kWavesPerBlock + w];
+    uint4 u, v;
+    u.x = p; u.y = u.x + a.x; u.z = u.y + a.y; u.w = u.z + a.z;
+    v.x = u.w + a.w; v.y = v.x + b.x; v.z = v.y + b.y; v.w = v.z + b.z;
+    uint4 *o = reinterpret_cast<uint4 *>(start + (size_t)t * kCoarseCells) + 2 * j;
+    o[0] = u;
+    o[1] = v;
+    if (j == kThreads - 1) start[(size_t)(t + 1) * kCoarseCells] = v.w + b.w;   // as the next tile's first
+    __syncthreads();
+}
+
+// Bead i into its run by its arrival number.
+__device__ inline void place_bead(int i, int n, const uint32_t *__restrict__ key, const uint32_t *__restrict__ rank,
+                                  const uint32_t *__restrict__ start, uint32_t *__restrict__ cell,
+                                  uint32_t *__restrict__ bead)
+{
+    const uint32_t k = min(key[i] & ~kWinTag, (uint32_t)kWinCells - 1u);
+    const uint32_t p = min(start[k] + rank[i], (uint32_t)n - 1u);   // in bounds also for counts of another build
+    cell[p] = k;
+    bead[p] = (uint32_t)i;
+}
+
+__global__ __launch_bounds__(kThreads) void k_scan_cells(WinBook wb, uint32_t *__restrict__ start)
+{
+    __shared__ uint32_t lds[2 * kWavesPerBlock];
+    scan_cells(blockIdx.x, wb, start, lds);
+}
+
+__global__ __launch_bounds__(kThreads) void k_place(int n, const uint32_t *__restrict__ key,
+                                                    const uint32_t *__restrict__ rank,
+                                                    const uint32_t *__restrict__ start, uint32_t *__restrict__ cell,
+                                                    uint32_t *__restrict__ bead)
+{
+    const int i = blockIdx.x * kThreads + threadIdx.x;
+    if (i < n) place_bead(i, n, key, rank, start, cell, bead);
+}
+
 struct WArgs {
     uint32_t *kA, *vA, *kB, *vB, *kC, *vC;
+    WinBook wb;
+    uint32_t *start;
     uint32_t *ghist;        // the cell indices' digit histograms [copies][4][256]
-    const uint32_t *ghw;    // the window digits' [copies][2][512]
-    const uint32_t *desc;   // this sort's window
-    const uint32_t *flag;   // set: a key outside the window
-    uint32_t *bbox;         // the fallback's occupied cell range, [copies][8]
-    uint32_t *ctr;          // 3 tile counters: each launch's first pass, the fallback's second
+    uint32_t *ctr;          // 2 tile counters: the fallback's second and third pass
     uint32_t *bar;          // 2 barrier counters
-    uint32_t *status;       // look-back words of the same three passes, tiles x 512 each
+    uint32_t *status;       // look-back words of the fallback's three passes, tiles x 256 each
     int *errflag;
     const DevRep *reps;     // the cell grid: replica 0's
     int tiles;
 };
 
 template <int kRounds>
-__global__ __launch_bounds__(kThreads) void k_sortw(int n, int launch, WArgs a)
+__global__ __launch_bounds__(kThreads) void k_window(int n, int launch, WArgs a)
 {
     __shared__ WLds<kRounds> L;
     const int t = threadIdx.x;
-    // the launch's first pass draws from counter `launch` and uses look-back words `launch`
-    // on either path, so its tile id and the window path's histogram sums are requested
-    // before the path is known
-    const uint32_t tile0 = draw_tile(a.ctr + launch);
-    uint32_t gw[2], gw8[1] = {0u};
-    hist_sums<2>(a.ghw + 512 * launch, gw);
-    if (launch != 0) hist_sums<1>(a.ghw + 512, gw8);   // the second digit read as 8 bits
-    const WinDesc w = load_win(a.desc);
-    const bool fallback = w.wx == 0u || *a.flag != 0u;
-    uint32_t *st0 = a.status, *st1 = st0 + (size_t)a.tiles * kWDig, *st2 = st1 + (size_t)a.tiles * kWDig;
-    if (t == 0) L.tile = tile0;
-    __syncthreads();
-    const int tile = (int)L.tile;
+    const WinDesc w = load_win(a.wb.desc);
+    const bool fallback = w.wx == 0u || *a.wb.flag != 0u;
     if (!fallback) {
         if (launch == 0) {
-            wpass<kRounds, 9, true>(L, n, 0, tile, gw, a.kA, a.vA, a.kB, a.vB, st0, a.errflag);
-        } else if (w.wx * w.wy * w.wz <= (1u << 17)) {   // window keys of 17 bits: an 8-bit second digit
-            wpass<kRounds, 8>(L, n, 9, tile, gw8, a.kB, a.vB, a.kA, a.vA, st1, a.errflag);
+            const int tiles = (int)((w.wx * w.wy * w.wz + kCoarseCells - 1) / kCoarseCells);
+            for (int c = blockIdx.x; c < tiles; c += gridDim.x) scan_cells(c, a.wb, a.start, L.scan);
         } else {
-            wpass<kRounds, 9>(L, n, 9, tile, gw, a.kB, a.vB, a.kA, a.vA, st1, a.errflag);
+            const int i = blockIdx.x * kThreads + t;
+            if (i < n) place_bead(i, n, a.kA, a.vA, a.start, a.kB, a.vB);
         }
         return;
     }
-    uint32_t g8[1];
+    uint32_t *st0 = a.status, *st1 = st0 + (size_t)a.tiles * 256, *st2 = st1 + (size_t)a.tiles * 256;
     if (launch != 0) {
-        hist_sums<1>(a.ghist + 512, g8);
-        wpass<kRounds, 8>(L, n, 16, tile, g8, a.kC, a.vC, a.kA, a.vA, st1, a.errflag);
+        // the counts of the keys that did lie in the window
+        if (w.wx != 0u)
+            for (int c = blockIdx.x * kThreads + t; c < kWinCells; c += gridDim.x * kThreads) a.wb.counts[c] = 0u;
+        if ((int)blockIdx.x >= a.tiles) return;   // workgroups past the tiles
+        if (t == 0) L.tile = atomicAdd(a.ctr + 1, 1u);
+        __syncthreads();
+        wpass<kRounds>(L, n, 16, (int)L.tile, hist_sum(a.ghist + 512), false, a.kC, a.vC, a.kA, a.vA, st2, a.errflag);
         return;
     }
     // every key back to its cell index (window keys), its three digits counted (the key
@@ -833,17 +755,15 @@ __global__ __launch_bounds__(kThreads) void k_sortw(int n, int launch, WArgs a)
     if (t < 6) {
         uint32_t v = 0u;
         for (int q = 0; q < kWavesPerBlock; q++) v = max(v, L.bb[q][t]);
-        if (v) atomicMax(&a.bbox[(blockIdx.x % kHistCopies) * 8 + t], v);
+        if (v) atomicMax(&a.wb.bbox[(blockIdx.x % kHistCopies) * 8 + t], v);
     }
     grid_sync(a.bar, gridDim.x, a.errflag);
-    hist_sums<1>(a.ghist, g8);
-    wpass<kRounds, 8, true>(L, n, 0, tile, g8, a.kA, a.vA, a.kB, a.vB, st0, a.errflag);
+    // all of the launch's workgroups are resident, so the first pass's tiles are theirs in order
+    wpass<kRounds>(L, n, 0, blockIdx.x, hist_sum(a.ghist), true, a.kA, a.vA, a.kB, a.vB, st0, a.errflag);
     grid_sync(a.bar + 1, gridDim.x, a.errflag);
-    const uint32_t tile1 = draw_tile(a.ctr + 2);
-    hist_sums<1>(a.ghist + 256, g8);
-    if (t == 0) L.tile = tile1;
+    if (t == 0) L.tile = atomicAdd(a.ctr, 1u);
     __syncthreads();
-    wpass<kRounds, 8>(L, n, 8, (int)L.tile, g8, a.kB, a.vB, a.kC, a.vC, st2, a.errflag);
+    wpass<kRounds>(L, n, 8, (int)L.tile, hist_sum(a.ghist + 256), false, a.kB, a.vB, a.kC, a.vC, st1, a.errflag);
 }
 
 }  // namespace
@@ -933,7 +853,7 @@ void sort_moved(hipStream_t st, SortBuffers &b, const MoveSort &m, int bits, int
 
 int move_blocks(int n) { return (n + 255) / 256; }
 
-// ---- the window sort: host side ----
+// ---- the counting builds: host side ----
 static int sortw_tiles(int n)
 {
     const int tile = kThreads * sort_rounds(n);
@@ -942,31 +862,39 @@ static int sortw_tiles(int n)
 
 bool sortw_fits(int n) { return n >= 1 && sortw_tiles(n) <= kWinMaxTiles && sort_rounds(n) != 12; }
 
-size_t sortw_words(int n) { return kWinKeyWords + (size_t)3 * sortw_tiles(n) * kWDig; }
+size_t sortw_words(int n, bool window) { return kWinKeyWords + (window ? (size_t)3 * sortw_tiles(n) * 256 : 0); }
 
 uint32_t *win_scratch(uint32_t *sort_scratch, int n) { return sort_scratch + sort_scratch_words(n, 4); }
 
-WinBook win_book(uint32_t *sort_scratch, int n, const uint32_t *desc)
+WinBook win_book(uint32_t *sort_scratch, int n, const uint32_t *desc, uint32_t *counts, uint32_t cells)
 {
     uint32_t *ws = win_scratch(sort_scratch, n);
-    return WinBook{desc, ws, ws + 16 * 1024, ws + 16 * 1024 + 16 * 8};
+    uint32_t *bbox = ws + (size_t)kCoarseCopies * kCoarse;
+    return WinBook{desc, ws, bbox, bbox + 16 * 8, counts, cells};
 }
 
-void sort_window(hipStream_t st, SortBuffers &b, uint32_t *k2, uint32_t *v2, int parity, const uint32_t *desc,
-                 const DevRep *reps)
+void count_build(hipStream_t st, SortBuffers &b, uint32_t *k2, uint32_t *v2, int parity, const WinBook &wb,
+                 uint32_t *start, const DevRep *reps)
 {
     const int n = b.n;
+    const int blocks = (n + kThreads - 1) / kThreads;
+    if (wb.cells != 0u) {
+        hipLaunchKernelGGL(k_scan_cells, dim3((wb.cells + kCoarseCells - 1) / kCoarseCells), dim3(kThreads), 0, st, wb, start);
+        hipLaunchKernelGGL(k_place, dim3(blocks), dim3(kThreads), 0, st, n, b.k0, b.v0, start, b.k1, b.v1);
+        return;
+    }
     const int tiles = sortw_tiles(n);
     b.tiles = tiles;
-    const WinBook wb = win_book(b.scratch[parity], n, desc);
-    uint32_t *misc = wb.flag;   // flag, 3 tile counters, 2 barrier counters
-    WArgs a{b.k0, b.v0, b.k1, b.v1, k2, v2, b.scratch[parity], wb.ghw, desc, wb.flag, wb.bbox, misc + 1, misc + 4,
-            win_scratch(b.scratch[parity], n) + kWinKeyWords, b.errflag, reps, tiles};
+    uint32_t *misc = wb.flag;   // flag, 2 tile counters, 2 barrier counters
+    const WArgs a{b.k0, b.v0, b.k1, b.v1, k2, v2, wb, start, b.scratch[parity], misc + 1, misc + 3,
+                  win_scratch(b.scratch[parity], n) + kWinKeyWords, b.errflag, reps, tiles};
+    // the window path's second launch has a thread a bead, more workgroups than the fallback's tiles
     for (int launch = 0; launch < 2; launch++) {
+        const dim3 grid(launch == 0 ? tiles : blocks);
         if (sort_rounds(n) == 2)
-            hipLaunchKernelGGL(k_sortw<2>, dim3(tiles), dim3(kThreads), 0, st, n, launch, a);
+            hipLaunchKernelGGL(k_window<2>, grid, dim3(kThreads), 0, st, n, launch, a);
         else
-            hipLaunchKernelGGL(k_sortw<8>, dim3(tiles), dim3(kThreads), 0, st, n, launch, a);
+            hipLaunchKernelGGL(k_window<8>, grid, dim3(kThreads), 0, st, n, launch, a);
     }
 }
 

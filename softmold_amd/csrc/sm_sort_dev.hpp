@@ -51,7 +51,7 @@ __device__ inline void hist_flush(uint32_t (*h)[256], uint32_t *ghist, int passe
         if (h[p][threadIdx.x]) atomicAdd(&g[p * 256 + threadIdx.x], h[p][threadIdx.x]);
 }
 
-// ---- the window sort: the key kernel's side ----------------------------------------------
+// ---- the counting builds: the key kernel's side ----------------------------------------------
 struct WinDesc {
     uint32_t x0, y0, z0, wx, wy, wz;
 };
@@ -60,36 +60,46 @@ __device__ inline WinDesc load_win(const uint32_t *d) { return WinDesc{d[0], d[1
 // occupied-range words hold max(c + 1) and max(kBoxEnc - c) per axis, so that zero is empty
 constexpr uint32_t kBoxEnc = 1u << 20;
 
-// The end of a key kernel's block in a window sort; every thread of the 256-thread block
-// calls it and gets the key to store.  A key in the window is counted by its two window
-// digits (bits 0-8 and 9-17); a key outside it sets the fallback flag.  With no window the
-// key is stored as it is (the fallback counts the digits).  hs: the block's 1024 LDS
-// words, zero on entry.
+// The end of a key kernel's block in a counting build; every thread of the 256-thread block
+// calls it and gets the key to store and the bead's arrival number in its cell.  A key in the
+// window (or any key, in a dense build) adds one to its cell's count and gets the count
+// before it: the lanes of a wave whose neighbours hold the same cell (the beads of one lipid)
+// add together, since the counts live beyond the L2s and take about 25 atomics a ns
+// (240k beads one by one: 8 us more than by runs).  The coarse counts are gathered per block
+// first.  A key outside the window sets the fallback flag.  hs: kCoarse LDS words, zero on
+// entry.
 __device__ inline uint32_t win_key_end(const WinBook &wb, const WinDesc &w, uint32_t *hs, uint32_t k, int cx, int cy,
-                                       int cz, bool valid)
+                                       int cz, bool valid, uint32_t &rank)
 {
     const int t = threadIdx.x, lane = t & (kWave - 1);
-    if (w.wx == 0u) return k;   // workgroup-uniform
-    bool inw = false;
-    uint32_t wk = 0u;
-    if (valid) {
+    const bool dense = wb.cells != 0u;
+    rank = 0u;
+    if (!dense && w.wx == 0u) return k;   // workgroup-uniform: no window
+    bool in = valid;
+    uint32_t wk = k;
+    if (!dense) {
         const uint32_t dx = (uint32_t)cx - w.x0, dy = (uint32_t)cy - w.y0, dz = (uint32_t)cz - w.z0;
-        inw = dx < w.wx && dy < w.wy && dz < w.wz;
+        in = valid && dx < w.wx && dy < w.wy && dz < w.wz;
         wk = (dz * w.wy + dy) * w.wx + dx;
+        if (__ballot(valid && !in) != 0ull && lane == 0) atomicOr(wb.flag, 1u);
     }
-    if (inw) {
-        atomicAdd(&hs[wk & 511u], 1u);
-        atomicAdd(&hs[512u + ((wk >> 9) & 511u)], 1u);
+    in = in && wk < (uint32_t)kWinCells;   // always, within a window or a dense table
+    const uint32_t id = in ? wk : ~0u;
+    const uint32_t prev = (uint32_t)__shfl_up((int)id, 1);
+    const unsigned long long heads = __ballot(lane == 0 || prev != id);
+    const unsigned long long upto = ~0ull >> (kWave - 1 - lane);   // this lane and those below
+    const int head = kWave - 1 - __clzll((long long)(heads & upto));
+    const unsigned long long later = heads & ~upto;
+    uint32_t first = 0u;
+    if (in && head == lane) {
+        const uint32_t run = (uint32_t)((later ? __ffsll((long long)later) - 1 : kWave) - lane);
+        first = atomicAdd(&wb.counts[wk], run);
+        atomicAdd(&hs[wk / kCoarseCells], run);
     }
-    if (__ballot(valid && !inw) != 0ull && lane == 0) atomicOr(wb.flag, 1u);
+    rank = (uint32_t)__shfl((int)first, head) + (uint32_t)(lane - head);
     __syncthreads();
-    uint32_t *g = wb.ghw + (size_t)(blockIdx.x % kHistCopies) * 1024;
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const uint32_t c = hs[t + 256 * j];
-        if (c) atomicAdd(&g[t + 256 * j], c);
-    }
-    return inw ? (kWinTag | wk) : k;
+    if (t < kCoarse && hs[t]) atomicAdd(&wb.coarse[(blockIdx.x % kCoarseCopies) * kCoarse + t], hs[t]);
+    return dense ? k : (in ? (kWinTag | wk) : k);
 }
 
 }  // namespace smdev
