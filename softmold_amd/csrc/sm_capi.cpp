@@ -1064,10 +1064,11 @@ sm_ctx *create(const sm_system *s, int nrep)
         }
         // sorted slots per wave in the pair kernel: short chunks keep small systems filling
         // the chip, longer ones cut the per-cell overhead of large ones (measured on the
-        // 15k, 240k and 3M-bead systems; every chunk gives the same forces); from half a
-        // million beads on 16 slots (3M vesicle 995 -> 950 us, 3M bilayer 1028 -> 1000, the
-        // 64-vesicle sweep 848 -> 813; at 360k beads even, at 240k 96.6 -> 103.4)
-        c->chunk = n >= 500000 ? 16 : (n >= 50000 ? 8 : 2);
+        // 15k, 240k and 3M-bead systems; every chunk gives the same forces); from one and a
+        // half million beads on 16 slots (pair kernel, 8 -> 16 slots: 3M vesicle 995 -> 950 us,
+        // 3M bilayer 1028 -> 1000, the 64-vesicle sweep 848 -> 813; whole steps: 1.8M beads in
+        // 12 bilayers 812 -> 807, one 1.35M bilayer 615 -> 620, 960k beads in 40 468 -> 477)
+        c->chunk = n >= 1500000 ? 16 : (n >= 50000 ? 8 : 2);
         c->ensure_capacity(0);
         HIPCHK(hipStreamSynchronize(st));
     } catch (...) {
