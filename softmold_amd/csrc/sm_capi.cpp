@@ -48,10 +48,10 @@ void dfree(T *&p)
     p = nullptr;
 }
 
-enum KClass { K_FIRST, K_SORT, K_REORDER, K_PAIR, K_BONDED, K_GATHER, K_CHAIN_E, K_KIN, K_MC, K_KICK_FIRST, K_NCLASS };
+enum KClass { K_FIRST, K_SORT, K_REORDER, K_PAIR, K_BONDED, K_GATHER, K_SUMS, K_MC, K_KICK_FIRST, K_NCLASS };
 const char *kClassName[K_NCLASS] = {"integrate_first+key", "radix_sort", "reorder+cell_table", "pair_force",
-                                    "bonded+langevin+kick", "pair_gather_fp64", "chain_energy_fp64",
-                                    "kinetic_fp64", "mc_move", "bonded+kick+next_first+key"};
+                                    "bonded+langevin+kick", "pair_gather_fp64", "energy_sums_fp64",
+                                    "mc_move", "bonded+kick+next_first+key"};
 
 // The pair kernels' constant table: each (home type, candidate type) row of the FP32 force
 // constants padded to 8 floats {r_m, C1, C2, r_c, C4, C5, 0, 0}, then the culling reach
@@ -112,7 +112,7 @@ struct RepHost {
 // Tiles of a segment set: ranges [begin_r, begin_r + len_r) cut into kSegTile pieces that
 // start at each range's start.
 struct SegHost {
-    std::vector<int2> tile;
+    std::vector<int4> tile;
     std::vector<int> rep_first;
 };
 
@@ -121,8 +121,9 @@ SegHost make_tiles(const std::vector<int> &begin, const std::vector<int> &len)
     SegHost h;
     for (size_t r = 0; r < begin.size(); r++) {
         h.rep_first.push_back((int)h.tile.size());
-        for (int t = 0; t < len[r]; t += kSegTile)
-            h.tile.push_back(make_int2(begin[r] + t, begin[r] + std::min(len[r], t + kSegTile)));
+        const int step = kSumTile * (int)(((long long)len[r] + kSumTile * kSumTiles - 1) / (kSumTile * kSumTiles));
+        for (int t = 0; t < len[r]; t += step)
+            h.tile.push_back(make_int4(begin[r] + t, begin[r] + std::min(len[r], t + step), (int)r, 0));
     }
     h.rep_first.push_back((int)h.tile.size());
     return h;
@@ -222,7 +223,8 @@ struct sm_ctx {
     double4 *pdC = nullptr;
     int pd_a = -1, pd_b = -1;
     size_t pd_tab = 0;
-    double *ebead = nullptr, *echain = nullptr, *dres = nullptr;   // dres: meas [R][3], then dU [R][2]
+    double *ebead = nullptr, *edelta = nullptr;   // a term per bead; a box-move step keeps its dU in edelta
+    double *dres = nullptr;                      // meas [R][3], then dU [R][2]; or one call's 8 R results
     SegTiles segB{}, segC{};
     int *dcounts = nullptr, *dpairs = nullptr;
     long long pairs_cap = 0;
@@ -287,10 +289,10 @@ struct sm_ctx {
         dfree(mbefore); dfree(cnt_b); dfree(cnt_i); dfree(cnt_s); dfree(mflags); dfree(mcount);
         dfree(reps); dfree(glob); dfree(fconstF); dfree(uconstD); dfree(fconstD); dfree(chainPerBead); dfree(chainList);
         dfree(gptr); dfree(gent); dfree(gconstD);
-        dfree(cconstD); dfree(ebead); dfree(echain); dfree(dres); dfree(dcounts); dfree(dpairs); dfree(dnp);
+        dfree(cconstD); dfree(ebead); dfree(edelta); dfree(dres); dfree(dcounts); dfree(dpairs); dfree(dnp);
         dfree(adjF); dfree(adjDF); dfree(adjDU); dfree(pdU); dfree(pdTab); dfree(pdC);
-        dfree(segB.tile); dfree(segB.rep_first); dfree(segB.tilesum);
-        dfree(segC.tile); dfree(segC.rep_first); dfree(segC.tilesum);
+        dfree(segB.tile); dfree(segB.rep_first); dfree(segB.tilesum); dfree(segB.ticket);
+        dfree(segC.tile); dfree(segC.rep_first); dfree(segC.tilesum); dfree(segC.ticket);
         if (st) (void)hipStreamDestroy(st);
     }
 
@@ -537,40 +539,55 @@ struct sm_ctx {
         timed(K_GATHER, [&] {
             launch_pair_gather(st, P, chunk, GATHER_U, sbeads, skey(), sidx(), cstart, cend, reps, fconstF, uconstD, ebead,
                                nullptr, nullptr, nullptr, 0);
-            launch_seg_sum(st, segB, ebead, meas_dev() + 0, 3);
         });
-        timed(K_CHAIN_E, [&] {
-            launch_chain_energy(st, nchains, chainList, cconstD, beads, reps, 0, echain);
-            launch_seg_sum(st, segC, echain, meas_dev() + 1, 3);
+        timed(K_SUMS, [&] {
+            SumArgs a = sums(ebead, meas_dev());
+            launch_sums(st, SUM_MEASURE, a);
             if (gptr) {
                 launch_gen_energy(st, n, gen(), beads, reps, 0, ebead);
-                launch_seg_sum(st, segB, ebead, meas_dev() + 1, 3, true);
+                add_column(ebead, meas_dev() + 1, 3);
             }
         });
-        timed(K_KIN, [&] {
-            launch_kinetic(st, n, vel, ebead);
-            launch_seg_sum(st, segB, ebead, meas_dev() + 2, 3);
-        });
+    }
+    SumArgs sums(const double *x, double *out) const
+    {
+        SumArgs a{};
+        a.B = segB;
+        a.C = segC;
+        a.x = x;
+        a.vel = vel;
+        a.chains = chainList;
+        a.cconst = cconstD;
+        a.beads = beads;
+        a.reps = reps;
+        a.out = out;
+        a.n = n;
+        return a;
+    }
+    void add_column(const double *x, double *out, int stride) const
+    {
+        SumArgs a = sums(x, out);
+        a.stride = stride;
+        a.add = 1;
+        launch_sums(st, SUM_COLUMN, a);
     }
     // U(old) - U(scaled) of every replica with its trial scale into dres[3R + 2r + 0..1]
     void delta_device()
     {
         timed(K_GATHER, [&] {
-            launch_pair_gather(st, P, chunk, GATHER_DU, sbeads, skey(), sidx(), cstart, cend, reps, fconstF, uconstD, ebead,
+            launch_pair_gather(st, P, chunk, GATHER_DU, sbeads, skey(), sidx(), cstart, cend, reps, fconstF, uconstD, edelta,
                                nullptr, nullptr, nullptr, 0);
-            launch_seg_sum(st, segB, ebead, du_dev() + 0, 2);
         });
-        delta_bonded();
+        delta_sums();
     }
-    // the CHAIN and generic-record part of the dU
-    void delta_bonded()
+    // the replicas' pair dU from the beads' (edelta), with the CHAIN and generic-record part
+    void delta_sums()
     {
-        timed(K_CHAIN_E, [&] {
-            launch_chain_energy(st, nchains, chainList, cconstD, beads, reps, 1, echain);
-            launch_seg_sum(st, segC, echain, du_dev() + 1, 2);
+        timed(K_SUMS, [&] {
+            launch_sums(st, SUM_DELTA, sums(edelta, du_dev()));
             if (gptr) {
                 launch_gen_energy(st, n, gen(), beads, reps, 1, ebead);
-                launch_seg_sum(st, segB, ebead, du_dev() + 1, 2, true);
+                add_column(ebead, du_dev() + 1, 2);
             }
         });
     }
@@ -602,8 +619,7 @@ struct sm_ctx {
     {
         timed(K_PAIR, [&] {
             launch_pair_force_du(st, P, chunk, sbeads, skey(), sidx(), cstart, cend, reps, fconstF, uconstD, fpair,
-                                 ebead);
-            launch_seg_sum(st, segB, ebead, du_dev() + 0, 2);
+                                 edelta);
         });
     }
     void pair_step(bool mc)
@@ -616,7 +632,7 @@ struct sm_ctx {
     void mc_finish()
     {
         if (mc_fused) {
-            delta_bonded();
+            delta_sums();
             mc_decide();
         } else {
             mc_move();
@@ -1019,18 +1035,19 @@ sm_ctx *create(const sm_system *s, int nrep)
         c->chainList = dalloc<int2>(list.size());
         c->cconstD = dalloc<double4>(ccD.size());
         c->ebead = dalloc<double>(n);
-        c->echain = dalloc<double>(nch);
-        c->dres = dalloc<double>(5 * (size_t)nrep);
+        c->edelta = dalloc<double>(n);
+        c->dres = dalloc<double>(8 * (size_t)nrep);
         c->dcounts = dalloc<int>(n);
         c->dnp = dalloc<unsigned long long>(1);
         auto upseg = [&](SegTiles &S, const SegHost &h) {
             S.ntiles = (int)h.tile.size();
-            S.nrep = nrep;
-            S.tile = dalloc<int2>(h.tile.size());
+            S.tile = dalloc<int4>(h.tile.size());
             S.rep_first = dalloc<int>(h.rep_first.size());
-            S.tilesum = dalloc<double>(h.tile.size());
+            S.tilesum = dalloc<double>(kSumCols * h.tile.size());
+            S.ticket = dalloc<uint32_t>(nrep);
+            HIPCHK(hipMemsetAsync(S.ticket, 0, sizeof(uint32_t) * nrep, c->st));
             if (!h.tile.empty())
-                HIPCHK(hipMemcpyAsync(S.tile, h.tile.data(), sizeof(int2) * h.tile.size(), hipMemcpyHostToDevice, c->st));
+                HIPCHK(hipMemcpyAsync(S.tile, h.tile.data(), sizeof(int4) * h.tile.size(), hipMemcpyHostToDevice, c->st));
             HIPCHK(hipMemcpyAsync(S.rep_first, h.rep_first.data(), sizeof(int) * h.rep_first.size(),
                                   hipMemcpyHostToDevice, c->st));
         };
@@ -1321,20 +1338,14 @@ int sm_bond_stats(sm_ctx *c, double *out)
         const int R = c->nrep;
         std::vector<double> h((size_t)4 * R, 0.0);
         if (c->gptr) {
-            double *w = dalloc<double>((size_t)4 * R);
-            try {
-                for (int what = 0; what < 4; what++) {
-                    launch_gen_stats(c->st, c->n, c->gen(), c->beads, c->reps, what, c->ebead);
-                    launch_seg_sum(c->st, c->segB, c->ebead, w + what, 4);
-                }
-                c->check_launch();
-                HIPCHK(hipMemcpyAsync(h.data(), w, sizeof(double) * h.size(), hipMemcpyDeviceToHost, c->st));
-                HIPCHK(hipStreamSynchronize(c->st));
-            } catch (...) {
-                dfree(w);
-                throw;
+            for (int what = 0; what < 4; what++) {
+                launch_gen_stats(c->st, c->n, c->gen(), c->beads, c->reps, what, c->ebead);
+                SumArgs a = c->sums(c->ebead, c->dres + what);
+                a.stride = 4;
+                launch_sums(c->st, SUM_COLUMN, a);
             }
-            dfree(w);
+            c->check_launch();
+            (void)c->link.fetch(c->st, c->glob, c->dres, h.size(), h.data());
         }
         for (int r = 0; r < R; r++) {
             // the divisions on the host, as the reference writes them: lBond / nBond even
@@ -1352,32 +1363,23 @@ int sm_bond_stats(sm_ctx *c, double *out)
     });
 }
 
+// the replicas' radii from their heads: `work` holds 8 doubles a replica, the radii last
+static void vesicle_radius(sm_ctx *c, int32_t head_type, double *work, double *radius)
+{
+    SumArgs a = c->sums(nullptr, work);
+    a.radius = work + 7 * (size_t)c->nrep;
+    a.head = head_type;
+    launch_sums(c->st, SUM_HEADS, a);
+    launch_sums(c->st, SUM_HEAD_DIST, a);
+    c->check_launch();
+    (void)c->link.fetch(c->st, c->glob, a.radius, (size_t)c->nrep, radius);
+}
+
 int sm_vesicle_radius(sm_ctx *c, int32_t head_type, double *radius)
 {
     return guarded([&] {
         if (!c || !radius) invalid("null argument");
-        const int R = c->nrep;
-        // [R][4] head sums, [R][3] centres, [R] distance sums
-        double *w = dalloc<double>((size_t)8 * R);
-        try {
-            double *sums = w, *com = w + 4 * R, *dist = w + 7 * R;
-            for (int what = 0; what < 4; what++) {
-                launch_head_terms(c->st, c->n, c->beads, c->reps, head_type, what, nullptr, c->ebead);
-                launch_seg_sum(c->st, c->segB, c->ebead, sums + what, 4);
-            }
-            launch_head_com(c->st, R, sums, com);
-            launch_head_terms(c->st, c->n, c->beads, c->reps, head_type, 4, com, c->ebead);
-            launch_seg_sum(c->st, c->segB, c->ebead, dist, 1);
-            c->check_launch();
-            std::vector<double> h((size_t)8 * R);
-            HIPCHK(hipMemcpyAsync(h.data(), w, sizeof(double) * h.size(), hipMemcpyDeviceToHost, c->st));
-            HIPCHK(hipStreamSynchronize(c->st));
-            for (int r = 0; r < R; r++) radius[r] = h[7 * R + r] / h[4 * r + 3];
-        } catch (...) {
-            dfree(w);
-            throw;
-        }
-        dfree(w);
+        vesicle_radius(c, head_type, c->dres, radius);
     });
 }
 
@@ -1391,21 +1393,8 @@ int sm_vesicle_radius_noalloc(sm_ctx *c, int32_t head_type, double *radius)
                         std::to_string(kNoAllocMaxReplicas) + "; use sm_vesicle_radius");
         double *w = noalloc_scratch(c->device);
         if (!w) throw ApiError(SM_ERR_STATE, "fixed scratch of this device was not set up");
-        // same kernels and layout as sm_vesicle_radius: [R][4] head sums, [R][3] centres,
-        // [R] distance sums; the radii then replace the centres.  Every word read is
-        // written first by this call, so nothing is cleared.
-        double *sums = w, *com = w + 4 * (size_t)R, *dist = w + 7 * (size_t)R;
-        for (int what = 0; what < 4; what++) {
-            launch_head_terms(c->st, c->n, c->beads, c->reps, head_type, what, nullptr, c->ebead);
-            launch_seg_sum(c->st, c->segB, c->ebead, sums + what, 4);
-        }
-        launch_head_com(c->st, R, sums, com);
-        launch_head_terms(c->st, c->n, c->beads, c->reps, head_type, 4, com, c->ebead);
-        launch_seg_sum(c->st, c->segB, c->ebead, dist, 1);
-        launch_head_radius(c->st, R, sums, dist, com);
-        c->check_launch();
-        HIPCHK(hipMemcpyAsync(radius, com, sizeof(double) * (size_t)R, hipMemcpyDeviceToHost, c->st));
-        HIPCHK(hipStreamSynchronize(c->st));
+        // every word read is written first by this call, so nothing is cleared
+        vesicle_radius(c, head_type, w, radius);
     });
 }
 
@@ -1512,14 +1501,11 @@ int sm_potential_delta(sm_ctx *c, const double *scale, double *du_pair, double *
 {
     return guarded([&] {
         if (!c || !scale) invalid("null argument");
-        std::vector<DevRep> hr = c->read_reps();
-        for (int r = 0; r < c->nrep; r++)
-            for (int d = 0; d < 3; d++) hr[r].scale[d] = scale[3 * r + d];
-        c->write_reps(hr);
+        c->link.send_scale(c->st, c->reps, c->nrep, scale);
         c->build(0, kStepKeep);
         if (c->mc_fused) {   // the traversal a box-move step runs (it also leaves the pair forces)
             c->pair_force_du();
-            c->delta_bonded();
+            c->delta_sums();
         } else {
             c->delta_device();
         }
@@ -1902,27 +1888,19 @@ int sm_param_derivative(sm_ctx *c, int32_t type_a, int32_t type_b, double *out)
         check_pair(c, type_a, type_b);
         upload_param_derivative_tables(c, type_a, type_b);
         c->build(0, kStepKeep);
-        const int R = c->nrep;
         const size_t nt = 6 * (size_t)c->P.nT * c->P.nT;
-        double *w = c->dres;   // 5 words per replica: the four derivatives, then free
-        for (int p = 0; p < 2; p++) {
+        double *e[2] = {c->ebead, c->edelta};
+        for (int p = 0; p < 2; p++)
             launch_pair_gather(c->st, c->P, c->chunk, GATHER_U, c->sbeads, c->skey(), c->sidx(), c->cstart, c->cend,
-                               c->reps, c->pdTab + p * c->pd_tab, c->pdU + p * nt, c->ebead, nullptr, nullptr, nullptr,
-                               0);
-            launch_seg_sum(c->st, c->segB, c->ebead, w + p, 5);
-        }
-        const size_t ncs = c->hcconst.size();
+                               c->reps, c->pdTab + p * c->pd_tab, c->pdU + p * nt, e[p], nullptr, nullptr, nullptr, 0);
         // the measurement words are free between calls (each measurement copies its own out)
-        if (c->nchains > 0)
-            for (int p = 0; p < 2; p++) {
-                launch_chain_energy(c->st, c->nchains, c->chainList, c->pdC + p * ncs, c->beads, c->reps, 0, c->echain);
-                launch_seg_sum(c->st, c->segC, c->echain, w + 2 + p, 5);
-            }
+        SumArgs a = c->sums(e[0], c->dres);
+        a.y = e[1];
+        a.cconst = c->pdC;
+        a.cconst2 = c->pdC + c->hcconst.size();
+        launch_sums(c->st, SUM_PARAM, a);
         c->check_launch();
-        std::vector<double> h((size_t)5 * R);
-        const int flags = c->link.fetch(c->st, c->glob, w, h.size(), h.data());
-        for (int r = 0; r < R; r++)
-            for (int p = 0; p < 4; p++) out[4 * (size_t)r + p] = (p >= 2 && c->nchains == 0) ? 0.0 : h[5 * r + p];
+        const int flags = c->link.fetch(c->st, c->glob, c->dres, 4 * (size_t)c->nrep, out);
         c->check_bits(flags);
     });
 }
@@ -2037,7 +2015,8 @@ int sm_adjoint(sm_ctx *c, int32_t type_a, int32_t type_b, int32_t nsteps, int32_
                 c->build(0, kStepKeep);
                 adjoint_forces(0.0, 0);
                 // per replica: grad[r * kNTheta + p]
-                for (int p = 0; p < kNTheta; p++) launch_seg_sum(st, c->segB, g + (size_t)p * n, gs + p, kNTheta);
+                static_assert(kNTheta == 4, "SUM_COLUMNS sums four");
+                launch_sums(st, SUM_COLUMNS, c->sums(g, gs));
                 c->check_launch();
                 HIPCHK(hipMemcpyAsync(grad, gs, sizeof(double) * kNTheta * R, hipMemcpyDeviceToHost, st));
                 HIPCHK(hipStreamSynchronize(st));

@@ -92,19 +92,42 @@ struct Params {
 // Counter-RNG stream tags (word 3 of the Philox counter).
 enum : unsigned { TAG_LANGEVIN = 0, TAG_MC = 1, TAG_LANGEVIN_INIT = 2 };
 
-// Deterministic segmented FP64 sums: a segment set is a list of ranges (one per replica)
-// cut into tiles of kSegTile elements that start at the range start, so a replica's sum
-// does not depend on the other replicas.
-constexpr int kSegTile = 2048;
+// Deterministic segmented FP64 sums: a segment set is a list of ranges (one per replica) cut
+// into tiles that start at the range start and whose length follows from the range's, so a
+// replica's sum does not depend on the other replicas.  At most kSumTiles tiles a range, of at
+// least kSumTile elements: one workgroup a tile, then the range's last one sums the tiles.
+constexpr int kSumTile = 512, kSumTiles = 1024, kSumCols = 4;
 struct SegTiles {
-    int2 *tile;        // (begin, end) per tile, device
+    int4 *tile;        // (begin, end, replica, -) per tile, device
     int *rep_first;    // first tile of each replica (R + 1 entries), device
+    uint32_t *ticket;  // tiles done per replica: zero between launches, device
+    double *tilesum;   // ntiles x kSumCols, device
     int ntiles;
-    int nrep;
-    double *tilesum;   // ntiles, device
 };
-// out[r * stride] = sum of x over replica r's range (add: out[r * stride] += that sum)
-void launch_seg_sum(hipStream_t st, const SegTiles &S, const double *x, double *out, int stride, bool add = false);
+// What a sum kernel adds up.  Each is one launch: the terms of up to four sums over the beads
+// and two over the CHAIN molecules are computed where they are added, and the tile that ends a
+// replica's last writes its results.
+enum SumKind : int {
+    SUM_COLUMN,      // out[r * stride] (+)= sum of x over the beads
+    SUM_COLUMNS,     // out[4r + 0..3] = sums of x, x + n, x + 2n, x + 3n over the beads
+    SUM_MEASURE,     // out[3r + 0..2] = sum of x, CHAIN energy, kinetic energy
+    SUM_DELTA,       // out[2r + 0..1] = sum of x, CHAIN U(old) - U(scaled)
+    SUM_PARAM,       // out[4r + 0..3] = sums of x and y, CHAIN energies with cconst and cconst2
+    SUM_HEADS,       // out[7r + 0..6] = head beads' x, y, z (imaged) and number, their centre
+    SUM_HEAD_DIST,   // radius[r] = mean distance of the heads to the centre out[7r + 4..6]
+};
+struct SumArgs {
+    SegTiles B, C;              // beads, CHAIN molecules
+    const double *x, *y;        // a term per bead
+    const float4 *vel;
+    const int2 *chains;
+    const double4 *cconst, *cconst2;
+    const Bead *beads;
+    const DevRep *reps;
+    double *out, *radius;
+    int n, stride, add, head;
+};
+void launch_sums(hipStream_t st, SumKind kind, const SumArgs &a);
 
 // ---- launchers (sm_kernels.hip) ---------------------------------------------------------
 // step_set >= 0: the device step counter is set to step_set; -1: it is advanced by one
@@ -218,9 +241,6 @@ void launch_pair_gather(hipStream_t st, const Params &P, int chunk, int mode, co
                         const uint32_t *skey, const uint32_t *sidx, const int *cstart, const int *cend,
                         const DevRep *reps, const float *tab, const double *uconst, double *energy, int *counts,
                         int *pairs, unsigned long long *npairs, long long cap);
-// One FP64 value per chain: its energy, or U(old) - U(scaled) when delta != 0.
-void launch_chain_energy(hipStream_t st, int nchains, const int2 *chains, const double4 *cconst, const Bead *beads,
-                         const DevRep *reps, int delta, double *e);
 // Generic-record energies, one FP64 value per bead: the records whose first bead it is,
 // U, or U(old) - U(scaled) when delta != 0.
 void launch_gen_energy(hipStream_t st, int n, const GenTables &gen, const Bead *beads, const DevRep *reps,
@@ -229,13 +249,6 @@ void launch_gen_energy(hipStream_t st, int n, const GenTables &gen, const Bead *
 // bend's arm lengths), over the records whose first bead it is.
 void launch_gen_stats(hipStream_t st, int n, const GenTables &gen, const Bead *beads, const DevRep *reps, int what,
                       double *e);
-// One FP64 kinetic energy per bead.
-void launch_kinetic(hipStream_t st, int n, const float4 *vel, double *e);
-// Vesicle-radius terms per bead (what 0..2: imaged head coordinate, 3: head count, 4: head
-// distance to com[3r..]); sums[4r..4r+3] -> com[3r..3r+2].
-void launch_head_terms(hipStream_t st, int n, const Bead *beads, const DevRep *reps, int head, int what,
-                       const double *com, double *e);
-void launch_head_com(hipStream_t st, int nrep, const double *sums, double *com);
 void launch_mc_propose(hipStream_t st, int nrep, DevRep *reps, const DevGlobal *glob);
 // du[r*2 + 0] = dU_pair, du[r*2 + 1] = dU_chain of replica r
 void launch_mc_decide(hipStream_t st, const Params &P, DevRep *reps, DevGlobal *glob, const double *du);
@@ -252,6 +265,8 @@ constexpr size_t kPackBytes = 3 * (sizeof(double) + 2 * sizeof(float));   // per
 void launch_post(hipStream_t st, const double *src, size_t count, const DevGlobal *glob, double *head);
 void launch_pack(hipStream_t st, int first, int count, const PackSrc &src, double *out, const DevRep *reps, int nrep,
                  const DevGlobal *glob, double *head);
+// reps[r].scale = scale[3r ..] (pinned host memory)
+void launch_set_scale(hipStream_t st, DevRep *reps, int nrep, const double *scale);
 // beads[first ..].x, y, z = pos (pinned host memory, 3 per bead)
 void launch_set_positions(hipStream_t st, int first, int count, const double *pos, Bead *beads);
 // fill kernel (graph-capturable replacement for hipMemsetAsync)
@@ -265,8 +280,6 @@ constexpr size_t kNoAllocScratchDoubles = 8 * (size_t)kNoAllocMaxReplicas;   // 
 hipError_t noalloc_scratch_init(int device);
 // The device's scratch address, or nullptr before noalloc_scratch_init(device).
 double *noalloc_scratch(int device);
-// radius[r] = dist[r] / sums[4r + 3], all device pointers
-void launch_head_radius(hipStream_t st, int nrep, const double *sums, const double *dist, double *radius);
 
 // ---- radix sort (sm_sort.hip) ---------------------------------------------------------
 struct SortBuffers {

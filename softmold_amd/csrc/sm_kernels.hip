@@ -523,46 +523,6 @@ __global__ __launch_bounds__(kBlock) void k_second(int n, const Bead *__restrict
     vel[i] = v;
 }
 
-// ---------------------------------------------------------------------------------------
-// Segmented FP64 sums with fixed-shape trees: the result is independent of scheduling
-// and of the other replicas.
-// ---------------------------------------------------------------------------------------
-__device__ inline double block_sum(double v, double *lds)
-{
-    lds[threadIdx.x] = v;
-    __syncthreads();
-    for (int off = kBlock / 2; off > 0; off >>= 1) {
-        if ((int)threadIdx.x < off) lds[threadIdx.x] += lds[threadIdx.x + off];
-        __syncthreads();
-    }
-    const double r = lds[0];
-    __syncthreads();
-    return r;
-}
-
-__global__ __launch_bounds__(kBlock) void k_seg_tiles(const double *__restrict__ x, const int2 *__restrict__ tile,
-                                                      double *__restrict__ tilesum)
-{
-    __shared__ double lds[kBlock];
-    const int2 t = tile[blockIdx.x];
-    double s = 0.0;
-    for (int i = t.x + (int)threadIdx.x; i < t.y; i += kBlock) s += x[i];
-    const double b = block_sum(s, lds);
-    if (threadIdx.x == 0) tilesum[blockIdx.x] = b;
-}
-
-__global__ __launch_bounds__(kBlock) void k_seg_final(const double *__restrict__ tilesum,
-                                                      const int *__restrict__ rep_first, double *__restrict__ out,
-                                                      int stride, int add)
-{
-    __shared__ double lds[kBlock];
-    const int r = blockIdx.x;
-    double s = 0.0;
-    for (int t = rep_first[r] + (int)threadIdx.x; t < rep_first[r + 1]; t += kBlock) s += tilesum[t];
-    const double b = block_sum(s, lds);
-    if (threadIdx.x == 0) out[(size_t)r * stride] = add ? out[(size_t)r * stride] + b : b;
-}
-
 // CHAIN energies in FP64 (harmonicP MD.h:422-431, bendP MD.h:769-789, walk
 // system.h:2487-2568 / dPotential system.h:3280-3384), one thread per chain.
 __device__ inline void mi3(const Bead &p, const Bead &q, const double *L, double d[3])
@@ -590,20 +550,12 @@ __device__ inline double bend_p(const double a[3], const double b[3], double c0,
     return kt * p * p * 0.5;
 }
 
-__global__ __launch_bounds__(kBlock) void k_chain_energy(int nch, const int2 *__restrict__ chains,
-                                                         const double4 *__restrict__ cconst,
-                                                         const Bead *__restrict__ beads,
-                                                         const DevRep *__restrict__ reps, int delta,
-                                                         double *__restrict__ e)
+// energy of the CHAIN molecule at (start, len), or U(old) - U(scaled)
+__device__ inline double chain_energy(int start, int len, const double4 &K, const Bead *__restrict__ beads,
+                                      const DevRep &R, bool delta)
 {
-    const int c = blockIdx.x * kBlock + threadIdx.x;
-    if (c >= nch) return;
-    const int2 ch = chains[c];
-    const int start = ch.x, len = ch.y & 0xFFFF;
-    const DevRep &R = reps[beads[start].rep];
     const double L[3] = {R.L[0], R.L[1], R.L[2]};
     const double S[3] = {R.scale[0], R.scale[1], R.scale[2]};
-    const double4 K = cconst[ch.y >> 16];
     double accu = 0.0;
     for (int l = start; l <= start + len - 3; l++) {
         const bool last = (l == start + len - 3);
@@ -623,7 +575,7 @@ __global__ __launch_bounds__(kBlock) void k_chain_energy(int nch, const int2 *__
             accu += u;
         }
     }
-    e[c] = accu;
+    return accu;
 }
 
 // Generic BOND / BEND energies (doBondPotential / doBendPotential, system.h:2718-2830;
@@ -709,28 +661,24 @@ __global__ __launch_bounds__(kBlock) void k_gen_stats(int n, GenTables gen, cons
     e[i] = accu;
 }
 
-// Kinetic::compute (dataCollection.h:667-673), one term per bead
-__global__ __launch_bounds__(kBlock) void k_kinetic(int n, const float4 *__restrict__ vel, double *__restrict__ e)
-{
-    const int i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= n) return;
-    const float4 v = vel[i];
-    const double x = v.x, y = v.y, z = v.z;
-    e[i] = (x * x + y * y + z * z) / 2.0;
-}
+// ---------------------------------------------------------------------------------------
+// Segmented FP64 sums with fixed-shape trees: the result is independent of scheduling
+// and of the other replicas.
+//
+// What bounds them is launches, not bytes: the beads of a measurement are a few MB, and each
+// of its sums took a kernel for its terms, one for the tiles and one for the total, 4 to 5 us
+// each on an MI355X whatever they read.  The terms are computed where they are added, a
+// measurement's sums share a launch, and the last tile of a replica (by a ticket) makes the
+// totals: a measurement at 90k beads has 2 kernels instead of 9, a vesicle radius 2 instead
+// of 16.  Tiles are short (512 elements, two a thread) because a CHAIN molecule's FP64 roots
+// and divisions are a long chain of their own.
+// ---------------------------------------------------------------------------------------
 
-// ---------------------------------------------------------------------------------------
-// Vesicle radius of each replica from its head beads (analysis/vesicleRadius.cpp:71-175),
-// one FP64 term per bead for the segmented sums:
-//   what 0..2: coordinate `what` of a head, moved by one box length towards the replica's
-//              first bead when farther than half a box from it (the centre-of-mass loop);
-//   what 3:    1 per head (the head count);
-//   what 4:    the head's distance to the centre com[3r..3r+2], with the second loop's
-//              image term, which the reference ADDS to the difference (d += minImg, :147-151):
-//              the two agree with a true minimum image whenever no head lies more than half
-//              a box from the centre, and differ, as the reference does, otherwise.
-// Non-head beads give 0.
-// ---------------------------------------------------------------------------------------
+// The head beads of a vesicle (analysis/vesicleRadius.cpp:71-175).  The centre-of-mass loop
+// moves a head by one box length towards the replica's first bead when farther than half a
+// box from it.  The distance loop's image term is ADDED to the difference (d += minImg,
+// :147-151): the two agree with a true minimum image whenever no head lies more than half a
+// box from the centre, and differ, as the reference does, otherwise.
 __device__ inline double image_shift(double d, double L)
 {
     double m = 0.0;
@@ -739,42 +687,145 @@ __device__ inline double image_shift(double d, double L)
     return m;
 }
 
-__global__ __launch_bounds__(kBlock) void k_head_terms(int n, const Bead *__restrict__ beads,
-                                                       const DevRep *__restrict__ reps, int head, int what,
-                                                       const double *__restrict__ com, double *__restrict__ e)
+__device__ inline void head_place(const Bead &b, const Bead &p0, const double *L, double *v)
 {
 #pragma clang fp contract(off)
-    const int i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= n) return;
-    const Bead b = beads[i];
-    double v = 0.0;
-    if (b.type == head) {
-        const DevRep &R = reps[b.rep];
-        if (what < 3) {
-            const Bead p0 = beads[R.first];
-            const double x = what == 0 ? b.x : (what == 1 ? b.y : b.z);
-            const double x0 = what == 0 ? p0.x : (what == 1 ? p0.y : p0.z);
-            v = x - image_shift(x - x0, R.L[what]);
-        } else if (what == 3) {
-            v = 1.0;
-        } else {
-            const double *c = com + 3 * b.rep;
-            double dx = b.x - c[0], dy = b.y - c[1], dz = b.z - c[2];
-            dx += image_shift(dx, R.L[0]);
-            dy += image_shift(dy, R.L[1]);
-            dz += image_shift(dz, R.L[2]);
-            v = sqrt(dx * dx + dy * dy + dz * dz);
-        }
-    }
-    e[i] = v;
+    v[0] += b.x - image_shift(b.x - p0.x, L[0]);
+    v[1] += b.y - image_shift(b.y - p0.y, L[1]);
+    v[2] += b.z - image_shift(b.z - p0.z, L[2]);
+    v[3] += 1.0;
 }
 
-// sums[4r + 0..3] = (sum x, sum y, sum z, heads) -> com[3r + 0..2]
-__global__ void k_head_com(int nrep, const double *__restrict__ sums, double *__restrict__ com)
+__device__ inline double head_distance(const Bead &b, const double *c, const double *L)
 {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= nrep) return;
-    for (int k = 0; k < 3; k++) com[3 * r + k] = sums[4 * r + k] / sums[4 * r + 3];
+#pragma clang fp contract(off)
+    double dx = b.x - c[0], dy = b.y - c[1], dz = b.z - c[2];
+    dx += image_shift(dx, L[0]);
+    dy += image_shift(dy, L[1]);
+    dz += image_shift(dz, L[2]);
+    return sqrt(dx * dx + dy * dy + dz * dz);
+}
+
+template <int KIND>
+__device__ inline void bead_terms(const SumArgs &a, int r, int i, double *v)
+{
+    if (KIND == SUM_HEADS || KIND == SUM_HEAD_DIST) {
+        const Bead b = a.beads[i];
+        if (b.type != a.head) return;
+        if (KIND == SUM_HEADS)
+            head_place(b, a.beads[a.reps[r].first], a.reps[r].L, v);
+        else
+            v[0] += head_distance(b, a.out + 7 * (size_t)r + 4, a.reps[r].L);
+        return;
+    }
+    v[0] += a.x[i];
+    if (KIND == SUM_COLUMNS)
+        for (int k = 1; k < 4; k++) v[k] += a.x[(size_t)k * a.n + i];
+    if (KIND == SUM_PARAM) v[1] += a.y[i];
+    if (KIND == SUM_MEASURE) {   // Kinetic::compute (dataCollection.h:667-673)
+        const float4 u = a.vel[i];
+        const double x = u.x, y = u.y, z = u.z;
+        v[1] += (x * x + y * y + z * z) / 2.0;
+    }
+}
+
+template <int KIND>
+__device__ inline void chain_terms(const SumArgs &a, int r, int c, double *v)
+{
+    const int2 ch = a.chains[c];
+    const int len = ch.y & 0xFFFF, set = ch.y >> 16;
+    v[0] += chain_energy(ch.x, len, a.cconst[set], a.beads, a.reps[r], KIND == SUM_DELTA);
+    if (KIND == SUM_PARAM) v[1] += chain_energy(ch.x, len, a.cconst2[set], a.beads, a.reps[r], false);
+}
+
+// replica r's totals: v[0 .. cols) over its beads, or over its chains
+template <int KIND>
+__device__ inline void store_sums(const SumArgs &a, int r, bool chain, const double *v)
+{
+    if (KIND == SUM_COLUMN) {
+        double *o = a.out + (size_t)r * a.stride;
+        *o = a.add ? *o + v[0] : v[0];
+    } else if (KIND == SUM_COLUMNS) {
+        for (int k = 0; k < 4; k++) a.out[4 * (size_t)r + k] = v[k];
+    } else if (KIND == SUM_MEASURE) {
+        double *o = a.out + 3 * (size_t)r;
+        if (chain) {
+            o[1] = v[0];
+        } else {
+            o[0] = v[0];
+            o[2] = v[1];
+        }
+    } else if (KIND == SUM_DELTA) {
+        a.out[2 * (size_t)r + (chain ? 1 : 0)] = v[0];
+    } else if (KIND == SUM_PARAM) {
+        for (int k = 0; k < 2; k++) a.out[4 * (size_t)r + (chain ? 2 : 0) + k] = v[k];
+    } else if (KIND == SUM_HEADS) {
+        double *o = a.out + 7 * (size_t)r;
+        for (int k = 0; k < 4; k++) o[k] = v[k];
+        for (int k = 0; k < 3; k++) o[4 + k] = v[k] / v[3];
+    } else if (KIND == SUM_HEAD_DIST) {
+        a.radius[r] = v[0] / a.out[7 * (size_t)r + 3];
+    }
+}
+
+// v[0 .. C) summed over the workgroup, in every thread
+template <int C>
+__device__ inline void block_sums(double *v, double (*lds)[kSumCols])
+{
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+#pragma unroll
+    for (int k = 0; k < C; k++)
+#pragma unroll
+        for (int o = kWave / 2; o > 0; o >>= 1) v[k] += __shfl_xor(v[k], o);
+    __syncthreads();
+    if (lane == 0)
+        for (int k = 0; k < C; k++) lds[wave][k] = v[k];
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < C; k++) v[k] = (lds[0][k] + lds[1][k]) + (lds[2][k] + lds[3][k]);
+}
+
+template <int KIND>
+__global__ __launch_bounds__(kBlock) void k_sums(SumArgs a)
+{
+    static_assert(kBlock == 4 * kWave, "block_sums adds four waves");
+    constexpr bool kChains = KIND == SUM_MEASURE || KIND == SUM_DELTA || KIND == SUM_PARAM;
+    constexpr int C = KIND == SUM_COLUMNS || KIND == SUM_HEADS ? 4 : (KIND == SUM_MEASURE || KIND == SUM_PARAM ? 2 : 1);
+    __shared__ double lds[kBlock / kWave][kSumCols];
+    __shared__ bool last;
+    const bool chain = kChains && (int)blockIdx.x >= a.B.ntiles;
+    const SegTiles &S = chain ? a.C : a.B;
+    const int tile = (int)blockIdx.x - (chain ? a.B.ntiles : 0);
+    const int4 t = S.tile[tile];
+    const int r = t.z, t0 = S.rep_first[r], t1 = S.rep_first[r + 1];
+    double v[kSumCols] = {0.0, 0.0, 0.0, 0.0};
+    if (chain)
+        for (int i = t.x + (int)threadIdx.x; i < t.y; i += kBlock) chain_terms<KIND>(a, r, i, v);
+    else
+        for (int i = t.x + (int)threadIdx.x; i < t.y; i += kBlock) bead_terms<KIND>(a, r, i, v);
+    block_sums<C>(v, lds);
+    if (t1 - t0 > 1) {
+        if (threadIdx.x == 0) {
+            for (int k = 0; k < C; k++)
+                __hip_atomic_store(S.tilesum + (size_t)tile * kSumCols + k, v[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            last = __hip_atomic_fetch_add(S.ticket + r, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) ==
+                   (uint32_t)(t1 - t0 - 1);
+        }
+        __syncthreads();
+        if (!last) return;
+        for (int k = 0; k < C; k++) v[k] = 0.0;
+        for (int j = t0 + (int)threadIdx.x; j < t1; j += kBlock)
+            for (int k = 0; k < C; k++)
+                v[k] += __hip_atomic_load(S.tilesum + (size_t)j * kSumCols + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        block_sums<C>(v, lds);
+        if (threadIdx.x == 0) S.ticket[r] = 0u;
+    }
+    if (threadIdx.x != 0) return;
+    store_sums<KIND>(a, r, chain, v);
+    if (kChains && !chain && a.C.rep_first[r] == a.C.rep_first[r + 1]) {   // no tile of its chains does
+        const double zero[kSumCols] = {0.0, 0.0, 0.0, 0.0};
+        store_sums<KIND>(a, r, true, zero);
+    }
 }
 
 // ---------------------------------------------------------------------------------------
@@ -883,6 +934,13 @@ __global__ __launch_bounds__(kBlock) void k_post(const double *__restrict__ src,
     if (i < count) head[1 + i] = src[i];
 }
 
+__global__ __launch_bounds__(kBlock) void k_set_scale(DevRep *__restrict__ reps, int nrep,
+                                                      const double *__restrict__ scale)
+{
+    const int i = blockIdx.x * kBlock + threadIdx.x;
+    if (i < 3 * nrep) reps[i / 3].scale[i % 3] = scale[i];
+}
+
 __global__ __launch_bounds__(kBlock) void k_pack(int first, int count, PackSrc src, double *__restrict__ out,
                                                  const DevRep *__restrict__ reps, int nrep,
                                                  const DevGlobal *__restrict__ glob, double *__restrict__ head)
@@ -975,12 +1033,18 @@ void launch_second(hipStream_t st, int n, const Bead *beads, const float4 *acc, 
     hipLaunchKernelGGL(k_second, dim3(blocks(n)), dim3(kBlock), 0, st, n, beads, acc, vel, halfdt);
 }
 
-void launch_seg_sum(hipStream_t st, const SegTiles &S, const double *x, double *out, int stride, bool add)
+void launch_sums(hipStream_t st, SumKind kind, const SumArgs &a)
 {
-    if (S.ntiles > 0)
-        hipLaunchKernelGGL(k_seg_tiles, dim3(S.ntiles), dim3(kBlock), 0, st, x, S.tile, S.tilesum);
-    hipLaunchKernelGGL(k_seg_final, dim3(S.nrep), dim3(kBlock), 0, st, S.tilesum, S.rep_first, out, stride,
-                       add ? 1 : 0);
+    const dim3 beads(a.B.ntiles), both(a.B.ntiles + a.C.ntiles), block(kBlock);
+    switch (kind) {
+    case SUM_COLUMN: hipLaunchKernelGGL(k_sums<SUM_COLUMN>, beads, block, 0, st, a); break;
+    case SUM_COLUMNS: hipLaunchKernelGGL(k_sums<SUM_COLUMNS>, beads, block, 0, st, a); break;
+    case SUM_MEASURE: hipLaunchKernelGGL(k_sums<SUM_MEASURE>, both, block, 0, st, a); break;
+    case SUM_DELTA: hipLaunchKernelGGL(k_sums<SUM_DELTA>, both, block, 0, st, a); break;
+    case SUM_PARAM: hipLaunchKernelGGL(k_sums<SUM_PARAM>, both, block, 0, st, a); break;
+    case SUM_HEADS: hipLaunchKernelGGL(k_sums<SUM_HEADS>, beads, block, 0, st, a); break;
+    case SUM_HEAD_DIST: hipLaunchKernelGGL(k_sums<SUM_HEAD_DIST>, beads, block, 0, st, a); break;
+    }
 }
 
 void launch_gen_stats(hipStream_t st, int n, const GenTables &gen, const Bead *beads, const DevRep *reps, int what,
@@ -993,30 +1057,6 @@ void launch_gen_energy(hipStream_t st, int n, const GenTables &gen, const Bead *
                        int delta, double *e)
 {
     hipLaunchKernelGGL(k_gen_energy, dim3(blocks(n)), dim3(kBlock), 0, st, n, gen, beads, reps, delta, e);
-}
-
-void launch_chain_energy(hipStream_t st, int nchains, const int2 *chains, const double4 *cconst, const Bead *beads,
-                         const DevRep *reps, int delta, double *e)
-{
-    if (nchains <= 0) return;
-    hipLaunchKernelGGL(k_chain_energy, dim3(blocks(nchains)), dim3(kBlock), 0, st, nchains, chains, cconst, beads,
-                       reps, delta, e);
-}
-
-void launch_kinetic(hipStream_t st, int n, const float4 *vel, double *e)
-{
-    hipLaunchKernelGGL(k_kinetic, dim3(blocks(n)), dim3(kBlock), 0, st, n, vel, e);
-}
-
-void launch_head_terms(hipStream_t st, int n, const Bead *beads, const DevRep *reps, int head, int what,
-                       const double *com, double *e)
-{
-    hipLaunchKernelGGL(k_head_terms, dim3(blocks(n)), dim3(kBlock), 0, st, n, beads, reps, head, what, com, e);
-}
-
-void launch_head_com(hipStream_t st, int nrep, const double *sums, double *com)
-{
-    hipLaunchKernelGGL(k_head_com, dim3(blocks(nrep)), dim3(kBlock), 0, st, nrep, sums, com);
 }
 
 void launch_mc_propose(hipStream_t st, int nrep, DevRep *reps, const DevGlobal *glob)
@@ -1044,6 +1084,11 @@ void launch_pack(hipStream_t st, int first, int count, const PackSrc &src, doubl
 {
     hipLaunchKernelGGL(k_pack, dim3(std::max(1, blocks(3ll * count))), dim3(kBlock), 0, st, first, count, src, out, reps,
                        nrep, glob, head);
+}
+
+void launch_set_scale(hipStream_t st, DevRep *reps, int nrep, const double *scale)
+{
+    hipLaunchKernelGGL(k_set_scale, dim3(blocks(3ll * nrep)), dim3(kBlock), 0, st, reps, nrep, scale);
 }
 
 void launch_set_positions(hipStream_t st, int first, int count, const double *pos, Bead *beads)

@@ -21,15 +21,6 @@ constexpr int kMaxDevices = 64;
 std::mutex g_mu;
 double *g_ptr[kMaxDevices] = {};
 
-// radius[r] = dist[r] / sums[4r + 3]: the division sm_vesicle_radius makes on the host
-__global__ void k_head_radius(int nrep, const double *__restrict__ sums, const double *__restrict__ dist,
-                              double *__restrict__ radius)
-{
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= nrep) return;
-    radius[r] = dist[r] / sums[4 * r + 3];
-}
-
 }  // namespace
 
 hipError_t noalloc_scratch_init(int device)
@@ -49,11 +40,6 @@ double *noalloc_scratch(int device)
     if (device < 0 || device >= kMaxDevices) return nullptr;
     std::lock_guard<std::mutex> lk(g_mu);
     return g_ptr[device];
-}
-
-void launch_head_radius(hipStream_t st, int nrep, const double *sums, const double *dist, double *radius)
-{
-    hipLaunchKernelGGL(k_head_radius, dim3((nrep + 63) / 64), dim3(64), 0, st, nrep, sums, dist, radius);
 }
 
 }  // namespace smdev

@@ -143,6 +143,16 @@ public:
         return flags();
     }
 
+    // reps[r].scale = scale[3r ..]; the caller's array is free again on return, the buffer after
+    // the next fetch
+    void send_scale(hipStream_t st, DevRep *reps, int nrep, const double *scale)
+    {
+        head(3 * (size_t)nrep);
+        std::memcpy(head_ + 1, scale, 3 * sizeof(double) * (size_t)nrep);
+        launch_set_scale(st, reps, nrep, head_ + 1);
+        check(hipGetLastError(), "scale");
+    }
+
     // beads[i].x, y, z = pos[3 i ..] for n beads; the caller's array is free again on return
     void send_positions(hipStream_t st, int n, const double *pos, Bead *beads)
     {
