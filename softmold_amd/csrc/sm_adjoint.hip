@@ -15,7 +15,11 @@
 // These kernels serve short fitting trajectories of small systems: stencil cells are read
 // straight from global memory, no LDS staging.  The pair term gives each bead 32 lanes,
 // one per stencil cell, and combines them by a fixed shuffle tree; with one thread per
-// bead the 12k-bead bilayer filled 47 workgroups and the pair term took 465 us a call.
+// bead the 12k-bead bilayer filled 47 workgroups and the pair term took 465 us a call.  The
+// lanes test their cells' beads and put the hits into a list, and 32 hits at a time are
+// evaluated, one a lane: a lane that evaluated its own hits as it found them left the other
+// 63 waiting through roots and divisions for nearly every candidate (86 us a call at 12k
+// beads, 38 now; what is left is the chain of loads behind a hit: bead, table row, adjoint).
 //
 // Reference: force law Force<double> (MD.h:795-848), potential (MD.h:895-930), constant
 // tables laradjiRevaleeFC/PC (potentials/laradjiRevalee.h:84-152), harmonicF/bendF
@@ -154,6 +158,8 @@ __device__ inline double lane_sum(double x)
     return x;
 }
 
+constexpr int kAdjHits = 2 * kAdjLanes;   // a bead's pending hits: fewer than 32, then up to 32 more
+
 __global__ __launch_bounds__(kBlock) void k_adj_pair(int n, int nT, double cut2, const Bead *__restrict__ sb,
                                                      const uint32_t *__restrict__ skey,
                                                      const uint32_t *__restrict__ sidx,
@@ -164,88 +170,130 @@ __global__ __launch_bounds__(kBlock) void k_adj_pair(int n, int nT, double cut2,
                                                      double4 *__restrict__ hvout, double *__restrict__ g, double obj,
                                                      int want_hv)
 {
+    __shared__ int2 hits[kBlock / kAdjLanes][kAdjHits];   // (sorted slot, stencil cell)
     const long long gt = (long long)blockIdx.x * kBlock + threadIdx.x;
     const int s = (int)(gt / kAdjLanes);   // sorted slot of the bead (uniform over its lanes)
     const int c = (int)(gt % kAdjLanes);   // its stencil cell
+    const int group = threadIdx.x / kAdjLanes;
     const bool live = s < n;
     double Fx = 0, Fy = 0, Fz = 0, Hx = 0, Hy = 0, Hz = 0;
     double gw[2] = {0.0, 0.0}, du[2] = {0.0, 0.0};
-    uint32_t me = 0;
-    if (live) {
-        const Bead hb = sb[s];
-        me = sidx[s];
-        const DevRep &R = reps[hb.rep];
-        const int nx = R.nc[0], ny = R.nc[1], nz = R.nc[2];
-        const uint32_t kbase = (uint32_t)R.cellbase;
-        const uint32_t k = skey[s] - kbase;
-        const int kx = (int)(k % (uint32_t)nx), ky = (int)((k / (uint32_t)nx) % (uint32_t)ny),
-                  kz = (int)(k / (uint32_t)(nx * ny));
-        const double4 wi = w[me];
-        const size_t tsz = 6 * (size_t)nT * nT;
-        if (c < 27) {
-            int X0 = kx + c % 3 - 1, Y0 = ky + (c / 3) % 3 - 1, Z0 = kz + c / 9 - 1;
-            const double sx = X0 < 0 ? -R.L[0] : (X0 >= nx ? R.L[0] : 0.0);
-            const double sy = Y0 < 0 ? -R.L[1] : (Y0 >= ny ? R.L[1] : 0.0);
-            const double sz = Z0 < 0 ? -R.L[2] : (Z0 >= nz ? R.L[2] : 0.0);
-            X0 = X0 < 0 ? X0 + nx : (X0 >= nx ? X0 - nx : X0);
-            Y0 = Y0 < 0 ? Y0 + ny : (Y0 >= ny ? Y0 - ny : Y0);
-            Z0 = Z0 < 0 ? Z0 + nz : (Z0 >= nz ? Z0 - nz : Z0);
-            const uint32_t kk = kbase + (uint32_t)(X0 + Y0 * nx + Z0 * nx * ny);
-            const int c0 = cstart[kk];
-            const int c1 = ((unsigned)c0 < (unsigned)n && skey[c0] == kk) ? cend[kk] : c0;
-            for (int j = c0; j < c1; j++) {
-                if (j == s) continue;
-                const Bead q = sb[j];
-                const double dx = hb.x - (q.x + sx), dy = hb.y - (q.y + sy), dz = hb.z - (q.z + sz);
-                const double r2 = sq3(dx, dy, dz);
-                if (!(r2 < cut2)) continue;
-                const double r = sqrt(r2);
-                // the row of the particle the reference's traversal makes first: across
-                // cells the one whose forward half shell (cellOpt.h:715) holds the other's
-                // cell, within a cell the lower index (cellOpt.h:572-585,780-795)
-                constexpr uint32_t fwd = forward_cells();
-                const bool first = c == 13 ? me < sidx[j] : ((fwd >> c) & 1u) != 0;
-                const size_t row = 6 * (first ? (size_t)hb.type * nT + q.type : (size_t)q.type * nT + hb.type);
-                const double *C = fc + row;
-                const int o = (r >= C[0]) ? 3 : 0;
-                const double m = C[o] - r;
-                const double f = (C[o + 1] - C[o + 2] * m) * m;        // force along d/r
-                const double fr = f / r;
-                Fx += dx * fr;
-                Fy += dy * fr;
-                Fz += dz * fr;
-                if (want_hv) {
-                    const double4 wj = w[sidx[j]];
-                    const double ux = wi.x - wj.x, uy = wi.y - wj.y, uz = wi.z - wj.z;
-                    const double fp = -(C[o + 1] - 2.0 * C[o + 2] * m);  // df/dr
-                    const double e = (dx * ux + dy * uy + dz * uz) / r;  // dr along the direction
-                    const double t = (fp / r - f / r2) * e;
-                    Hx += ux * fr + dx * t;
-                    Hy += uy * fr + dy * t;
-                    Hz += uz * fr + dz * t;
+    const int slot = live ? s : n - 1;
+    const Bead hb = sb[slot];
+    const uint32_t me = sidx[slot];
+    const DevRep &R = reps[hb.rep];
+    const int nx = R.nc[0], ny = R.nc[1], nz = R.nc[2];
+    const double L0 = R.L[0], L1 = R.L[1], L2 = R.L[2];
+    const uint32_t kbase = (uint32_t)R.cellbase;
+    const uint32_t k = skey[slot] - kbase;
+    const int kx = (int)(k % (uint32_t)nx), ky = (int)((k / (uint32_t)nx) % (uint32_t)ny),
+              kz = (int)(k / (uint32_t)(nx * ny));
+    const double4 wi = w[me];
+    const size_t tsz = 6 * (size_t)nT * nT;
+    // the box length to add to the beads of stencil cell q along an axis
+    auto shift = [](int cell, int cells, double L) { return cell < 0 ? -L : (cell >= cells ? L : 0.0); };
+    double sx = 0.0, sy = 0.0, sz = 0.0;
+    int j = 0, end = 0;
+    if (live && c < 27) {
+        int X0 = kx + c % 3 - 1, Y0 = ky + (c / 3) % 3 - 1, Z0 = kz + c / 9 - 1;
+        sx = shift(X0, nx, L0);
+        sy = shift(Y0, ny, L1);
+        sz = shift(Z0, nz, L2);
+        X0 = X0 < 0 ? X0 + nx : (X0 >= nx ? X0 - nx : X0);
+        Y0 = Y0 < 0 ? Y0 + ny : (Y0 >= ny ? Y0 - ny : Y0);
+        Z0 = Z0 < 0 ? Z0 + nz : (Z0 >= nz ? Z0 - nz : Z0);
+        const uint32_t kk = kbase + (uint32_t)(X0 + Y0 * nx + Z0 * nx * ny);
+        j = cstart[kk];
+        end = ((unsigned)j < (unsigned)n && skey[j] == kk) ? cend[kk] : j;
+    }
+    // one hit: bead hj of stencil cell hc, within the cutoff
+    auto evaluate = [&](int hj, int hc) {
+        const Bead q = sb[hj];
+        const uint32_t other = sidx[hj];
+        const double dx = hb.x - (q.x + shift(kx + hc % 3 - 1, nx, L0));
+        const double dy = hb.y - (q.y + shift(ky + (hc / 3) % 3 - 1, ny, L1));
+        const double dz = hb.z - (q.z + shift(kz + hc / 9 - 1, nz, L2));
+        const double r2 = sq3(dx, dy, dz);
+        const double r = sqrt(r2);
+        // the row of the particle the reference's traversal makes first: across
+        // cells the one whose forward half shell (cellOpt.h:715) holds the other's
+        // cell, within a cell the lower index (cellOpt.h:572-585,780-795)
+        constexpr uint32_t fwd = forward_cells();
+        const bool first = hc == 13 ? me < other : ((fwd >> hc) & 1u) != 0;
+        const size_t row = 6 * (first ? (size_t)hb.type * nT + q.type : (size_t)q.type * nT + hb.type);
+        const double *C = fc + row;
+        const int o = (r >= C[0]) ? 3 : 0;
+        const double m = C[o] - r;
+        const double f = (C[o + 1] - C[o + 2] * m) * m;        // force along d/r
+        const double ri = 1.0 / r, fr = f * ri;
+        Fx += dx * fr;
+        Fy += dy * fr;
+        Fz += dz * fr;
+        if (want_hv) {
+            const double4 wj = w[other];
+            const double ux = wi.x - wj.x, uy = wi.y - wj.y, uz = wi.z - wj.z;
+            const double fp = -(C[o + 1] - 2.0 * C[o + 2] * m);  // df/dr
+            const double e = (dx * ux + dy * uy + dz * uz) * ri;  // dr along the direction
+            const double t = (fp - fr) * ri * e;
+            Hx += ux * fr + dx * t;
+            Hy += uy * fr + dy * t;
+            Hz += uz * fr + dz * t;
+        }
+        const double wd = (wi.x * dx + wi.y * dy + wi.z * dz) * ri;
+        const double *U = duc + row;   // only C1, C2, C4, C5 of the U row depend on theta
+        for (int p = 0; p < 2; p++) {
+            const double *D = dfc + p * tsz + row;
+            gw[p] += wd * ((D[o + 1] - D[o + 2] * m) * m);
+            if (obj != 0.0) {
+                const double *E = U + p * tsz;
+                double d;
+                if (r <= C[0]) {
+                    const double mu = C[0] - r;
+                    d = E[1] * mu * mu + E[2];
+                } else {
+                    const double mu = C[3] - r;
+                    d = mu * mu * (E[4] - mu * E[5]);
                 }
-                const double wd = (wi.x * dx + wi.y * dy + wi.z * dz) / r;
-                const double *U = duc + row;   // only C1, C2, C4, C5 of the U row depend on theta
-                for (int p = 0; p < 2; p++) {
-                    const double *D = dfc + p * tsz + row;
-                    gw[p] += wd * ((D[o + 1] - D[o + 2] * m) * m);
-                    if (obj != 0.0) {
-                        const double *E = U + p * tsz;
-                        double d;
-                        if (r <= C[0]) {
-                            const double mu = C[0] - r;
-                            d = E[1] * mu * mu + E[2];
-                        } else {
-                            const double mu = C[3] - r;
-                            d = mu * mu * (E[4] - mu * E[5]);
-                        }
-                        du[p] += 0.5 * d;
-                    }
-                }
+                du[p] += 0.5 * d;
             }
         }
+    };
+    int head = 0, count = 0;   // the bead's pending hits (uniform over its lanes)
+    const double *at = &sb[j < end ? j : slot].x;
+    double qx = at[0], qy = at[1], qz = at[2];
+    for (;;) {
+        // a candidate a lane, its next one's load in flight
+        const bool more = j < end;
+        const bool any = __any(more);
+        const double dx = hb.x - (qx + sx), dy = hb.y - (qy + sy), dz = hb.z - (qz + sz);
+        const bool hit = more && j != s && sq3(dx, dy, dz) < cut2;
+        const int2 mine = make_int2(j, c);
+        if (more) j++;
+        if (j < end) {
+            at = &sb[j].x;
+            qx = at[0];
+            qy = at[1];
+            qz = at[2];
+        }
+        const unsigned long long wave = __ballot(hit);
+        const uint32_t found = (uint32_t)((threadIdx.x & kAdjLanes) ? wave >> kAdjLanes : wave);
+        if (hit) hits[group][(head + count + __popc(found & ((1u << c) - 1u))) % kAdjHits] = mine;
+        count += __popc(found);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (count >= kAdjLanes || (!any && count > 0)) {
+            const int take = min(count, kAdjLanes);
+            if (c < take) {
+                const int2 h = hits[group][(head + c) % kAdjHits];
+                evaluate(h.x, h.y);
+            }
+            head += take;
+            count -= take;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (!any && !__any(count > 0)) break;
     }
-    // every lane of the group takes part in the tree, live or not
     Fx = lane_sum(Fx);
     Fy = lane_sum(Fy);
     Fz = lane_sum(Fz);
