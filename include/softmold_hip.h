@@ -224,8 +224,10 @@ int sm_get_params(sm_ctx *ctx, int32_t type_a, int32_t type_b, double *theta);
  * U_pair + U_chain (with the generic records' energy) after each step's kick, one value
  * per replica.  If grad != NULL it receives dJ/dtheta (4 values per replica, replica
  * after replica) from the discrete adjoint of the step in FP64, recomputing the trajectory
- * from checkpoints every `checkpoint` steps; MC accept/reject decisions are held fixed
- * (the pathwise derivative).  The context state is left as it was. */
+ * from checkpoints every `checkpoint` steps, or further apart while the positions of the
+ * steps between them (32 bytes a bead and step) fit 256 MiB; the steps after the last
+ * checkpoint are not recomputed.  MC accept/reject decisions are held fixed (the pathwise
+ * derivative).  The context state is left as it was. */
 int sm_adjoint(sm_ctx *ctx, int32_t type_a, int32_t type_b, int32_t nsteps, int32_t checkpoint, double *J,
                double *grad);
 

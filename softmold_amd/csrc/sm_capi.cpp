@@ -216,6 +216,24 @@ struct sm_ctx {
     std::vector<double> hfconst, huconst;
     std::vector<double4> hcconst;
     double *adjF = nullptr, *adjDF = nullptr, *adjDU = nullptr;   // FP64 F table, d/dtheta tables
+    // the adjoint's workspace (AdjointRun)
+    char *adj_ws = nullptr;
+    size_t adj_ws_bytes = 0;
+    char *adj_workspace(size_t bytes)
+    {
+        if (bytes > adj_ws_bytes) {
+            free_adj_workspace();
+            adj_ws = dalloc<char>(bytes);
+            adj_ws_bytes = bytes;
+        }
+        return adj_ws;
+    }
+    void free_adj_workspace()
+    {
+        dfree(adj_ws);
+        adj_ws = nullptr;
+        adj_ws_bytes = 0;
+    }
     // sm_param_derivative: the U table's d/dUmin and d/dUmax forms of one type pair, their
     // culling tables, and the CHAIN constant sets with (k_bond, k_bend) = (1, 0) and (0, 1)
     double *pdU = nullptr;
@@ -290,6 +308,7 @@ struct sm_ctx {
         dfree(reps); dfree(glob); dfree(fconstF); dfree(uconstD); dfree(fconstD); dfree(chainPerBead); dfree(chainList);
         dfree(gptr); dfree(gent); dfree(gconstD);
         dfree(cconstD); dfree(ebead); dfree(edelta); dfree(dres); dfree(dcounts); dfree(dpairs); dfree(dnp);
+        free_adj_workspace();
         dfree(adjF); dfree(adjDF); dfree(adjDU); dfree(pdU); dfree(pdTab); dfree(pdC);
         dfree(segB.tile); dfree(segB.rep_first); dfree(segB.tilesum); dfree(segB.ticket);
         dfree(segC.tile); dfree(segC.rep_first); dfree(segC.tilesum); dfree(segC.ticket);
@@ -563,6 +582,21 @@ struct sm_ctx {
         a.out = out;
         a.n = n;
         return a;
+    }
+    // out[2r + 0..1] += {U_pair, U_chain} of the resident order
+    void add_energies(double *out)
+    {
+        timed(K_GATHER, [&] {
+            launch_pair_gather(st, P, chunk, GATHER_U, sbeads, skey(), sidx(), cstart, cend, reps, fconstF, uconstD, ebead,
+                               nullptr, nullptr, nullptr, 0);
+        });
+        timed(K_SUMS, [&] {
+            launch_sums(st, SUM_ENERGY, sums(ebead, out));
+            if (gptr) {
+                launch_gen_energy(st, n, gen(), beads, reps, 0, ebead);
+                add_column(ebead, out + 1, 2);
+            }
+        });
     }
     void add_column(const double *x, double *out, int stride) const
     {
@@ -1814,37 +1848,167 @@ void upload_param_derivative_tables(sm_ctx *c, int a, int b)
     c->pd_b = b;
 }
 
-// device copy of the evolving state
-struct StateCopy {
-    Bead *beads = nullptr;
-    float4 *vel = nullptr, *acc = nullptr;
-    DevRep *reps = nullptr;
-    DevGlobal *glob = nullptr;
-    void alloc(const sm_ctx *c)
+// The adjoint's trajectory in a context: the solver's beads, velocities, replicas and step
+// counter stand aside (put back on every way out) while the steps run on copies in the
+// context's workspace, a buffer of beads per step, so a step's positions stay for the reverse
+// pass without a copy.
+//
+// What bounds a gradient is launches and recomputation: at 12k beads a step's kernels take 5
+// to 40 us each.  The reverse pass needs each step's positions only, 32 bytes a bead; the steps
+// since the last checkpoint are kept as the forward pass makes them, and checkpoints are set no
+// closer than kKeepBytes allows, so a trajectory that fits is run once and not twice.  With
+// the copies of each step's beads and replicas, the objective read back after each step and
+// the workspace allocated anew, 24 steps took 5.5 ms instead of 3.5.
+struct AdjointRun {
+    static constexpr size_t kKeepBytes = 256ull << 20;    // positions kept whatever checkpoint asks for
+    static constexpr size_t kIdleBytes = 512ull << 20;    // workspace a context holds between calls
+
+    sm_ctx *c;
+    const int n, nrep, S;   // beads, replicas, steps
+    int k, nseg;            // steps between checkpoints, segments
+    struct State {
+        Bead *beads;
+        float4 *vel, *acc;
+        DevRep *reps;
+        DevGlobal *glob;
+    };
+    State own;                        // the context's
+    Bead *own_alt;
+    bool own_fused;
+    std::vector<Bead *> x;            // x[t]: a segment's positions after its t-th step, before that step's box move
+    std::vector<State> checkpoint;    // states at steps k, 2k, ...; [0] at step 0
+    DevRep *pre = nullptr, *post = nullptr;   // a segment's box moves: the replicas before and after each
+    double *sums = nullptr;           // sums over the steps of U_pair, U_chain per replica
+    double4 *X = nullptr, *V = nullptr, *A = nullptr, *F = nullptr, *HV = nullptr;
+    double *g = nullptr, *gs = nullptr;
+
+    AdjointRun(sm_ctx *ctx, int steps, int want_k, bool grad) : c(ctx), n(ctx->n), nrep(ctx->nrep), S(steps)
     {
-        beads = dalloc<Bead>(c->n);
-        vel = dalloc<float4>(c->n);
-        acc = dalloc<float4>(c->n);
-        reps = dalloc<DevRep>(c->nrep);
-        glob = dalloc<DevGlobal>(1);
+        const long long fit = (long long)(kKeepBytes / (sizeof(Bead) * (size_t)n));
+        k = (int)std::min<long long>(S, std::max<long long>(want_k, fit));
+        nseg = (S + k - 1) / k;
+        own = State{c->beads, c->vel, c->acc, c->reps, c->glob};
+        own_alt = c->beads_alt;
+        own_fused = c->mc_fused;
+        // two passes over one list: the workspace's size, then its addresses
+        State cur{};
+        for (int pass = 0; pass < 2; pass++) {
+            size_t at = 0;
+            char *base = pass ? c->adj_workspace(words) : nullptr;
+            auto take = [&](auto *&p, size_t count) {
+                using T = std::remove_reference_t<decltype(*p)>;
+                p = reinterpret_cast<T *>(base + at);
+                at += (sizeof(T) * count + 255) / 256 * 256;
+            };
+            x.resize(k + 2);
+            for (Bead *&b : x) take(b, n);
+            auto state = [&](State &s, bool beads) {
+                if (beads) take(s.beads, n);
+                take(s.vel, n);
+                take(s.acc, n);
+                take(s.reps, nrep);
+                take(s.glob, 1);
+            };
+            state(cur, false);
+            checkpoint.resize(grad ? nseg - 1 : 0);
+            for (State &s : checkpoint) state(s, true);
+            take(pre, (size_t)(k / 8 + 1) * nrep);
+            take(post, (size_t)(k / 8 + 1) * nrep);
+            take(sums, 2 * (size_t)nrep);
+            if (grad) {
+                for (double4 **p : {&X, &V, &A, &F, &HV}) take(*p, n);
+                take(g, kNTheta * (size_t)n);
+                take(gs, kNTheta * (size_t)nrep);
+            }
+            words = at;
+        }
+        copy(x[0], own.beads, n);
+        copy(cur.vel, own.vel, n);
+        copy(cur.acc, own.acc, n);
+        copy(cur.reps, own.reps, nrep);
+        copy(cur.glob, own.glob, 1);
+        c->beads = x[0];
+        c->vel = cur.vel;
+        c->acc = cur.acc;
+        c->reps = cur.reps;
+        c->glob = cur.glob;
+        // the forward run and the recomputed segments take their box-move dU the same way
+        // (the gather after the kick), so they make the same decisions
+        c->mc_fused = false;
+        c->drop_graph();
     }
-    void release() { dfree(beads); dfree(vel); dfree(acc); dfree(reps); dfree(glob); }
-    void save(const sm_ctx *c)
+    ~AdjointRun()
     {
-        HIPCHK(hipMemcpyAsync(beads, c->beads, sizeof(Bead) * c->n, hipMemcpyDeviceToDevice, c->st));
-        HIPCHK(hipMemcpyAsync(vel, c->vel, sizeof(float4) * c->n, hipMemcpyDeviceToDevice, c->st));
-        HIPCHK(hipMemcpyAsync(acc, c->acc, sizeof(float4) * c->n, hipMemcpyDeviceToDevice, c->st));
-        HIPCHK(hipMemcpyAsync(reps, c->reps, sizeof(DevRep) * c->nrep, hipMemcpyDeviceToDevice, c->st));
-        HIPCHK(hipMemcpyAsync(glob, c->glob, sizeof(DevGlobal), hipMemcpyDeviceToDevice, c->st));
-    }
-    void load(sm_ctx *c) const
-    {
+        (void)hipStreamSynchronize(c->st);
+        c->beads = own.beads;
+        c->beads_alt = own_alt;
+        c->vel = own.vel;
+        c->acc = own.acc;
+        c->reps = own.reps;
+        c->glob = own.glob;
+        c->mc_fused = own_fused;
         c->forget_boxes();
-        HIPCHK(hipMemcpyAsync(c->beads, beads, sizeof(Bead) * c->n, hipMemcpyDeviceToDevice, c->st));
-        HIPCHK(hipMemcpyAsync(c->vel, vel, sizeof(float4) * c->n, hipMemcpyDeviceToDevice, c->st));
-        HIPCHK(hipMemcpyAsync(c->acc, acc, sizeof(float4) * c->n, hipMemcpyDeviceToDevice, c->st));
-        HIPCHK(hipMemcpyAsync(c->reps, reps, sizeof(DevRep) * c->nrep, hipMemcpyDeviceToDevice, c->st));
-        HIPCHK(hipMemcpyAsync(c->glob, glob, sizeof(DevGlobal), hipMemcpyDeviceToDevice, c->st));
+        if (c->adj_ws_bytes > kIdleBytes) c->free_adj_workspace();
+    }
+    AdjointRun(const AdjointRun &) = delete;
+    AdjointRun &operator=(const AdjointRun &) = delete;
+
+    // index among the segment's box moves of the one at step s
+    int move(int s, int s0) const { return s / 8 - s0 / 8 - 1; }
+
+    // Steps s0 + 1 .. s1 (a segment's, from its state with the positions in x[0]): the context
+    // is left in the state at s1.  objective: add each step's energies to the sums.
+    void steps(int s0, int s1, bool objective)
+    {
+        const size_t rn = nrep;
+        copy(x[1], x[0], n);
+        c->beads = x[1];
+        c->step_first(s0 + 1);
+        for (int s = s0 + 1; s <= s1; s++) {
+            const int t = s - s0;
+            const bool mc = c->mc_step(s);
+            c->sort_and_reorder();
+            c->pair_force();
+            if (objective) c->add_energies(sums);
+            if (!mc && s < s1) {
+                c->beads_alt = x[t + 1];
+                c->kick_first(s);   // x[t] stays as it is
+                continue;
+            }
+            c->bonded(KICK_STEP, nullptr);
+            if (mc) {
+                copy(pre + move(s, s0) * rn, c->reps, rn);
+                copy(x[t + 1], x[t], n);
+                c->beads = x[t + 1];
+                c->mc_move();
+                copy(post + move(s, s0) * rn, c->reps, rn);
+                if (s < s1) c->step_first(s + 1);
+            }
+        }
+    }
+    void save(const State &to)
+    {
+        copy(to.beads, c->beads, n);
+        copy(to.vel, c->vel, n);
+        copy(to.acc, c->acc, n);
+        copy(to.reps, c->reps, nrep);
+        copy(to.glob, c->glob, 1);
+    }
+    void load(const State &from)
+    {
+        copy(x[0], from.beads, n);
+        copy(c->vel, from.vel, n);
+        copy(c->acc, from.acc, n);
+        copy(c->reps, from.reps, nrep);
+        copy(c->glob, from.glob, 1);
+    }
+
+private:
+    size_t words = 0;   // the workspace's bytes
+    template <class T>
+    void copy(T *to, const T *from, size_t count)
+    {
+        if (to != from) HIPCHK(hipMemcpyAsync(to, from, sizeof(T) * count, hipMemcpyDeviceToDevice, c->st));
     }
 };
 
@@ -1913,123 +2077,75 @@ int sm_adjoint(sm_ctx *c, int32_t type_a, int32_t type_b, int32_t nsteps, int32_
         if (nsteps < 1 || checkpoint < 1 || checkpoint > nsteps) invalid("need 1 <= checkpoint <= nsteps");
         const int R = c->nrep;
         check_pair(c, type_a, type_b);
-        const int n = c->n, S = nsteps, k = checkpoint;
+        const int n = c->n, S = nsteps;
         const double obj = 1.0 / S;
         long long moves = 0;
         for (long long s = 1; s <= S; s++)
             if (c->mc_step(s)) moves++;
         c->ensure_capacity(moves);
         upload_adjoint_tables(c, type_a, type_b);
+        AdjointRun run(c, S, checkpoint, grad != nullptr);
+        const int k = run.k, nseg = run.nseg;
+        hipStream_t st = c->st;
 
-        const int ncp = (S + k - 1) / k;   // checkpoints at steps 0, k, 2k, ...
-        // the forward run and the recomputed segments take their box-move dU the same way
-        // (the gather after the kick), so they make the same decisions
-        struct KeepFused {
-            sm_ctx *c;
-            bool v;
-            ~KeepFused() { c->mc_fused = v; }
-        } keep{c, c->mc_fused};
-        c->mc_fused = false;
-        StateCopy entry;
-        std::vector<StateCopy> cps(ncp);
-        Bead *segBeads = nullptr;
-        DevRep *segPre = nullptr, *segPost = nullptr;
-        double4 *X = nullptr, *V = nullptr, *A = nullptr, *F = nullptr, *HV = nullptr;
-        double *g = nullptr, *gs = nullptr;
-        auto cleanup = [&] {
-            entry.release();
-            for (auto &cp : cps) cp.release();
-            dfree(segBeads); dfree(segPre); dfree(segPost);
-            dfree(X); dfree(V); dfree(A); dfree(F); dfree(HV); dfree(g); dfree(gs);
-        };
-        try {
-            hipStream_t st = c->st;
-            entry.alloc(c);
-            entry.save(c);
-            for (auto &cp : cps) cp.alloc(c);
-
-            // forward: init forces, then steps 1..S, J = mean of U after each kick
-            c->build(0, 0);
-            c->pair_force();
-            c->bonded(KICK_INIT, nullptr);
-            cps[0].save(c);
-            std::vector<double> Jsum(R, 0.0), m(3 * (size_t)R);
-            for (int s = 1; s <= S; s++) {
-                c->step_first(s);
-                c->step_finish(true, c->mc_step(s));
-                c->link.fetch(st, c->glob, c->meas_dev(), m.size(), m.data());
-                for (int r = 0; r < R; r++) Jsum[r] += m[3 * r] + m[3 * r + 1];
-                if (s % k == 0 && s / k < ncp) cps[s / k].save(c);
-            }
-            c->check_launch();
-            c->check_flags();
-            for (int r = 0; r < R; r++) J[r] = Jsum[r] * obj;
-
-            if (grad) {
-                segBeads = dalloc<Bead>((size_t)k * n);
-                segPre = dalloc<DevRep>((size_t)k * c->nrep);
-                segPost = dalloc<DevRep>((size_t)k * c->nrep);
-                X = dalloc<double4>(n); V = dalloc<double4>(n); A = dalloc<double4>(n);
-                F = dalloc<double4>(n); HV = dalloc<double4>(n);
-                g = dalloc<double>(kNTheta * (size_t)n);
-                gs = dalloc<double>(kNTheta * (size_t)R);
-                for (double4 *p : {X, V, A, F, HV}) HIPCHK(hipMemsetAsync(p, 0, sizeof(double4) * n, st));
-                HIPCHK(hipMemsetAsync(g, 0, sizeof(double) * kNTheta * n, st));
-                const AdjTables T{c->adjF, c->adjDF, c->adjDU};
-                auto adjoint_forces = [&](double o, int hv) {
-                    launch_adj_pair(st, c->P, c->sbeads, c->skey(), c->sidx(), c->cstart, c->cend, c->reps, T, A, F,
-                                    HV, g, o, hv);
-                    launch_adj_chain(st, c->P, c->beads, c->chainPerBead, c->cconstD, c->reps, A, F, HV, g, o, hv);
-                    if (c->gptr) launch_adj_gen(st, c->P, c->gen(), c->beads, c->reps, A, F, HV, hv);
-                };
-                for (int seg = ncp - 1; seg >= 0; seg--) {
-                    const int s0 = seg * k, s1 = std::min(S, s0 + k);
-                    // recompute the segment, keeping each step's positions before its MC move
-                    cps[seg].load(c);
-                    for (int s = s0 + 1; s <= s1; s++) {
-                        const int t = s - s0 - 1;
-                        c->step_first(s);
-                        c->step_finish(false, false);
-                        HIPCHK(hipMemcpyAsync(segBeads + (size_t)t * n, c->beads, sizeof(Bead) * n,
-                                              hipMemcpyDeviceToDevice, st));
-                        HIPCHK(hipMemcpyAsync(segPre + (size_t)t * c->nrep, c->reps, sizeof(DevRep) * c->nrep,
-                                              hipMemcpyDeviceToDevice, st));
-                        if (c->mc_step(s)) c->mc_move();
-                        HIPCHK(hipMemcpyAsync(segPost + (size_t)t * c->nrep, c->reps, sizeof(DevRep) * c->nrep,
-                                              hipMemcpyDeviceToDevice, st));
-                    }
-                    for (int s = s1; s > s0; s--) {
-                        const int t = s - s0 - 1;
-                        HIPCHK(hipMemcpyAsync(c->beads, segBeads + (size_t)t * n, sizeof(Bead) * n,
-                                              hipMemcpyDeviceToDevice, st));
-                        HIPCHK(hipMemcpyAsync(c->reps, segPre + (size_t)t * c->nrep, sizeof(DevRep) * c->nrep,
-                                              hipMemcpyDeviceToDevice, st));
-                        c->build(0, kStepKeep);
-                        adjoint_forces(obj, 1);
-                        launch_adj_step(st, c->P, c->beads, segPost + (size_t)t * c->nrep, c->mc_step(s) ? 1 : 0,
-                                        X, V, A, F, HV, obj, s - 1 >= 1 ? 1 : 0);
-                    }
-                }
-                // a_0 = F(x_0) + ...: its adjoint meets dF/dtheta at the initial positions
-                cps[0].load(c);
-                c->build(0, kStepKeep);
-                adjoint_forces(0.0, 0);
-                // per replica: grad[r * kNTheta + p]
-                static_assert(kNTheta == 4, "SUM_COLUMNS sums four");
-                launch_sums(st, SUM_COLUMNS, c->sums(g, gs));
-                c->check_launch();
-                HIPCHK(hipMemcpyAsync(grad, gs, sizeof(double) * kNTheta * R, hipMemcpyDeviceToHost, st));
-                HIPCHK(hipStreamSynchronize(st));
-            }
-            entry.load(c);
-            HIPCHK(hipStreamSynchronize(st));
-            c->drop_graph();
-        } catch (...) {
-            (void)hipStreamSynchronize(c->st);
-            cleanup();
-            throw;
+        // forward: init forces, then steps 1..S, J = mean of U after each kick
+        HIPCHK(hipMemsetAsync(run.sums, 0, sizeof(double) * 2 * (size_t)R, st));
+        c->build(0, 0);
+        c->pair_force();
+        c->bonded(KICK_INIT, nullptr);
+        for (int seg = 0; seg < nseg; seg++) {
+            if (seg + 1 < nseg && grad) run.save(run.checkpoint[seg]);
+            run.steps(seg * k, std::min(S, seg * k + k), true);
+            if (seg + 1 < nseg) HIPCHK(hipMemcpyAsync(run.x[0], c->beads, sizeof(Bead) * n, hipMemcpyDeviceToDevice, st));
+            if (seg + 1 < nseg) c->beads = run.x[0];
         }
-        cleanup();
+        c->check_launch();
+        std::vector<double> h(2 * (size_t)R);
+        c->check_bits(c->link.fetch(st, c->glob, run.sums, h.size(), h.data()));
+        for (int r = 0; r < R; r++) J[r] = (h[2 * r] + h[2 * r + 1]) * obj;
+        if (!grad) return;
+
+        const auto zero = [&](void *p, size_t bytes) { HIPCHK(hipMemsetAsync(p, 0, bytes, st)); };
+        for (double4 *p : {run.X, run.V, run.A}) zero(p, sizeof(double4) * n);
+        zero(run.g, sizeof(double) * kNTheta * n);
+        const AdjTables T{c->adjF, c->adjDF, c->adjDU};
+        auto adjoint_forces = [&](double o, int hv) {
+            launch_adj_pair(st, c->P, c->sbeads, c->skey(), c->sidx(), c->cstart, c->cend, c->reps, T, run.A, run.F,
+                            run.HV, run.g, o, hv);
+            launch_adj_chain(st, c->P, c->beads, c->chainPerBead, c->cconstD, c->reps, run.A, run.F, run.HV, run.g, o,
+                             hv);
+            if (c->gptr) launch_adj_gen(st, c->P, c->gen(), c->beads, c->reps, run.A, run.F, run.HV, hv);
+        };
+        for (int seg = nseg - 1; seg >= 0; seg--) {
+            const int s0 = seg * k, s1 = std::min(S, s0 + k);
+            if (seg + 1 < nseg) {   // the last segment's positions are there from the forward pass
+                run.load(run.checkpoint[seg]);
+                run.steps(s0, s1, false);
+            }
+            for (int s = s1; s > s0; s--) {
+                const bool mc = c->mc_step(s);
+                const DevRep *post = c->reps;
+                c->beads = run.x[s - s0];
+                if (mc) {
+                    const size_t m = (size_t)run.move(s, s0) * R;
+                    HIPCHK(hipMemcpyAsync(c->reps, run.pre + m, sizeof(DevRep) * R, hipMemcpyDeviceToDevice, st));
+                    post = run.post + m;
+                }
+                c->build(0, kStepKeep);
+                adjoint_forces(obj, 1);
+                launch_adj_step(st, c->P, c->beads, post, mc ? 1 : 0, run.X, run.V, run.A, run.F, run.HV, obj,
+                                s - 1 >= 1 ? 1 : 0);
+            }
+        }
+        // a_0 = F(x_0) + ...: its adjoint meets dF/dtheta at the initial positions
+        c->beads = run.x[0];
+        c->build(0, kStepKeep);
+        adjoint_forces(0.0, 0);
+        // per replica: grad[r * kNTheta + p]
+        static_assert(kNTheta == 4, "SUM_COLUMNS sums four");
+        launch_sums(st, SUM_COLUMNS, c->sums(run.g, run.gs));
+        c->check_launch();
+        (void)c->link.fetch(st, c->glob, run.gs, kNTheta * (size_t)R, grad);
     });
 }
 

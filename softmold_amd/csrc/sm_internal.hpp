@@ -111,6 +111,7 @@ enum SumKind : int {
     SUM_COLUMN,      // out[r * stride] (+)= sum of x over the beads
     SUM_COLUMNS,     // out[4r + 0..3] = sums of x, x + n, x + 2n, x + 3n over the beads
     SUM_MEASURE,     // out[3r + 0..2] = sum of x, CHAIN energy, kinetic energy
+    SUM_ENERGY,      // out[2r + 0..1] += sum of x, CHAIN energy
     SUM_DELTA,       // out[2r + 0..1] = sum of x, CHAIN U(old) - U(scaled)
     SUM_PARAM,       // out[4r + 0..3] = sums of x and y, CHAIN energies with cconst and cconst2
     SUM_HEADS,       // out[7r + 0..6] = head beads' x, y, z (imaged) and number, their centre

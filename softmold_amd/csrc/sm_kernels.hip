@@ -755,6 +755,8 @@ __device__ inline void store_sums(const SumArgs &a, int r, bool chain, const dou
             o[0] = v[0];
             o[2] = v[1];
         }
+    } else if (KIND == SUM_ENERGY) {
+        a.out[2 * (size_t)r + (chain ? 1 : 0)] += v[0];
     } else if (KIND == SUM_DELTA) {
         a.out[2 * (size_t)r + (chain ? 1 : 0)] = v[0];
     } else if (KIND == SUM_PARAM) {
@@ -789,7 +791,8 @@ template <int KIND>
 __global__ __launch_bounds__(kBlock) void k_sums(SumArgs a)
 {
     static_assert(kBlock == 4 * kWave, "block_sums adds four waves");
-    constexpr bool kChains = KIND == SUM_MEASURE || KIND == SUM_DELTA || KIND == SUM_PARAM;
+    constexpr bool kChains =
+        KIND == SUM_MEASURE || KIND == SUM_ENERGY || KIND == SUM_DELTA || KIND == SUM_PARAM;
     constexpr int C = KIND == SUM_COLUMNS || KIND == SUM_HEADS ? 4 : (KIND == SUM_MEASURE || KIND == SUM_PARAM ? 2 : 1);
     __shared__ double lds[kBlock / kWave][kSumCols];
     __shared__ bool last;
@@ -1040,6 +1043,7 @@ void launch_sums(hipStream_t st, SumKind kind, const SumArgs &a)
     case SUM_COLUMN: hipLaunchKernelGGL(k_sums<SUM_COLUMN>, beads, block, 0, st, a); break;
     case SUM_COLUMNS: hipLaunchKernelGGL(k_sums<SUM_COLUMNS>, beads, block, 0, st, a); break;
     case SUM_MEASURE: hipLaunchKernelGGL(k_sums<SUM_MEASURE>, both, block, 0, st, a); break;
+    case SUM_ENERGY: hipLaunchKernelGGL(k_sums<SUM_ENERGY>, both, block, 0, st, a); break;
     case SUM_DELTA: hipLaunchKernelGGL(k_sums<SUM_DELTA>, both, block, 0, st, a); break;
     case SUM_PARAM: hipLaunchKernelGGL(k_sums<SUM_PARAM>, both, block, 0, st, a); break;
     case SUM_HEADS: hipLaunchKernelGGL(k_sums<SUM_HEADS>, beads, block, 0, st, a); break;
