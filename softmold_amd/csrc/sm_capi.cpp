@@ -255,9 +255,11 @@ struct sm_ctx {
     int sorted_sel = 0;   // which sort buffer pair holds the sorted result
     // captured 8-step graph
     bool use_graph = false;
-    // one graph per sort-scratch parity at the start of the block (8 sorts return to it)
-    hipGraph_t graph[2] = {nullptr, nullptr};
-    hipGraphExec_t gexec[2] = {nullptr, nullptr};
+    // one graph per sort-scratch parity and bead buffer at the start of the block (8 sorts and 8
+    // changes of buffer return to them): [2 * parity + (beads is not beads_home)]
+    hipGraph_t graph[4] = {};
+    hipGraphExec_t gexec[4] = {};
+    const Bead *beads_home = nullptr;
     // profiling
     bool prof = false;
     struct Rec { int cls; hipEvent_t a, b; };
@@ -317,7 +319,7 @@ struct sm_ctx {
 
     void drop_graph()
     {
-        for (int p = 0; p < 2; p++) {
+        for (int p = 0; p < 4; p++) {
             if (gexec[p]) (void)hipGraphExecDestroy(gexec[p]);
             if (graph[p]) (void)hipGraphDestroy(graph[p]);
             gexec[p] = nullptr;
@@ -478,7 +480,8 @@ struct sm_ctx {
 
     // keys (optionally after Verlet::first) with the next sort's digit histograms, sort,
     // reorder + dense cell table (clearing the other sort scratch)
-    void first_and_keys(int integrate, long long step_set, bool for_sort = true)
+    // away: the beads go to the other buffer
+    void first_and_keys(int integrate, long long step_set, bool for_sort = true, bool away = false)
     {
         uint32_t *gh = for_sort ? hist[sort_parity] : nullptr;
         // keys computed twice before a sort (sm_step_first called twice): start over
@@ -487,12 +490,13 @@ struct sm_ctx {
         const int passes = sort_passes(sort_bits);
         timed(K_FIRST, [&] {
             if (for_sort)
-                launch_first(st, P, beads, vel, acc, reps, glob, key_out(), idx_out(), integrate, step_set, gh, passes,
-                             move_book(), win_keys(sort_parity));
+                launch_first(st, P, beads, away ? beads_alt : beads, vel, acc, reps, glob, key_out(), idx_out(),
+                             integrate, step_set, gh, passes, move_book(), win_keys(sort_parity));
             else   // keys only (no sort follows): into the mover buffer, which no sort state holds
-                launch_first(st, P, beads, vel, acc, reps, glob, k0, nullptr, integrate, step_set, nullptr, passes,
+                launch_first(st, P, beads, beads, vel, acc, reps, glob, k0, nullptr, integrate, step_set, nullptr, passes,
                              MoveBook{nullptr, nullptr});
         });
+        if (away) std::swap(beads, beads_alt);
     }
     void sort_and_reorder()
     {
@@ -676,17 +680,17 @@ struct sm_ctx {
 
     // Step s's bonded + Langevin forces and second half kick, with step s + 1's first half,
     // keys and digit histograms, as one kernel (same arithmetic as bonded() then
-    // step_first(s + 1)); the new positions land in the other bead buffer.
-    void kick_first(long long s)
+    // step_first(s + 1)); the new positions land in the other bead buffer.  from_base: s counts
+    // from the captured block's start.
+    void kick_first(long long s, bool from_base = false)
     {
-        if (gexec[0] || gexec[1]) drop_graph();   // captured graphs hold the bead buffer
         uint32_t *gh = hist[sort_parity];
         if (hist_pending) restart_hist(gh);
         hist_pending = true;
         const int passes = sort_passes(sort_bits);
         timed(K_KICK_FIRST, [&] {
             launch_kick_first(st, P, beads, beads_alt, chainPerBead, cconstD, gen(), fpair, vel, reps, glob, s,
-                              key_out(), idx_out(), gh, passes, move_book(), win_keys(sort_parity));
+                              from_base, key_out(), idx_out(), gh, passes, move_book(), win_keys(sort_parity));
         });
         std::swap(beads, beads_alt);
     }
@@ -708,34 +712,70 @@ struct sm_ctx {
 
     // Steps s .. s+7 with s % 8 == 1 as one graph: the step counter advances on the
     // device, so the same graph serves every such block; the MC move (if any replica
-    // has one) falls on the block's last step.
+    // has one) falls on the block's last step.  The kernels are run()'s: seven fused kicks, and
+    // the block's first half step moves the beads to the other buffer too, so that the block
+    // ends in the buffer it began in and the next replays the same graph.  16 steps of the
+    // 12k-bead bilayer with their download took 831 us with the halves apart, 793 now.
     void graph_block(long long s)
     {
         if (sort_mode == 1 && !order_valid) {
             // the graph would replay a first sort without a previous order: step this block
             // eagerly, after which the order is there to capture against
-            for (int k = 0; k < 8; k++) eager_step(s + k);
+            eager(s, s + 8);
             return;
         }
-        const int p = sort_parity;   // 8 sorts later the parity is p again
-        if (!gexec[p]) {
+        if (hist_pending) {   // keys computed but not sorted: the graph's are the first
+            restart_hist(hist[sort_parity]);
+            hist_pending = false;
+        }
+        const int p = sort_parity, q = 2 * p + (beads != beads_home ? 1 : 0);
+        if (!gexec[q]) {
             HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
+            first_and_keys(1, kStepAdvance, true, true);
             for (int k = 0; k < 8; k++) {
-                step_first(kStepAdvance);
-                step_finish(false, k == 7 && any_mc);
+                const bool mc = k == 7 && any_mc;
+                sort_and_reorder();
+                pair_step(mc);
+                if (k < 7) {
+                    kick_first(k + 1, true);
+                    continue;
+                }
+                bonded(KICK_STEP, nullptr);
+                if (mc) mc_finish();
             }
-            hipError_t e = hipStreamEndCapture(st, &graph[p]);
+            hipError_t e = hipStreamEndCapture(st, &graph[q]);
             if (e != hipSuccess) {
-                graph[p] = nullptr;
+                graph[q] = nullptr;
                 HIPCHK(e);
             }
-            HIPCHK(hipGraphInstantiate(&gexec[p], graph[p], nullptr, nullptr, 0));
+            HIPCHK(hipGraphInstantiate(&gexec[q], graph[q], nullptr, nullptr, 0));
+            if (any_mc) moves_since--;   // capture only recorded the move
         }
-        sort_parity = p;   // capture only recorded the toggles
+        sort_parity = p;   // and the toggles
         if (any_mc) moves_since++;
         // the block advances from step s - 1
         launch_set_step(st, glob, s - 1);
-        HIPCHK(hipGraphLaunch(gexec[p], st));
+        HIPCHK(hipGraphLaunch(gexec[q], st));
+    }
+
+    // Steps [s, end): one without a box move ends in the fused kernel that also does the next
+    // step's first half; a box-move step and the last step end unfused.
+    void eager(long long s, long long end)
+    {
+        bool first_done = false;
+        for (; s < end; s++) {
+            if (!first_done) step_first(s);
+            const bool mc = mc_step(s);
+            sort_and_reorder();
+            pair_step(mc);
+            first_done = !mc && s + 1 < end;
+            if (first_done) {
+                kick_first(s);
+                continue;
+            }
+            bonded(KICK_STEP, nullptr);
+            if (mc) mc_finish();
+        }
     }
 
     void run(long long first, long long nsteps)
@@ -747,31 +787,11 @@ struct sm_ctx {
         long long s = first;
         const long long end = first + nsteps;
         if (use_graph && !prof) {
-            while (s < end && s % 8 != 1) eager_step(s++);
-            while (end - s >= 8) {
-                graph_block(s);
-                s += 8;
-            }
-            while (s < end) eager_step(s++);
-            return;
+            const long long lead = std::min(end, s + (9 - s % 8) % 8);   // up to the next s % 8 == 1
+            eager(s, lead);
+            for (s = lead; end - s >= 8; s += 8) graph_block(s);
         }
-        // eager: a step without a box move ends in the fused kernel that also does the next
-        // step's first half; a box-move step and the run's last step end unfused
-        bool first_done = false;
-        for (; s < end; s++) {
-            if (!first_done) step_first(s);
-            const bool mc = mc_step(s);
-            sort_and_reorder();
-            pair_step(mc);
-            if (!mc && s + 1 < end) {
-                kick_first(s);
-                first_done = true;
-            } else {
-                bonded(KICK_STEP, nullptr);
-                if (mc) mc_finish();
-                first_done = false;
-            }
-        }
+        eager(s, end);
     }
 };
 
@@ -1028,6 +1048,7 @@ sm_ctx *create(const sm_system *s, int nrep)
         c->beads = dalloc<Bead>(n);
         c->sbeads = dalloc<Bead>(n);
         c->beads_alt = dalloc<Bead>(n);
+        c->beads_home = c->beads;
         c->vel = dalloc<float4>(n);
         c->acc = dalloc<float4>(n);
         c->fpair = dalloc<float4>(n);

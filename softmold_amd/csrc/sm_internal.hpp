@@ -71,6 +71,7 @@ struct DevGlobal {
     int flags;
     int pad;
     long long step;            // step index of the step in progress (Philox counter)
+    long long base;            // the step before the captured block in progress
 };
 
 enum : int { FLAG_BAD_POSITION = 1, FLAG_CELL_OVERFLOW = 2, FLAG_SORT_TIMEOUT = 4, FLAG_SORT_COUNT = 8 };
@@ -183,7 +184,8 @@ size_t sortw_words(int n, bool window);
 uint32_t *win_scratch(uint32_t *sort_scratch, int n);   // where it starts in a sort's scratch
 WinBook win_book(uint32_t *sort_scratch, int n, const uint32_t *desc, uint32_t *counts, uint32_t cells);
 bool sortw_fits(int n);   // the tiles of n keys are few enough for the window build's launches
-void launch_first(hipStream_t st, const Params &P, Bead *beads, float4 *vel, const float4 *acc, const DevRep *reps,
+// out: where the beads go (beads itself, or another buffer)
+void launch_first(hipStream_t st, const Params &P, const Bead *beads, Bead *out, float4 *vel, const float4 *acc, const DevRep *reps,
                   DevGlobal *glob, uint32_t *key, uint32_t *idx, int integrate, long long step_set, uint32_t *ghist,
                   int passes, const MoveBook &book, const WinBook &wb = WinBook{});
 // also zeroes clear[0 .. clear_words) (the next sort's scratch)
@@ -225,7 +227,7 @@ enum : int { KICK_STEP = 0, KICK_INIT = 1, KICK_NONE = 2 };
 // histograms of step + 1 (positions written to beads_out; the device step becomes step + 1)
 void launch_kick_first(hipStream_t st, const Params &P, const Bead *beads, Bead *beads_out, const int2 *chain,
                        const double4 *cconst, const GenTables &gen, const float4 *fpair, float4 *vel,
-                       const DevRep *reps, DevGlobal *glob, long long step, uint32_t *key, uint32_t *idx,
+                       const DevRep *reps, DevGlobal *glob, long long step, bool from_base, uint32_t *key, uint32_t *idx,
                        uint32_t *ghist, int passes, const MoveBook &book,
                        const WinBook &wb = WinBook{});
 void launch_second(hipStream_t st, int n, const Bead *beads, const float4 *acc, float4 *vel, float dt);

@@ -98,7 +98,7 @@ __device__ inline uint32_t bead_key(const Bead &b, const DevRep &R, DevGlobal *_
 }
 
 // Verlet::first of bead i and its cell key
-__device__ inline uint32_t first_one(int i, Bead *__restrict__ beads, float4 *__restrict__ vel,
+__device__ inline uint32_t first_one(int i, const Bead *beads, Bead *out, float4 *__restrict__ vel,
                                      const float4 *__restrict__ acc, const DevRep *__restrict__ reps,
                                      DevGlobal *__restrict__ glob, float halfdt, double dt, int integrate, int &cx,
                                      int &cy, int &cz)
@@ -110,8 +110,9 @@ __device__ inline uint32_t first_one(int i, Bead *__restrict__ beads, float4 *__
         half_kick(v, acc[i], halfdt);
         drift_wrap(b, v, dt, R.L[0], R.L[1], R.L[2]);
         vel[i] = v;
-        beads[i] = b;
+        if (out == beads) out[i] = b;
     }
+    if (out != beads) out[i] = b;
     return bead_key(b, R, glob, cx, cy, cz);
 }
 
@@ -129,7 +130,7 @@ __device__ inline void flush_moves(const MoveBook &book, int nmoved)
     if (book.cnt_b && threadIdx.x == 0) book.cnt_b[blockIdx.x] = (uint32_t)nmoved;
 }
 
-__global__ __launch_bounds__(kBlock) void k_first(int n, Bead *__restrict__ beads, float4 *__restrict__ vel,
+__global__ __launch_bounds__(kBlock) void k_first(int n, const Bead *beads, Bead *out, float4 *__restrict__ vel,
                                                   const float4 *__restrict__ acc, const DevRep *__restrict__ reps,
                                                   DevGlobal *__restrict__ glob, uint32_t *__restrict__ key,
                                                   uint32_t *__restrict__ idx, float halfdt, double dt, int integrate,
@@ -152,7 +153,7 @@ __global__ __launch_bounds__(kBlock) void k_first(int n, Bead *__restrict__ bead
     }
     uint32_t k = 0u, rank = (uint32_t)i;
     int cx = 0, cy = 0, cz = 0;
-    if (i < n) k = first_one(i, beads, vel, acc, reps, glob, halfdt, dt, integrate, cx, cy, cz);
+    if (i < n) k = first_one(i, beads, out, vel, acc, reps, glob, halfdt, dt, integrate, cx, cy, cz);
     if (ghist && win) {
         k = win_key_end(wb, w, hs, k, cx, cy, cz, i < n, rank);
     } else if (ghist) {
@@ -464,7 +465,7 @@ __global__ __launch_bounds__(kBlock) void k_kick_first(int n, const Bead *__rest
                                                        const float4 *__restrict__ fpair, float4 *__restrict__ vel,
                                                        const DevRep *__restrict__ reps,
                                                        DevGlobal *__restrict__ glob, float halfdt, double dt,
-                                                       long long step, uint32_t *__restrict__ key,
+                                                       long long step, int from_base, uint32_t *__restrict__ key,
                                                        uint32_t *__restrict__ idx, uint32_t *__restrict__ ghist,
                                                        int passes, MoveBook book, WinBook wb)
 {
@@ -473,6 +474,7 @@ __global__ __launch_bounds__(kBlock) void k_kick_first(int n, const Bead *__rest
     const int i = blockIdx.x * kBlock + threadIdx.x;
     WinDesc w{};
     if (WIN && wb.desc) w = load_win(wb.desc);
+    if (from_base) step += glob->base;   // in a captured block, whose steps count from there
     if (i == 0) glob->step = step + 1;
     if (WIN)
         hs[threadIdx.x] = 0u;
@@ -919,7 +921,7 @@ __global__ __launch_bounds__(kBlock) void k_rescale(int n, Bead *__restrict__ be
     beads[i] = b;
 }
 
-__global__ void k_set_step(DevGlobal *glob, long long step) { glob->step = step; }
+__global__ void k_set_step(DevGlobal *glob, long long step) { glob->step = glob->base = step; }
 
 __global__ __launch_bounds__(kBlock) void k_fill_u32(uint32_t *__restrict__ p, size_t count, uint32_t value)
 {
@@ -975,12 +977,12 @@ inline int blocks(long long n) { return (int)((n + kBlock - 1) / kBlock); }
 // ---------------------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------------------
-void launch_first(hipStream_t st, const Params &P, Bead *beads, float4 *vel, const float4 *acc, const DevRep *reps,
+void launch_first(hipStream_t st, const Params &P, const Bead *beads, Bead *out, float4 *vel, const float4 *acc, const DevRep *reps,
                   DevGlobal *glob, uint32_t *key, uint32_t *idx, int integrate, long long step_set, uint32_t *ghist,
                   int passes, const MoveBook &book, const WinBook &wb)
 {
-    hipLaunchKernelGGL(k_first, dim3(blocks(P.n)), dim3(kBlock), 0, st, P.n, beads, vel, acc, reps, glob, key, idx,
-                       (float)(0.5 * P.dt), P.dt, integrate, step_set, ghist, passes, book, wb);
+    hipLaunchKernelGGL(k_first, dim3(blocks(P.n)), dim3(kBlock), 0, st, P.n, beads, out, vel, acc, reps, glob, key,
+                       idx, (float)(0.5 * P.dt), P.dt, integrate, step_set, ghist, passes, book, wb);
 }
 
 void launch_reorder(hipStream_t st, int n, const uint32_t *skey, const uint32_t *sidx, const Bead *beads,
@@ -1009,25 +1011,25 @@ void launch_bonded_kick(hipStream_t st, const Params &P, const Bead *beads, cons
 
 void launch_kick_first(hipStream_t st, const Params &P, const Bead *beads, Bead *beads_out, const int2 *chain,
                        const double4 *cconst, const GenTables &gen, const float4 *fpair, float4 *vel,
-                       const DevRep *reps, DevGlobal *glob, long long step, uint32_t *key, uint32_t *idx,
+                       const DevRep *reps, DevGlobal *glob, long long step, bool from_base, uint32_t *key, uint32_t *idx,
                        uint32_t *ghist, int passes, const MoveBook &book, const WinBook &wb)
 {
     const float halfdt = (float)(P.dt * 0.5);
     if (P.nrep > 1 && wb.counts)
         hipLaunchKernelGGL((k_kick_first<false, true>), dim3(blocks(P.n)), dim3(kBlock), 0, st, P.n, beads, beads_out,
-                           chain, cconst, gen, fpair, vel, reps, glob, halfdt, P.dt, step, key, idx, ghist, passes,
+                           chain, cconst, gen, fpair, vel, reps, glob, halfdt, P.dt, step, from_base ? 1 : 0, key, idx, ghist, passes,
                            book, wb);
     else if (wb.counts)
         hipLaunchKernelGGL((k_kick_first<true, true>), dim3(blocks(P.n)), dim3(kBlock), 0, st, P.n, beads, beads_out,
-                           chain, cconst, gen, fpair, vel, reps, glob, halfdt, P.dt, step, key, idx, ghist,
+                           chain, cconst, gen, fpair, vel, reps, glob, halfdt, P.dt, step, from_base ? 1 : 0, key, idx, ghist,
                            passes, book, wb);
     else if (P.nrep == 1)
         hipLaunchKernelGGL((k_kick_first<true, false>), dim3(blocks(P.n)), dim3(kBlock), 0, st, P.n, beads,
-                           beads_out, chain, cconst, gen, fpair, vel, reps, glob, halfdt, P.dt, step, key, idx,
+                           beads_out, chain, cconst, gen, fpair, vel, reps, glob, halfdt, P.dt, step, from_base ? 1 : 0, key, idx,
                            ghist, passes, book, wb);
     else
         hipLaunchKernelGGL((k_kick_first<false, false>), dim3(blocks(P.n)), dim3(kBlock), 0, st, P.n, beads,
-                           beads_out, chain, cconst, gen, fpair, vel, reps, glob, halfdt, P.dt, step, key, idx,
+                           beads_out, chain, cconst, gen, fpair, vel, reps, glob, halfdt, P.dt, step, from_base ? 1 : 0, key, idx,
                            ghist, passes, book, wb);
 }
 
