@@ -33,6 +33,14 @@
 // the pair in the 13-cell half shell (cellOpt.h:715) minus the imaged other.  The energy
 // gathers (U, dU) stage only the home cell and its forward half shell and use the same
 // quarter-cell culling, with the reach radius widened by the trial scale for dU.
+//
+// What bounds it: vector instructions.  At 240k beads and 16 waves a CU the force issues 2270
+// of them per occupied cell, 78 % of the issue slots (92 us); with 12 waves a CU it takes 113.
+// So instructions are what counts outside the candidate loop (40 a candidate): the quarters
+// are taken from the comparisons' lane masks, the lists hold byte offsets, scans run in DPP
+// steps, the small divisions by reciprocals, a chunk without a cell leaves at once, and the
+// tables take the LDS of the types there are.  Together 95.7 -> 92 us for that force, the
+// force with dU 195 -> 178, U 87.6 -> 84.4; 3M-bead bilayer 955 -> 931 and 1705 -> 1555.
 #include "sm_internal.hpp"
 
 namespace smdev {
@@ -49,16 +57,6 @@ struct __align__(16) Cand {
     int t, c;
 };
 
-__device__ inline int wave_incl_scan(int v, int lane)
-{
-#pragma unroll
-    for (int off = 1; off < kWave; off <<= 1) {
-        const int t = __shfl_up(v, off);
-        if (lane >= off) v += t;
-    }
-    return v;
-}
-
 // Inclusive prefix maximum over the wave of non-negative values, in DPP steps: shifts by
 // 1, 2, 4, 8 within each 16-lane row, then row 0's and row 2's last lanes into rows 1 and
 // 3, then lane 31 into rows 2 and 3.  Lanes a step does not reach keep their value.
@@ -71,6 +69,24 @@ __device__ inline int wave_max_scan(int v)
     v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false));  // row_bcast:15
     v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false));  // row_bcast:31
     return v;
+}
+
+// Inclusive prefix sum over the wave, in the same steps.
+__device__ inline int wave_sum_scan(int v)
+{
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
+    return v;
+}
+
+// base + the number of lanes of m below this one
+__device__ inline int lanes_before(unsigned long long m, int base)
+{
+    return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, (uint32_t)base));
 }
 
 // Image shift of one stencil cell: the box length added to a candidate's coordinates
@@ -274,9 +290,10 @@ __device__ inline void force_term(const Bead &hb, const Cand &q, bool other, dou
     const double dyd = hb.y - q.y;
     const double dzd = hb.z - q.z;
     const double r2 = sq3(dxd, dyd, dzd);
-    // the type bound keeps the type's LDS read ahead of the branch, with the position
-    if (r2 < cut2 && other && (unsigned)q.t < (unsigned)kMaxTypes)
-        force_law(dxd, dyd, dzd, r2, C8 + 2 * q.t, fx, fy, fz);
+    // the empty asm keeps the type's LDS read ahead of the branch, with the position
+    int t = q.t;
+    asm volatile("" : "+v"(t));
+    if (r2 < cut2 && other) force_law(dxd, dyd, dzd, r2, C8 + 2 * t, fx, fy, fz);
 }
 
 // Which side of a pair the reference's half-shell traversal makes its first particle p1,
@@ -366,8 +383,11 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
     constexpr int kMaxC = (k2P || kE || kFDU) ? 128 : 192;
     constexpr int kStageIters = kMaxC / kWave;
     static_assert(kMaxC % kWave == 0, "staging rounds cover whole waves");
-    __shared__ float4 sC8[kF ? 2 * kMaxTypes * kMaxTypes : 1];   // rows padded to 8 floats
-    __shared__ double sCd[(kF && !kFDU) ? 1 : 6 * kMaxTypes * kMaxTypes];
+    // the constant rows, sized by the types there are (tables_bytes): six types leave room for
+    // 16 waves a CU where the bound of eight left 14 or 15
+    extern __shared__ float4 sTables[];
+    float4 *const sC8 = sTables;   // rows padded to 8 floats
+    double *const sCd = reinterpret_cast<double *>(sTables + (kF ? 2 * nT * nT : 0));
     __shared__ Cand sCand[kWaves][kMaxC];   // staged candidates of the current pass
     __shared__ float4 sRel[k2P ? kWaves : 1][k2P ? kMaxC : 1];
     __shared__ uint8_t sList[k2P ? kWaves : 1][k2P ? kList : 1][kWave];   // per-lane hit lists, lane-minor
@@ -377,10 +397,11 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
     __shared__ int sDelta[kWaves][27];
     // per pass: the stencil cell at each cell's first staged slot (0 elsewhere), then, in
     // the same memory once the slots are staged, the candidate lists of the four quarters
-    // of the home cell packed one after another (list q at q * kMaxC) and padded so the
+    // of the home cell (byte offsets into sCand) packed one after another (list q at
+    // q * kMaxC) and padded so the
     // force loop's reads one trip ahead (at most 3 x 64 entries past the end of a list)
     // stay inside the array
-    constexpr int kListBytes = kCull ? 4 * kMaxC + 3 * kWave : kMaxC;
+    constexpr int kListBytes = kCull ? 2 * (4 * kMaxC + 3 * kWave) : kMaxC;
     static_assert(kListBytes % 4 == 0, "the map is cleared in 32-bit words");
     __shared__ uint32_t sLists[kWaves][kListBytes / 4];
 
@@ -405,7 +426,8 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
         if (a + lane > 0) kp = skey[a + lane - 1];
     }
     // the constant tables: every load first (indices clamped in bounds, so no branch holds
-    // one back), then the LDS stores, so the staging costs one memory trip
+    // one back), then the LDS stores, so the staging costs one memory trip; a chunk inside
+    // one cell's run owns nothing and leaves before the tables arrive
     constexpr int kThreads = kWaves * kWave;
     constexpr int kC8Per = (2 * kMaxTypes * kMaxTypes + kThreads - 1) / kThreads;
     constexpr int kCdPer = (6 * kMaxTypes * kMaxTypes + kThreads - 1) / kThreads;
@@ -432,23 +454,22 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
         rf = tab[8 * nT * nT + treach];
         re = tab[8 * nT * nT + kMaxTypes + treach];
     }
-    // stored whole (entries past the table hold copies of its last one and are never read),
-    // so that no branch sinks a load down to its store
-    static_assert(kC8Per * kThreads <= 2 * kMaxTypes * kMaxTypes && kCdPer * kThreads <= 6 * kMaxTypes * kMaxTypes,
-                  "the tables are stored whole");
+    static_assert(kWaves == 1, "a wave may leave by itself");
+    if (chunk <= kWave && !__any(a + lane < aend && (a + lane == 0 || kp != kc))) return;
     if (kF) {
 #pragma unroll
-        for (int k = 0; k < kC8Per; k++) sC8[threadIdx.x + k * kThreads] = c8[k];
+        for (int k = 0; k < kC8Per; k++)
+            if ((int)threadIdx.x + k * kThreads < 2 * nT * nT) sC8[threadIdx.x + k * kThreads] = c8[k];
     }
     if (!kF || kFDU) {
 #pragma unroll
-        for (int k = 0; k < kCdPer; k++) sCd[threadIdx.x + k * kThreads] = cd[k];
+        for (int k = 0; k < kCdPer; k++)
+            if ((int)threadIdx.x + k * kThreads < 6 * nT * nT) sCd[threadIdx.x + k * kThreads] = cd[k];
     }
     // every thread stores (those past nT the last type's value again, the same bits)
     if (kCull) sReach2[treach] = kFDU ? fmaxf(rf, re) : (kE ? re : rf);
     __syncthreads();
 
-    const unsigned long long lanes_lt = lane ? (~0ull >> (64 - lane)) : 0ull;
     constexpr uint32_t fwd = forward_mask();
     Cand *Cw = sCand[wave];
     float4 *Rw = sRel[k2P ? wave : 0];
@@ -519,7 +540,7 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
                 ncnt = ok ? c1 - c0 : 0;
             }
             // 2. layout of the candidates
-            const int incl = wave_incl_scan(ncnt, lane);
+            const int incl = wave_sum_scan(ncnt);
             const int excl = incl - ncnt;
             const int total = __builtin_amdgcn_readlane(incl, 26);
             const int selfOff = __builtin_amdgcn_readlane(excl, 13);
@@ -532,11 +553,18 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
                 sDelta[wave][lane] = nst - excl;
             }
             uint8_t *mapW = reinterpret_cast<uint8_t *>(sLists[wave]);   // map, then lists
+            uint16_t *listW = reinterpret_cast<uint16_t *>(sLists[wave]);
+            const auto cand_at = [&](int offset) {
+                return load_cand(reinterpret_cast<const Cand *>(reinterpret_cast<const char *>(Cw) + offset));
+            };
 
             for (int h0 = 0; h0 < nh; h0 += kWave) {
                 const int H = min(kWave, nh - h0);
-                const int tpp = kWave / H;
-                const int hi = lane / tpp;
+                // 64 / H and lane / tpp by FP32 reciprocals: H, tpp and lane are at most 64, so a
+                // quotient is at least 1/64 from the next integer, or on one, and the offsets
+                // settle it
+                const int tpp = (int)fmaf((float)kWave, __builtin_amdgcn_rcpf((float)H), 0.005f);
+                const int hi = (int)(((float)lane + 0.5f) * __builtin_amdgcn_rcpf((float)tpp));
                 const int sub = lane - hi * tpp;
                 const bool act = hi < H;
                 // the home particle and its index: loaded for every lane (an idle lane takes the
@@ -577,12 +605,13 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
                     Bead qb[kStageIters];
 #pragma unroll
                     for (int it = 0; it < kStageIters; it++)
-                        if (it < iters && src[it] >= 0) qb[it] = sb[src[it]];
-                    int reach[kStageIters];
+                        if (it < iters) qb[it] = sb[max(src[it], 0)];
+                    bool near[kStageIters][4];   // the quarters of the home cell it can reach
 #pragma unroll
                     for (int it = 0; it < kStageIters; it++) {
-                        reach[it] = 0;
-                        if (it >= iters || src[it] < 0) continue;
+#pragma unroll
+                        for (int q = 0; q < 4; q++) near[it][q] = false;
+                        if (it >= iters) continue;
                         const int c = cel[it];
                         Cand cd;
                         const Shift sh = ShW[c];
@@ -594,7 +623,7 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
                         if (kCull) {
                             // which quarters of the home cell (x below / above the centre,
                             // times y below / above) the candidate can reach: box distance
-                            // below the reach radius; bit qx + 2 qy
+                            // below the reach radius; quarter qx + 2 qy
                             const float rx = (float)(ix - ox0), ry = (float)(iy - oy0), rz = (float)(iz - oz0);
                             const float gz = fmaxf(fabsf(rz) - hcz, 0.f);
                             const float gx0 = fmaxf(fmaxf(rx, -hcx - rx), 0.f), gx1 = fmaxf(fmaxf(-rx, rx - hcx), 0.f);
@@ -602,9 +631,12 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
                             const float z2 = gz * gz;
                             const float a0 = fmaf(gx0, gx0, z2), a1 = fmaf(gx1, gx1, z2);
                             const float b0 = gy0 * gy0, b1 = gy1 * gy1;
-                            const float r2max = sReach2[qb[it].type] * reachS;
-                            reach[it] = (a0 + b0 < r2max ? 1 : 0) | (a1 + b0 < r2max ? 2 : 0) |
-                                        (a0 + b1 < r2max ? 4 : 0) | (a1 + b1 < r2max ? 8 : 0);
+                            const float r2max = src[it] >= 0 ? sReach2[qb[it].type] * reachS : -1.f;
+                            const float c0 = r2max - b0, c1 = r2max - b1;
+                            near[it][0] = a0 < c0;
+                            near[it][1] = a1 < c0;
+                            near[it][2] = a0 < c1;
+                            near[it][3] = a1 < c1;
                         }
                         // forces and energy gathers stage imaged positions (q + shift, the
                         // one rounding the reference's minImg makes of the same operands);
@@ -631,9 +663,10 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
                             if (it >= iters) break;
 #pragma unroll
                             for (int q = 0; q < 4; q++) {
-                                const bool r = (reach[it] >> q) & 1;
-                                const unsigned long long b = __ballot(r);
-                                if (r) mapW[q * kMaxC + nq[q] + __popcll(b & lanes_lt)] = (uint8_t)(lane + it * kWave);
+                                const unsigned long long b = __ballot(near[it][q]);
+                                if (near[it][q])
+                                    listW[lanes_before(b, q * kMaxC + nq[q])] =
+                                        (uint16_t)((lane + it * kWave) * (int)sizeof(Cand));
                                 nq[q] += __popcll(b);
                             }
                         }
@@ -651,7 +684,7 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
                         // (forward half shell; the higher slot within the home cell), the
                         // FP64 dU term with the row of the particle the reference makes first
                         const int quad = (hfx >= 0.f ? 1 : 0) + (hfy >= 0.f ? 2 : 0);
-                        const uint8_t *lst = mapW + quad * kMaxC;
+                        const uint16_t *lst = listW + quad * kMaxC;
                         const int nl = quad == 0 ? nq[0] : (quad == 1 ? nq[1] : (quad == 2 ? nq[2] : nq[3]));
                         // the next entry is read one iteration ahead (entries past nl fall in
                         // the next list or the padding and are never used)
@@ -659,7 +692,7 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
                         for (int jj = sub; jj < nl; jj += tpp) {
                             const int i0 = inext;
                             inext = lst[jj + tpp];
-                            const Cand q = load_cand(Cw + i0);
+                            const Cand q = cand_at(i0);
                             const int tq = q.t & 0xff, c = q.t >> 8;
                             const double dxd = hb.x - q.x, dyd = hb.y - q.y, dzd = hb.z - q.z;
                             const double r2 = sq3(dxd, dyd, dzd);
@@ -680,18 +713,18 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
                         const float4 *C8 = sC8 + 2 * hb.type * nT;
                         const double *Cd = sCd + 6 * hb.type * nT;
                         const int quad = (hfx >= 0.f ? 1 : 0) + (hfy >= 0.f ? 2 : 0);
-                        const uint8_t *lst = mapW + quad * kMaxC;
+                        const uint16_t *lst = listW + quad * kMaxC;
                         const int nl = quad == 0 ? nq[0] : (quad == 1 ? nq[1] : (quad == 2 ? nq[2] : nq[3]));
                         // the next trip's list entries are read one trip ahead (entries past
                         // nl fall in the next list or the padding and are never used)
                         int j = sub;
-                        const uint8_t *lp = lst + sub;
+                        const uint16_t *lp = lst + sub;
                         int i0 = lp[0], i1 = lp[tpp];
                         for (; j + tpp < nl; j += 2 * tpp) {
                             lp += 2 * tpp;
                             const int n0 = lp[0], n1 = lp[tpp];
-                            const Cand q0 = load_cand(Cw + i0);
-                            const Cand q1 = load_cand(Cw + i1);
+                            const Cand q0 = cand_at(i0);
+                            const Cand q1 = cand_at(i1);
                             if (kFC) {
                                 count_term<ASYM>(hb, q0, q0.c != hslot, cut2, Cd, sCd, nT, me, sidx, cnt);
                                 count_term<ASYM>(hb, q1, q1.c != hslot, cut2, Cd, sCd, nT, me, sidx, cnt);
@@ -706,7 +739,7 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
                             i1 = n1;
                         }
                         if (j < nl) {
-                            const Cand q0 = load_cand(Cw + i0);
+                            const Cand q0 = cand_at(i0);
                             if (kFC)
                                 count_term<ASYM>(hb, q0, q0.c != hslot, cut2, Cd, sCd, nT, me, sidx, cnt);
                             else if (ASYM)
@@ -750,7 +783,7 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
                         // its forward half shell are staged, and within the home cell the
                         // lower slot owns the pair
                         const int quad = (hfx >= 0.f ? 1 : 0) + (hfy >= 0.f ? 2 : 0);
-                        const uint8_t *lst = mapW + quad * kMaxC;
+                        const uint16_t *lst = listW + quad * kMaxC;
                         const int nl = quad == 0 ? nq[0] : (quad == 1 ? nq[1] : (quad == 2 ? nq[2] : nq[3]));
                         const double *Ch = sCd + 6 * hb.type * nT;
                         // one owned pair's share: U, or U(old) - U(scaled) (du_pair)
@@ -771,13 +804,13 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
                         for (int jj = sub; jj < nl; jj += tpp) {
                             const int i0 = inext;
                             inext = lst[jj + tpp];
-                            accu += term(Cw[i0], cb + i0);
+                            accu += term(cand_at(i0), cb + i0 / (int)sizeof(Cand));
                         }
                     } else if (!kF && act) {
                         // neighbour counts and pair lists see both sides of every pair
                         for (int j = cb + sub; j < ce; j += tpp) {
                             if (j == self) continue;
-                            const Cand q = Cw[j - cb];
+                            const Cand q = load_cand(Cw + (j - cb));
                             const int c = q.t >> 8;
                             const Shift sh = ShW[c];
                             const double sx = sh.x, sy = sh.y, sz = sh.z;
@@ -869,7 +902,9 @@ void launch_cells(hipStream_t st, const Params &P, int chunk, const Bead *sbeads
     // The half-shell energy gathers gain on both in groups of 64.
     const bool energy = MODE == M_U || MODE == M_DU;
     const int turn = energy ? 6 : (P.flat ? 7 : 0);
-    hipLaunchKernelGGL((k_cells<MODE, ASYM, ONE>), dim3(nb), dim3(kWaves * kWave), 0, st, P.n, P.nT, chunk, nb, cut2, cut2pre,
+    const bool floats = MODE == M_FORCE || MODE == M_FORCE1 || MODE == M_FDU, doubles = !floats || MODE == M_FDU;
+    const size_t tables_bytes = (size_t)P.nT * P.nT * ((floats ? 2 * sizeof(float4) : 0) + (doubles ? 6 * sizeof(double) : 0));
+    hipLaunchKernelGGL((k_cells<MODE, ASYM, ONE>), dim3(nb), dim3(kWaves * kWave), tables_bytes, st, P.n, P.nT, chunk, nb, cut2, cut2pre,
                        sbeads, skey, sidx, cstart, cend, reps, fconst, uconst, turn, out);
 }
 
