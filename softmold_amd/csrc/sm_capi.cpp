@@ -169,27 +169,42 @@ struct sm_ctx {
     bool order_valid = false;
     // Counting builds (sm_internal.hpp).  Window: sort_mode 2, when win_ok (a single replica of
     // at most 256 sort tiles), while the keys have 17 to 24 bits; wdesc + 8p is the window of
-    // the build with scratch parity p, which the previous build's reorder derived on the device.
-    // Dense: otherwise, sort_mode 0 or 2 with at most kCountBeads beads, while the cell table
-    // holds at most kWinCells cells.  counts and start: the cells' beads and first slots; k2
-    // then holds the sorted cell indices and v0 the bead indices ((k2, v2) is also the window
-    // fallback's third buffer pair).  cnt_last: the last build was a counting build, win_last:
-    // by a window.
+    // the build with scratch parity p, which the previous build derived on the device.  Dense:
+    // otherwise, sort_mode 0 or 2 with at most 256 tiles, while the cell table holds at most
+    // kWinCells cells.  counts[p] and counted[p]: the cells' beads, and the cells counted
+    // in, by the build with parity p; k2 then holds the sorted cell indices and v0 the bead
+    // indices ((k2, v2) is also the fallback's third buffer pair).  cnt_last: the last build
+    // was a counting build, win_last: by a window.
     bool win_ok = false, win_last = false, cnt_last = false;
-    uint32_t *k2 = nullptr, *v2 = nullptr, *wdesc = nullptr, *counts = nullptr, *start = nullptr;
+    uint32_t *k2 = nullptr, *v2 = nullptr, *wdesc = nullptr, *counts[2] = {}, *counted[2] = {}, *bucket = nullptr;
+    size_t count_cells = 0;   // cells that counts and bucket hold
+    bool counters_ready = false;   // the last build was a counting build with these buffers
     bool win_now() const { return sort_mode == 2 && win_ok && sort_bits >= 17 && sort_bits <= 24; }
     bool dense_now() const
     {
-        return !win_now() && sort_mode != 1 && counts && capacity <= kWinCells && n <= kCountBeads;
+        return !win_now() && sort_mode != 1 && bucket && capacity <= kWinCells && sortw_fits(n);
     }
     bool count_now() const { return dense_now() || win_now(); }
+    // room to count in windows, or in the whole table while that is small
     void alloc_counts()
     {
-        if (counts) return;
-        counts = dalloc<uint32_t>(kWinCells);
-        start = dalloc<uint32_t>(kStartWords);
+        if (!sortw_fits(n)) return;
+        size_t cells = win_ok ? count_limit(n) : 0;
+        if (capacity <= kWinCells) cells = std::max(cells, ((size_t)capacity + kCoarseCells - 1) / kCoarseCells * kCoarseCells);
+        if (cells <= count_cells) return;
+        dfree(bucket);
+        bucket = dalloc<uint32_t>(cells * kBucket);
         if (!k2) k2 = dalloc<uint32_t>(n);
-        HIPCHK(hipMemsetAsync(counts, 0, sizeof(uint32_t) * kWinCells, st));
+        if (!v2) v2 = dalloc<uint32_t>(n);
+        for (int p = 0; p < 2; p++) {
+            dfree(counts[p]);
+            counts[p] = dalloc<uint32_t>(cells);
+            if (counted[p]) continue;
+            counted[p] = dalloc<uint32_t>(n);
+            HIPCHK(hipMemsetAsync(counted[p], 0, sizeof(uint32_t) * n, st));
+        }
+        count_cells = cells;
+        counters_ready = false;
     }
     int *cstart = nullptr, *cend = nullptr;
     long long capacity = 0;   // cells in the dense table, all replicas
@@ -272,20 +287,30 @@ struct sm_ctx {
     const uint32_t *sidx() const { return sort_mode == 1 ? sv[scur] : (cnt_last ? v0 : (sorted_sel ? v1 : v0)); }
     // the key kernel's outputs and bookkeeping for the next sort
     uint32_t *key_out() const { return sort_mode == 1 ? kidx[kcur] : k0; }
-    // bead indices for the every-key sort, arrival numbers for a counting build
-    uint32_t *idx_out() const { return sort_mode == 1 ? nullptr : v0; }
+    // bead indices for the every-key sort (a counting build's are in its buckets)
+    uint32_t *idx_out() const { return sort_mode == 1 || count_now() ? nullptr : v0; }
     WinBook win_keys(int p) const
     {
         if (!count_now()) return WinBook{};
         const bool win = win_now();
-        return win_book(hist[p], n, win ? wdesc + 8 * p : nullptr, counts, win ? 0u : (uint32_t)capacity);
+        return win_book(hist[p], n, win ? wdesc + 8 * p : nullptr, counts[p], bucket, win ? 0u : (uint32_t)capacity,
+                        (uint32_t)count_cells);
     }
     // a key kernel ran without its sort: zero what it added to the sort's scratch
     void restart_hist(uint32_t *gh)
     {
         launch_fill_u32(st, gh, sort_hist_words(), 0u);
         launch_fill_u32(st, win_scratch(gh, n), kWinKeyWords, 0u);
-        if (counts) launch_fill_u32(st, counts, kWinCells, 0u);
+        if (counts[0]) launch_fill_u32(st, counts[sort_parity], count_cells, 0u);
+    }
+    // before a key kernel: its scratch holds nothing yet
+    void begin_keys()
+    {
+        if (hist_pending) restart_hist(hist[sort_parity]);   // keys computed twice before a sort: start over
+        hist_pending = true;
+        // a counting build clears the counters of the one right before it only
+        if (count_now() && !counters_ready)
+            for (uint32_t *c : counts) launch_fill_u32(st, c, count_cells, 0u);
     }
     MoveBook move_book() const
     {
@@ -304,7 +329,8 @@ struct sm_ctx {
         for (auto e : pool) (void)hipEventDestroy(e);
         dfree(beads); dfree(sbeads); dfree(beads_alt); dfree(vel); dfree(acc); dfree(fpair); dfree(fscratch);
         dfree(k0); dfree(v0); dfree(k1); dfree(v1); dfree(hist[0]); dfree(hist[1]); dfree(cstart); dfree(cend);
-        dfree(k2); dfree(v2); dfree(wdesc); dfree(counts); dfree(start);
+        dfree(k2); dfree(v2); dfree(wdesc); dfree(bucket);
+        for (int p = 0; p < 2; p++) { dfree(counts[p]); dfree(counted[p]); }
         for (int p = 0; p < 2; p++) { dfree(kidx[p]); dfree(sk[p]); dfree(sv[p]); }
         dfree(mbefore); dfree(cnt_b); dfree(cnt_i); dfree(cnt_s); dfree(mflags); dfree(mcount);
         dfree(reps); dfree(glob); dfree(fconstF); dfree(uconstD); dfree(fconstD); dfree(chainPerBead); dfree(chainList);
@@ -475,7 +501,7 @@ struct sm_ctx {
         int bits = 1;
         while ((1ll << bits) < base) bits++;
         sort_bits = bits;
-        if (win_ok || (capacity <= kWinCells && n <= kCountBeads)) alloc_counts();
+        alloc_counts();
     }
 
     // keys (optionally after Verlet::first) with the next sort's digit histograms, sort,
@@ -484,9 +510,7 @@ struct sm_ctx {
     void first_and_keys(int integrate, long long step_set, bool for_sort = true, bool away = false)
     {
         uint32_t *gh = for_sort ? hist[sort_parity] : nullptr;
-        // keys computed twice before a sort (sm_step_first called twice): start over
-        if (for_sort && hist_pending) restart_hist(gh);
-        hist_pending = hist_pending || for_sort;
+        if (for_sort) begin_keys();
         const int passes = sort_passes(sort_bits);
         timed(K_FIRST, [&] {
             if (for_sort)
@@ -502,7 +526,20 @@ struct sm_ctx {
     {
         const int p = sort_parity;
         const bool count = count_now();
-        const WinBook wb = win_keys(p);
+        win_last = count && win_now();
+        cnt_last = counters_ready = count;
+        if (count) {
+            timed(K_REORDER, [&] {
+                launch_build(st, n, BuildArgs{k0, v0, k1, v1, k2, v2, win_keys(p), counts[1 - p], counted[1 - p],
+                                              counted[p], wdesc ? wdesc + 8 * (1 - p) : nullptr, beads, sbeads, cstart,
+                                              cend, hist[1 - p], hist_words, reps, hist[p],
+                                              win_scratch(hist[p], n) + kWinKeyWords, &glob->flags, build_tiles(n)});
+            });
+            order_valid = false;
+            sort_parity = 1 - p;
+            hist_pending = false;
+            return;
+        }
         if (sort_mode == 1) {
             timed(K_SORT, [&] {
                 SortBuffers sb{k0, v0, k1, v1, {hist[0], hist[1]}, &glob->flags, n, 0};
@@ -513,12 +550,6 @@ struct sm_ctx {
             scur = 1 - scur;
             kcur = 1 - kcur;
             order_valid = true;
-        } else if (count) {
-            timed(K_SORT, [&] {
-                SortBuffers sb{k0, v0, k1, v1, {hist[0], hist[1]}, &glob->flags, n, 0};
-                count_build(st, sb, k2, v2, p, wb, start, reps);
-            });
-            order_valid = false;
         } else {
             timed(K_SORT, [&] {
                 SortBuffers sb{k0, v0, k1, v1, {hist[0], hist[1]}, &glob->flags, n, 0};
@@ -526,14 +557,8 @@ struct sm_ctx {
             });
             order_valid = false;
         }
-        win_last = count && wb.desc;
-        cnt_last = count;
         timed(K_REORDER, [&] {
-            if (count)
-                launch_reorder_count(st, n, k0, v0, k1, v1, k2, start, beads, sbeads, cstart, cend, hist[1 - p],
-                                     hist_words, wb, wdesc ? wdesc + 8 * (1 - p) : nullptr, reps);
-            else
-                launch_reorder(st, n, skey(), sidx(), beads, sbeads, cstart, cend, hist[1 - p], hist_words);
+            launch_reorder(st, n, skey(), sidx(), beads, sbeads, cstart, cend, hist[1 - p], hist_words);
         });
         sort_parity = 1 - p;
         hist_pending = false;
@@ -685,8 +710,7 @@ struct sm_ctx {
     void kick_first(long long s, bool from_base = false)
     {
         uint32_t *gh = hist[sort_parity];
-        if (hist_pending) restart_hist(gh);
-        hist_pending = true;
+        begin_keys();
         const int passes = sort_passes(sort_bits);
         timed(K_KICK_FIRST, [&] {
             launch_kick_first(st, P, beads, beads_alt, chainPerBead, cconstD, gen(), fpair, vel, reps, glob, s,
@@ -718,9 +742,9 @@ struct sm_ctx {
     // 12k-bead bilayer with their download took 831 us with the halves apart, 793 now.
     void graph_block(long long s)
     {
-        if (sort_mode == 1 && !order_valid) {
-            // the graph would replay a first sort without a previous order: step this block
-            // eagerly, after which the order is there to capture against
+        if ((sort_mode == 1 && !order_valid) || (count_now() && !counters_ready)) {
+            // the graph would replay a first sort without a previous order, or a first counting
+            // build: step this block eagerly, after which there is one to capture against
             eager(s, s + 8);
             return;
         }
@@ -1076,7 +1100,7 @@ sm_ctx *create(const sm_system *s, int nrep)
         c->cnt_s = dalloc<uint32_t>(move_tiles(n));
         c->mflags = dalloc<unsigned long long>(((size_t)n + 63) / 64);
         c->mcount = dalloc<int>(1);
-        c->hist_words = sort_scratch_words(n, 4) + sortw_words(n, c->win_ok);
+        c->hist_words = sort_scratch_words(n, 4) + sortw_words(n, sortw_fits(n));
         for (int p = 0; p < 2; p++) {
             c->hist[p] = dalloc<uint32_t>(c->hist_words);
             HIPCHK(hipMemsetAsync(c->hist[p], 0, sizeof(uint32_t) * c->hist_words, c->st));
@@ -1620,7 +1644,7 @@ int sm_tune_get(sm_ctx *c, const char *knob, int32_t *value)
                 const int lp = 1 - c->sort_parity;
                 uint32_t wx = 0, flag = 0;
                 HIPCHK(hipMemcpyAsync(&wx, c->wdesc + 8 * lp + 3, sizeof(uint32_t), hipMemcpyDeviceToHost, c->st));
-                HIPCHK(hipMemcpyAsync(&flag, win_book(c->hist[lp], c->n, nullptr, nullptr, 0u).flag, sizeof(uint32_t),
+                HIPCHK(hipMemcpyAsync(&flag, win_book(c->hist[lp], c->n, nullptr, nullptr, nullptr, 0u, 0u).flag, sizeof(uint32_t),
                                       hipMemcpyDeviceToHost, c->st));
                 HIPCHK(hipStreamSynchronize(c->st));
                 *value = (wx != 0 && flag == 0) ? 1 : 0;

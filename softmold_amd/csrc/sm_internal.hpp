@@ -143,27 +143,28 @@ struct MoveBook {
     const uint32_t *kold;
     uint32_t *cnt_b;
 };
-// The counting builds: the key kernel counts the beads of each cell (an atomic that also gives
-// the bead's arrival number), a scan of the counts gives each cell's first slot, the beads go
-// to their cell's run in arrival order and the reorder puts each run into index order, which
-// makes the order the stable sort's.
+// The counting builds: the key kernel counts the beads of each cell with an atomic that also
+// gives a bead's arrival number, under which it enters the cell's bucket; one kernel
+// (launch_build) then scans the counts, takes each run from its bucket and puts it into index
+// order, which makes the order the stable sort's.
 //  - window (sort_mode 2: one replica, every key sorted, keys of 17 to 24 bits, at most
 //    kWinMaxTiles tiles of keys): each build has a window of cells, the previous measured
 //    occupied cell range widened by one cell on each side, used when it holds at most
-//    kWinCells cells.  A key whose cell lies in it is stored as kWinTag | the cell's index in
-//    the window's own (z, y, x) order, which orders keys as the cell index does.  A key
-//    outside the window raises the build's fallback flag; the same launches then sort the
-//    cell indices in three 8-bit passes.
-//  - dense (sort_mode 0 or 2, any context of at most kCountBeads beads whose cell table holds
-//    at most kWinCells cells): the cell index itself; nothing to fall back from.  The counters
-//    take 25 atomics a ns whatever the table, the radix passes cost 5 us each at least: per
-//    step 130 us counted against 144 sorted at 192k beads in 16 bilayers, 261 against 261 at
-//    470k, 478 against 471 at 960k.
+//    count_limit(n) cells: four a bead, 2^14 to 2^18, so that a small context's buckets are
+//    small too (a vesicle's window has half a cell a bead at most).  A key whose cell lies in it is stored as kWinTag | the cell's index in
+//    the window's own (z, y, x) order, which orders keys as the cell index does.
+//  - dense (sort_mode 0 or 2, any context of at most kWinMaxTiles tiles of keys, 524288 beads,
+//    whose cell table holds at most kWinCells cells): the cell index itself.  The counters take
+//    25 atomics a ns, a radix pass 5 us at least: per step 119 us counted against 144
+//    sorted at 192k beads in 16 bilayers, 252 against 262 at 470k; the fallback's workgroups
+//    must fit the card together, which ends it there.
+// A key outside the window, or a cell of more beads than a bucket holds, raises the build's
+// fallback flag; the same launch then sorts the cell indices in three 8-bit passes.
 // desc == NULL and cells == 0: neither.
 constexpr uint32_t kWinTag = 1u << 31;
 constexpr int kWinMaxTiles = 256;
 constexpr int kWinCells = 1 << 18;
-constexpr int kCountBeads = 1 << 19;
+constexpr int kBucket = 64;                              // beads of a cell's bucket: 8 a unit volume
 constexpr int kCoarseCells = 2048;                       // cells a scan tile holds
 constexpr int kCoarse = kWinCells / kCoarseCells;        // coarse counts: beads of each scan tile
 constexpr int kCoarseCopies = 4;
@@ -171,19 +172,22 @@ struct WinBook {
     const uint32_t *desc;   // this build's window {x0, y0, z0, wx, wy, wz}; wx == 0: none
     uint32_t *coarse;       // [kCoarseCopies][kCoarse]
     uint32_t *bbox;         // [16 copies][8]: max of cx + 1, cy + 1, cz + 1, 2^20 - cx, 2^20 - cy, 2^20 - cz
-    uint32_t *flag;         // nonzero: some key fell outside the window
-    uint32_t *counts;       // beads per cell: zero before the key kernel, and again after the scan
+    uint32_t *flag;         // nonzero: the build falls back
+    uint32_t *counts;       // beads per cell: zero before the key kernel, and again two builds on
+    uint32_t *bucket;       // [cells][kBucket]: bead indices by arrival
     uint32_t cells;         // dense: the table's cells
+    uint32_t limit;         // cells that counts and bucket hold (a multiple of kCoarseCells)
 };
 // the counting builds' scratch, after the sort_scratch_words(n, 4) words of the every-key sort:
-// coarse, bbox, {flag, 2 tile counters, 2 barrier counters, pad}, then, for windows, 3 passes x
-// tiles x 256 look-back words; the key kernel writes the first kWinKeyWords of it
+// coarse, bbox, {flag, 4 barrier counters, pad}, then 3 passes x tiles x 256 look-back words;
+// the key kernel writes the first kWinKeyWords of it
 constexpr size_t kWinKeyWords = (size_t)kCoarseCopies * kCoarse + 16 * 8 + 8;
-constexpr size_t kStartWords = (size_t)kWinCells + kCoarseCells;   // first slots, and one past the last
-size_t sortw_words(int n, bool window);
+size_t sortw_words(int n, bool counting);
 uint32_t *win_scratch(uint32_t *sort_scratch, int n);   // where it starts in a sort's scratch
-WinBook win_book(uint32_t *sort_scratch, int n, const uint32_t *desc, uint32_t *counts, uint32_t cells);
-bool sortw_fits(int n);   // the tiles of n keys are few enough for the window build's launches
+WinBook win_book(uint32_t *sort_scratch, int n, const uint32_t *desc, uint32_t *counts, uint32_t *bucket,
+                 uint32_t cells, uint32_t limit);
+size_t count_limit(int n);
+bool sortw_fits(int n);   // the tiles of n keys are few enough for the build's fallback
 // out: where the beads go (beads itself, or another buffer)
 void launch_first(hipStream_t st, const Params &P, const Bead *beads, Bead *out, float4 *vel, const float4 *acc, const DevRep *reps,
                   DevGlobal *glob, uint32_t *key, uint32_t *idx, int integrate, long long step_set, uint32_t *ghist,
@@ -191,16 +195,6 @@ void launch_first(hipStream_t st, const Params &P, const Bead *beads, Bead *out,
 // also zeroes clear[0 .. clear_words) (the next sort's scratch)
 void launch_reorder(hipStream_t st, int n, const uint32_t *skey, const uint32_t *sidx, const Bead *beads,
                     Bead *sbeads, int *cstart, int *cend, uint32_t *clear, size_t clear_words);
-// A counting build's reorder.  Window or dense path: (k1, v1) holds each run's cell (in the
-// window's or the table's order) and bead indices in arrival order, start the runs' first
-// slots.  Fallback: (k0, v0) holds the sorted cell indices and bead indices.  k2 and v0 receive
-// the sorted cell indices and bead indices; it also derives the next build's window (desc_next)
-// from this build's occupied range.  The cell grid of a window is replica 0's, read on the
-// device.
-void launch_reorder_count(hipStream_t st, int n, const uint32_t *k0, uint32_t *v0, const uint32_t *k1,
-                          const uint32_t *v1, uint32_t *k2, const uint32_t *start, const Bead *beads, Bead *sbeads,
-                          int *cstart, int *cend, uint32_t *clear, size_t clear_words, const WinBook &wb,
-                          uint32_t *desc_next, const DevRep *reps);
 // variant 0: one phase (FP64 test, force law under the branch) over per-quarter-cell culled
 // candidate lists; 1: FP32 screen into a per-lane hit list, then FP64 test + force law on
 // the hits
@@ -321,10 +315,32 @@ struct MoveSort {
     uint32_t *skey, *sidx;                   // the new sorted order
 };
 void sort_moved(hipStream_t st, SortBuffers &b, const MoveSort &m, int bits, int parity);
-// The counting build of the keys k0 and arrival numbers v0 by bead index (from a key kernel
-// given wb): the runs' first slots into start and the runs into (k1, v1); wb.desc: a window,
-// whose fallback sorts into (k0, v0) through (k1, v1) and (k2, v2) instead (needs sortw_fits(n)).
-void count_build(hipStream_t st, SortBuffers &b, uint32_t *k2, uint32_t *v2, int parity, const WinBook &wb,
-                 uint32_t *start, const DevRep *reps);
+// The counting build of the keys b.k0 by bead index (from a key kernel given wb): the sorted
+// cell indices into k2 and bead indices into b.v0, the beads in that order into sbeads, the
+// occupied cells' slots into cstart and cend; and the next build's window (desc_next) from this
+// build's occupied range.  The fallback goes through (k1, v1) and (k2, v2) into (k0, v0).
+// cells_now receives the cells that this build counted in; the counters counts_old are zeroed
+// at the cells cells_old of the build before.  Zeroes clear[0 .. clear_words) (the next
+// build's scratch).  Needs sortw_fits(n).
+struct BuildArgs {
+    uint32_t *k0, *v0, *k1, *v1, *k2, *v2;
+    WinBook wb;
+    uint32_t *counts_old;
+    const uint32_t *cells_old;
+    uint32_t *cells_now;
+    uint32_t *desc_next;
+    const Bead *beads;
+    Bead *sbeads;
+    int *cstart, *cend;
+    uint32_t *clear;
+    size_t clear_words;
+    const DevRep *reps;     // a window's cell grid: replica 0's
+    uint32_t *ghist;        // the cell indices' digit histograms [copies][4][256]
+    uint32_t *status;       // look-back words of the fallback's three passes, tiles x 256 each
+    int *errflag;
+    int tiles;              // the fallback's tiles
+};
+void launch_build(hipStream_t st, int n, const BuildArgs &a);
+int build_tiles(int n);
 
 }  // namespace smdev

@@ -151,11 +151,11 @@ __global__ __launch_bounds__(kBlock) void k_first(int n, const Bead *beads, Bead
             for (int p = 0; p < passes; p++) h[p][threadIdx.x] = 0u;
         __syncthreads();
     }
-    uint32_t k = 0u, rank = (uint32_t)i;
+    uint32_t k = 0u;
     int cx = 0, cy = 0, cz = 0;
     if (i < n) k = first_one(i, beads, out, vel, acc, reps, glob, halfdt, dt, integrate, cx, cy, cz);
     if (ghist && win) {
-        k = win_key_end(wb, w, hs, k, cx, cy, cz, i < n, rank);
+        k = win_key_end(wb, w, hs, k, cx, cy, cz, i, i < n);
     } else if (ghist) {
         // the sort's digit histograms while the key is in a register (all lanes: ballots)
         const bool counted = note_move(book, i, k, i < n);
@@ -166,7 +166,7 @@ __global__ __launch_bounds__(kBlock) void k_first(int n, const Bead *beads, Bead
     }
     if (i < n) {
         key[i] = k;
-        if (idx) idx[i] = rank;
+        if (idx) idx[i] = (uint32_t)i;
     }
 }
 
@@ -188,92 +188,6 @@ __global__ __launch_bounds__(kBlock) void k_reorder(int n, const uint32_t *__res
     sbeads[s] = beads[sidx[s]];
     if (s == 0 || kprev != k) cstart[k] = s;
     if (s == n - 1 || knext != k) cend[k] = s + 1;
-}
-
-// The reorder of a counting build (see launch_reorder_count).  On the window or dense path a
-// bead's slot is its run's first slot plus the run's beads of lower index: a run is a cell's
-// dozen beads, read by every one of its threads from the caches.  Block 0 also sets the next
-// build's window: this build's after the window path; after the fallback, the occupied cell
-// range the fallback measured, widened by one cell on each side and clipped to the grid, or
-// none (wx = 0) when that holds more than kWinCells cells.
-__global__ __launch_bounds__(kBlock) void k_reorder_count(int n, const uint32_t *__restrict__ k0,
-                                                          uint32_t *__restrict__ v0, const uint32_t *__restrict__ k1,
-                                                          const uint32_t *__restrict__ v1, uint32_t *__restrict__ k2,
-                                                          const uint32_t *__restrict__ start,
-                                                          const Bead *__restrict__ beads, Bead *__restrict__ sbeads,
-                                                          int *__restrict__ cstart, int *__restrict__ cend,
-                                                          uint32_t *__restrict__ clear, size_t clear_words, WinBook wb,
-                                                          uint32_t *__restrict__ desc_next,
-                                                          const DevRep *__restrict__ reps)
-{
-    const int s = blockIdx.x * kBlock + threadIdx.x;
-    for (size_t w = (size_t)s; w < clear_words; w += (size_t)gridDim.x * kBlock) clear[w] = 0u;
-    const bool dense = wb.cells != 0u;
-    WinDesc w{};
-    bool fallback = false;
-    int nx = 1, ny = 1;
-    if (!dense) {
-        nx = reps[0].nc[0];
-        ny = reps[0].nc[1];
-        w = load_win(wb.desc);
-        fallback = w.wx == 0u || *wb.flag != 0u;
-    }
-    if (!dense && blockIdx.x == 0 && threadIdx.x < kWave) {
-        const int t = threadIdx.x;
-        uint32_t v = 0u;
-        if (fallback && t < 6)
-            for (int c = 0; c < kHistCopies; c++) v = max(v, wb.bbox[c * 8 + t]);
-        uint32_t f[6];
-#pragma unroll
-        for (int j = 0; j < 6; j++) f[j] = (uint32_t)__shfl((int)v, j);
-        if (t == 0) {
-            uint32_t d[6] = {w.x0, w.y0, w.z0, w.wx, w.wy, w.wz};
-            if (fallback) {
-                for (int j = 0; j < 6; j++) d[j] = 0u;
-                if (f[0] != 0u) {
-                    const int ncell[3] = {nx, ny, reps[0].nc[2]};
-                    unsigned long long cells = 1ull;
-                    for (int a = 0; a < 3; a++) {
-                        const int lo = max((int)(kBoxEnc - f[3 + a]) - 1, 0);
-                        const int hi = min((int)f[a], ncell[a] - 1);   // f = highest cell + 1
-                        d[a] = (uint32_t)lo;
-                        d[3 + a] = (uint32_t)(hi - lo + 1);
-                        cells *= (unsigned long long)(hi - lo + 1);
-                    }
-                    if (cells > (unsigned long long)kWinCells)
-                        for (int j = 0; j < 6; j++) d[j] = 0u;
-                }
-            }
-            for (int j = 0; j < 6; j++) desc_next[j] = d[j];
-        }
-    }
-    if (s >= n) return;
-    if (fallback) {   // (k0, v0) is sorted
-        const uint32_t k = k0[s], kprev = k0[s > 0 ? s - 1 : 0], knext = k0[s < n - 1 ? s + 1 : s];
-        sbeads[s] = beads[v0[s]];
-        k2[s] = k;
-        if (s == 0 || kprev != k) cstart[k] = s;
-        if (s == n - 1 || knext != k) cend[k] = s + 1;
-        return;
-    }
-    const uint32_t wk = min(k1[s], (uint32_t)kWinCells - 1u), i = min(v1[s], (uint32_t)n - 1u);
-    const Bead b = beads[i];
-    const uint32_t c0 = min(start[wk], (uint32_t)n - 1u), c1 = min(start[wk + 1], (uint32_t)n);
-    uint32_t pos = c0;
-    for (uint32_t j = c0; j < c1; j++) pos += v1[j] < i ? 1u : 0u;
-    pos = min(pos, (uint32_t)n - 1u);   // in bounds also for counts that are not this build's
-    uint32_t full = wk;
-    if (!dense) {
-        const uint32_t q = wk / w.wx, x = wk - q * w.wx, z = q / w.wy, y = q - z * w.wy;
-        full = ((z + w.z0) * (uint32_t)ny + (y + w.y0)) * (uint32_t)nx + (x + w.x0);
-    }
-    sbeads[pos] = b;
-    v0[pos] = i;
-    k2[pos] = full;
-    if (pos == c0) {
-        cstart[full] = (int)c0;
-        cend[full] = (int)c1;
-    }
 }
 
 // ---------------------------------------------------------------------------------------
@@ -456,7 +370,7 @@ __global__ __launch_bounds__(kBlock) void k_bonded_kick(int n, const Bead *__res
 // traffic, 128 instead of 144 bytes a bead).
 // ONE: a single-replica context, whose replica constants are read from reps[0] without
 // waiting for the bead's replica index
-// WIN: keys and arrival numbers for a counting build (wb)
+// WIN: keys and buckets for a counting build (wb)
 template <bool ONE, bool WIN>
 __global__ __launch_bounds__(kBlock) void k_kick_first(int n, const Bead *__restrict__ beads,
                                                        Bead *__restrict__ beads_out,
@@ -481,7 +395,7 @@ __global__ __launch_bounds__(kBlock) void k_kick_first(int n, const Bead *__rest
     else
         for (int p = 0; p < passes; p++) h[p][threadIdx.x] = 0u;
     __syncthreads();
-    uint32_t k = 0u, rank = (uint32_t)i;
+    uint32_t k = 0u;
     int cx = 0, cy = 0, cz = 0;
     if (i < n) {
         Bead b = beads[i];
@@ -499,7 +413,7 @@ __global__ __launch_bounds__(kBlock) void k_kick_first(int n, const Bead *__rest
         k = bead_key(b, R, glob, cx, cy, cz);
     }
     if (WIN) {
-        k = win_key_end(wb, w, hs, k, cx, cy, cz, i < n, rank);
+        k = win_key_end(wb, w, hs, k, cx, cy, cz, i, i < n);
     } else {
         const bool counted = note_move(book, i, k, i < n);
         hist_add(h, k, counted, passes);
@@ -509,7 +423,7 @@ __global__ __launch_bounds__(kBlock) void k_kick_first(int n, const Bead *__rest
     }
     if (i < n) {
         key[i] = k;
-        if (idx) idx[i] = rank;
+        if (idx) idx[i] = (uint32_t)i;
     }
 }
 
@@ -990,15 +904,6 @@ void launch_reorder(hipStream_t st, int n, const uint32_t *skey, const uint32_t 
 {
     hipLaunchKernelGGL(k_reorder, dim3(blocks(n)), dim3(kBlock), 0, st, n, skey, sidx, beads, sbeads, cstart, cend,
                        clear, clear_words);
-}
-
-void launch_reorder_count(hipStream_t st, int n, const uint32_t *k0, uint32_t *v0, const uint32_t *k1,
-                          const uint32_t *v1, uint32_t *k2, const uint32_t *start, const Bead *beads, Bead *sbeads,
-                          int *cstart, int *cend, uint32_t *clear, size_t clear_words, const WinBook &wb,
-                          uint32_t *desc_next, const DevRep *reps)
-{
-    hipLaunchKernelGGL(k_reorder_count, dim3(blocks(n)), dim3(kBlock), 0, st, n, k0, v0, k1, v1, k2, start, beads,
-                       sbeads, cstart, cend, clear, clear_words, wb, desc_next, reps);
 }
 
 void launch_bonded_kick(hipStream_t st, const Params &P, const Bead *beads, const int2 *chain,

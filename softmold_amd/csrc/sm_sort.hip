@@ -30,14 +30,8 @@
 //
 // Counting builds: where the cells of a build fit 2^18 counters -- the whole table (dense), or
 // a window around the previous build's occupied cells (sort_mode 2, one replica) -- the key
-// kernel counts the beads of each cell while the keys are in registers.  k_scan_cells turns the
-// counts into first slots, k_place puts each bead into its cell's run by its arrival number,
-// and the reorder puts each run into index order, so the order is the stable sort's without a
-// sort.  A vesicle of 240k beads in a 200^3-cell grid has 23-bit keys but a 50^3-cell window:
-// 36 us of radix passes and reorder became 19 us (scan and place 10.6, reorder 8.6, and 2 us
-// more in the key kernel); 15k beads 20 -> 13 us, 1.5k beads 14 -> 12 us.
-// If a key fell outside the window (or there is none), the same launches sort the cell indices
-// in three 8-bit passes and measure the occupied range for the next window.
+// kernel counts the beads of each cell while the keys are in registers and drops them into the
+// cell's bucket; k_build does the rest in one launch, without a sort.
 #include <algorithm>
 
 #include "sm_sort_dev.hpp"
@@ -452,11 +446,22 @@ __global__ __launch_bounds__(kThreads) void k_merge(int n, const int *__restrict
 
 
 // ---------------------------------------------------------------------------------------
-// The counting builds, and the window build's fallback: three 8-bit passes over the cell
-// indices.  Its first launch converts any window keys back to cell indices and counts their
-// digits, then runs two passes with a grid-wide barrier before each (a launch has at most
-// kWinMaxTiles workgroups that stay, so all of them are resident together); the second launch
-// runs the third.  Each launch reads which path to take from the device.
+// k_build: the counting builds.
+//
+// What bounds it: launches and chains of loads.  A vesicle of 240k beads in a 200^3-cell grid
+// has 23-bit keys but a 50^3-cell window: two or three radix passes with their look-back and
+// the reorder took 36 us, a scan of the counts, a scatter and the reorder as three kernels
+// 19, one kernel 12; at 1.5k beads 14, 12 and 7.  A workgroup owns 256 slots of the new order
+// (so the work is even, however the cells fill): it sums the coarse counts to find the scan
+// tile of its first slot, scans that tile's counts (and the next ones' until its slots end),
+// and marks where the runs begin; a max-scan gives each thread its run and its place in it.
+// The thread's bead goes to the run's first slot plus the run's beads of lower index, counted
+// in the bucket, a row that the run's threads share in the caches.
+//
+// The fallback: three 8-bit passes over the cell indices and the reorder, with a grid-wide
+// barrier before each.  It turns window keys back into cell indices, counts their digits and
+// measures the occupied range for the next window.  Its at most kWinMaxTiles workgroups are
+// the only ones that wait, and all of them fit the card together.
 // ---------------------------------------------------------------------------------------
 template <int kRounds>
 struct WLds {
@@ -465,7 +470,6 @@ struct WLds {
     uint32_t h[3][256];                          // digit counts of a tile's cell indices
     uint32_t bb[kWavesPerBlock][6];              // occupied cell range of each wave's keys
     uint32_t scan[kWavesPerBlock];
-    uint32_t tile;
 };
 
 // Sum of the counts of digit d over the tiles before `tile` (decoupled look-back over
@@ -587,159 +591,179 @@ __device__ inline uint32_t hist_sum(const uint32_t *__restrict__ ghist)
     return g;
 }
 
-// Every workgroup of the launch arrives at *ctr before any goes on; its stores before are
-// visible to every workgroup's loads after.  Bounded like the look-back.
+// `count` workgroups arrive at *ctr before any goes on; its stores before are visible to
+// every workgroup's loads after: the workgroup barrier orders the threads' stores before thread
+// 0's release, and its acquire before their loads (one cache write-back and one invalidation
+// a workgroup, not one a wave).  Bounded like the look-back.
 __device__ inline void grid_sync(uint32_t *ctr, uint32_t count, int *errflag)
 {
-    __threadfence();
     __syncthreads();
     if (threadIdx.x == 0) {
         __hip_atomic_fetch_add(ctr, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
         int spins = 0;
-        while (__hip_atomic_load(ctr, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) < count) {
+        while (__hip_atomic_load(ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < count) {
             if (++spins >= kSpinLimit) {
                 atomicOr(errflag, FLAG_SORT_TIMEOUT);
                 break;
             }
             __builtin_amdgcn_s_sleep(1);
         }
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     }
     __syncthreads();
-    __threadfence();
 }
 
-// First slots of scan tile t's kCoarseCells cells from their counts, which it clears for the
-// next key kernel.  The beads before the tile are the coarse counts of the tiles before it, so
-// no tile waits for another; eight cells a thread, in two 16-byte loads.  3 us at 125k cells.
-__device__ inline void scan_cells(int t, const WinBook &wb, uint32_t *__restrict__ start, uint32_t *lds)
+// what a workgroup of the fast path holds
+struct BLds {
+    uint32_t pre[kCoarse + 1];   // beads before each scan tile
+    uint32_t scan[kWavesPerBlock];
+    uint32_t first;              // the scan tile of the workgroup's first slot
+    uint32_t cell[kThreads], start[kThreads], count[kThreads];   // of the run that begins at a slot, or 0
+};
+
+__device__ inline uint32_t wave_scan_add(uint32_t x)
 {
-    static_assert(kCoarseCells == 8 * kThreads && kCoarse <= kThreads, "eight cells and at most one tile a thread");
-    const int j = threadIdx.x, lane = j & (kWave - 1), wave = j / kWave;
-    uint4 *c = reinterpret_cast<uint4 *>(wb.counts + (size_t)t * kCoarseCells) + 2 * j;
-    const uint4 a = c[0], b = c[1];
-    uint32_t before = 0u;
-    if (j < kCoarse && j < t)
-        for (int k = 0; k < kCoarseCopies; k++) before += wb.coarse[k * kCoarse + j];
-    c[0] = c[1] = make_uint4(0u, 0u, 0u, 0u);
-    const uint32_t mine = a.x + a.y + a.z + a.w + b.x + b.y + b.z + b.w;
-    uint32_t x = mine;
+    const int lane = threadIdx.x & (kWave - 1);
 #pragma unroll
     for (int o = 1; o < kWave; o <<= 1) {
         const uint32_t y = __shfl_up(x, o);
         if (lane >= o) x += y;
     }
-#pragma unroll
-    for (int o = kWave / 2; o > 0; o >>= 1) before += __shfl_xor(before, o);
-    if (lane == kWave - 1) {
-        lds[wave] = x;
-        lds[kWavesPerBlock + wave] = before;
+    return x;
+}
+
+__device__ void build_slots(BLds &L, int n, const BuildArgs &a, const WinDesc &w, bool dense)
+{
+    static_assert(kCoarseCells == 8 * kThreads && kCoarse <= 2 * kWave, "eight cells a thread, the tiles in two waves");
+    const int t = threadIdx.x, wave = t / kWave, lane = t & (kWave - 1);
+    const uint32_t lo = blockIdx.x * kThreads, hi = min(lo + kThreads, (uint32_t)n);
+    const int s = (int)lo + t;
+    // this thread's share of the counters of the build before (see cells_old)
+    if (s < n) a.counts_old[min(a.cells_old[s], a.wb.limit - 1u)] = 0u;
+    uint32_t c = 0u;
+    if (t < kCoarse)
+        for (int k = 0; k < kCoarseCopies; k++) c += a.wb.coarse[k * kCoarse + t];
+    uint32_t x = wave_scan_add(c);
+    if (lane == kWave - 1) L.scan[wave] = x;
+    L.cell[t] = 0u;
+    if (t == 0) L.first = 0u;
+    __syncthreads();
+    if (wave == 1) x += L.scan[0];
+    if (t < kCoarse) {
+        L.pre[t + 1] = x;
+        if (x - c <= lo && x > lo) L.first = (uint32_t)t;
+    }
+    if (t == 0) L.pre[0] = 0u;
+    __syncthreads();
+    for (int tile = (int)L.first; tile < kCoarse && L.pre[tile] < hi; tile++) {
+        if (L.pre[tile] == L.pre[tile + 1]) continue;   // uniform
+        const uint4 *p = reinterpret_cast<const uint4 *>(a.wb.counts + (size_t)tile * kCoarseCells) + 2 * t;
+        const uint4 u = p[0], v = p[1];
+        const uint32_t m[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+        uint32_t sum = 0u;
+        for (int k = 0; k < 8; k++) sum += m[k];
+        uint32_t y = wave_scan_add(sum);
+        __syncthreads();   // the tile before is done with L.scan
+        if (lane == kWave - 1) L.scan[wave] = y;
+        __syncthreads();
+        y += L.pre[tile] - sum;
+        for (int q = 0; q < wave; q++) y += L.scan[q];
+        for (int k = 0; k < 8; k++) {
+            if (m[k] != 0u && y < hi && y + m[k] > lo) {
+                const uint32_t at = max(y, lo) - lo;
+                L.cell[at] = (uint32_t)(tile * kCoarseCells + 8 * t + k) + 1u;
+                L.start[at] = y;
+                L.count[at] = m[k];
+            }
+            y += m[k];
+        }
     }
     __syncthreads();
-    uint32_t p = x - mine;
-    for (int w = 0; w < kWavesPerBlock; w++) p += (w < wave ? lds[w] : 0u) + lds[kWavesPerBlock + w];
-    uint4 u, v;
-    u.x = p; u.y = u.x + a.x; u.z = u.y + a.y; u.w = u.z + a.z;
-    v.x = u.w + a.w; v.y = v.x + b.x; v.z = v.y + b.y; v.w = v.z + b.z;
-    uint4 *o = reinterpret_cast<uint4 *>(start + (size_t)t * kCoarseCells) + 2 * j;
-    o[0] = u;
-    o[1] = v;
-    if (j == kThreads - 1) start[(size_t)(t + 1) * kCoarseCells] = v.w + b.w;   // as the next tile's first
+    // the slot where this thread's run begins in the workgroup: the last mark up to it
+    int head = L.cell[t] != 0u ? t : 0;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+        const int y = __shfl_up(head, o);
+        if (lane >= o) head = max(head, y);
+    }
+    if (lane == kWave - 1) L.scan[wave] = (uint32_t)head;
     __syncthreads();
+    for (int q = 0; q < wave; q++) head = max(head, (int)L.scan[q]);
+    if (s >= n) return;
+    const uint32_t wk = min(L.cell[head] - 1u, a.wb.limit - 1u);
+    const uint32_t start = L.start[head], count = min(L.count[head], (uint32_t)kBucket);
+    const uint32_t *row = a.wb.bucket + (size_t)wk * kBucket;
+    const uint32_t i = min(row[min((uint32_t)s - start, (uint32_t)kBucket - 1u)], (uint32_t)n - 1u);
+    const Bead b = a.beads[i];
+    uint32_t pos = start;
+    const uint4 *row4 = reinterpret_cast<const uint4 *>(row);
+    for (uint32_t q = 0; q < count; q += 4) {
+        const uint4 e = row4[q / 4];
+        pos += (e.x < i ? 1u : 0u) + (q + 1 < count && e.y < i ? 1u : 0u) + (q + 2 < count && e.z < i ? 1u : 0u) +
+               (q + 3 < count && e.w < i ? 1u : 0u);
+    }
+    pos = min(pos, (uint32_t)n - 1u);   // in bounds also for counts that are not this build's
+    uint32_t full = wk;
+    if (!dense) {
+        const uint32_t nx = (uint32_t)a.reps[0].nc[0], ny = (uint32_t)a.reps[0].nc[1];
+        const uint32_t q = wk / w.wx, cx = wk - q * w.wx, cz = q / w.wy, cy = q - cz * w.wy;
+        full = ((cz + w.z0) * ny + (cy + w.y0)) * nx + (cx + w.x0);
+    }
+    a.sbeads[pos] = b;
+    a.v0[pos] = i;
+    a.k2[pos] = full;
+    a.cells_now[s] = wk;
+    if (pos == start) {
+        a.cstart[full] = (int)start;
+        a.cend[full] = (int)(start + count);
+    }
 }
-
-// Bead i into its run by its arrival number.
-__device__ inline void place_bead(int i, int n, const uint32_t *__restrict__ key, const uint32_t *__restrict__ rank,
-                                  const uint32_t *__restrict__ start, uint32_t *__restrict__ cell,
-                                  uint32_t *__restrict__ bead)
-{
-    const uint32_t k = min(key[i] & ~kWinTag, (uint32_t)kWinCells - 1u);
-    const uint32_t p = min(start[k] + rank[i], (uint32_t)n - 1u);   // in bounds also for counts of another build
-    cell[p] = k;
-    bead[p] = (uint32_t)i;
-}
-
-__global__ __launch_bounds__(kThreads) void k_scan_cells(WinBook wb, uint32_t *__restrict__ start)
-{
-    __shared__ uint32_t lds[2 * kWavesPerBlock];
-    scan_cells(blockIdx.x, wb, start, lds);
-}
-
-__global__ __launch_bounds__(kThreads) void k_place(int n, const uint32_t *__restrict__ key,
-                                                    const uint32_t *__restrict__ rank,
-                                                    const uint32_t *__restrict__ start, uint32_t *__restrict__ cell,
-                                                    uint32_t *__restrict__ bead)
-{
-    const int i = blockIdx.x * kThreads + threadIdx.x;
-    if (i < n) place_bead(i, n, key, rank, start, cell, bead);
-}
-
-struct WArgs {
-    uint32_t *kA, *vA, *kB, *vB, *kC, *vC;
-    WinBook wb;
-    uint32_t *start;
-    uint32_t *ghist;        // the cell indices' digit histograms [copies][4][256]
-    uint32_t *ctr;          // 2 tile counters: the fallback's second and third pass
-    uint32_t *bar;          // 2 barrier counters
-    uint32_t *status;       // look-back words of the fallback's three passes, tiles x 256 each
-    int *errflag;
-    const DevRep *reps;     // the cell grid: replica 0's
-    int tiles;
-};
 
 template <int kRounds>
-__global__ __launch_bounds__(kThreads) void k_window(int n, int launch, WArgs a)
+__device__ void build_sorted(WLds<kRounds> &L, int n, const BuildArgs &a, const WinDesc &w, bool dense)
 {
-    __shared__ WLds<kRounds> L;
-    const int t = threadIdx.x;
-    const WinDesc w = load_win(a.wb.desc);
-    const bool fallback = w.wx == 0u || *a.wb.flag != 0u;
-    if (!fallback) {
-        if (launch == 0) {
-            const int tiles = (int)((w.wx * w.wy * w.wz + kCoarseCells - 1) / kCoarseCells);
-            for (int c = blockIdx.x; c < tiles; c += gridDim.x) scan_cells(c, a.wb, a.start, L.scan);
-        } else {
-            const int i = blockIdx.x * kThreads + t;
-            if (i < n) place_bead(i, n, a.kA, a.vA, a.start, a.kB, a.vB);
-        }
-        return;
-    }
+    const int t = threadIdx.x, lane = t & (kWave - 1), wave = t / kWave, tile = blockIdx.x;
     uint32_t *st0 = a.status, *st1 = st0 + (size_t)a.tiles * 256, *st2 = st1 + (size_t)a.tiles * 256;
-    if (launch != 0) {
-        // the counts of the keys that did lie in the window
-        if (w.wx != 0u)
-            for (int c = blockIdx.x * kThreads + t; c < kWinCells; c += gridDim.x * kThreads) a.wb.counts[c] = 0u;
-        if ((int)blockIdx.x >= a.tiles) return;   // workgroups past the tiles
-        if (t == 0) L.tile = atomicAdd(a.ctr + 1, 1u);
-        __syncthreads();
-        wpass<kRounds>(L, n, 16, (int)L.tile, hist_sum(a.ghist + 512), false, a.kC, a.vC, a.kA, a.vA, st2, a.errflag);
-        return;
-    }
+    uint32_t *bar = a.wb.flag + 1;
+    // the counts of the keys that did lie in the window
+    if (dense || w.wx != 0u)
+        for (uint32_t c = tile * kThreads + t; c < a.wb.limit; c += a.tiles * kThreads) a.wb.counts[c] = 0u;
     // every key back to its cell index (window keys), its three digits counted (the key
     // kernel counted none), and the occupied cell range measured for the next window
     const uint32_t nx = (uint32_t)a.reps[0].nc[0], ny = (uint32_t)a.reps[0].nc[1];
-    const int lane = t & (kWave - 1), wave = t / kWave;
     for (int p = 0; p < 3; p++) L.h[p][t] = 0u;
     __syncthreads();
     uint32_t m[6] = {0u, 0u, 0u, 0u, 0u, 0u};
-    const int base = blockIdx.x * kThreads * kRounds;
+    const int base = tile * kThreads * kRounds;
+    uint32_t kr[kRounds], cr[kRounds];
+#pragma unroll
+    for (int r = 0; r < kRounds; r++) {
+        const int i = min(base + r * kThreads + t, n - 1);
+        kr[r] = a.k0[i];
+        cr[r] = min(a.cells_old[i], a.wb.limit - 1u);
+    }
+#pragma unroll
     for (int r = 0; r < kRounds; r++) {
         const int i = base + r * kThreads + t;
         if (i < n) {
-            uint32_t k = a.kA[i];
+            a.counts_old[cr[r]] = 0u;
+            uint32_t k = kr[r];
             if (k & kWinTag) {
                 const uint32_t wk = k & ~kWinTag;
                 const uint32_t q = wk / w.wx, x = wk - q * w.wx, z = q / w.wy, y = q - z * w.wy;
                 k = ((z + w.z0) * ny + (y + w.y0)) * nx + (x + w.x0);
-                a.kA[i] = k;
+                a.k0[i] = k;
             }
             for (int p = 0; p < 3; p++) atomicAdd(&L.h[p][(k >> (8 * p)) & 255u], 1u);
-            const uint32_t q = k / nx, cx = k - q * nx, cz = q / ny, cy = q - cz * ny;
-            m[0] = max(m[0], cx + 1u);
-            m[1] = max(m[1], cy + 1u);
-            m[2] = max(m[2], cz + 1u);
-            m[3] = max(m[3], kBoxEnc - cx);
-            m[4] = max(m[4], kBoxEnc - cy);
-            m[5] = max(m[5], kBoxEnc - cz);
+            if (!dense) {
+                const uint32_t q = k / nx, cx = k - q * nx, cz = q / ny, cy = q - cz * ny;
+                m[0] = max(m[0], cx + 1u);
+                m[1] = max(m[1], cy + 1u);
+                m[2] = max(m[2], cz + 1u);
+                m[3] = max(m[3], kBoxEnc - cx);
+                m[4] = max(m[4], kBoxEnc - cy);
+                m[5] = max(m[5], kBoxEnc - cz);
+            }
         }
     }
 #pragma unroll
@@ -749,21 +773,92 @@ __global__ __launch_bounds__(kThreads) void k_window(int n, int launch, WArgs a)
     if (lane == 0)
         for (int j = 0; j < 6; j++) L.bb[wave][j] = m[j];
     __syncthreads();
-    uint32_t *gh = a.ghist + (size_t)(blockIdx.x % kHistCopies) * 1024;
+    uint32_t *gh = a.ghist + (size_t)(tile % kHistCopies) * 1024;
     for (int p = 0; p < 3; p++)
         if (L.h[p][t]) atomicAdd(&gh[p * 256 + t], L.h[p][t]);
     if (t < 6) {
         uint32_t v = 0u;
         for (int q = 0; q < kWavesPerBlock; q++) v = max(v, L.bb[q][t]);
-        if (v) atomicMax(&a.wb.bbox[(blockIdx.x % kHistCopies) * 8 + t], v);
+        if (v) atomicMax(&a.wb.bbox[(tile % kHistCopies) * 8 + t], v);
     }
-    grid_sync(a.bar, gridDim.x, a.errflag);
-    // all of the launch's workgroups are resident, so the first pass's tiles are theirs in order
-    wpass<kRounds>(L, n, 0, blockIdx.x, hist_sum(a.ghist), true, a.kA, a.vA, a.kB, a.vB, st0, a.errflag);
-    grid_sync(a.bar + 1, gridDim.x, a.errflag);
-    if (t == 0) L.tile = atomicAdd(a.ctr, 1u);
-    __syncthreads();
-    wpass<kRounds>(L, n, 8, (int)L.tile, hist_sum(a.ghist + 256), false, a.kB, a.vB, a.kC, a.vC, st1, a.errflag);
+    // all the tiles' workgroups are resident, so each pass's tiles are theirs in order
+    grid_sync(bar, a.tiles, a.errflag);
+    wpass<kRounds>(L, n, 0, tile, hist_sum(a.ghist), true, a.k0, a.v0, a.k1, a.v1, st0, a.errflag);
+    grid_sync(bar + 1, a.tiles, a.errflag);
+    wpass<kRounds>(L, n, 8, tile, hist_sum(a.ghist + 256), false, a.k1, a.v1, a.k2, a.v2, st1, a.errflag);
+    grid_sync(bar + 2, a.tiles, a.errflag);
+    wpass<kRounds>(L, n, 16, tile, hist_sum(a.ghist + 512), false, a.k2, a.v2, a.k0, a.v0, st2, a.errflag);
+    grid_sync(bar + 3, a.tiles, a.errflag);
+    uint32_t vr[kRounds];
+#pragma unroll
+    for (int r = 0; r < kRounds; r++) vr[r] = min(a.v0[min(base + r * kThreads + t, n - 1)], (uint32_t)n - 1u);
+    Bead br[kRounds];
+#pragma unroll
+    for (int r = 0; r < kRounds; r++) br[r] = a.beads[vr[r]];
+#pragma unroll
+    for (int r = 0; r < kRounds; r++) {
+        const int s = base + r * kThreads + t;
+        if (s < n) {
+            const uint32_t k = a.k0[s], kprev = a.k0[s > 0 ? s - 1 : 0], knext = a.k0[s < n - 1 ? s + 1 : s];
+            a.sbeads[s] = br[r];
+            a.k2[s] = k;
+            if (s == 0 || kprev != k) a.cstart[k] = s;
+            if (s == n - 1 || knext != k) a.cend[k] = s + 1;
+        }
+    }
+}
+
+// The next build's window: this build's after the fast path; after the fallback, the
+// occupied cell range that it measured, widened by one cell on each side and clipped to the grid,
+// or none (wx = 0) when that holds more cells than there are counters.  By the first wave of a workgroup
+// that has passed the range's barrier.
+__device__ inline void next_window(const BuildArgs &a, const WinDesc &w, bool fallback)
+{
+    const int t = threadIdx.x;
+    uint32_t v = 0u;
+    if (fallback && t < 6)
+        for (int c = 0; c < kHistCopies; c++) v = max(v, a.wb.bbox[c * 8 + t]);
+    uint32_t f[6];
+#pragma unroll
+    for (int j = 0; j < 6; j++) f[j] = __shfl(v, j);
+    if (t != 0) return;
+    uint32_t d[6] = {w.x0, w.y0, w.z0, w.wx, w.wy, w.wz};
+    if (fallback) {
+        for (int j = 0; j < 6; j++) d[j] = 0u;
+        if (f[0] != 0u) {
+            unsigned long long cells = 1ull;
+            for (int x = 0; x < 3; x++) {
+                const int lo = max((int)(kBoxEnc - f[3 + x]) - 1, 0);
+                const int hi = min((int)f[x], a.reps[0].nc[x] - 1);
+                d[x] = (uint32_t)lo;
+                d[3 + x] = (uint32_t)(hi - lo + 1);
+                cells *= (unsigned long long)(hi - lo + 1);
+            }
+            if (cells > (unsigned long long)a.wb.limit)
+                for (int j = 0; j < 6; j++) d[j] = 0u;
+        }
+    }
+    for (int j = 0; j < 6; j++) a.desc_next[j] = d[j];
+}
+
+template <int kRounds>
+__global__ __launch_bounds__(kThreads) void k_build(int n, BuildArgs a)
+{
+    __shared__ union {
+        WLds<kRounds> w;
+        BLds b;
+    } L;
+    for (size_t i = (size_t)blockIdx.x * kThreads + threadIdx.x; i < a.clear_words; i += (size_t)gridDim.x * kThreads)
+        a.clear[i] = 0u;
+    const bool dense = a.wb.cells != 0u;
+    WinDesc w{};
+    if (!dense) w = load_win(a.wb.desc);
+    const bool fallback = (!dense && w.wx == 0u) || *a.wb.flag != 0u;   // the same in every workgroup
+    if (!fallback)
+        build_slots(L.b, n, a, w, dense);
+    else if ((int)blockIdx.x < a.tiles)
+        build_sorted<kRounds>(L.w, n, a, w, dense);
+    if (!dense && blockIdx.x == 0 && threadIdx.x < kWave) next_window(a, w, fallback);
 }
 
 }  // namespace
@@ -854,48 +949,39 @@ void sort_moved(hipStream_t st, SortBuffers &b, const MoveSort &m, int bits, int
 int move_blocks(int n) { return (n + 255) / 256; }
 
 // ---- the counting builds: host side ----
-static int sortw_tiles(int n)
+int build_tiles(int n)
 {
     const int tile = kThreads * sort_rounds(n);
     return (n + tile - 1) / tile;
 }
 
-bool sortw_fits(int n) { return n >= 1 && sortw_tiles(n) <= kWinMaxTiles && sort_rounds(n) != 12; }
+bool sortw_fits(int n) { return n >= 1 && build_tiles(n) <= kWinMaxTiles && sort_rounds(n) != 12; }
 
-size_t sortw_words(int n, bool window) { return kWinKeyWords + (window ? (size_t)3 * sortw_tiles(n) * 256 : 0); }
+size_t sortw_words(int n, bool counting) { return kWinKeyWords + (counting ? (size_t)3 * build_tiles(n) * 256 : 0); }
 
 uint32_t *win_scratch(uint32_t *sort_scratch, int n) { return sort_scratch + sort_scratch_words(n, 4); }
 
-WinBook win_book(uint32_t *sort_scratch, int n, const uint32_t *desc, uint32_t *counts, uint32_t cells)
+size_t count_limit(int n)
+{
+    const long long want = std::min<long long>(std::max<long long>(4ll * n, 1 << 14), kWinCells);
+    return (size_t)((want + kCoarseCells - 1) / kCoarseCells * kCoarseCells);
+}
+
+WinBook win_book(uint32_t *sort_scratch, int n, const uint32_t *desc, uint32_t *counts, uint32_t *bucket,
+                 uint32_t cells, uint32_t limit)
 {
     uint32_t *ws = win_scratch(sort_scratch, n);
     uint32_t *bbox = ws + (size_t)kCoarseCopies * kCoarse;
-    return WinBook{desc, ws, bbox, bbox + 16 * 8, counts, cells};
+    return WinBook{desc, ws, bbox, bbox + 16 * 8, counts, bucket, cells, limit};
 }
 
-void count_build(hipStream_t st, SortBuffers &b, uint32_t *k2, uint32_t *v2, int parity, const WinBook &wb,
-                 uint32_t *start, const DevRep *reps)
+void launch_build(hipStream_t st, int n, const BuildArgs &a)
 {
-    const int n = b.n;
-    const int blocks = (n + kThreads - 1) / kThreads;
-    if (wb.cells != 0u) {
-        hipLaunchKernelGGL(k_scan_cells, dim3((wb.cells + kCoarseCells - 1) / kCoarseCells), dim3(kThreads), 0, st, wb, start);
-        hipLaunchKernelGGL(k_place, dim3(blocks), dim3(kThreads), 0, st, n, b.k0, b.v0, start, b.k1, b.v1);
-        return;
-    }
-    const int tiles = sortw_tiles(n);
-    b.tiles = tiles;
-    uint32_t *misc = wb.flag;   // flag, 2 tile counters, 2 barrier counters
-    const WArgs a{b.k0, b.v0, b.k1, b.v1, k2, v2, wb, start, b.scratch[parity], misc + 1, misc + 3,
-                  win_scratch(b.scratch[parity], n) + kWinKeyWords, b.errflag, reps, tiles};
-    // the window path's second launch has a thread a bead, more workgroups than the fallback's tiles
-    for (int launch = 0; launch < 2; launch++) {
-        const dim3 grid(launch == 0 ? tiles : blocks);
-        if (sort_rounds(n) == 2)
-            hipLaunchKernelGGL(k_window<2>, grid, dim3(kThreads), 0, st, n, launch, a);
-        else
-            hipLaunchKernelGGL(k_window<8>, grid, dim3(kThreads), 0, st, n, launch, a);
-    }
+    const dim3 grid((n + kThreads - 1) / kThreads), block(kThreads);
+    if (sort_rounds(n) == 2)
+        hipLaunchKernelGGL(k_build<2>, grid, block, 0, st, n, a);
+    else
+        hipLaunchKernelGGL(k_build<8>, grid, block, 0, st, n, a);
 }
 
 }  // namespace smdev

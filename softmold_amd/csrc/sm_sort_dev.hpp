@@ -61,29 +61,29 @@ __device__ inline WinDesc load_win(const uint32_t *d) { return WinDesc{d[0], d[1
 constexpr uint32_t kBoxEnc = 1u << 20;
 
 // The end of a key kernel's block in a counting build; every thread of the 256-thread block
-// calls it and gets the key to store and the bead's arrival number in its cell.  A key in the
-// window (or any key, in a dense build) adds one to its cell's count and gets the count
-// before it: the lanes of a wave whose neighbours hold the same cell (the beads of one lipid)
+// calls it and gets the key to store.  A key in the window (or any key, in a dense build) adds
+// one to its cell's count and enters bead i into the cell's bucket under the count before it:
+// the lanes of a wave whose neighbours hold the same cell (the beads of one lipid)
 // add together, since the counts live beyond the L2s and take about 25 atomics a ns
 // (240k beads one by one: 8 us more than by runs).  The coarse counts are gathered per block
-// first.  A key outside the window sets the fallback flag.  hs: kCoarse LDS words, zero on
-// entry.
+// first.  A key outside the window, or past the bucket, sets the fallback flag.  hs: kCoarse
+// LDS words, zero on entry.
 __device__ inline uint32_t win_key_end(const WinBook &wb, const WinDesc &w, uint32_t *hs, uint32_t k, int cx, int cy,
-                                       int cz, bool valid, uint32_t &rank)
+                                       int cz, int i, bool valid)
 {
     const int t = threadIdx.x, lane = t & (kWave - 1);
     const bool dense = wb.cells != 0u;
-    rank = 0u;
     if (!dense && w.wx == 0u) return k;   // workgroup-uniform: no window
     bool in = valid;
     uint32_t wk = k;
+    bool bad = false;
     if (!dense) {
         const uint32_t dx = (uint32_t)cx - w.x0, dy = (uint32_t)cy - w.y0, dz = (uint32_t)cz - w.z0;
         in = valid && dx < w.wx && dy < w.wy && dz < w.wz;
         wk = (dz * w.wy + dy) * w.wx + dx;
-        if (__ballot(valid && !in) != 0ull && lane == 0) atomicOr(wb.flag, 1u);
+        bad = valid && !in;
     }
-    in = in && wk < (uint32_t)kWinCells;   // always, within a window or a dense table
+    in = in && wk < wb.limit;   // always, within a window or a dense table
     const uint32_t id = in ? wk : ~0u;
     const uint32_t prev = (uint32_t)__shfl_up((int)id, 1);
     const unsigned long long heads = __ballot(lane == 0 || prev != id);
@@ -96,7 +96,9 @@ __device__ inline uint32_t win_key_end(const WinBook &wb, const WinDesc &w, uint
         first = atomicAdd(&wb.counts[wk], run);
         atomicAdd(&hs[wk / kCoarseCells], run);
     }
-    rank = (uint32_t)__shfl((int)first, head) + (uint32_t)(lane - head);
+    const uint32_t rank = (uint32_t)__shfl((int)first, head) + (uint32_t)(lane - head);
+    if (in && rank < (uint32_t)kBucket) wb.bucket[(size_t)wk * kBucket + rank] = (uint32_t)i;
+    if (__ballot(bad || (in && rank >= (uint32_t)kBucket)) != 0ull && lane == 0) atomicOr(wb.flag, 1u);
     __syncthreads();
     if (t < kCoarse && hs[t]) atomicAdd(&wb.coarse[(blockIdx.x % kCoarseCopies) * kCoarse + t], hs[t]);
     return dense ? k : (in ? (kWinTag | wk) : k);
