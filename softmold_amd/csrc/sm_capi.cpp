@@ -1158,13 +1158,15 @@ sm_ctx *create(const sm_system *s, int nrep)
             HIPCHK(hipMemcpyAsync(c->chainList, list.data(), sizeof(int2) * list.size(), hipMemcpyHostToDevice, st));
             HIPCHK(hipMemcpyAsync(c->cconstD, ccD.data(), sizeof(double4) * ccD.size(), hipMemcpyHostToDevice, st));
         }
-        // sorted slots per wave in the pair kernel: short chunks keep small systems filling
-        // the chip, longer ones cut the per-cell overhead of large ones (measured on the
-        // 15k, 240k and 3M-bead systems; every chunk gives the same forces); from one and a
-        // half million beads on 16 slots (pair kernel, 8 -> 16 slots: 3M vesicle 995 -> 950 us,
-        // 3M bilayer 1028 -> 1000, the 64-vesicle sweep 848 -> 813; whole steps: 1.8M beads in
-        // 12 bilayers 812 -> 807, one 1.35M bilayer 615 -> 620, 960k beads in 40 468 -> 477)
-        c->chunk = n >= 1500000 ? 16 : (n >= 50000 ? 8 : 2);
+        // sorted slots per wave in the pair kernels: short chunks keep small systems filling the
+        // chip and even out flat ones, longer ones cut the overhead per wave (every chunk gives
+        // the same forces).  Whole steps in us at 2, 4, 8, 16 slots: 1.5k vesicle 27.1, 28 at 4;
+        // 18k bilayer 48.0, 46.7; 90k vesicle 63.7, 62.3, 61.7; 120k 74.5, 72.5, 71.7; 300k
+        // bilayer 148 at 4, 158, 178; 990k bilayer 450 at 4, 451, 468; 3M bilayer 1216 at 4,
+        // 1188, 1191; 1.35M vesicle 530 at 8, 522; 3M vesicle 1123 at 8, 1098; 1.5M beads in 64
+        // bilayers 648 at 8, 658.
+        const int many = c->P.flat ? 1000000 : 100000;
+        c->chunk = n < 10000 ? 2 : (n < many ? 4 : (n < 2000000 || c->P.flat ? 8 : 16));
         c->ensure_capacity(0);
         HIPCHK(hipStreamSynchronize(st));
     } catch (...) {

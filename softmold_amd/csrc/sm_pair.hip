@@ -358,8 +358,8 @@ struct Out {
 // of the particle the reference's traversal makes first (home_first).  ONE: a
 // single-replica context, whose box and grid are read from reps[0] once rather than per
 // cell after the home bead's replica index.
-template <int MODE, bool ASYM, bool ONE = false>
-__global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(4))) void k_cells(
+template <int MODE, bool ASYM, bool ONE, int MAXC, int WAVES>
+__global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(WAVES))) void k_cells(
     int n, int nT, int chunk, int nblocks, double cut2, float cut2pre, const Bead *__restrict__ sb,
     const uint32_t *__restrict__ skey, const uint32_t *__restrict__ sidx, const int *__restrict__ cstart,
     const int *__restrict__ cend, const DevRep *__restrict__ reps, const float *__restrict__ tab,
@@ -377,10 +377,10 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
     // instead of evaluating them: same staging, culling, lists and FP64 test
     constexpr bool kFC = MODE == M_FCOUNT;
     constexpr bool kCull = kF1 || kE || kFC;           // candidates culled per quarter of the home cell
-    // staged candidates per pass: the force kernel measured fastest at 192; the two-phase
-    // force and the FP64 energy gathers at 128 (their larger constant tables and registers
-    // leave less LDS per resident wave)
-    constexpr int kMaxC = (k2P || kE || kFDU) ? 128 : 192;
+    // staged candidates per pass: the two-phase force and the FP64 energy gathers measured
+    // fastest at 128 (U of 240k beads 84 us, 92 with 192; with dU 177 and 205), the force see
+    // kManyBeads
+    constexpr int kMaxC = MAXC;
     constexpr int kStageIters = kMaxC / kWave;
     static_assert(kMaxC % kWave == 0, "staging rounds cover whole waves");
     // the constant rows, sized by the types there are (tables_bytes): six types leave room for
@@ -577,6 +577,10 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
                 double fx = 0.0, fy = 0.0, fz = 0.0;
                 double accu = 0.0;
                 int cnt = 0;
+                // a lane's next candidate in its quarter's list; past a pass's end it goes on
+                // into the next one's, so that every tpp-th candidate of the cell is this
+                // lane's however the passes cut the list, and the sums do not depend on kMaxC
+                int next = sub;
                 for (int cb = 0; cb < total; cb += kMaxC) {
                     const int ce = min(total, cb + kMaxC);
                     // staging rounds this pass needs (wave-uniform): the unrolled rounds
@@ -586,7 +590,7 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
                     // map of the pass: every stencil cell with slots in [cb, ce) marks its
                     // first one with its index (the cell holding slot cb marks position 0),
                     // and a max-scan over the positions gives each slot its cell
-                    if (lane < kMaxC / 4) sLists[wave][lane] = 0u;
+                    for (int t = lane; t < kMaxC / 4; t += kWave) sLists[wave][t] = 0u;
                     if (lane < 27 && ncnt > 0 && incl > cb && excl < ce) mapW[max(excl, cb) - cb] = (uint8_t)lane;
                     wave_lds_sync();
                     int src[kStageIters], cel[kStageIters];
@@ -688,10 +692,10 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
                         const int nl = quad == 0 ? nq[0] : (quad == 1 ? nq[1] : (quad == 2 ? nq[2] : nq[3]));
                         // the next entry is read one iteration ahead (entries past nl fall in
                         // the next list or the padding and are never used)
-                        int inext = lst[sub];
-                        for (int jj = sub; jj < nl; jj += tpp) {
+                        int inext = lst[next];
+                        for (; next < nl; next += tpp) {
                             const int i0 = inext;
-                            inext = lst[jj + tpp];
+                            inext = lst[next + tpp];
                             const Cand q = cand_at(i0);
                             const int tq = q.t & 0xff, c = q.t >> 8;
                             const double dxd = hb.x - q.x, dyd = hb.y - q.y, dzd = hb.z - q.z;
@@ -706,6 +710,7 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
                             const bool owned = c == 13 ? q.c > hslot : ((fwd >> c) & 1u) != 0;
                             if (owned) accu += du_pair(dxd, dyd, dzd, r2, sCd + 6 * row, cut2, s2x, s2y, s2z, dseries);
                         }
+                        next -= nl;
                     } else if ((MODE == M_FORCE1 || kFC) && act) {
                         // one phase over the home's quarter list: FP64 test, force law under
                         // the branch; two candidates per trip so both LDS reads are in
@@ -717,8 +722,8 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
                         const int nl = quad == 0 ? nq[0] : (quad == 1 ? nq[1] : (quad == 2 ? nq[2] : nq[3]));
                         // the next trip's list entries are read one trip ahead (entries past
                         // nl fall in the next list or the padding and are never used)
-                        int j = sub;
-                        const uint16_t *lp = lst + sub;
+                        int j = next;
+                        const uint16_t *lp = lst + next;
                         int i0 = lp[0], i1 = lp[tpp];
                         for (; j + tpp < nl; j += 2 * tpp) {
                             lp += 2 * tpp;
@@ -746,7 +751,9 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
                                 force_term_asym(hb, q0, q0.c != hslot, cut2, sC8, nT, me, sidx, fx, fy, fz);
                             else
                                 force_term(hb, q0, q0.c != hslot, cut2, C8, fx, fy, fz);
+                            j += tpp;
                         }
+                        next = j - nl;
                     } else if (k2P) {
                         const float4 *C8 = sC8 + 2 * hb.type * nT;
                         uint8_t *lst = &sList[k2P ? wave : 0][0][lane];
@@ -800,12 +807,13 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
                             if (MODE == M_U) return r2 < cut2 ? pair_u_any(r2, C) : 0.0;
                             return du_pair(dx, dy, dz, r2, C, cut2, s2x, s2y, s2z, dseries);
                         };
-                        int inext = lst[sub];   // read one iteration ahead, as above
-                        for (int jj = sub; jj < nl; jj += tpp) {
+                        int inext = lst[next];   // read one iteration ahead, as above
+                        for (; next < nl; next += tpp) {
                             const int i0 = inext;
-                            inext = lst[jj + tpp];
+                            inext = lst[next + tpp];
                             accu += term(cand_at(i0), cb + i0 / (int)sizeof(Cand));
                         }
+                        next -= nl;
                     } else if (!kF && act) {
                         // neighbour counts and pair lists see both sides of every pair
                         for (int j = cb + sub; j < ce; j += tpp) {
@@ -879,7 +887,7 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
     }
 }
 
-template <int MODE, bool ASYM = false, bool ONE = false>
+template <int MODE, bool ASYM = false, bool ONE = false, int MAXC = 128, int WAVES = 4>
 void launch_cells(hipStream_t st, const Params &P, int chunk, const Bead *sbeads, const uint32_t *skey,
                   const uint32_t *sidx, const int *cstart, const int *cend, const DevRep *reps,
                   const float *fconst, const double *uconst, const Out &out)
@@ -904,9 +912,32 @@ void launch_cells(hipStream_t st, const Params &P, int chunk, const Bead *sbeads
     const int turn = energy ? 6 : (P.flat ? 7 : 0);
     const bool floats = MODE == M_FORCE || MODE == M_FORCE1 || MODE == M_FDU, doubles = !floats || MODE == M_FDU;
     const size_t tables_bytes = (size_t)P.nT * P.nT * ((floats ? 2 * sizeof(float4) : 0) + (doubles ? 6 * sizeof(double) : 0));
-    hipLaunchKernelGGL((k_cells<MODE, ASYM, ONE>), dim3(nb), dim3(kWaves * kWave), tables_bytes, st, P.n, P.nT, chunk, nb, cut2, cut2pre,
+    hipLaunchKernelGGL((k_cells<MODE, ASYM, ONE, MAXC, WAVES>), dim3(nb), dim3(kWaves * kWave), tables_bytes, st, P.n, P.nT, chunk, nb, cut2, cut2pre,
                        sbeads, skey, sidx, cstart, cend, reps, fconst, uconst, turn, out);
 }
+
+// the instance for the tables' symmetry and, where ONEs says so, for one replica
+template <int MODE, int MAXC, int WAVES, bool ONES, class... A>
+void launch_for(const Params &P, hipStream_t st, const A &...args)
+{
+    const bool one = ONES && P.nrep == 1;
+    if (P.asym && one)
+        launch_cells<MODE, true, ONES, MAXC, WAVES>(st, P, args...);
+    else if (P.asym)
+        launch_cells<MODE, true, false, MAXC, WAVES>(st, P, args...);
+    else if (one)
+        launch_cells<MODE, false, ONES, MAXC, WAVES>(st, P, args...);
+    else
+        launch_cells<MODE, false, false, MAXC, WAVES>(st, P, args...);
+}
+
+// Candidates per pass and waves per SIMD of the force.  From 100k beads on the waves that are
+// ready to issue count: 128 candidates leave registers and LDS for five waves instead of the
+// four that 192 leave (240k vesicle 91.4 -> 89.2 us, the 64-vesicle sweep 739 -> 702).
+// Smaller systems have few waves a SIMD as it is, and a pass less is worth more (12k bilayer
+// 24.5 us with 192, 26.0 with 128; 29k 29.8 and 32.1; 60k vesicle 36.5 and 36.8).  The sums are
+// the same bit for bit.
+constexpr int kManyBeads = 100000;
 
 }  // namespace
 
@@ -921,18 +952,12 @@ void launch_pair_force(hipStream_t st, const Params &P, int chunk, int variant, 
                        const DevRep *reps, const float *fconst, float4 *fpair)
 {
     Out o{fpair, nullptr, nullptr, nullptr, nullptr, 0};
-    if (variant == 1 && P.asym)
-        launch_cells<M_FORCE, true>(st, P, chunk, sbeads, skey, sidx, cstart, cend, reps, fconst, nullptr, o);
-    else if (variant == 1)
-        launch_cells<M_FORCE>(st, P, chunk, sbeads, skey, sidx, cstart, cend, reps, fconst, nullptr, o);
-    else if (P.asym && P.nrep == 1)
-        launch_cells<M_FORCE1, true, true>(st, P, chunk, sbeads, skey, sidx, cstart, cend, reps, fconst, nullptr, o);
-    else if (P.asym)
-        launch_cells<M_FORCE1, true>(st, P, chunk, sbeads, skey, sidx, cstart, cend, reps, fconst, nullptr, o);
-    else if (P.nrep == 1)
-        launch_cells<M_FORCE1, false, true>(st, P, chunk, sbeads, skey, sidx, cstart, cend, reps, fconst, nullptr, o);
+    if (variant == 1)
+        launch_for<M_FORCE, 128, 4, false>(P, st, chunk, sbeads, skey, sidx, cstart, cend, reps, fconst, nullptr, o);
+    else if (P.n >= kManyBeads)
+        launch_for<M_FORCE1, 128, 5, true>(P, st, chunk, sbeads, skey, sidx, cstart, cend, reps, fconst, nullptr, o);
     else
-        launch_cells<M_FORCE1>(st, P, chunk, sbeads, skey, sidx, cstart, cend, reps, fconst, nullptr, o);
+        launch_for<M_FORCE1, 192, 4, true>(P, st, chunk, sbeads, skey, sidx, cstart, cend, reps, fconst, nullptr, o);
 }
 
 void launch_pair_force_du(hipStream_t st, const Params &P, int chunk, const Bead *sbeads, const uint32_t *skey,
@@ -940,14 +965,7 @@ void launch_pair_force_du(hipStream_t st, const Params &P, int chunk, const Bead
                           const float *fconst, const double *uconst, float4 *fpair, double *energy)
 {
     Out o{fpair, energy, nullptr, nullptr, nullptr, 0};
-    if (P.asym && P.nrep == 1)
-        launch_cells<M_FDU, true, true>(st, P, chunk, sbeads, skey, sidx, cstart, cend, reps, fconst, uconst, o);
-    else if (P.asym)
-        launch_cells<M_FDU, true>(st, P, chunk, sbeads, skey, sidx, cstart, cend, reps, fconst, uconst, o);
-    else if (P.nrep == 1)
-        launch_cells<M_FDU, false, true>(st, P, chunk, sbeads, skey, sidx, cstart, cend, reps, fconst, uconst, o);
-    else
-        launch_cells<M_FDU>(st, P, chunk, sbeads, skey, sidx, cstart, cend, reps, fconst, uconst, o);
+    launch_for<M_FDU, 128, 4, true>(P, st, chunk, sbeads, skey, sidx, cstart, cend, reps, fconst, uconst, o);
 }
 
 void launch_pair_gather(hipStream_t st, const Params &P, int chunk, int mode, const Bead *sbeads,
@@ -958,25 +976,16 @@ void launch_pair_gather(hipStream_t st, const Params &P, int chunk, int mode, co
     Out o{nullptr, energy, counts, pairs, npairs, cap};
     switch (mode) {
     case GATHER_U:
-        if (P.asym)
-            launch_cells<M_U, true>(st, P, chunk, sbeads, skey, sidx, cstart, cend, reps, tab, uconst, o);
-        else
-            launch_cells<M_U>(st, P, chunk, sbeads, skey, sidx, cstart, cend, reps, tab, uconst, o);
+        launch_for<M_U, 128, 4, false>(P, st, chunk, sbeads, skey, sidx, cstart, cend, reps, tab, uconst, o);
         break;
     case GATHER_DU:
-        if (P.asym)
-            launch_cells<M_DU, true>(st, P, chunk, sbeads, skey, sidx, cstart, cend, reps, tab, uconst, o);
-        else
-            launch_cells<M_DU>(st, P, chunk, sbeads, skey, sidx, cstart, cend, reps, tab, uconst, o);
+        launch_for<M_DU, 128, 4, false>(P, st, chunk, sbeads, skey, sidx, cstart, cend, reps, tab, uconst, o);
         break;
     case GATHER_COUNT:
         launch_cells<M_COUNT>(st, P, chunk, sbeads, skey, sidx, cstart, cend, reps, tab, uconst, o);
         break;
     case GATHER_FCOUNT:
-        if (P.asym)
-            launch_cells<M_FCOUNT, true>(st, P, chunk, sbeads, skey, sidx, cstart, cend, reps, tab, uconst, o);
-        else
-            launch_cells<M_FCOUNT>(st, P, chunk, sbeads, skey, sidx, cstart, cend, reps, tab, uconst, o);
+        launch_for<M_FCOUNT, 192, 4, false>(P, st, chunk, sbeads, skey, sidx, cstart, cend, reps, tab, uconst, o);
         break;
     default: launch_cells<M_LIST>(st, P, chunk, sbeads, skey, sidx, cstart, cend, reps, tab, uconst, o); break;
     }
