@@ -262,7 +262,7 @@ struct sm_ctx {
     int *dcounts = nullptr, *dpairs = nullptr;
     long long pairs_cap = 0;
     unsigned long long *dnp = nullptr;
-    int chunk = 8;
+    int chunk = 8, echunk = 8;   // sorted slots per wave: the force and the counts; the FP64 energy traversals
     int pair_variant = 0;
     // box-move steps: the pair dU in the same traversal as the step's pair force (1) or in
     // a gather of its own after the kick (0, as the adjoint uses)
@@ -585,7 +585,7 @@ struct sm_ctx {
     void measure_device()
     {
         timed(K_GATHER, [&] {
-            launch_pair_gather(st, P, chunk, GATHER_U, sbeads, skey(), sidx(), cstart, cend, reps, fconstF, uconstD, ebead,
+            launch_pair_gather(st, P, echunk, GATHER_U, sbeads, skey(), sidx(), cstart, cend, reps, fconstF, uconstD, ebead,
                                nullptr, nullptr, nullptr, 0);
         });
         timed(K_SUMS, [&] {
@@ -616,7 +616,7 @@ struct sm_ctx {
     void add_energies(double *out)
     {
         timed(K_GATHER, [&] {
-            launch_pair_gather(st, P, chunk, GATHER_U, sbeads, skey(), sidx(), cstart, cend, reps, fconstF, uconstD, ebead,
+            launch_pair_gather(st, P, echunk, GATHER_U, sbeads, skey(), sidx(), cstart, cend, reps, fconstF, uconstD, ebead,
                                nullptr, nullptr, nullptr, 0);
         });
         timed(K_SUMS, [&] {
@@ -638,7 +638,7 @@ struct sm_ctx {
     void delta_device()
     {
         timed(K_GATHER, [&] {
-            launch_pair_gather(st, P, chunk, GATHER_DU, sbeads, skey(), sidx(), cstart, cend, reps, fconstF, uconstD, edelta,
+            launch_pair_gather(st, P, echunk, GATHER_DU, sbeads, skey(), sidx(), cstart, cend, reps, fconstF, uconstD, edelta,
                                nullptr, nullptr, nullptr, 0);
         });
         delta_sums();
@@ -681,7 +681,7 @@ struct sm_ctx {
     void pair_force_du()
     {
         timed(K_PAIR, [&] {
-            launch_pair_force_du(st, P, chunk, sbeads, skey(), sidx(), cstart, cend, reps, fconstF, uconstD, fpair,
+            launch_pair_force_du(st, P, echunk, sbeads, skey(), sidx(), cstart, cend, reps, fconstF, uconstD, fpair,
                                  edelta);
         });
     }
@@ -1167,6 +1167,12 @@ sm_ctx *create(const sm_system *s, int nrep)
         // bilayers 648 at 8, 658.
         const int many = c->P.flat ? 1000000 : 100000;
         c->chunk = n < 10000 ? 2 : (n < many ? 4 : (n < 2000000 || c->P.flat ? 8 : 16));
+        // The energy traversals do more per candidate.  Force with dU and U in us: 1.5k vesicle
+        // 24 and 15.0 at 2, 31 and 19.4 at 8; 12k bilayer 57 and 29.4 at 2, 46 and 25.4 at 8; 37k
+        // vesicle 54 and 29.2 at 2, 51 and 27.1 at 4, 49 and 29.6 at 8; 90k bilayer 84 and 44.2
+        // at 4, 82 and 43.0 at 8; 1.2M vesicle 687 and 325 at 8, 677 and 317 at 16; 1.2M bilayer
+        // 653 and 311 at 8, 667 and 317 at 16.
+        c->echunk = n < 10000 ? 2 : (c->P.flat ? 8 : (n < 50000 ? 4 : (n < 1000000 ? 8 : 16)));
         c->ensure_capacity(0);
         HIPCHK(hipStreamSynchronize(st));
     } catch (...) {
@@ -1607,7 +1613,7 @@ int sm_tune(sm_ctx *c, const char *knob, int32_t value)
         if (!c || !knob) invalid("null argument");
         if (std::strcmp(knob, "pair_chunk") == 0) {
             if (value < 1 || value > 4096) invalid("pair_chunk must be in [1, 4096]");
-            c->chunk = value;
+            c->chunk = c->echunk = value;
         } else if (std::strcmp(knob, "pair_variant") == 0) {
             if (value < 0 || value > 1) invalid("pair_variant must be 0 or 1");
             c->pair_variant = value;
@@ -2102,7 +2108,7 @@ int sm_param_derivative(sm_ctx *c, int32_t type_a, int32_t type_b, double *out)
         const size_t nt = 6 * (size_t)c->P.nT * c->P.nT;
         double *e[2] = {c->ebead, c->edelta};
         for (int p = 0; p < 2; p++)
-            launch_pair_gather(c->st, c->P, c->chunk, GATHER_U, c->sbeads, c->skey(), c->sidx(), c->cstart, c->cend,
+            launch_pair_gather(c->st, c->P, c->echunk, GATHER_U, c->sbeads, c->skey(), c->sidx(), c->cstart, c->cend,
                                c->reps, c->pdTab + p * c->pd_tab, c->pdU + p * nt, e[p], nullptr, nullptr, nullptr, 0);
         // the measurement words are free between calls (each measurement copies its own out)
         SumArgs a = c->sums(e[0], c->dres);
