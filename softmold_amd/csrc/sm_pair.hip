@@ -376,7 +376,13 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
     // the one-phase force traversal counting its accepted pairs with a nonzero term
     // instead of evaluating them: same staging, culling, lists and FP64 test
     constexpr bool kFC = MODE == M_FCOUNT;
-    constexpr bool kCull = kF1 || kE || kFC;           // candidates culled per quarter of the home cell
+    constexpr bool kCull = kF1 || kE || kFC;           // candidates culled per quarter of a box:
+    // the home cell's, or that of its homes, which a membrane leaves a third smaller.  The
+    // homes' box saves 10 to 14 % of the candidate tests for 75 instructions a cell: 6 % of the
+    // 90k bilayer's force with dU (90.9 -> 85.4 us), 3 % of the 240k vesicle's (177 -> 171), 5 and
+    // 1 % of their U; the force alone has cheaper tests and no registers left for it (240k 89.2
+    // -> 94.8 us)
+    constexpr bool kTight = kFDU || kE;
     // staged candidates per pass: the two-phase force and the FP64 energy gathers measured
     // fastest at 128 (U of 240k beads 84 us, 92 with 192; with dU 177 and 205), the force see
     // kManyBeads
@@ -581,6 +587,7 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
                 // into the next one's, so that every tpp-th candidate of the cell is this
                 // lane's however the passes cut the list, and the sums do not depend on kMaxC
                 int next = sub;
+                [[maybe_unused]] float xlo = 0.f, xmid = 0.f, xhi = 0.f, ylo = 0.f, ymid = 0.f, yhi = 0.f, zlo = 0.f, zhi = 0.f;
                 for (int cb = 0; cb < total; cb += kMaxC) {
                     const int ce = min(total, cb + kMaxC);
                     // staging rounds this pass needs (wave-uniform): the unrolled rounds
@@ -610,7 +617,28 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
                     for (int it = 0; it < kStageIters; it++)
                         if (it < iters) qb[it] = sb[max(src[it], 0)];
-                    bool near[kStageIters][4];   // the quarters of the home cell it can reach
+                    // the box of the batch's homes, relative to the cell centre, and its middle in
+                    // x and y (the loads of the pass are in flight); the largest of offset +- rel,
+                    // which is positive, through its bits
+                    if (kTight && cb == 0) {
+                        const float rx = (float)(hb0.x - ox0), ry = (float)(hb0.y - oy0), rz = (float)(hb0.z - oz0);
+                        const auto most = [](float v) {
+                            return __int_as_float(__builtin_amdgcn_readlane(wave_max_scan(__float_as_int(v)), kWave - 1));
+                        };
+                        const float ax2 = 2.f * hcx, ay2 = 2.f * hcy, az2 = 2.f * hcz;
+                        const auto uniform = [](float v) {   // into a scalar register
+                            return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
+                        };
+                        xhi = uniform(most(ax2 + rx) - ax2);
+                        xlo = uniform(ax2 - most(ax2 - rx));
+                        yhi = uniform(most(ay2 + ry) - ay2);
+                        ylo = uniform(ay2 - most(ay2 - ry));
+                        zhi = uniform(most(az2 + rz) - az2);
+                        zlo = uniform(az2 - most(az2 - rz));
+                        xmid = uniform(0.5f * (xlo + xhi));
+                        ymid = uniform(0.5f * (ylo + yhi));
+                    }
+                    bool near[kStageIters][4];   // the quarters of the box it can reach
 #pragma unroll
                     for (int it = 0; it < kStageIters; it++) {
 #pragma unroll
@@ -625,13 +653,21 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
                         if (k2P)
                             Rw[lane + it * kWave] = make_float4((float)(ix - ox0), (float)(iy - oy0), (float)(iz - oz0), 0.f);
                         if (kCull) {
-                            // which quarters of the home cell (x below / above the centre,
+                            // which quarters of the box (x below / above its middle,
                             // times y below / above) the candidate can reach: box distance
                             // below the reach radius; quarter qx + 2 qy
                             const float rx = (float)(ix - ox0), ry = (float)(iy - oy0), rz = (float)(iz - oz0);
-                            const float gz = fmaxf(fabsf(rz) - hcz, 0.f);
-                            const float gx0 = fmaxf(fmaxf(rx, -hcx - rx), 0.f), gx1 = fmaxf(fmaxf(-rx, rx - hcx), 0.f);
-                            const float gy0 = fmaxf(fmaxf(ry, -hcy - ry), 0.f), gy1 = fmaxf(fmaxf(-ry, ry - hcy), 0.f);
+                            float gz, gx0, gx1, gy0, gy1;
+                            if constexpr (kTight) {
+                                const float xm = rx - xmid, ym = ry - ymid;
+                                gz = fmaxf(fmaxf(zlo - rz, rz - zhi), 0.f);
+                                gx0 = fmaxf(fmaxf(xlo - rx, xm), 0.f), gx1 = fmaxf(fmaxf(-xm, rx - xhi), 0.f);
+                                gy0 = fmaxf(fmaxf(ylo - ry, ym), 0.f), gy1 = fmaxf(fmaxf(-ym, ry - yhi), 0.f);
+                            } else {
+                                gz = fmaxf(fabsf(rz) - hcz, 0.f);
+                                gx0 = fmaxf(fmaxf(rx, -hcx - rx), 0.f), gx1 = fmaxf(fmaxf(-rx, rx - hcx), 0.f);
+                                gy0 = fmaxf(fmaxf(ry, -hcy - ry), 0.f), gy1 = fmaxf(fmaxf(-ry, ry - hcy), 0.f);
+                            }
                             const float z2 = gz * gz;
                             const float a0 = fmaf(gx0, gx0, z2), a1 = fmaf(gx1, gx1, z2);
                             const float b0 = gy0 * gy0, b1 = gy1 * gy1;
@@ -687,7 +723,7 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
                         // the force of every candidate and, for each pair this side owns
                         // (forward half shell; the higher slot within the home cell), the
                         // FP64 dU term with the row of the particle the reference makes first
-                        const int quad = (hfx >= 0.f ? 1 : 0) + (hfy >= 0.f ? 2 : 0);
+                        const int quad = (hfx >= xmid ? 1 : 0) + (hfy >= ymid ? 2 : 0);
                         const uint16_t *lst = listW + quad * kMaxC;
                         const int nl = quad == 0 ? nq[0] : (quad == 1 ? nq[1] : (quad == 2 ? nq[2] : nq[3]));
                         // the next entry is read one iteration ahead (entries past nl fall in
@@ -717,7 +753,7 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
                         // flight before either is used
                         const float4 *C8 = sC8 + 2 * hb.type * nT;
                         const double *Cd = sCd + 6 * hb.type * nT;
-                        const int quad = (hfx >= 0.f ? 1 : 0) + (hfy >= 0.f ? 2 : 0);
+                        const int quad = (hfx >= xmid ? 1 : 0) + (hfy >= ymid ? 2 : 0);
                         const uint16_t *lst = listW + quad * kMaxC;
                         const int nl = quad == 0 ? nq[0] : (quad == 1 ? nq[1] : (quad == 2 ? nq[2] : nq[3]));
                         // the next trip's list entries are read one trip ahead (entries past
@@ -789,7 +825,7 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
                         // each pair once, from the side that owns it: only the home cell and
                         // its forward half shell are staged, and within the home cell the
                         // lower slot owns the pair
-                        const int quad = (hfx >= 0.f ? 1 : 0) + (hfy >= 0.f ? 2 : 0);
+                        const int quad = (hfx >= xmid ? 1 : 0) + (hfy >= ymid ? 2 : 0);
                         const uint16_t *lst = listW + quad * kMaxC;
                         const int nl = quad == 0 ? nq[0] : (quad == 1 ? nq[1] : (quad == 2 ? nq[2] : nq[3]));
                         const double *Ch = sCd + 6 * hb.type * nT;
