@@ -310,19 +310,77 @@ __global__ __launch_bounds__(kBlock) void k_adj_pair(int n, int nT, double cut2,
     }
 }
 
+// Reverse of one step s, given the adjoints (X, V, A) of (x_s, v_s, a_s), where A already
+// holds c V_s for type != 0 (the v_s = v_h + c a_s term):
+//   X~ = S X (accepted MC move) - obj F(x~_s) + (dF/dx) A     (objective obj U(x~_s))
+//   V_h = V - gamma A (+ dt X~ for type != 0)
+//   X_{s-1} = X~,  V_{s-1} = V_h,  A_{s-1} = c V_h (type != 0), plus c V_{s-1} when the
+//   previous step is a full step (prep_next) rather than the initial force evaluation.
+// A_{s-1} goes to another buffer: other beads' chains still read A_s.
+struct AdjStep {
+    const DevRep *post;   // the replicas after this step's box move
+    int mc;               // whether it has one
+    double4 *X, *V, *A_next;
+    double c, dt;
+    int prep_next;
+};
+
+__device__ inline void adj_step_one(const AdjStep &p, int i, const Bead &b, double4 f, double4 h, const double4 &a,
+                                    double obj)
+{
+    const DevRep &R = p.post[b.rep];
+    double4 x = p.X[i];
+    if (p.mc && R.accept) {
+        x.x *= R.scale[0];
+        x.y *= R.scale[1];
+        x.z *= R.scale[2];
+    }
+    const double4 v = p.V[i];
+    x.x += h.x - obj * f.x;
+    x.y += h.y - obj * f.y;
+    x.z += h.z - obj * f.z;
+    const double gamma = R.gamma;
+    double4 vh = make_double4(v.x - gamma * a.x, v.y - gamma * a.y, v.z - gamma * a.z, 0.0);
+    double4 an = make_double4(0, 0, 0, 0);
+    if (b.type != 0) {
+        vh.x += p.dt * x.x;
+        vh.y += p.dt * x.y;
+        vh.z += p.dt * x.z;
+        const double k = p.prep_next ? 2.0 * p.c : p.c;
+        an = make_double4(k * vh.x, k * vh.y, k * vh.z, 0.0);
+    }
+    p.X[i] = x;
+    p.V[i] = vh;
+    p.A_next[i] = an;
+}
+
+__global__ __launch_bounds__(kBlock) void k_adj_step(int n, const Bead *__restrict__ beads, AdjStep p,
+                                                     const double4 *__restrict__ A, const double4 *__restrict__ F,
+                                                     const double4 *__restrict__ HV, double obj)
+{
+    const int i = blockIdx.x * kBlock + threadIdx.x;
+    if (i < n) adj_step_one(p, i, beads[i], F[i], HV[i], A[i], obj);
+}
+
+// STEP: the reverse step of the bead in the same pass, from the pair kernel's F and HV with the
+// chain's (5 us and a launch a step less at 12k beads)
+template <bool STEP>
 __global__ __launch_bounds__(kBlock) void k_adj_chain(int n, const Bead *__restrict__ beads,
                                                       const int2 *__restrict__ chain,
                                                       const double4 *__restrict__ cconst,
                                                       const DevRep *__restrict__ reps,
                                                       const double4 *__restrict__ w, double4 *__restrict__ fout,
                                                       double4 *__restrict__ hvout, double *__restrict__ g, double obj,
-                                                      int want_hv)
+                                                      int want_hv, AdjStep next)
 {
     const int i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= n) return;
     const int2 ci = chain[i];
-    if (ci.x < 0) return;
     const Bead b0 = beads[i];
+    if (ci.x < 0) {
+        if (STEP) adj_step_one(next, i, b0, fout[i], hvout[i], w[i], obj);
+        return;
+    }
     const DevRep &R = reps[b0.rep];
     const double L[3] = {R.L[0], R.L[1], R.L[2]};
     const int start = ci.x, len = ci.y & 0xFFFF, j = i - start;
@@ -344,11 +402,14 @@ __global__ __launch_bounds__(kBlock) void k_adj_chain(int n, const Bead *__restr
     const V3<Dual> f = chain_force(pd, j, len, L, K.x, K.y, K.z, K.w);
     double4 fo = fout[i];
     fo.x += f.x.v; fo.y += f.y.v; fo.z += f.z.v;
-    fout[i] = fo;
-    if (want_hv) {
+    if (!STEP) fout[i] = fo;
+    if (STEP || want_hv) {
         double4 h = hvout[i];
         h.x += f.x.d; h.y += f.y.d; h.z += f.z.d;
-        hvout[i] = h;
+        if (STEP)
+            adj_step_one(next, i, b0, fo, h, w[i], obj);
+        else
+            hvout[i] = h;
     }
     // theta derivatives: the bond part of the force is linear in k_bond, the bend part in
     // k_bend, so dF/dk is the force at k = 1 with the other stiffness off
@@ -425,47 +486,6 @@ __global__ __launch_bounds__(kBlock) void k_adj_gen(int n, GenTables gen, const 
     }
 }
 
-// Reverse of one step s, given the adjoints (X, V, A) of (x_s, v_s, a_s), where A already
-// holds c V_s for type != 0 (the v_s = v_h + c a_s term):
-//   X~ = S X (accepted MC move) - obj F(x~_s) + (dF/dx) A     (objective obj U(x~_s))
-//   V_h = V - gamma A (+ dt X~ for type != 0)
-//   X_{s-1} = X~,  V_{s-1} = V_h,  A_{s-1} = c V_h (type != 0), plus c V_{s-1} when the
-//   previous step is a full step (prep_next) rather than the initial force evaluation.
-__global__ __launch_bounds__(kBlock) void k_adj_step(int n, const Bead *__restrict__ beads,
-                                                     const DevRep *__restrict__ post, int mc, double4 *__restrict__ X,
-                                                     double4 *__restrict__ V, double4 *__restrict__ A,
-                                                     const double4 *__restrict__ F, const double4 *__restrict__ HV,
-                                                     double obj, double c, double dt, int prep_next)
-{
-    const int i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= n) return;
-    const Bead b = beads[i];
-    const DevRep &R = post[b.rep];
-    double4 x = X[i];
-    if (mc && R.accept) {
-        x.x *= R.scale[0];
-        x.y *= R.scale[1];
-        x.z *= R.scale[2];
-    }
-    const double4 f = F[i], h = HV[i], a = A[i], v = V[i];
-    x.x += h.x - obj * f.x;
-    x.y += h.y - obj * f.y;
-    x.z += h.z - obj * f.z;
-    const double gamma = R.gamma;
-    double4 vh = make_double4(v.x - gamma * a.x, v.y - gamma * a.y, v.z - gamma * a.z, 0.0);
-    double4 an = make_double4(0, 0, 0, 0);
-    if (b.type != 0) {
-        vh.x += dt * x.x;
-        vh.y += dt * x.y;
-        vh.z += dt * x.z;
-        const double k = prep_next ? 2.0 * c : c;
-        an = make_double4(k * vh.x, k * vh.y, k * vh.z, 0.0);
-    }
-    X[i] = x;
-    V[i] = vh;
-    A[i] = an;
-}
-
 }  // namespace
 
 void launch_adj_pair(hipStream_t st, const Params &P, const Bead *sbeads, const uint32_t *skey, const uint32_t *sidx,
@@ -488,15 +508,25 @@ void launch_adj_chain(hipStream_t st, const Params &P, const Bead *beads, const 
                       const DevRep *reps, const double4 *w, double4 *fout, double4 *hvout, double *g, double obj,
                       int want_hv)
 {
-    hipLaunchKernelGGL(k_adj_chain, dim3(blocks(P.n)), dim3(kBlock), 0, st, P.n, beads, chain, cconst, reps, w, fout,
-                       hvout, g, obj, want_hv);
+    hipLaunchKernelGGL(k_adj_chain<false>, dim3(blocks(P.n)), dim3(kBlock), 0, st, P.n, beads, chain, cconst, reps, w,
+                       fout, hvout, g, obj, want_hv, AdjStep{});
+}
+
+void launch_adj_chain_step(hipStream_t st, const Params &P, const Bead *beads, const int2 *chain,
+                           const double4 *cconst, const DevRep *reps, const DevRep *post, int mc, double4 *X,
+                           double4 *V, const double4 *A, double4 *A_next, double4 *F, double4 *HV, double *g,
+                           double obj, int prep_next)
+{
+    hipLaunchKernelGGL(k_adj_chain<true>, dim3(blocks(P.n)), dim3(kBlock), 0, st, P.n, beads, chain, cconst, reps, A, F,
+                       HV, g, obj, 1, AdjStep{post, mc, X, V, A_next, 0.5 * P.dt, P.dt, prep_next});
 }
 
 void launch_adj_step(hipStream_t st, const Params &P, const Bead *beads, const DevRep *post, int mc, double4 *X,
-                     double4 *V, double4 *A, const double4 *F, const double4 *HV, double obj, int prep_next)
+                     double4 *V, const double4 *A, double4 *A_next, const double4 *F, const double4 *HV, double obj,
+                     int prep_next)
 {
-    hipLaunchKernelGGL(k_adj_step, dim3(blocks(P.n)), dim3(kBlock), 0, st, P.n, beads, post, mc, X, V, A, F, HV, obj,
-                       0.5 * P.dt, P.dt, prep_next);
+    hipLaunchKernelGGL(k_adj_step, dim3(blocks(P.n)), dim3(kBlock), 0, st, P.n, beads,
+                       AdjStep{post, mc, X, V, A_next, 0.5 * P.dt, P.dt, prep_next}, A, F, HV, obj);
 }
 
 }  // namespace smdev

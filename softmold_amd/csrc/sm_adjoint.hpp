@@ -27,8 +27,16 @@ void launch_adj_chain(hipStream_t st, const Params &P, const Bead *beads, const 
 // Per bead: the generic BOND / BEND / BALL records' force (+=) and its (dF/dx) w (+=).
 void launch_adj_gen(hipStream_t st, const Params &P, const GenTables &gen, const Bead *beads, const DevRep *reps,
                     const double4 *w, double4 *fout, double4 *hvout, int want_hv);
-// One reverse step (see sm_adjoint.hip); post = the replicas after this step's MC move.
+// One reverse step (see sm_adjoint.hip); post = the replicas after this step's MC move.  A_next is
+// not A.
 void launch_adj_step(hipStream_t st, const Params &P, const Bead *beads, const DevRep *post, int mc, double4 *X,
-                     double4 *V, double4 *A, const double4 *F, const double4 *HV, double obj, int prep_next);
+                     double4 *V, const double4 *A, double4 *A_next, const double4 *F, const double4 *HV, double obj,
+                     int prep_next);
+// launch_adj_chain with want_hv, then the reverse step, in one pass (F and HV are left as the
+// pair kernel wrote them).
+void launch_adj_chain_step(hipStream_t st, const Params &P, const Bead *beads, const int2 *chain,
+                           const double4 *cconst, const DevRep *reps, const DevRep *post, int mc, double4 *X,
+                           double4 *V, const double4 *A, double4 *A_next, double4 *F, double4 *HV, double *g,
+                           double obj, int prep_next);
 
 }  // namespace smdev

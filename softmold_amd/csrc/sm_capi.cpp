@@ -1932,7 +1932,7 @@ struct AdjointRun {
     std::vector<State> checkpoint;    // states at steps k, 2k, ...; [0] at step 0
     DevRep *pre = nullptr, *post = nullptr;   // a segment's box moves: the replicas before and after each
     double *sums = nullptr;           // sums over the steps of U_pair, U_chain per replica
-    double4 *X = nullptr, *V = nullptr, *A = nullptr, *F = nullptr, *HV = nullptr;
+    double4 *X = nullptr, *V = nullptr, *A = nullptr, *A_next = nullptr, *F = nullptr, *HV = nullptr;
     double *g = nullptr, *gs = nullptr;
 
     AdjointRun(sm_ctx *ctx, int steps, int want_k, bool grad) : c(ctx), n(ctx->n), nrep(ctx->nrep), S(steps)
@@ -1969,7 +1969,7 @@ struct AdjointRun {
             take(post, (size_t)(k / 8 + 1) * nrep);
             take(sums, 2 * (size_t)nrep);
             if (grad) {
-                for (double4 **p : {&X, &V, &A, &F, &HV}) take(*p, n);
+                for (double4 **p : {&X, &V, &A, &A_next, &F, &HV}) take(*p, n);
                 take(g, kNTheta * (size_t)n);
                 take(gs, kNTheta * (size_t)nrep);
             }
@@ -2162,9 +2162,11 @@ int sm_adjoint(sm_ctx *c, int32_t type_a, int32_t type_b, int32_t nsteps, int32_
         for (double4 *p : {run.X, run.V, run.A}) zero(p, sizeof(double4) * n);
         zero(run.g, sizeof(double) * kNTheta * n);
         const AdjTables T{c->adjF, c->adjDF, c->adjDU};
-        auto adjoint_forces = [&](double o, int hv) {
+        auto pair_terms = [&](double o, int hv) {
             launch_adj_pair(st, c->P, c->sbeads, c->skey(), c->sidx(), c->cstart, c->cend, c->reps, T, run.A, run.F,
                             run.HV, run.g, o, hv);
+        };
+        auto chain_terms = [&](double o, int hv) {
             launch_adj_chain(st, c->P, c->beads, c->chainPerBead, c->cconstD, c->reps, run.A, run.F, run.HV, run.g, o,
                              hv);
             if (c->gptr) launch_adj_gen(st, c->P, c->gen(), c->beads, c->reps, run.A, run.F, run.HV, hv);
@@ -2185,15 +2187,24 @@ int sm_adjoint(sm_ctx *c, int32_t type_a, int32_t type_b, int32_t nsteps, int32_
                     post = run.post + m;
                 }
                 c->build(0, kStepKeep);
-                adjoint_forces(obj, 1);
-                launch_adj_step(st, c->P, c->beads, post, mc ? 1 : 0, run.X, run.V, run.A, run.F, run.HV, obj,
-                                s - 1 >= 1 ? 1 : 0);
+                pair_terms(obj, 1);
+                const int prep = s - 1 >= 1 ? 1 : 0;
+                if (c->gptr) {
+                    chain_terms(obj, 1);
+                    launch_adj_step(st, c->P, c->beads, post, mc ? 1 : 0, run.X, run.V, run.A, run.A_next, run.F,
+                                    run.HV, obj, prep);
+                } else {
+                    launch_adj_chain_step(st, c->P, c->beads, c->chainPerBead, c->cconstD, c->reps, post, mc ? 1 : 0,
+                                          run.X, run.V, run.A, run.A_next, run.F, run.HV, run.g, obj, prep);
+                }
+                std::swap(run.A, run.A_next);
             }
         }
         // a_0 = F(x_0) + ...: its adjoint meets dF/dtheta at the initial positions
         c->beads = run.x[0];
         c->build(0, kStepKeep);
-        adjoint_forces(0.0, 0);
+        pair_terms(0.0, 0);
+        chain_terms(0.0, 0);
         // per replica: grad[r * kNTheta + p]
         static_assert(kNTheta == 4, "SUM_COLUMNS sums four");
         launch_sums(st, SUM_COLUMNS, c->sums(run.g, run.gs));
