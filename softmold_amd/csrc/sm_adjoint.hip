@@ -19,7 +19,8 @@
 // lanes test their cells' beads and put the hits into a list, and 32 hits at a time are
 // evaluated, one a lane: a lane that evaluated its own hits as it found them left the other
 // 63 waiting through roots and divisions for nearly every candidate (86 us a call at 12k
-// beads, 38 now; what is left is the chain of loads behind a hit: bead, table row, adjoint).
+// beads, 38 so, and 32 with the tables in LDS and the theta terms for the fitted pair only; what
+// is left is the chain of loads behind a hit, bead and adjoint).
 //
 // Reference: force law Force<double> (MD.h:795-848), potential (MD.h:895-930), constant
 // tables laradjiRevaleeFC/PC (potentials/laradjiRevalee.h:84-152), harmonicF/bendF
@@ -164,13 +165,22 @@ __global__ __launch_bounds__(kBlock) void k_adj_pair(int n, int nT, double cut2,
                                                      const uint32_t *__restrict__ skey,
                                                      const uint32_t *__restrict__ sidx,
                                                      const int *__restrict__ cstart, const int *__restrict__ cend,
-                                                     const DevRep *__restrict__ reps, const double *__restrict__ fc,
-                                                     const double *__restrict__ dfc, const double *__restrict__ duc,
+                                                     const DevRep *__restrict__ reps, AdjTables T,
                                                      const double4 *__restrict__ w, double4 *__restrict__ fout,
                                                      double4 *__restrict__ hvout, double *__restrict__ g, double obj,
                                                      int want_hv)
 {
     __shared__ int2 hits[kBlock / kAdjLanes][kAdjHits];   // (sorted slot, stencil cell)
+    // the force rows, and the theta derivatives' rows of the fitted pair, (a, b) then (b, a):
+    // {dF/dUmin, dF/dUmax, dU/dUmin, dU/dUmax}, every other row's being zero
+    __shared__ double sC[6 * kMaxTypes * kMaxTypes], sTheta[2][4][6];
+    const size_t tsz = 6 * (size_t)nT * nT;
+    for (int t = threadIdx.x; t < (int)tsz; t += kBlock) sC[t] = T.fc[t];
+    if (threadIdx.x < 48) {
+        const int r = threadIdx.x / 24, p = threadIdx.x / 6 % 4, k = threadIdx.x % 6;
+        sTheta[r][p][k] = (p < 2 ? T.dfc : T.duc)[(p & 1) * tsz + (r ? T.row_ba : T.row_ab) + k];
+    }
+    __syncthreads();
     const long long gt = (long long)blockIdx.x * kBlock + threadIdx.x;
     const int s = (int)(gt / kAdjLanes);   // sorted slot of the bead (uniform over its lanes)
     const int c = (int)(gt % kAdjLanes);   // its stencil cell
@@ -189,7 +199,6 @@ __global__ __launch_bounds__(kBlock) void k_adj_pair(int n, int nT, double cut2,
     const int kx = (int)(k % (uint32_t)nx), ky = (int)((k / (uint32_t)nx) % (uint32_t)ny),
               kz = (int)(k / (uint32_t)(nx * ny));
     const double4 wi = w[me];
-    const size_t tsz = 6 * (size_t)nT * nT;
     // the box length to add to the beads of stencil cell q along an axis
     auto shift = [](int cell, int cells, double L) { return cell < 0 ? -L : (cell >= cells ? L : 0.0); };
     double sx = 0.0, sy = 0.0, sz = 0.0;
@@ -220,8 +229,8 @@ __global__ __launch_bounds__(kBlock) void k_adj_pair(int n, int nT, double cut2,
         // cell, within a cell the lower index (cellOpt.h:572-585,780-795)
         constexpr uint32_t fwd = forward_cells();
         const bool first = hc == 13 ? me < other : ((fwd >> hc) & 1u) != 0;
-        const size_t row = 6 * (first ? (size_t)hb.type * nT + q.type : (size_t)q.type * nT + hb.type);
-        const double *C = fc + row;
+        const int row = 6 * (first ? hb.type * nT + q.type : q.type * nT + hb.type);
+        const double *C = sC + row;
         const int o = (r >= C[0]) ? 3 : 0;
         const double m = C[o] - r;
         const double f = (C[o + 1] - C[o + 2] * m) * m;        // force along d/r
@@ -240,12 +249,12 @@ __global__ __launch_bounds__(kBlock) void k_adj_pair(int n, int nT, double cut2,
             Hz += uz * fr + dz * t;
         }
         const double wd = (wi.x * dx + wi.y * dy + wi.z * dz) * ri;
-        const double *U = duc + row;   // only C1, C2, C4, C5 of the U row depend on theta
+        if (row != T.row_ab && row != T.row_ba) return;
+        const double (*D)[6] = sTheta[row == T.row_ab ? 0 : 1];
         for (int p = 0; p < 2; p++) {
-            const double *D = dfc + p * tsz + row;
-            gw[p] += wd * ((D[o + 1] - D[o + 2] * m) * m);
+            gw[p] += wd * ((D[p][o + 1] - D[p][o + 2] * m) * m);
             if (obj != 0.0) {
-                const double *E = U + p * tsz;
+                const double *E = D[2 + p];   // only C1, C2, C4, C5 of the U row depend on theta
                 double d;
                 if (r <= C[0]) {
                     const double mu = C[0] - r;
@@ -494,7 +503,7 @@ void launch_adj_pair(hipStream_t st, const Params &P, const Bead *sbeads, const 
 {
     hipLaunchKernelGGL(k_adj_pair, dim3(blocks((long long)P.n * kAdjLanes)), dim3(kBlock), 0, st, P.n, P.nT,
                        P.cutoff * P.cutoff, sbeads,
-                       skey, sidx, cstart, cend, reps, T.fc, T.dfc, T.duc, w, fout, hvout, g, obj, want_hv);
+                       skey, sidx, cstart, cend, reps, T, w, fout, hvout, g, obj, want_hv);
 }
 
 void launch_adj_gen(hipStream_t st, const Params &P, const GenTables &gen, const Bead *beads, const DevRep *reps,

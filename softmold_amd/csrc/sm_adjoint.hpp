@@ -11,6 +11,7 @@ struct AdjTables {
     const double *fc;    // F constants, FP64, 6 nT^2
     const double *dfc;   // dF-constants / d(Umin), d(Umax): 2 x 6 nT^2
     const double *duc;   // dU-constants / d(Umin), d(Umax): 2 x 6 nT^2
+    int row_ab, row_ba;  // the fitted pair's rows, the only ones of dfc and duc that are not zero
 };
 
 // Per sorted slot: FP64 pair force F (=), (dF/dx) w (=, if want_hv), and into the per-bead

@@ -2161,7 +2161,8 @@ int sm_adjoint(sm_ctx *c, int32_t type_a, int32_t type_b, int32_t nsteps, int32_
         const auto zero = [&](void *p, size_t bytes) { HIPCHK(hipMemsetAsync(p, 0, bytes, st)); };
         for (double4 *p : {run.X, run.V, run.A}) zero(p, sizeof(double4) * n);
         zero(run.g, sizeof(double) * kNTheta * n);
-        const AdjTables T{c->adjF, c->adjDF, c->adjDU};
+        const int nT = c->P.nT;
+        const AdjTables T{c->adjF, c->adjDF, c->adjDU, 6 * (type_a * nT + type_b), 6 * (type_b * nT + type_a)};
         auto pair_terms = [&](double o, int hv) {
             launch_adj_pair(st, c->P, c->sbeads, c->skey(), c->sidx(), c->cstart, c->cend, c->reps, T, run.A, run.F,
                             run.HV, run.g, o, hv);
