@@ -431,6 +431,15 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
         kc = skey[a + lane];
         if (a + lane > 0) kp = skey[a + lane - 1];
     }
+    // one replica: its box and grid while the keys are on their way (the compiler would load each
+    // part at its first use and wait there): the 240k vesicle's force 89.4 -> 87.7 us.  A wave
+    // that is alone on its SIMD only starts later for it (1.5k vesicle 17.9 -> 18.6 us), so the
+    // instances of small systems, and the energy traversals, do without.
+    if constexpr (ONE && MODE == M_FORCE1 && WAVES > 4) {
+        const DevRep &R = reps[0];
+        asm volatile("" ::"s"(R.L[0]), "s"(R.L[1]), "s"(R.L[2]), "s"(R.cs[0]), "s"(R.cs[1]), "s"(R.cs[2]), "s"(R.nc[0]),
+                     "s"(R.nc[1]), "s"(R.nc[2]), "s"((uint32_t)R.cellbase));
+    }
     // the constant tables: every load first (indices clamped in bounds, so no branch holds
     // one back), then the LDS stores, so the staging costs one memory trip; a chunk inside
     // one cell's run owns nothing and leaves before the tables arrive
