@@ -612,13 +612,18 @@ struct sm_ctx {
         a.n = n;
         return a;
     }
-    // out[2r + 0..1] += {U_pair, U_chain} of the resident order
+    // the pair force with each bead's share of U_pair in ebead: one traversal of 32 us where the
+    // force and U took 23 and 24 at 12k beads
+    void pair_force_u()
+    {
+        timed(K_PAIR, [&] {
+            launch_pair_force_u(st, P, echunk, sbeads, skey(), sidx(), cstart, cend, reps, fconstF, uconstD, fpair,
+                                ebead);
+        });
+    }
+    // out[2r + 0..1] += {U_pair (from ebead), U_chain}
     void add_energies(double *out)
     {
-        timed(K_GATHER, [&] {
-            launch_pair_gather(st, P, echunk, GATHER_U, sbeads, skey(), sidx(), cstart, cend, reps, fconstF, uconstD, ebead,
-                               nullptr, nullptr, nullptr, 0);
-        });
         timed(K_SUMS, [&] {
             launch_sums(st, SUM_ENERGY, sums(ebead, out));
             if (gptr) {
@@ -2021,7 +2026,7 @@ struct AdjointRun {
             const int t = s - s0;
             const bool mc = c->mc_step(s);
             c->sort_and_reorder();
-            c->pair_force();
+            c->pair_force_u();   // in the recomputed segments too, whose steps must be the same
             if (objective) c->add_energies(sums);
             if (!mc && s < s1) {
                 c->beads_alt = x[t + 1];

@@ -207,6 +207,10 @@ void launch_pair_force(hipStream_t st, const Params &P, int chunk, int variant, 
 void launch_pair_force_du(hipStream_t st, const Params &P, int chunk, const Bead *sbeads, const uint32_t *skey,
                           const uint32_t *sidx, const int *cstart, const int *cend, const DevRep *reps,
                           const float *fconst, const double *uconst, float4 *fpair, double *energy);
+// The same with each pair's U instead.
+void launch_pair_force_u(hipStream_t st, const Params &P, int chunk, const Bead *sbeads, const uint32_t *skey,
+                         const uint32_t *sidx, const int *cstart, const int *cend, const DevRep *reps,
+                         const float *fconst, const double *uconst, float4 *fpair, double *energy);
 // gptr == NULL: CHAIN terms only; else also the generic records of each bead
 struct GenTables {
     const int *gptr;

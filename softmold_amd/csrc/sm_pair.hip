@@ -50,7 +50,7 @@ namespace {
 constexpr int kWaves = 1;   // waves per workgroup: one, so a finished wave frees its slot at once
 constexpr int kList = 32;      // candidates a lane screens before evaluating its hits
 
-enum : int { M_FORCE = 0, M_U = 1, M_DU = 2, M_COUNT = 3, M_LIST = 4, M_FORCE1 = 5, M_FCOUNT = 6, M_FDU = 7 };
+enum : int { M_FORCE = 0, M_U = 1, M_DU = 2, M_COUNT = 3, M_LIST = 4, M_FORCE1 = 5, M_FCOUNT = 6, M_FDU = 7, M_FU = 8 };
 
 struct __align__(16) Cand {
     double x, y, z;
@@ -369,9 +369,12 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
     // the home particle owns, in the same traversal (the box move's dU at the positions the
     // force sees)
     constexpr bool kFDU = MODE == M_FDU;
-    constexpr bool kF = MODE == M_FORCE || MODE == M_FORCE1 || kFDU;   // force (two-phase / one-phase)
+    // the one-phase force with the FP64 U of each pair the home particle owns
+    constexpr bool kFU = MODE == M_FU;
+    constexpr bool kFE = kFDU || kFU;
+    constexpr bool kF = MODE == M_FORCE || MODE == M_FORCE1 || kFE;   // force (two-phase / one-phase)
     constexpr bool k2P = MODE == M_FORCE;
-    constexpr bool kF1 = MODE == M_FORCE1 || kFDU;
+    constexpr bool kF1 = MODE == M_FORCE1 || kFE;
     constexpr bool kE = MODE == M_U || MODE == M_DU;   // FP64 energy gathers
     // the one-phase force traversal counting its accepted pairs with a nonzero term
     // instead of evaluating them: same staging, culling, lists and FP64 test
@@ -382,7 +385,7 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
     // 90k bilayer's force with dU (90.9 -> 85.4 us), 3 % of the 240k vesicle's (177 -> 171), 5 and
     // 1 % of their U; the force alone has cheaper tests and no registers left for it (240k 89.2
     // -> 94.8 us)
-    constexpr bool kTight = kFDU || kE;
+    constexpr bool kTight = kFE || kE;
     // staged candidates per pass: the two-phase force and the FP64 energy gathers measured
     // fastest at 128 (U of 240k beads 84 us, 92 with 192; with dU 177 and 205), the force see
     // kManyBeads
@@ -447,7 +450,7 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
     constexpr int kC8Per = (2 * kMaxTypes * kMaxTypes + kThreads - 1) / kThreads;
     constexpr int kCdPer = (6 * kMaxTypes * kMaxTypes + kThreads - 1) / kThreads;
     float4 c8[kF ? kC8Per : 1];
-    double cd[(!kF || kFDU) ? kCdPer : 1];
+    double cd[(!kF || kFE) ? kCdPer : 1];
     float rf = 0.f, re = 0.f;
     if (kF) {
         const float4 *t8 = reinterpret_cast<const float4 *>(tab);
@@ -457,7 +460,7 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
             c8[k] = t8[min(t, 2 * nT * nT - 1)];
         }
     }
-    if (!kF || kFDU) {
+    if (!kF || kFE) {
 #pragma unroll
         for (int k = 0; k < kCdPer; k++) {
             const int t = threadIdx.x + k * kThreads;
@@ -476,13 +479,13 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
         for (int k = 0; k < kC8Per; k++)
             if ((int)threadIdx.x + k * kThreads < 2 * nT * nT) sC8[threadIdx.x + k * kThreads] = c8[k];
     }
-    if (!kF || kFDU) {
+    if (!kF || kFE) {
 #pragma unroll
         for (int k = 0; k < kCdPer; k++)
             if ((int)threadIdx.x + k * kThreads < 6 * nT * nT) sCd[threadIdx.x + k * kThreads] = cd[k];
     }
     // every thread stores (those past nT the last type's value again, the same bits)
-    if (kCull) sReach2[treach] = kFDU ? fmaxf(rf, re) : (kE ? re : rf);
+    if (kCull) sReach2[treach] = kFE ? fmaxf(rf, re) : (kE ? re : rf);
     __syncthreads();
 
     constexpr uint32_t fwd = forward_mask();
@@ -699,7 +702,7 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
                         // count and list gathers, and the force over an asymmetric table: the
                         // slot, with the stencil cell above the type's bits (types are below
                         // kMaxTypes <= 256)
-                        constexpr bool kSlotCell = MODE == M_COUNT || MODE == M_LIST || kFDU || (ASYM && (kF || kFC));
+                        constexpr bool kSlotCell = MODE == M_COUNT || MODE == M_LIST || kFE || (ASYM && (kF || kFC));
                         cd.t = kSlotCell ? (qb[it].type | (c << 8)) : qb[it].type;
                         cd.c = (kF || kFC || kSlotCell) ? src[it] : c;
                         Cw[lane + it * kWave] = cd;
@@ -728,10 +731,10 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
                     asm volatile("" : "+v"(hb.x), "+v"(hb.y), "+v"(hb.z), "+v"(hb.type));
                     // home position relative to the cell centre (its quarter; the two-phase screen)
                     const float hfx = (float)(hb.x - ox0), hfy = (float)(hb.y - oy0), hfz = (float)(hb.z - oz0);
-                    if (kFDU && act) {
+                    if (kFE && act) {
                         // the force of every candidate and, for each pair this side owns
                         // (forward half shell; the higher slot within the home cell), the
-                        // FP64 dU term with the row of the particle the reference makes first
+                        // FP64 dU (or U) term with the row of the particle the reference makes first
                         const int quad = (hfx >= xmid ? 1 : 0) + (hfy >= ymid ? 2 : 0);
                         const uint16_t *lst = listW + quad * kMaxC;
                         const int nl = quad == 0 ? nq[0] : (quad == 1 ? nq[1] : (quad == 2 ? nq[2] : nq[3]));
@@ -753,7 +756,11 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
                             if (r2 < cut2 && q.c != hslot) force_law(dxd, dyd, dzd, r2, sC8 + 2 * row, fx, fy, fz);
                             // owned: a forward half-shell cell, or the higher slot in the home cell
                             const bool owned = c == 13 ? q.c > hslot : ((fwd >> c) & 1u) != 0;
-                            if (owned) accu += du_pair(dxd, dyd, dzd, r2, sCd + 6 * row, cut2, s2x, s2y, s2z, dseries);
+                            if (kFU) {
+                                if (owned && r2 < cut2) accu += pair_u_any(r2, sCd + 6 * row);
+                            } else if (owned) {
+                                accu += du_pair(dxd, dyd, dzd, r2, sCd + 6 * row, cut2, s2x, s2y, s2z, dseries);
+                            }
                         }
                         next -= nl;
                     } else if ((MODE == M_FORCE1 || kFC) && act) {
@@ -906,7 +913,7 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
                         }
                     }
                     if (act && sub == 0) out.force[me] = make_float4((float)fx, (float)fy, (float)fz, 0.f);
-                    if (kFDU) {
+                    if (kFE) {
                         for (int st = 1; st < tpp; st <<= 1) {
                             const double o = __shfl(accu, lane + st);
                             if ((sub & (2 * st - 1)) == 0 && sub + st < tpp) accu += o;
@@ -955,7 +962,8 @@ void launch_cells(hipStream_t st, const Params &P, int chunk, const Bead *sbeads
     // The half-shell energy gathers gain on both in groups of 64.
     const bool energy = MODE == M_U || MODE == M_DU;
     const int turn = energy ? 6 : (P.flat ? 7 : 0);
-    const bool floats = MODE == M_FORCE || MODE == M_FORCE1 || MODE == M_FDU, doubles = !floats || MODE == M_FDU;
+    const bool both = MODE == M_FDU || MODE == M_FU;
+    const bool floats = MODE == M_FORCE || MODE == M_FORCE1 || both, doubles = !floats || both;
     const size_t tables_bytes = (size_t)P.nT * P.nT * ((floats ? 2 * sizeof(float4) : 0) + (doubles ? 6 * sizeof(double) : 0));
     hipLaunchKernelGGL((k_cells<MODE, ASYM, ONE, MAXC, WAVES>), dim3(nb), dim3(kWaves * kWave), tables_bytes, st, P.n, P.nT, chunk, nb, cut2, cut2pre,
                        sbeads, skey, sidx, cstart, cend, reps, fconst, uconst, turn, out);
@@ -1011,6 +1019,14 @@ void launch_pair_force_du(hipStream_t st, const Params &P, int chunk, const Bead
 {
     Out o{fpair, energy, nullptr, nullptr, nullptr, 0};
     launch_for<M_FDU, 128, 4, true>(P, st, chunk, sbeads, skey, sidx, cstart, cend, reps, fconst, uconst, o);
+}
+
+void launch_pair_force_u(hipStream_t st, const Params &P, int chunk, const Bead *sbeads, const uint32_t *skey,
+                         const uint32_t *sidx, const int *cstart, const int *cend, const DevRep *reps,
+                         const float *fconst, const double *uconst, float4 *fpair, double *energy)
+{
+    Out o{fpair, energy, nullptr, nullptr, nullptr, 0};
+    launch_for<M_FU, 128, 4, true>(P, st, chunk, sbeads, skey, sidx, cstart, cend, reps, fconst, uconst, o);
 }
 
 void launch_pair_gather(hipStream_t st, const Params &P, int chunk, int mode, const Bead *sbeads,

@@ -37,3 +37,28 @@ def test_two_segments_equal_one(lipids, segment):
     assert np.array_equal(g1, g2) and np.all(np.isfinite(g1)) and np.any(g1 != 0)
     for x, y in zip(before, s.download()):
         assert np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("asymmetric", [False, True])
+@pytest.mark.parametrize("model,lipids", [("bilayer", 300), ("liposome", 2500)])
+def test_objective_of_one_step_is_the_measured_energy(model, lipids, asymmetric):
+    """The objective's U comes with the pair force, a measurement's from its own traversal: the
+    same terms in other orders.  The positions after one step are the same (they follow from the
+    initial forces), so J is U_pair + U_chain there, to the roundings of a sum of terms of both
+    signs: n_pairs * 2^-53 of the terms' sum, of which U is a good part; 1e-11 is asserted."""
+    m = getattr(sm.Mpd, model)(11, lipids, 3.45)
+    d = dict(m.system())
+    m.close()
+    d["delta_lxy"] = 0.0
+    if asymmetric:
+        f, u = np.array(d["fconst"]), np.array(d["uconst"])
+        row = 6 * (2 * d["n_types"] + 3)
+        f[row + 1] *= 1.25
+        u[row + 1] *= 1.25
+        d["fconst"], d["uconst"] = f, u
+    s = sm.Solver.from_system(d)
+    J, _ = objective(s, PAIR, 1, 1, grad=False)
+    s.init_forces()
+    s.run(1, 1)
+    e = np.asarray(s.measure()).reshape(-1)
+    assert J == pytest.approx(e[0] + e[1], rel=1e-11)
