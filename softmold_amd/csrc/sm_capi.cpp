@@ -2110,14 +2110,11 @@ int sm_param_derivative(sm_ctx *c, int32_t type_a, int32_t type_b, double *out)
         check_pair(c, type_a, type_b);
         upload_param_derivative_tables(c, type_a, type_b);
         c->build(0, kStepKeep);
-        const size_t nt = 6 * (size_t)c->P.nT * c->P.nT;
-        double *e[2] = {c->ebead, c->edelta};
-        for (int p = 0; p < 2; p++)
-            launch_pair_gather(c->st, c->P, c->echunk, GATHER_U, c->sbeads, c->skey(), c->sidx(), c->cstart, c->cend,
-                               c->reps, c->pdTab + p * c->pd_tab, c->pdU + p * nt, e[p], nullptr, nullptr, nullptr, 0);
+        launch_pair_gather_u2(c->st, c->P, c->echunk, c->sbeads, c->skey(), c->sidx(), c->cstart, c->cend, c->reps,
+                              c->pdTab, c->pdU, c->ebead, c->edelta);
         // the measurement words are free between calls (each measurement copies its own out)
-        SumArgs a = c->sums(e[0], c->dres);
-        a.y = e[1];
+        SumArgs a = c->sums(c->ebead, c->dres);
+        a.y = c->edelta;
         a.cconst = c->pdC;
         a.cconst2 = c->pdC + c->hcconst.size();
         launch_sums(c->st, SUM_PARAM, a);

@@ -242,6 +242,10 @@ void launch_pair_gather(hipStream_t st, const Params &P, int chunk, int mode, co
                         const uint32_t *skey, const uint32_t *sidx, const int *cstart, const int *cend,
                         const DevRep *reps, const float *tab, const double *uconst, double *energy, int *counts,
                         int *pairs, unsigned long long *npairs, long long cap);
+// GATHER_U under two potential tables at once (tab and uconst hold both, one after the other).
+void launch_pair_gather_u2(hipStream_t st, const Params &P, int chunk, const Bead *sbeads, const uint32_t *skey,
+                           const uint32_t *sidx, const int *cstart, const int *cend, const DevRep *reps,
+                           const float *tab, const double *uconst, double *energy, double *energy2);
 // Generic-record energies, one FP64 value per bead: the records whose first bead it is,
 // U, or U(old) - U(scaled) when delta != 0.
 void launch_gen_energy(hipStream_t st, int n, const GenTables &gen, const Bead *beads, const DevRep *reps,

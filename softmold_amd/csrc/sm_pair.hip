@@ -50,7 +50,7 @@ namespace {
 constexpr int kWaves = 1;   // waves per workgroup: one, so a finished wave frees its slot at once
 constexpr int kList = 32;      // candidates a lane screens before evaluating its hits
 
-enum : int { M_FORCE = 0, M_U = 1, M_DU = 2, M_COUNT = 3, M_LIST = 4, M_FORCE1 = 5, M_FCOUNT = 6, M_FDU = 7, M_FU = 8 };
+enum : int { M_FORCE = 0, M_U = 1, M_DU = 2, M_COUNT = 3, M_LIST = 4, M_FORCE1 = 5, M_FCOUNT = 6, M_FDU = 7, M_FU = 8, M_U2 = 9 };
 
 struct __align__(16) Cand {
     double x, y, z;
@@ -347,7 +347,7 @@ __device__ inline void count_term(const Bead &hb, const Cand &q, bool other, dou
 
 struct Out {
     float4 *force;            // M_FORCE, original order
-    double *energy;           // M_U, M_DU: one FP64 value per sorted slot
+    double *energy, *energy2; // M_U, M_DU, M_U2: one FP64 value (a table) per sorted slot
     int *counts;              // M_COUNT, original order
     int *pairs;               // M_LIST
     unsigned long long *npairs;
@@ -375,7 +375,9 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
     constexpr bool kF = MODE == M_FORCE || MODE == M_FORCE1 || kFE;   // force (two-phase / one-phase)
     constexpr bool k2P = MODE == M_FORCE;
     constexpr bool kF1 = MODE == M_FORCE1 || kFE;
-    constexpr bool kE = MODE == M_U || MODE == M_DU;   // FP64 energy gathers
+    // FP64 energy gathers; U2: U with two potential tables, one after the other in uconst and tab
+    constexpr bool kU2 = MODE == M_U2;
+    constexpr bool kE = MODE == M_U || MODE == M_DU || kU2;
     // the one-phase force traversal counting its accepted pairs with a nonzero term
     // instead of evaluating them: same staging, culling, lists and FP64 test
     constexpr bool kFC = MODE == M_FCOUNT;
@@ -448,7 +450,8 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
     // one cell's run owns nothing and leaves before the tables arrive
     constexpr int kThreads = kWaves * kWave;
     constexpr int kC8Per = (2 * kMaxTypes * kMaxTypes + kThreads - 1) / kThreads;
-    constexpr int kCdPer = (6 * kMaxTypes * kMaxTypes + kThreads - 1) / kThreads;
+    constexpr int kCdPer = ((kU2 ? 12 : 6) * kMaxTypes * kMaxTypes + kThreads - 1) / kThreads;
+    const int ncd = (kU2 ? 12 : 6) * nT * nT;
     float4 c8[kF ? kC8Per : 1];
     double cd[(!kF || kFE) ? kCdPer : 1];
     float rf = 0.f, re = 0.f;
@@ -464,13 +467,14 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
         for (int k = 0; k < kCdPer; k++) {
             const int t = threadIdx.x + k * kThreads;
-            cd[k] = uconst[min(t, 6 * nT * nT - 1)];
+            cd[k] = uconst[min(t, ncd - 1)];
         }
     }
     const int treach = min((int)threadIdx.x, nT - 1);   // threads past nT repeat the last type
     if (kCull) {
         rf = tab[8 * nT * nT + treach];
         re = tab[8 * nT * nT + kMaxTypes + treach];
+        if (kU2) re = fmaxf(re, tab[16 * nT * nT + 3 * kMaxTypes + treach]);
     }
     static_assert(kWaves == 1, "a wave may leave by itself");
     if (chunk <= kWave && !__any(a + lane < aend && (a + lane == 0 || kp != kc))) return;
@@ -482,7 +486,7 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
     if (!kF || kFE) {
 #pragma unroll
         for (int k = 0; k < kCdPer; k++)
-            if ((int)threadIdx.x + k * kThreads < 6 * nT * nT) sCd[threadIdx.x + k * kThreads] = cd[k];
+            if ((int)threadIdx.x + k * kThreads < ncd) sCd[threadIdx.x + k * kThreads] = cd[k];
     }
     // every thread stores (those past nT the last type's value again, the same bits)
     if (kCull) sReach2[treach] = kFE ? fmaxf(rf, re) : (kE ? re : rf);
@@ -533,7 +537,7 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
             // 1. stencil lookups, one cell per lane; the energy gathers take each pair from
             // the side that owns it, so they stage only the home cell and its forward half
             // shell
-            constexpr bool kOwnedOnly = MODE == M_U || MODE == M_DU;
+            constexpr bool kOwnedOnly = kE;
             int nst = 0, ncnt = 0;
             Shift shl;
             shl.x = shl.y = shl.z = shl.pad = 0.0;
@@ -593,7 +597,7 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
                 const Bead hb0 = sb[act ? hslot : s0];
                 const uint32_t me = sidx[act ? hslot : s0];
                 double fx = 0.0, fy = 0.0, fz = 0.0;
-                double accu = 0.0;
+                double accu = 0.0, accu2 = 0.0;
                 int cnt = 0;
                 // a lane's next candidate in its quarter's list; past a pass's end it goes on
                 // into the next one's, so that every tpp-th candidate of the cell is this
@@ -857,6 +861,12 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
                             const double dx = hb.x - q.x, dy = hb.y - q.y, dz = hb.z - q.z;   // staged imaged
                             const double r2 = sq3(dx, dy, dz);
                             if (MODE == M_U) return r2 < cut2 ? pair_u_any(r2, C) : 0.0;
+                            if (kU2) {
+                                if (!(r2 < cut2)) return 0.0;
+                                const double dr = sqrt_pos(r2);
+                                accu2 += pair_u_r(dr, C + 6 * nT * nT);
+                                return pair_u_r(dr, C);
+                            }
                             return du_pair(dx, dy, dz, r2, C, cut2, s2x, s2y, s2z, dseries);
                         };
                         int inext = lst[next];   // read one iteration ahead, as above
@@ -926,13 +936,20 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
                         if ((sub & (2 * st - 1)) == 0 && sub + st < tpp) cnt += o;
                     }
                     if (act && sub == 0) out.counts[me] = cnt;
-                } else if (MODE == M_U || MODE == M_DU) {
+                } else if (kE) {
                     // the home particle's share, its lanes combined by the same fixed tree
                     for (int st = 1; st < tpp; st <<= 1) {
                         const double o = __shfl(accu, lane + st);
                         if ((sub & (2 * st - 1)) == 0 && sub + st < tpp) accu += o;
                     }
                     if (act && sub == 0) out.energy[s0 + h0 + hi] = accu;
+                    if (kU2) {
+                        for (int st = 1; st < tpp; st <<= 1) {
+                            const double o = __shfl(accu2, lane + st);
+                            if ((sub & (2 * st - 1)) == 0 && sub + st < tpp) accu2 += o;
+                        }
+                        if (act && sub == 0) out.energy2[s0 + h0 + hi] = accu2;
+                    }
                 }
             }
         }
@@ -960,11 +977,11 @@ void launch_cells(hipStream_t st, const Params &P, int chunk, const Bead *sbeads
     // XCDs cost 5-16 % (3M bilayer 1072 -> 1000 us with 16 slots a chunk, 300k bilayer 128 ->
     // 119); over a vesicle the ranges are even and turns cost 1-2 % (240k: 96.6 -> 98.0 us).
     // The half-shell energy gathers gain on both in groups of 64.
-    const bool energy = MODE == M_U || MODE == M_DU;
+    const bool energy = MODE == M_U || MODE == M_DU || MODE == M_U2;
     const int turn = energy ? 6 : (P.flat ? 7 : 0);
     const bool both = MODE == M_FDU || MODE == M_FU;
     const bool floats = MODE == M_FORCE || MODE == M_FORCE1 || both, doubles = !floats || both;
-    const size_t tables_bytes = (size_t)P.nT * P.nT * ((floats ? 2 * sizeof(float4) : 0) + (doubles ? 6 * sizeof(double) : 0));
+    const size_t tables_bytes = (size_t)P.nT * P.nT * ((floats ? 2 * sizeof(float4) : 0) + (doubles ? (MODE == M_U2 ? 12 : 6) * sizeof(double) : 0));
     hipLaunchKernelGGL((k_cells<MODE, ASYM, ONE, MAXC, WAVES>), dim3(nb), dim3(kWaves * kWave), tables_bytes, st, P.n, P.nT, chunk, nb, cut2, cut2pre,
                        sbeads, skey, sidx, cstart, cend, reps, fconst, uconst, turn, out);
 }
@@ -1004,7 +1021,7 @@ void launch_pair_force(hipStream_t st, const Params &P, int chunk, int variant, 
                        const uint32_t *skey, const uint32_t *sidx, const int *cstart, const int *cend,
                        const DevRep *reps, const float *fconst, float4 *fpair)
 {
-    Out o{fpair, nullptr, nullptr, nullptr, nullptr, 0};
+    Out o{fpair, nullptr, nullptr, nullptr, nullptr, nullptr, 0};
     if (variant == 1)
         launch_for<M_FORCE, 128, 4, false>(P, st, chunk, sbeads, skey, sidx, cstart, cend, reps, fconst, nullptr, o);
     else if (P.n >= kManyBeads)
@@ -1017,7 +1034,7 @@ void launch_pair_force_du(hipStream_t st, const Params &P, int chunk, const Bead
                           const uint32_t *sidx, const int *cstart, const int *cend, const DevRep *reps,
                           const float *fconst, const double *uconst, float4 *fpair, double *energy)
 {
-    Out o{fpair, energy, nullptr, nullptr, nullptr, 0};
+    Out o{fpair, energy, nullptr, nullptr, nullptr, nullptr, 0};
     launch_for<M_FDU, 128, 4, true>(P, st, chunk, sbeads, skey, sidx, cstart, cend, reps, fconst, uconst, o);
 }
 
@@ -1025,8 +1042,16 @@ void launch_pair_force_u(hipStream_t st, const Params &P, int chunk, const Bead 
                          const uint32_t *sidx, const int *cstart, const int *cend, const DevRep *reps,
                          const float *fconst, const double *uconst, float4 *fpair, double *energy)
 {
-    Out o{fpair, energy, nullptr, nullptr, nullptr, 0};
+    Out o{fpair, energy, nullptr, nullptr, nullptr, nullptr, 0};
     launch_for<M_FU, 128, 4, true>(P, st, chunk, sbeads, skey, sidx, cstart, cend, reps, fconst, uconst, o);
+}
+
+void launch_pair_gather_u2(hipStream_t st, const Params &P, int chunk, const Bead *sbeads, const uint32_t *skey,
+                           const uint32_t *sidx, const int *cstart, const int *cend, const DevRep *reps,
+                           const float *tab, const double *uconst, double *energy, double *energy2)
+{
+    Out o{nullptr, energy, energy2, nullptr, nullptr, nullptr, 0};
+    launch_for<M_U2, 128, 4, false>(P, st, chunk, sbeads, skey, sidx, cstart, cend, reps, tab, uconst, o);
 }
 
 void launch_pair_gather(hipStream_t st, const Params &P, int chunk, int mode, const Bead *sbeads,
@@ -1034,7 +1059,7 @@ void launch_pair_gather(hipStream_t st, const Params &P, int chunk, int mode, co
                         const DevRep *reps, const float *tab, const double *uconst, double *energy, int *counts,
                         int *pairs, unsigned long long *npairs, long long cap)
 {
-    Out o{nullptr, energy, counts, pairs, npairs, cap};
+    Out o{nullptr, energy, nullptr, counts, pairs, npairs, cap};
     switch (mode) {
     case GATHER_U:
         launch_for<M_U, 128, 4, false>(P, st, chunk, sbeads, skey, sidx, cstart, cend, reps, tab, uconst, o);
