@@ -1128,8 +1128,8 @@ sm_ctx *create(const sm_system *s, int nrep)
             S.tile = dalloc<int4>(h.tile.size());
             S.rep_first = dalloc<int>(h.rep_first.size());
             S.tilesum = dalloc<double>(kSumCols * h.tile.size());
-            S.ticket = dalloc<uint32_t>(nrep);
-            HIPCHK(hipMemsetAsync(S.ticket, 0, sizeof(uint32_t) * nrep, c->st));
+            S.ticket = dalloc<uint32_t>((size_t)kTicketWords * nrep);
+            HIPCHK(hipMemsetAsync(S.ticket, 0, sizeof(uint32_t) * kTicketWords * nrep, c->st));
             if (!h.tile.empty())
                 HIPCHK(hipMemcpyAsync(S.tile, h.tile.data(), sizeof(int4) * h.tile.size(), hipMemcpyHostToDevice, c->st));
             HIPCHK(hipMemcpyAsync(S.rep_first, h.rep_first.data(), sizeof(int) * h.rep_first.size(),

@@ -98,10 +98,11 @@ enum : unsigned { TAG_LANGEVIN = 0, TAG_MC = 1, TAG_LANGEVIN_INIT = 2 };
 // replica's sum does not depend on the other replicas.  At most kSumTiles tiles a range, of at
 // least kSumTile elements: one workgroup a tile, then the range's last one sums the tiles.
 constexpr int kSumTile = 512, kSumTiles = 1024, kSumCols = 4;
+constexpr int kTicketWords = 32;   // a replica's ticket has a cache line: adds to one line queue
 struct SegTiles {
     int4 *tile;        // (begin, end, replica, -) per tile, device
     int *rep_first;    // first tile of each replica (R + 1 entries), device
-    uint32_t *ticket;  // tiles done per replica: zero between launches, device
+    uint32_t *ticket;  // tiles done per replica, kTicketWords apart: zero between launches, device
     double *tilesum;   // ntiles x kSumCols, device
     int ntiles;
 };
