@@ -7,8 +7,8 @@
 Workload (`value`): the 80,000-lipid vesicle (240,000 beads) from the liposome generator
 (seed 1234, areal density 3.45, box 400^3, dt 0.02, T 3, gamma 1, tension 0 so no box
 moves), built in memory with the product's generator (byte-identical to the reference
-generator).  A step is one full MD step: Verlet first half + cell key, radix sort,
-reorder + cell table, pair force, CHAIN forces + Langevin + second half-kick.  Inputs are
+generator).  A step is one full MD step: Verlet first half + cell key, cell build
+(sort, reorder, cell table), pair force, CHAIN forces + Langevin + second half-kick.  Inputs are
 resident in HBM before timing starts; no measurement or file output inside the timed loop.
 
 `batched`: the 64-replica tension x temperature sweep (softmold_amd.sweep) stepped as one
@@ -293,7 +293,7 @@ def main():
                     help="with --batched-only: step the batch with these knobs, without the autotuner "
                          "and without the sequential baseline")
     ap.add_argument("--sort-mode", type=int, choices=(0, 1, 2), default=None,
-                    help="the plain workload's cell sort: 0 every key, 1 incremental, 2 every key in a window "
+                    help="the plain workload's cell sort: 0 every key, 1 incremental, 2 counted per cell of a window "
                          "(default: the solver's)")
     args = ap.parse_args()
     if args.calib_copy:
@@ -363,10 +363,10 @@ def main():
     # the whole step against HBM: the per-bead algorithmic bytes of an unfused FP32 step
     # (integrate + key 76, radix sort 16 per pass, reorder 36, pair 28, bonded 40,
     # scatter 16, second half + Langevin 36) and 8 B per occupied cell; the sort takes
-    # ceil(bits / 8) passes over the cell indices, or two over the keys of a window of at
-    # most 2^18 cells
+    # ceil(bits / 8) passes over the cell indices, or one where the beads are counted per cell
+    # of a window (each goes into its cell's bucket and out of it)
     bits = max(1, int(np.ceil(np.log2(float(np.prod(nc))))))
-    passes = 2 if window_path else (bits + 7) // 8
+    passes = 1 if window_path else (bits + 7) // 8
     step_bytes = (232.0 + 16.0 * passes) * n + 8.0 * occ
     step_gbs = step_bytes / (ms_per_step * 1e-3) / 1e9
 

@@ -157,7 +157,7 @@ struct sm_ctx {
     // MI355X: 38.4 against 48.9 us per step at 240k beads (the movers' passes and the
     // merge are latency-bound launches), 126 against 115 us at 3M, 156 against 118 us for
     // the 64-replica sweep of 2.8M; contexts of a million beads or more start in mode 1,
-    // single replicas that the window sort fits start in mode 2, and the autotuner tries
+    // single replicas whose builds count beads start in mode 2, and the autotuner tries
     // every mode the context allows.
     int sort_mode = 0;
     uint32_t *kidx[2] = {nullptr, nullptr};

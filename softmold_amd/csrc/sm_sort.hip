@@ -808,10 +808,10 @@ __device__ void build_sorted(WLds<kRounds> &L, int n, const BuildArgs &a, const 
     }
 }
 
-// The next build's window: this build's after the fast path; after the fallback, the
-// occupied cell range that it measured, widened by one cell on each side and clipped to the grid,
-// or none (wx = 0) when that holds more cells than there are counters.  By the first wave of a workgroup
-// that has passed the range's barrier.
+// The next build's window: this build's after the fast path; after the fallback, the occupied
+// cell range that it measured, widened by one cell on each side and clipped to the grid, or none
+// (wx = 0) when that holds more cells than there are counters.  By the first wave of a
+// workgroup that has passed the range's barrier.
 __device__ inline void next_window(const BuildArgs &a, const WinDesc &w, bool fallback)
 {
     const int t = threadIdx.x;
