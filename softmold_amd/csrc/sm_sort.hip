@@ -592,11 +592,13 @@ __device__ inline uint32_t hist_sum(const uint32_t *__restrict__ ghist)
 }
 
 // `count` workgroups arrive at *ctr before any goes on; its stores before are visible to
-// every workgroup's loads after: the workgroup barrier orders the threads' stores before thread
-// 0's release, and its acquire before their loads (one cache write-back and one invalidation
-// a workgroup, not one a wave).  Bounded like the look-back.
+// every workgroup's loads after.  Thread 0 releases and acquires for the workgroup (one cache
+// write-back and one invalidation, not one a wave), which reaches what the other waves wrote
+// once their memory operations are complete: each wave waits for its own, since the workgroup
+// barrier does not.  Bounded like the look-back.
 __device__ inline void grid_sync(uint32_t *ctr, uint32_t count, int *errflag)
 {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (threadIdx.x == 0) {
         __hip_atomic_fetch_add(ctr, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
