@@ -190,8 +190,9 @@ int sm_potential_delta(sm_ctx *ctx, const double *scale, double *du_pair, double
  * "mc_fused" = 1 (default) to take a box-move step's pair dU in the traversal of
  * that step's pair force, 0 in a gather of its own after the kick (sm_potential_delta
  * follows the same knob); the two sum the same FP64 terms in different orders.
- * sm_tune_get also reads "sort_window_path": 1 if the last build's sort took the window
- * path (it synchronises the context's stream). */
+ * sm_tune_get also reads "sort_count_path": 1 if the last build counted its beads per cell
+ * and did not fall back to sorting them, and "sort_window_path": 1 if it did so within a
+ * window (both synchronise the context's stream). */
 int sm_tune(sm_ctx *ctx, const char *knob, int32_t value);
 int sm_tune_get(sm_ctx *ctx, const char *knob, int32_t *value);
 /* Autotuner (no reference counterpart): times `steps` steps of this context's own work

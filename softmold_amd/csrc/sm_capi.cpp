@@ -296,6 +296,19 @@ struct sm_ctx {
         return win_book(hist[p], n, win ? wdesc + 8 * p : nullptr, counts[p], bucket, win ? 0u : (uint32_t)capacity,
                         (uint32_t)count_cells);
     }
+    // whether the last build counted its beads, and did not fall back to sorting them (waits for
+    // the stream); its window and flag: its scratch is cleared only by the next build
+    bool counted_last()
+    {
+        if (!cnt_last) return false;
+        const int lp = 1 - sort_parity;
+        uint32_t wx = 1, flag = 0;
+        if (win_last) HIPCHK(hipMemcpyAsync(&wx, wdesc + 8 * lp + 3, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
+        const uint32_t *f = win_book(hist[lp], n, nullptr, nullptr, nullptr, 0u, 0u).flag;
+        HIPCHK(hipMemcpyAsync(&flag, f, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
+        HIPCHK(hipStreamSynchronize(st));
+        return wx != 0 && flag == 0;
+    }
     // a key kernel ran without its sort: zero what it added to the sort's scratch
     void restart_hist(uint32_t *gh)
     {
@@ -1649,20 +1662,9 @@ int sm_tune_get(sm_ctx *c, const char *knob, int32_t *value)
         else if (std::strcmp(knob, "graph") == 0) *value = c->use_graph ? 1 : 0;
         else if (std::strcmp(knob, "sort_mode") == 0) *value = c->sort_mode;
         else if (std::strcmp(knob, "mc_fused") == 0) *value = c->mc_fused ? 1 : 0;
-        else if (std::strcmp(knob, "sort_window_path") == 0) {
-            *value = 0;
-            if (c->win_last) {
-                // the last sort's window and fallback flag: its scratch is cleared only by the
-                // next sort's reorder
-                const int lp = 1 - c->sort_parity;
-                uint32_t wx = 0, flag = 0;
-                HIPCHK(hipMemcpyAsync(&wx, c->wdesc + 8 * lp + 3, sizeof(uint32_t), hipMemcpyDeviceToHost, c->st));
-                HIPCHK(hipMemcpyAsync(&flag, win_book(c->hist[lp], c->n, nullptr, nullptr, nullptr, 0u, 0u).flag, sizeof(uint32_t),
-                                      hipMemcpyDeviceToHost, c->st));
-                HIPCHK(hipStreamSynchronize(c->st));
-                *value = (wx != 0 && flag == 0) ? 1 : 0;
-            }
-        } else invalid(std::string("unknown knob ") + knob);
+        else if (std::strcmp(knob, "sort_window_path") == 0) *value = c->win_last && c->counted_last() ? 1 : 0;
+        else if (std::strcmp(knob, "sort_count_path") == 0) *value = c->counted_last() ? 1 : 0;
+        else invalid(std::string("unknown knob ") + knob);
     });
 }
 
