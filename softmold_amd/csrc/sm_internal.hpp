@@ -158,8 +158,7 @@ struct MoveBook {
 //  - dense (sort_mode 0 or 2, any context of at most kWinMaxTiles tiles of keys, 524288 beads,
 //    whose cell table holds at most kWinCells cells): the cell index itself.  The counters take
 //    25 atomics a ns, a radix pass 5 us at least: per step 119 us counted against 144
-//    sorted at 192k beads in 16 bilayers, 252 against 262 at 470k; the fallback's workgroups
-//    must fit the card together, which ends it there.
+//    sorted at 192k beads in 16 bilayers, 252 against 262 at 470k, so the gain ends there.
 // A key outside the window, or a cell of more beads than a bucket holds, raises the build's
 // fallback flag; the same launch then sorts the cell indices in three 8-bit passes.
 // desc == NULL and cells == 0: neither.
@@ -181,7 +180,7 @@ struct WinBook {
     uint32_t limit;         // cells that counts and bucket hold (a multiple of kCoarseCells)
 };
 // the counting builds' scratch, after the sort_scratch_words(n, 4) words of the every-key sort:
-// coarse, bbox, {flag, 4 barrier counters, pad}, then 3 passes x tiles x 256 look-back words;
+// coarse, bbox, {flag, piece counter, 5 stage counters, pad}, then 3 passes x tiles x 256 look-back words;
 // the key kernel writes the first kWinKeyWords of it
 constexpr size_t kWinKeyWords = (size_t)kCoarseCopies * kCoarse + 16 * 8 + 8;
 size_t sortw_words(int n, bool counting);

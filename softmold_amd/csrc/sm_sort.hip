@@ -458,10 +458,12 @@ __global__ __launch_bounds__(kThreads) void k_merge(int n, const int *__restrict
 // The thread's bead goes to the run's first slot plus the run's beads of lower index, counted
 // in the bucket, a row that the run's threads share in the caches.
 //
-// The fallback: three 8-bit passes over the cell indices and the reorder, with a grid-wide
-// barrier before each.  It turns window keys back into cell indices, counts their digits and
-// measures the occupied range for the next window.  Its at most kWinMaxTiles workgroups are
-// the only ones that wait, and all of them fit the card together.
+// The fallback: five stages -- window keys back to cell indices, with their digits counted and
+// the occupied range measured for the next window; three 8-bit passes over the cell indices;
+// the reorder -- of one piece a tile.  Workgroups draw the pieces in order from a counter, and a
+// piece waits only for pieces drawn before it (the whole stage before, and the look-back's lower
+// tiles), so the one that was drawn first of those unfinished never waits: the build ends
+// however few of the workgroups are on the card together, whatever else runs there.
 // ---------------------------------------------------------------------------------------
 template <int kRounds>
 struct WLds {
@@ -591,17 +593,10 @@ __device__ inline uint32_t hist_sum(const uint32_t *__restrict__ ghist)
     return g;
 }
 
-// `count` workgroups arrive at *ctr before any goes on; its stores before are visible to
-// every workgroup's loads after.  Thread 0 releases and acquires for the workgroup (one cache
-// write-back and one invalidation, not one a wave), which reaches what the other waves wrote
-// once their memory operations are complete: each wave waits for its own, since the workgroup
-// barrier does not.  Bounded like the look-back.
-__device__ inline void grid_sync(uint32_t *ctr, uint32_t count, int *errflag)
+// Waits for `count` arrivals, bounded like the look-back.
+__device__ inline void await(uint32_t *ctr, uint32_t count, int *errflag)
 {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
     if (threadIdx.x == 0) {
-        __hip_atomic_fetch_add(ctr, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
         int spins = 0;
         while (__hip_atomic_load(ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < count) {
             if (++spins >= kSpinLimit) {
@@ -722,11 +717,9 @@ __device__ void build_slots(BLds &L, int n, const BuildArgs &a, const WinDesc &w
 }
 
 template <int kRounds>
-__device__ void build_sorted(WLds<kRounds> &L, int n, const BuildArgs &a, const WinDesc &w, bool dense)
+__device__ void build_count(WLds<kRounds> &L, int n, int tile, const BuildArgs &a, const WinDesc &w, bool dense)
 {
-    const int t = threadIdx.x, lane = t & (kWave - 1), wave = t / kWave, tile = blockIdx.x;
-    uint32_t *st0 = a.status, *st1 = st0 + (size_t)a.tiles * 256, *st2 = st1 + (size_t)a.tiles * 256;
-    uint32_t *bar = a.wb.flag + 1;
+    const int t = threadIdx.x, lane = t & (kWave - 1), wave = t / kWave;
     // the counts of the keys that did lie in the window
     if (dense || w.wx != 0u)
         for (uint32_t c = tile * kThreads + t; c < a.wb.limit; c += a.tiles * kThreads) a.wb.counts[c] = 0u;
@@ -783,14 +776,12 @@ __device__ void build_sorted(WLds<kRounds> &L, int n, const BuildArgs &a, const 
         for (int q = 0; q < kWavesPerBlock; q++) v = max(v, L.bb[q][t]);
         if (v) atomicMax(&a.wb.bbox[(tile % kHistCopies) * 8 + t], v);
     }
-    // all the tiles' workgroups are resident, so each pass's tiles are theirs in order
-    grid_sync(bar, a.tiles, a.errflag);
-    wpass<kRounds>(L, n, 0, tile, hist_sum(a.ghist), true, a.k0, a.v0, a.k1, a.v1, st0, a.errflag);
-    grid_sync(bar + 1, a.tiles, a.errflag);
-    wpass<kRounds>(L, n, 8, tile, hist_sum(a.ghist + 256), false, a.k1, a.v1, a.k2, a.v2, st1, a.errflag);
-    grid_sync(bar + 2, a.tiles, a.errflag);
-    wpass<kRounds>(L, n, 16, tile, hist_sum(a.ghist + 512), false, a.k2, a.v2, a.k0, a.v0, st2, a.errflag);
-    grid_sync(bar + 3, a.tiles, a.errflag);
+}
+
+template <int kRounds>
+__device__ void build_reorder(int n, int tile, const BuildArgs &a)
+{
+    const int t = threadIdx.x, base = tile * kThreads * kRounds;
     uint32_t vr[kRounds];
 #pragma unroll
     for (int r = 0; r < kRounds; r++) vr[r] = min(a.v0[min(base + r * kThreads + t, n - 1)], (uint32_t)n - 1u);
@@ -812,8 +803,8 @@ __device__ void build_sorted(WLds<kRounds> &L, int n, const BuildArgs &a, const 
 
 // The next build's window: this build's after the fast path; after the fallback, the occupied
 // cell range that it measured, widened by one cell on each side and clipped to the grid, or none
-// (wx = 0) when that holds more cells than there are counters.  By the first wave of a
-// workgroup that has passed the range's barrier.
+// (wx = 0) when that holds more cells than there are counters.  By one wave, which has waited for
+// the range.
 __device__ inline void next_window(const BuildArgs &a, const WinDesc &w, bool fallback)
 {
     const int t = threadIdx.x;
@@ -843,6 +834,47 @@ __device__ inline void next_window(const BuildArgs &a, const WinDesc &w, bool fa
     for (int j = 0; j < 6; j++) a.desc_next[j] = d[j];
 }
 
+// The fallback's pieces of this workgroup: it draws them from *next and counts each stage's in
+// done[stage].  A piece's stores are visible to the workgroups that see its count: thread 0
+// releases for the workgroup (one cache write-back, not one a wave), which reaches what the
+// other waves wrote once their memory operations are complete; each wave waits for its own, since
+// the workgroup barrier does not.  Counting a piece and drawing the next are one block of thread
+// 0 between barriers, and the piece is a scalar: with a block at either end of the loop the
+// compiler let the other lanes go round it without thread 0.
+template <int kRounds>
+__device__ void build_sorted(WLds<kRounds> &L, int n, const BuildArgs &a, const WinDesc &w, bool dense)
+{
+    __shared__ uint32_t s_piece;
+    uint32_t *const next = a.wb.flag + 1, *const done = next + 1;
+    const uint32_t tiles = (uint32_t)a.tiles;
+    if (threadIdx.x == 0) s_piece = __hip_atomic_fetch_add(next, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    for (;;) {
+        const uint32_t piece = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_piece), stage = piece / tiles;
+        const int tile = (int)(piece - stage * tiles);
+        if (stage > 4u) return;
+        if (stage > 0u) await(done + stage - 1u, tiles, a.errflag);
+        if (stage == 0u) {
+            build_count<kRounds>(L, n, tile, a, w, dense);
+        } else if (stage < 4u) {
+            const uint32_t p = stage - 1u;
+            uint32_t *const k[4] = {a.k0, a.k1, a.k2, a.k0}, *const v[4] = {a.v0, a.v1, a.v2, a.v0};
+            wpass<kRounds>(L, n, (int)(8u * p), tile, hist_sum(a.ghist + 256u * p), p == 0u, k[p], v[p], k[p + 1u],
+                           v[p + 1u], a.status + (size_t)p * tiles * 256u, a.errflag);
+        } else {
+            if (!dense && tile == 0 && threadIdx.x < kWave) next_window(a, w, true);
+            build_reorder<kRounds>(n, tile, a);
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            __hip_atomic_fetch_add(done + stage, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+            s_piece = __hip_atomic_fetch_add(next, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        __syncthreads();
+    }
+}
+
 template <int kRounds>
 __global__ __launch_bounds__(kThreads) void k_build(int n, BuildArgs a)
 {
@@ -856,11 +888,12 @@ __global__ __launch_bounds__(kThreads) void k_build(int n, BuildArgs a)
     WinDesc w{};
     if (!dense) w = load_win(a.wb.desc);
     const bool fallback = (!dense && w.wx == 0u) || *a.wb.flag != 0u;   // the same in every workgroup
-    if (!fallback)
-        build_slots(L.b, n, a, w, dense);
-    else if ((int)blockIdx.x < a.tiles)
-        build_sorted<kRounds>(L.w, n, a, w, dense);
-    if (!dense && blockIdx.x == 0 && threadIdx.x < kWave) next_window(a, w, fallback);
+    if (fallback) {
+        if ((int)blockIdx.x < a.tiles) build_sorted<kRounds>(L.w, n, a, w, dense);
+        return;
+    }
+    build_slots(L.b, n, a, w, dense);
+    if (!dense && blockIdx.x == 0 && threadIdx.x < kWave) next_window(a, w, false);
 }
 
 }  // namespace
