@@ -950,6 +950,7 @@ sm_ctx *create(const sm_system *s, int nrep)
         // once per device while it is current
         HIPCHK(hipGetDevice(&c->device));
         HIPCHK(noalloc_scratch_init(c->device));
+        c->link.create(nrep);
 
         // chains: per-bead role table and per-chain list, replica after replica
         std::vector<int2> perBead(n, make_int2(-1, 0));

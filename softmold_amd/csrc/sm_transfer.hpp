@@ -24,6 +24,19 @@ public:
     static constexpr int kChunk = 65536;          // beads a pinned buffer holds
     static constexpr int kThreadBeads = 65536;    // fewer beads are unpacked by the caller alone
     static constexpr int kWorkers = 8;
+    static constexpr size_t kResults = 4;         // doubles a replica that one fetch returns, at most
+
+    // With the context's device current: what every call needs -- the events, which belong to the
+    // device that is current when they are made, and the buffer of the largest result of
+    // `replicas` replicas -- so that no call depends on the device current then, and a result's
+    // first fetch allocates nothing.
+    void create(int replicas)
+    {
+        check(hipGetDevice(&device_), "device");
+        for (hipEvent_t &e : ev_) check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "event");
+        room_ = kResults * (size_t)replicas;
+        check(hipHostMalloc(reinterpret_cast<void **>(&head_), (room_ + 1) * sizeof(double), hipHostMallocDefault), "buffer");
+    }
 
     void destroy()
     {
@@ -42,7 +55,7 @@ public:
     // `count` doubles from device memory with the context's state flags: returns the flags
     int fetch(hipStream_t st, const DevGlobal *glob, const double *src, size_t count, double *dst)
     {
-        head(count);
+        if (count > room_) throw smapi::ApiError(SM_ERR_STATE, "a result larger than its buffer");
         launch_post(st, src, count, glob, head_);
         check(hipGetLastError(), "post");
         finish(st, 0);
@@ -53,7 +66,6 @@ public:
     // The box lengths of every replica and the state flags.
     int fetch_boxes(hipStream_t st, const DevGlobal *glob, const DevRep *reps, int nrep, double *box)
     {
-        head(3 * (size_t)nrep);
         launch_pack(st, 0, 0, PackSrc{nullptr, nullptr, nullptr}, nullptr, reps, nrep, glob, head_);
         check(hipGetLastError(), "pack");
         finish(st, 0);
@@ -68,7 +80,6 @@ public:
     {
         const PackSrc s{pos ? src.beads : nullptr, a ? src.a : nullptr, b ? src.b : nullptr};
         const int chunks = (n + kChunk - 1) / kChunk;
-        head(3 * (size_t)nrep);
         buffers(std::min(n, kChunk), chunks > 1 ? 2 : 1);
         auto launch = [&](int c) {
             const int first = c * kChunk, count = std::min(kChunk, n - first);
@@ -147,7 +158,6 @@ public:
     // the next fetch
     void send_scale(hipStream_t st, DevRep *reps, int nrep, const double *scale)
     {
-        head(3 * (size_t)nrep);
         std::memcpy(head_ + 1, scale, 3 * sizeof(double) * (size_t)nrep);
         launch_set_scale(st, reps, nrep, head_ + 1);
         check(hipGetLastError(), "scale");
@@ -156,7 +166,6 @@ public:
     // beads[i].x, y, z = pos[3 i ..] for n beads; the caller's array is free again on return
     void send_positions(hipStream_t st, int n, const double *pos, Bead *beads)
     {
-        events();
         const int chunks = (n + kChunk - 1) / kChunk;
         buffers(std::min(n, kChunk), chunks > 1 ? 2 : 1);
         for (int c = 0; c < chunks; c++) {
@@ -172,8 +181,9 @@ public:
 private:
     void *buf_[2] = {nullptr, nullptr};
     size_t beads_[2] = {0, 0};
-    double *head_ = nullptr;      // flags, then up to head_count_ doubles
-    size_t head_count_ = 0;
+    double *head_ = nullptr;      // flags, then room_ doubles
+    size_t room_ = 0;
+    int device_ = 0;              // the context's
     hipEvent_t ev_[2] = {nullptr, nullptr};
 
     static void check(hipError_t e, const char *what)
@@ -181,25 +191,11 @@ private:
         if (e != hipSuccess)
             throw smapi::ApiError(SM_ERR_HIP, std::string(hipGetErrorName(e)) + " in a " + what + " of a result transfer");
     }
-    void events()
-    {
-        for (hipEvent_t &e : ev_)
-            if (!e) check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "event");
-    }
-    void head(size_t count)
-    {
-        events();
-        if (head_ && count <= head_count_) return;
-        if (head_) (void)hipHostFree(head_);
-        head_ = nullptr;
-        head_count_ = 0;
-        check(hipHostMalloc(reinterpret_cast<void **>(&head_), (count + 1) * sizeof(double), hipHostMallocDefault), "buffer");
-        head_count_ = count;
-    }
     void buffers(int beads, int want)
     {
         for (int i = 0; i < want; i++) {
             if (buf_[i] && (size_t)beads <= beads_[i]) continue;
+            OnDevice here(device_);
             if (buf_[i]) (void)hipHostFree(buf_[i]);
             buf_[i] = nullptr;
             beads_[i] = 0;
@@ -207,6 +203,22 @@ private:
             beads_[i] = (size_t)beads;
         }
     }
+    // the context's device current, then again the caller's
+    struct OnDevice {
+        int was = -1;
+        explicit OnDevice(int device)
+        {
+            int now;
+            check(hipGetDevice(&now), "device");
+            if (now == device) return;
+            check(hipSetDevice(device), "device");
+            was = now;
+        }
+        ~OnDevice()
+        {
+            if (was >= 0) (void)hipSetDevice(was);
+        }
+    };
     void finish(hipStream_t st, int e)
     {
         check(hipEventRecord(ev_[e], st), "event");

@@ -1,0 +1,181 @@
+// Drives HostLink (softmold_amd/csrc/sm_transfer.hpp) without a GPU: the HIP calls it makes and
+// the kernels it launches are played here on host memory, with a device to a stream, an event
+// and an allocation.  Usage: transfer_harness SCENARIO; exit code 0 if it held.
+#include "sm_transfer.hpp"
+
+#include <cstdio>
+#include <cstdlib>
+#include <string>
+
+namespace {
+
+struct FakeStream { int device; };
+struct FakeEvent { int device; };
+
+int g_device = 0;                          // the current device
+int g_allocations = 0, g_events = 0;       // made so far
+int g_buffer_device = -1;                  // current at the last pinned allocation
+
+#define EXPECT(cond)                                                       \
+    do {                                                                   \
+        if (!(cond)) {                                                     \
+            std::fprintf(stderr, "line %d: %s\n", __LINE__, #cond);        \
+            std::exit(1);                                                  \
+        }                                                                  \
+    } while (0)
+
+}  // namespace
+
+thread_local std::string smapi::g_err;
+
+extern "C" {
+hipError_t hipGetDevice(int *d) { *d = g_device; return hipSuccess; }
+hipError_t hipSetDevice(int d) { g_device = d; return hipSuccess; }
+hipError_t hipGetLastError() { return hipSuccess; }
+const char *hipGetErrorName(hipError_t e) { return e == hipSuccess ? "hipSuccess" : "hipError"; }
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned)
+{
+    g_events++;
+    *e = reinterpret_cast<hipEvent_t>(new FakeEvent{g_device});
+    return hipSuccess;
+}
+hipError_t hipEventDestroy(hipEvent_t e) { delete reinterpret_cast<FakeEvent *>(e); return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t st)
+{
+    return reinterpret_cast<FakeEvent *>(e)->device == reinterpret_cast<FakeStream *>(st)->device ? hipSuccess
+                                                                                                  : hipErrorInvalidHandle;
+}
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipHostMalloc(void **p, size_t bytes, unsigned)
+{
+    g_allocations++;
+    g_buffer_device = g_device;
+    *p = std::malloc(bytes);
+    return hipSuccess;
+}
+hipError_t hipHostFree(void *p) { std::free(p); return hipSuccess; }
+}
+
+namespace smdev {
+void launch_post(hipStream_t, const double *src, size_t count, const DevGlobal *glob, double *head)
+{
+    *reinterpret_cast<long long *>(head) = glob->flags;
+    for (size_t i = 0; i < count; i++) head[1 + i] = src[i];
+}
+void launch_pack(hipStream_t, int first, int count, const PackSrc &src, double *out, const DevRep *reps, int nrep,
+                 const DevGlobal *glob, double *head)
+{
+    if (head) {
+        *reinterpret_cast<long long *>(head) = glob->flags;
+        for (int i = 0; i < 3 * nrep; i++) head[1 + i] = reps[i / 3].L[i % 3];
+    }
+    float *f = reinterpret_cast<float *>(out + (src.beads ? 3 * (size_t)count : 0));
+    for (int e = 0; e < 3 * count; e++) {
+        const int i = first + e / 3, c = e % 3;
+        if (src.beads) out[e] = (&src.beads[i].x)[c];
+        if (src.a) f[e] = (&src.a[i].x)[c];
+        if (src.b) f[(src.a ? 3 * (size_t)count : 0) + e] = (&src.b[i].x)[c];
+    }
+}
+void launch_set_scale(hipStream_t, DevRep *reps, int nrep, const double *scale)
+{
+    for (int i = 0; i < 3 * nrep; i++) reps[i / 3].scale[i % 3] = scale[i];
+}
+void launch_set_positions(hipStream_t, int first, int count, const double *pos, Bead *beads)
+{
+    for (int e = 0; e < 3 * count; e++) (&beads[first + e / 3].x)[e % 3] = pos[e];
+}
+}  // namespace smdev
+
+using namespace smdev;
+
+namespace {
+
+// A context's state: n beads of R replicas on device `device`.
+struct State {
+    int n, R;
+    FakeStream stream;
+    std::vector<Bead> beads;
+    std::vector<float4> vel;
+    std::vector<DevRep> reps;
+    DevGlobal glob{};
+    State(int n_, int r_, int device) : n(n_), R(r_), stream{device}, beads(n_), vel(n_), reps(r_)
+    {
+        for (int i = 0; i < n; i++) {
+            beads[i].x = 0.5 + i, beads[i].y = 2.0 * i, beads[i].z = -1.0 * i;
+            vel[i].x = 0.25f * i, vel[i].y = 1.0f, vel[i].z = -0.5f * i;
+        }
+        for (int r = 0; r < R; r++)
+            for (int d = 0; d < 3; d++) reps[r].L[d] = 10.0 * r + d;
+        glob.flags = 5;
+    }
+    hipStream_t st() { return reinterpret_cast<hipStream_t>(&stream); }
+    PackSrc src() { return PackSrc{beads.data(), vel.data(), nullptr}; }
+};
+
+void check_download(State &s, HostLink &link)
+{
+    std::vector<double> pos(3 * (size_t)s.n, 7.0), vel(pos), box(3 * (size_t)s.R);
+    EXPECT(link.fetch_beads(s.st(), s.n, s.src(), pos.data(), vel.data(), nullptr, &s.glob, s.reps.data(), s.R, box.data()) == 5);
+    for (int i = 0; i < s.n; i++)
+        for (int c = 0; c < 3; c++) {
+            EXPECT(pos[3 * (size_t)i + c] == (&s.beads[i].x)[c]);
+            EXPECT(vel[3 * (size_t)i + c] == (&s.vel[i].x)[c]);
+        }
+    for (int i = 0; i < 3 * s.R; i++) EXPECT(box[i] == s.reps[i / 3].L[i % 3]);
+}
+
+// Calls made while another device is current than the context's.
+int other_device()
+{
+    State s(200001, 3, 1);
+    HostLink link;
+    g_device = 1;
+    link.create(s.R);
+    g_device = 0;
+    std::vector<double> res(4 * (size_t)s.R, 3.25), got(res.size()), box(3 * (size_t)s.R);
+    EXPECT(link.fetch(s.st(), &s.glob, res.data(), res.size(), got.data()) == 5 && got == res);
+    EXPECT(link.fetch_boxes(s.st(), &s.glob, s.reps.data(), s.R, box.data()) == 5 && box[4] == 11.0);
+    check_download(s, link);
+    EXPECT(g_buffer_device == 1 && g_device == 0);
+    std::vector<double> pos(3 * (size_t)s.n);
+    for (size_t e = 0; e < pos.size(); e++) pos[e] = 0.125 * e;
+    link.send_positions(s.st(), s.n, pos.data(), s.beads.data());
+    for (int i = 0; i < s.n; i++) EXPECT(s.beads[i].y == pos[3 * (size_t)i + 1]);
+    link.send_scale(s.st(), s.reps.data(), s.R, pos.data());
+    EXPECT(s.reps[2].scale[1] == pos[7]);
+    link.destroy();
+    return 0;
+}
+
+// The first result of a new context, and the largest.
+int no_allocation()
+{
+    State s(10, 5, 0);
+    HostLink link;
+    link.create(s.R);
+    const int made = g_allocations + g_events;
+    std::vector<double> res(4 * (size_t)s.R, -2.0), got(res.size());
+    for (size_t count : {(size_t)s.R, res.size(), (size_t)0}) link.fetch(s.st(), &s.glob, res.data(), count, got.data());
+    EXPECT(got == res);
+    link.fetch_boxes(s.st(), &s.glob, s.reps.data(), s.R, got.data());
+    EXPECT(g_allocations + g_events == made);
+    link.destroy();
+    return 0;
+}
+
+}  // namespace
+
+int main(int argc, char **argv)
+{
+    const std::string what = argc > 1 ? argv[1] : "";
+    try {
+        if (what == "other_device") return other_device();
+        if (what == "no_allocation") return no_allocation();
+    } catch (const std::exception &e) {
+        std::fprintf(stderr, "%s: %s\n", what.c_str(), e.what());
+        return 1;
+    }
+    std::fprintf(stderr, "unknown scenario\n");
+    return 2;
+}
