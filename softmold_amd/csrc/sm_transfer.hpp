@@ -5,7 +5,7 @@
 // One pack kernel and one event take 13 us on an MI355X where every pageable copy takes 25 us
 // (a download was five of them); at 3M beads the 144 MB cross the bus in 3 ms, but one thread
 // fills the 216 MB of doubles in 46 ms, eight in 10 ms.  Large states therefore go in chunks
-// through two pinned buffers while up to kWorkers threads unpack the chunk before.
+// through pinned buffers while up to kWorkers threads unpack the chunk before.
 #pragma once
 #include "sm_errors.hpp"
 #include "sm_internal.hpp"
@@ -21,7 +21,19 @@ namespace smdev {
 
 class HostLink {
 public:
-    static constexpr int kChunk = 65536;          // beads a pinned buffer holds
+    // Chunks: beads that a pinned buffer holds, and buffers.  A context's first transfer allocates
+    // them: 45 us for 1.5 MiB, 290 and more from 3 MiB on, which made the first download of 72k
+    // beads 950 us where pageable copies took 600 (335 with the short ones).  A large download
+    // pays little for that and more for each chunk that is handed over: 240k beads 1050 to 1100
+    // us long, 1050 to 1500 short; 1M beads 3.0 and 4.1 ms.
+    struct Chunks {
+        int beads, buffers, count;
+        explicit Chunks(int n)
+            : beads(n > 196608 ? 65536 : 32768), buffers(n > 196608 ? 2 : 4), count((n + beads - 1) / beads)
+        {
+        }
+    };
+    static constexpr int kBuffers = 4;            // at most
     static constexpr int kThreadBeads = 65536;    // fewer beads are unpacked by the caller alone
     static constexpr int kWorkers = 8;
     static constexpr size_t kResults = 4;         // doubles a replica that one fetch returns, at most
@@ -79,21 +91,22 @@ public:
                     const DevGlobal *glob, const DevRep *reps, int nrep, double *box)
     {
         const PackSrc s{pos ? src.beads : nullptr, a ? src.a : nullptr, b ? src.b : nullptr};
-        const int chunks = (n + kChunk - 1) / kChunk;
-        buffers(std::min(n, kChunk), chunks > 1 ? 2 : 1);
+        const Chunks ch(n);
+        const int chunks = ch.count;
+        buffers(std::min(n, ch.beads), std::min(chunks, ch.buffers));
         auto launch = [&](int c) {
-            const int first = c * kChunk, count = std::min(kChunk, n - first);
-            launch_pack(st, first, count, s, static_cast<double *>(buf_[c & 1]), reps, c == 0 ? nrep : 0, glob,
+            const int first = c * ch.beads, count = std::min(ch.beads, n - first);
+            launch_pack(st, first, count, s, static_cast<double *>(buf_[c % ch.buffers]), reps, c == 0 ? nrep : 0, glob,
                         c == 0 ? head_ : nullptr);
             check(hipGetLastError(), "pack");
-            check(hipEventRecord(ev_[c & 1], st), "event");
+            check(hipEventRecord(ev_[c % ch.buffers], st), "event");
         };
-        auto wait = [&](int c) { check(hipEventSynchronize(ev_[c & 1]), "event"); };
+        auto wait = [&](int c) { check(hipEventSynchronize(ev_[c % ch.buffers]), "event"); };
         // beads [count i / parts, count (i + 1) / parts) of chunk c into the caller's arrays
         auto unpack = [&](int c, int i, int parts) {
-            const int first = c * kChunk, count = std::min(kChunk, n - first);
+            const int first = c * ch.beads, count = std::min(ch.beads, n - first);
             const size_t e0 = 3 * ((size_t)count * i / parts), e1 = 3 * ((size_t)count * (i + 1) / parts);
-            const double *p = static_cast<const double *>(buf_[c & 1]);
+            const double *p = static_cast<const double *>(buf_[c % ch.buffers]);
             const float *f = reinterpret_cast<const float *>(p + (s.beads ? 3 * (size_t)count : 0));
             const size_t o = 3 * (size_t)first;
             if (s.beads) std::memcpy(pos + o + e0, p + e0, (e1 - e0) * sizeof(double));
@@ -141,13 +154,13 @@ public:
             }
             parts = 1 + (int)team.size();
             size.store(parts, std::memory_order_release);
-            if (chunks > 1) launch(1);
+            for (int c = 1; c < std::min(chunks, ch.buffers); c++) launch(c);
             for (int c = 0; c < chunks; c++) {
                 wait(c);
                 ready.store(c + 1, std::memory_order_release);
                 unpack(c, 0, parts);
                 while (done.load(std::memory_order_acquire) < (c + 1) * (parts - 1)) std::this_thread::yield();
-                if (c + 2 < chunks) launch(c + 2);
+                if (c + ch.buffers < chunks) launch(c + ch.buffers);
             }
         }
         if (box) std::memcpy(box, head_ + 1, 3 * sizeof(double) * (size_t)nrep);
@@ -166,25 +179,26 @@ public:
     // beads[i].x, y, z = pos[3 i ..] for n beads; the caller's array is free again on return
     void send_positions(hipStream_t st, int n, const double *pos, Bead *beads)
     {
-        const int chunks = (n + kChunk - 1) / kChunk;
-        buffers(std::min(n, kChunk), chunks > 1 ? 2 : 1);
+        const Chunks ch(n);
+        const int chunks = ch.count;
+        buffers(std::min(n, ch.beads), std::min(chunks, ch.buffers));
         for (int c = 0; c < chunks; c++) {
-            const int first = c * kChunk, count = std::min(kChunk, n - first);
-            check(hipEventSynchronize(ev_[c & 1]), "event");   // the buffer's last kernel is done
-            std::memcpy(buf_[c & 1], pos + 3 * (size_t)first, 3 * sizeof(double) * (size_t)count);
-            launch_set_positions(st, first, count, static_cast<const double *>(buf_[c & 1]), beads);
+            const int first = c * ch.beads, count = std::min(ch.beads, n - first);
+            check(hipEventSynchronize(ev_[c % ch.buffers]), "event");   // the buffer's last kernel is done
+            std::memcpy(buf_[c % ch.buffers], pos + 3 * (size_t)first, 3 * sizeof(double) * (size_t)count);
+            launch_set_positions(st, first, count, static_cast<const double *>(buf_[c % ch.buffers]), beads);
             check(hipGetLastError(), "unpack");
-            check(hipEventRecord(ev_[c & 1], st), "event");
+            check(hipEventRecord(ev_[c % ch.buffers], st), "event");
         }
     }
 
 private:
-    void *buf_[2] = {nullptr, nullptr};
-    size_t beads_[2] = {0, 0};
+    void *buf_[kBuffers] = {};
+    size_t beads_[kBuffers] = {};
     double *head_ = nullptr;      // flags, then room_ doubles
     size_t room_ = 0;
     int device_ = 0;              // the context's
-    hipEvent_t ev_[2] = {nullptr, nullptr};
+    hipEvent_t ev_[kBuffers] = {};
 
     static void check(hipError_t e, const char *what)
     {

@@ -15,6 +15,7 @@ struct FakeEvent { int device; };
 int g_device = 0;                          // the current device
 int g_allocations = 0, g_events = 0;       // made so far
 int g_buffer_device = -1;                  // current at the last pinned allocation
+size_t g_largest = 0;                      // pinned allocation, bytes
 
 #define EXPECT(cond)                                                       \
     do {                                                                   \
@@ -50,6 +51,7 @@ hipError_t hipHostMalloc(void **p, size_t bytes, unsigned)
 {
     g_allocations++;
     g_buffer_device = g_device;
+    g_largest = std::max(g_largest, bytes);
     *p = std::malloc(bytes);
     return hipSuccess;
 }
@@ -164,6 +166,22 @@ int no_allocation()
     return 0;
 }
 
+// The pinned buffers of a first download: none of the length whose allocation costs more than
+// the download of a few chunks saves.
+int first_buffers()
+{
+    for (int n : {1, 32768, 32769, 72000, 196608, 196609, 500000}) {
+        State s(n, 1, 0);
+        HostLink link;
+        link.create(s.R);
+        g_largest = 0;
+        check_download(s, link);
+        if (n <= 196608) EXPECT(g_largest <= 2u << 20);
+        link.destroy();
+    }
+    return 0;
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
@@ -172,6 +190,7 @@ int main(int argc, char **argv)
     try {
         if (what == "other_device") return other_device();
         if (what == "no_allocation") return no_allocation();
+        if (what == "first_buffers") return first_buffers();
     } catch (const std::exception &e) {
         std::fprintf(stderr, "%s: %s\n", what.c_str(), e.what());
         return 1;

@@ -5,6 +5,8 @@ the device of every stream, event and allocation.
 - other_device: a context's calls work, and give the right values, whatever device is current
   when they are made, as the copies on its stream did that they replace.
 - no_allocation: a context's first result allocates nothing (sm_vesicle_radius_noalloc).
+- first_buffers: the pinned buffers stay below the length (2 to 3 MiB) from which one takes
+  hundreds of microseconds to allocate; and downloads of one chunk, its edge and many.
 """
 import os
 import shutil
@@ -30,7 +32,7 @@ def harness(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("scenario", ["other_device", "no_allocation"])
+@pytest.mark.parametrize("scenario", ["other_device", "no_allocation", "first_buffers"])
 def test_transfer(harness, scenario):
     env = dict(os.environ, ASAN_OPTIONS="verify_asan_link_order=0:detect_leaks=0")
     r = subprocess.run([harness, scenario], env=env, capture_output=True, text=True, timeout=60)
