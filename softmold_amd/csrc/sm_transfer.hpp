@@ -13,7 +13,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
-#include <system_error>
+#include <exception>
 #include <thread>
 #include <vector>
 
@@ -118,9 +118,23 @@ public:
         };
         const int want = n < kThreadBeads ? 1 : std::max(1, std::min(kWorkers, (int)std::thread::hardware_concurrency() / 2));
         std::atomic<int> ready{0}, done{0};
+        std::atomic<int> size{0};   // parts, once every worker that could be started was
         std::atomic<bool> quit{false};
+        const auto work = [&](int i) {
+            while (size.load(std::memory_order_acquire) == 0)
+                if (quit.load()) return;
+                else std::this_thread::yield();
+            const int parts = size.load();
+            for (int c = 0; c < chunks; c++) {
+                while (ready.load(std::memory_order_acquire) <= c)
+                    if (quit.load()) return;
+                    else std::this_thread::yield();
+                unpack(c, i, parts);
+                done.fetch_add(1, std::memory_order_release);
+            }
+        };
         std::vector<std::thread> team;
-        struct Join {
+        struct Join {   // the last of what the workers use, so the first to go
             std::vector<std::thread> &t;
             std::atomic<bool> &quit;
             ~Join()
@@ -129,30 +143,15 @@ public:
                 for (auto &x : t) x.join();
             }
         };
-        int parts = 1;
         {
             Join join{team, quit};
             launch(0);
-            std::atomic<int> size{0};   // parts, once every worker that could be started was
-            auto work = [&](int i) {
-                while (size.load(std::memory_order_acquire) == 0)
-                    if (quit.load()) return;
-                    else std::this_thread::yield();
-                const int parts = size.load();
-                for (int c = 0; c < chunks; c++) {
-                    while (ready.load(std::memory_order_acquire) <= c)
-                        if (quit.load()) return;
-                        else std::this_thread::yield();
-                    unpack(c, i, parts);
-                    done.fetch_add(1, std::memory_order_release);
-                }
-            };
             try {
                 team.reserve(want);
                 for (int i = 1; i < want; i++) team.emplace_back(work, i);
-            } catch (const std::system_error &) {   // fewer threads then
+            } catch (const std::exception &) {   // no thread, or no memory for one: those there are
             }
-            parts = 1 + (int)team.size();
+            const int parts = 1 + (int)team.size();
             size.store(parts, std::memory_order_release);
             for (int c = 1; c < std::min(chunks, ch.buffers); c++) launch(c);
             for (int c = 0; c < chunks; c++) {

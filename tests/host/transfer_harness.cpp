@@ -16,6 +16,8 @@ int g_device = 0;                          // the current device
 int g_allocations = 0, g_events = 0;       // made so far
 int g_buffer_device = -1;                  // current at the last pinned allocation
 size_t g_largest = 0;                      // pinned allocation, bytes
+std::atomic<int> g_bad_wait{-1};           // the wait for an event that fails, counted down
+thread_local int g_bad_new = -1;           // this thread's allocation that fails, counted down
 
 #define EXPECT(cond)                                                       \
     do {                                                                   \
@@ -28,6 +30,15 @@ size_t g_largest = 0;                      // pinned allocation, bytes
 }  // namespace
 
 thread_local std::string smapi::g_err;
+
+void *operator new(size_t bytes)
+{
+    if (g_bad_new >= 0 && g_bad_new-- == 0) throw std::bad_alloc();
+    if (void *p = std::malloc(bytes ? bytes : 1)) return p;
+    throw std::bad_alloc();
+}
+void operator delete(void *p) noexcept { std::free(p); }
+void operator delete(void *p, size_t) noexcept { std::free(p); }
 
 extern "C" {
 hipError_t hipGetDevice(int *d) { *d = g_device; return hipSuccess; }
@@ -46,7 +57,7 @@ hipError_t hipEventRecord(hipEvent_t e, hipStream_t st)
     return reinterpret_cast<FakeEvent *>(e)->device == reinterpret_cast<FakeStream *>(st)->device ? hipSuccess
                                                                                                   : hipErrorInvalidHandle;
 }
-hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return g_bad_wait >= 0 && g_bad_wait-- == 0 ? hipErrorUnknown : hipSuccess; }
 hipError_t hipHostMalloc(void **p, size_t bytes, unsigned)
 {
     g_allocations++;
@@ -182,6 +193,37 @@ int first_buffers()
     return 0;
 }
 
+// Downloads whose workers cannot all be started, and downloads that fail under way.
+int troubled_team()
+{
+    State s(300000, 1, 0);
+    HostLink link;
+    link.create(s.R);
+    check_download(s, link);
+    std::vector<double> pos(3 * (size_t)s.n), box(3);
+    for (int k = 0; k < 8; k++) {   // the k-th allocation of the call: the team's room, then a worker each
+        std::fill(pos.begin(), pos.end(), 7.0);
+        g_bad_new = k;
+        EXPECT(link.fetch_beads(s.st(), s.n, s.src(), pos.data(), nullptr, nullptr, &s.glob, s.reps.data(), 1, box.data()) == 5);
+        g_bad_new = -1;
+        for (int i = 0; i < s.n; i++) EXPECT(pos[3 * (size_t)i + 2] == s.beads[i].z);
+    }
+    for (int k = 0; k < 5; k++)
+        for (int rep = 0; rep < 20; rep++) {
+            bool thrown = false;
+            g_bad_wait = k;
+            try {
+                link.fetch_beads(s.st(), s.n, s.src(), pos.data(), nullptr, nullptr, &s.glob, s.reps.data(), 1, box.data());
+            } catch (const smapi::ApiError &) {
+                thrown = true;
+            }
+            g_bad_wait = -1;
+            EXPECT(thrown);
+        }
+    link.destroy();
+    return 0;
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
@@ -191,6 +233,7 @@ int main(int argc, char **argv)
         if (what == "other_device") return other_device();
         if (what == "no_allocation") return no_allocation();
         if (what == "first_buffers") return first_buffers();
+        if (what == "troubled_team") return troubled_team();
     } catch (const std::exception &e) {
         std::fprintf(stderr, "%s: %s\n", what.c_str(), e.what());
         return 1;

@@ -7,6 +7,8 @@ the device of every stream, event and allocation.
 - no_allocation: a context's first result allocates nothing (sm_vesicle_radius_noalloc).
 - first_buffers: the pinned buffers stay below the length (2 to 3 MiB) from which one takes
   hundreds of microseconds to allocate; and downloads of one chunk, its edge and many.
+- troubled_team: a worker that cannot be started leaves a download to the others, and one that
+  fails under way ends its workers before what they use (under the address sanitizer).
 """
 import os
 import shutil
@@ -32,7 +34,7 @@ def harness(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("scenario", ["other_device", "no_allocation", "first_buffers"])
+@pytest.mark.parametrize("scenario", ["other_device", "no_allocation", "first_buffers", "troubled_team"])
 def test_transfer(harness, scenario):
     env = dict(os.environ, ASAN_OPTIONS="verify_asan_link_order=0:detect_leaks=0")
     r = subprocess.run([harness, scenario], env=env, capture_output=True, text=True, timeout=60)
