@@ -12,8 +12,10 @@
 
 #include <algorithm>
 #include <atomic>
+#include <condition_variable>
 #include <cstring>
 #include <exception>
+#include <mutex>
 #include <thread>
 #include <vector>
 
@@ -118,13 +120,20 @@ public:
         };
         const int want = n < kThreadBeads ? 1 : std::max(1, std::min(kWorkers, (int)std::thread::hardware_concurrency() / 2));
         std::atomic<int> ready{0}, done{0};
-        std::atomic<int> size{0};   // parts, once every worker that could be started was
+        // The workers sleep until the first chunk is there: the GPU may have any amount of queued
+        // work before it (seven of them polling took as many cores for a whole stretch of steps).
+        // After it, chunks come as fast as they are unpacked, and they poll.
+        std::mutex mu;
+        std::condition_variable wake;
+        int size = 0;   // parts, once the first chunk is there
         std::atomic<bool> quit{false};
         const auto work = [&](int i) {
-            while (size.load(std::memory_order_acquire) == 0)
-                if (quit.load()) return;
-                else std::this_thread::yield();
-            const int parts = size.load();
+            int parts;
+            {
+                std::unique_lock<std::mutex> lock(mu);
+                wake.wait(lock, [&] { return size != 0 || quit.load(); });
+                parts = size;
+            }
             for (int c = 0; c < chunks; c++) {
                 while (ready.load(std::memory_order_acquire) <= c)
                     if (quit.load()) return;
@@ -136,15 +145,21 @@ public:
         std::vector<std::thread> team;
         struct Join {   // the last of what the workers use, so the first to go
             std::vector<std::thread> &t;
+            std::mutex &mu;
+            std::condition_variable &wake;
             std::atomic<bool> &quit;
             ~Join()
             {
-                quit.store(true);
+                {
+                    std::lock_guard<std::mutex> lock(mu);
+                    quit.store(true);
+                }
+                wake.notify_all();
                 for (auto &x : t) x.join();
             }
         };
         {
-            Join join{team, quit};
+            Join join{team, mu, wake, quit};
             launch(0);
             try {
                 team.reserve(want);
@@ -152,10 +167,15 @@ public:
             } catch (const std::exception &) {   // no thread, or no memory for one: those there are
             }
             const int parts = 1 + (int)team.size();
-            size.store(parts, std::memory_order_release);
             for (int c = 1; c < std::min(chunks, ch.buffers); c++) launch(c);
+            wait(0);
+            {
+                std::lock_guard<std::mutex> lock(mu);
+                size = parts;
+            }
+            wake.notify_all();
             for (int c = 0; c < chunks; c++) {
-                wait(c);
+                if (c > 0) wait(c);
                 ready.store(c + 1, std::memory_order_release);
                 unpack(c, 0, parts);
                 while (done.load(std::memory_order_acquire) < (c + 1) * (parts - 1)) std::this_thread::yield();

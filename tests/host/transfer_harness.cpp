@@ -3,8 +3,10 @@
 // and an allocation.  Usage: transfer_harness SCENARIO; exit code 0 if it held.
 #include "sm_transfer.hpp"
 
+#include <chrono>
 #include <cstdio>
 #include <cstdlib>
+#include <ctime>
 #include <string>
 
 namespace {
@@ -17,6 +19,7 @@ int g_allocations = 0, g_events = 0;       // made so far
 int g_buffer_device = -1;                  // current at the last pinned allocation
 size_t g_largest = 0;                      // pinned allocation, bytes
 std::atomic<int> g_bad_wait{-1};           // the wait for an event that fails, counted down
+std::atomic<int> g_busy_ms{0};             // the GPU's queued work: the next wait lasts so long
 thread_local int g_bad_new = -1;           // this thread's allocation that fails, counted down
 
 #define EXPECT(cond)                                                       \
@@ -57,7 +60,11 @@ hipError_t hipEventRecord(hipEvent_t e, hipStream_t st)
     return reinterpret_cast<FakeEvent *>(e)->device == reinterpret_cast<FakeStream *>(st)->device ? hipSuccess
                                                                                                   : hipErrorInvalidHandle;
 }
-hipError_t hipEventSynchronize(hipEvent_t) { return g_bad_wait >= 0 && g_bad_wait-- == 0 ? hipErrorUnknown : hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t)
+{
+    std::this_thread::sleep_for(std::chrono::milliseconds(g_busy_ms.exchange(0)));
+    return g_bad_wait >= 0 && g_bad_wait-- == 0 ? hipErrorUnknown : hipSuccess;
+}
 hipError_t hipHostMalloc(void **p, size_t bytes, unsigned)
 {
     g_allocations++;
@@ -224,6 +231,25 @@ int troubled_team()
     return 0;
 }
 
+// A download behind 600 ms of the GPU's work: the host's threads sleep meanwhile.
+int behind_work()
+{
+    State s(300000, 1, 0);
+    HostLink link;
+    link.create(s.R);
+    check_download(s, link);
+    const std::clock_t idle = std::clock();
+    check_download(s, link);
+    const std::clock_t start = std::clock();
+    g_busy_ms = 600;
+    check_download(s, link);
+    const double plain = double(start - idle) / CLOCKS_PER_SEC, behind = double(std::clock() - start) / CLOCKS_PER_SEC;
+    std::fprintf(stderr, "CPU seconds: %.3f alone, %.3f behind the work\n", plain, behind);
+    EXPECT(behind < plain + 0.3);
+    link.destroy();
+    return 0;
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
@@ -234,6 +260,7 @@ int main(int argc, char **argv)
         if (what == "no_allocation") return no_allocation();
         if (what == "first_buffers") return first_buffers();
         if (what == "troubled_team") return troubled_team();
+        if (what == "behind_work") return behind_work();
     } catch (const std::exception &e) {
         std::fprintf(stderr, "%s: %s\n", what.c_str(), e.what());
         return 1;

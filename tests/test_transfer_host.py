@@ -9,6 +9,8 @@ the device of every stream, event and allocation.
   hundreds of microseconds to allocate; and downloads of one chunk, its edge and many.
 - troubled_team: a worker that cannot be started leaves a download to the others, and one that
   fails under way ends its workers before what they use (under the address sanitizer).
+- behind_work: no host thread is busy while a download waits for the GPU's queued work (the
+  processor time of the call; spinning, its workers used 600 ms each).
 """
 import os
 import shutil
@@ -34,7 +36,7 @@ def harness(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("scenario", ["other_device", "no_allocation", "first_buffers", "troubled_team"])
+@pytest.mark.parametrize("scenario", ["other_device", "no_allocation", "first_buffers", "troubled_team", "behind_work"])
 def test_transfer(harness, scenario):
     env = dict(os.environ, ASAN_OPTIONS="verify_asan_link_order=0:detect_leaks=0")
     r = subprocess.run([harness, scenario], env=env, capture_output=True, text=True, timeout=60)
