@@ -175,9 +175,11 @@ int sm_potential_delta(sm_ctx *ctx, const double *scale, double *du_pair, double
 /* ---- launch shapes ------------------------------------------------------------------ */
 /* Set a launch-shape knob of this build; no counterpart in the reference (its launches are
  * fixed, include/cuda/other.h:6-11).  Knobs: "pair_chunk" = sorted slots per wave64 in
- * the pair kernels (1..4096; by default the energy traversals have a length of their own); "pair_variant" = 0 one-phase force kernel with the
- * home cell's candidates culled per quarter cell (default), 1 two-phase (FP32 screen into
- * per-lane hit lists, then the FP64 test on the hits);
+ * the pair kernels (1..4096; by default the energy traversals have a length of their own,
+ * which sm_tune_get reads as "energy_chunk", and which setting or autotuning pair_chunk makes
+ * the same); "pair_variant" = 0 one-phase force kernel with the home cell's candidates culled
+ * per quarter cell (default), 1 two-phase (FP32 screen into per-lane hit lists, then the FP64
+ * test on the hits);
  * "graph" = 1 to replay sm_run's aligned 8-step blocks as one captured hipGraph;
  * "sort_mode" = 1 to re-sort the cell keys incrementally -- the beads whose cell changed
  * are sorted and merged into the previous order (the default from a million beads up) --

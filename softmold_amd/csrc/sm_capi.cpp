@@ -1659,6 +1659,7 @@ int sm_tune_get(sm_ctx *c, const char *knob, int32_t *value)
     return guarded([&] {
         if (!c || !knob || !value) invalid("null argument");
         if (std::strcmp(knob, "pair_chunk") == 0) *value = c->chunk;
+        else if (std::strcmp(knob, "energy_chunk") == 0) *value = c->echunk;
         else if (std::strcmp(knob, "pair_variant") == 0) *value = c->pair_variant;
         else if (std::strcmp(knob, "graph") == 0) *value = c->use_graph ? 1 : 0;
         else if (std::strcmp(knob, "sort_mode") == 0) *value = c->sort_mode;
@@ -1722,7 +1723,7 @@ int sm_autotune(sm_ctx *c, int32_t steps, double *best_ms_per_step)
             double best = 1e300;
             Cand bestc{c->chunk, c->pair_variant, c->use_graph ? 1 : 0, c->sort_mode};
             auto trial = [&](const Cand &k) {
-                c->chunk = k.chunk;
+                c->chunk = c->echunk = k.chunk;   // as sm_tune sets them
                 c->pair_variant = k.variant;
                 c->use_graph = k.graph != 0;
                 if (c->sort_mode != k.sort) {
@@ -1751,7 +1752,7 @@ int sm_autotune(sm_ctx *c, int32_t steps, double *best_ms_per_step)
             for (int m = 0; m <= 2; m++)   // the other sort modes
                 if (m != b0.sort && (m != 2 || c->win_ok)) trial({b0.chunk, b0.variant, 1, m});
             trial({bestc.chunk, bestc.variant, 0, bestc.sort});       // is the graph worth it here
-            c->chunk = bestc.chunk;
+            c->chunk = c->echunk = bestc.chunk;
             c->pair_variant = bestc.variant;
             c->use_graph = bestc.graph != 0;
             if (c->sort_mode != bestc.sort) {
