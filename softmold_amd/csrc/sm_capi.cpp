@@ -1937,17 +1937,21 @@ struct AdjointRun {
     State own;                        // the context's
     Bead *own_alt;
     bool own_fused;
-    std::vector<Bead *> x;            // x[t]: a segment's positions after its t-th step, before that step's box move
+    // x[t]: a segment's positions after its t-th step, before that step's box move.  An
+    // objective alone needs the step before only: two buffers in turns (at), and no segments.
+    std::vector<Bead *> x;
+    const bool keep;
+    Bead *at(int t) const { return x[keep ? t : t & 1]; }
     std::vector<State> checkpoint;    // states at steps k, 2k, ...; [0] at step 0
     DevRep *pre = nullptr, *post = nullptr;   // a segment's box moves: the replicas before and after each
     double *sums = nullptr;           // sums over the steps of U_pair, U_chain per replica
     double4 *X = nullptr, *V = nullptr, *A = nullptr, *A_next = nullptr, *F = nullptr, *HV = nullptr;
     double *g = nullptr, *gs = nullptr;
 
-    AdjointRun(sm_ctx *ctx, int steps, int want_k, bool grad) : c(ctx), n(ctx->n), nrep(ctx->nrep), S(steps)
+    AdjointRun(sm_ctx *ctx, int steps, int want_k, bool grad) : c(ctx), n(ctx->n), nrep(ctx->nrep), S(steps), keep(grad)
     {
         const long long fit = (long long)(kKeepBytes / (sizeof(Bead) * (size_t)n));
-        k = (int)std::min<long long>(S, std::max<long long>(want_k, fit));
+        k = keep ? (int)std::min<long long>(S, std::max<long long>(want_k, fit)) : S;
         nseg = (S + k - 1) / k;
         own = State{c->beads, c->vel, c->acc, c->reps, c->glob};
         own_alt = c->beads_alt;
@@ -1962,7 +1966,7 @@ struct AdjointRun {
                 p = reinterpret_cast<T *>(base + at);
                 at += (sizeof(T) * count + 255) / 256 * 256;
             };
-            x.resize(k + 2);
+            x.resize(keep ? k + 2 : 2);
             for (Bead *&b : x) take(b, n);
             auto state = [&](State &s, bool beads) {
                 if (beads) take(s.beads, n);
@@ -1972,12 +1976,12 @@ struct AdjointRun {
                 take(s.glob, 1);
             };
             state(cur, false);
-            checkpoint.resize(grad ? nseg - 1 : 0);
+            checkpoint.resize(nseg - 1);
             for (State &s : checkpoint) state(s, true);
-            take(pre, (size_t)(k / 8 + 1) * nrep);
-            take(post, (size_t)(k / 8 + 1) * nrep);
             take(sums, 2 * (size_t)nrep);
-            if (grad) {
+            if (keep) {
+                take(pre, (size_t)(k / 8 + 1) * nrep);
+                take(post, (size_t)(k / 8 + 1) * nrep);
                 for (double4 **p : {&X, &V, &A, &A_next, &F, &HV}) take(*p, n);
                 take(g, kNTheta * (size_t)n);
                 take(gs, kNTheta * (size_t)nrep);
@@ -2023,8 +2027,8 @@ struct AdjointRun {
     void steps(int s0, int s1, bool objective)
     {
         const size_t rn = nrep;
-        copy(x[1], x[0], n);
-        c->beads = x[1];
+        copy(at(1), at(0), n);
+        c->beads = at(1);
         c->step_first(s0 + 1);
         for (int s = s0 + 1; s <= s1; s++) {
             const int t = s - s0;
@@ -2033,17 +2037,17 @@ struct AdjointRun {
             c->pair_force_u();   // in the recomputed segments too, whose steps must be the same
             if (objective) c->add_energies(sums);
             if (!mc && s < s1) {
-                c->beads_alt = x[t + 1];
-                c->kick_first(s);   // x[t] stays as it is
+                c->beads_alt = at(t + 1);
+                c->kick_first(s);   // at(t) stays as it is
                 continue;
             }
             c->bonded(KICK_STEP, nullptr);
             if (mc) {
-                copy(pre + move(s, s0) * rn, c->reps, rn);
-                copy(x[t + 1], x[t], n);
-                c->beads = x[t + 1];
+                if (keep) copy(pre + move(s, s0) * rn, c->reps, rn);
+                copy(at(t + 1), at(t), n);
+                c->beads = at(t + 1);
                 c->mc_move();
-                copy(post + move(s, s0) * rn, c->reps, rn);
+                if (keep) copy(post + move(s, s0) * rn, c->reps, rn);
                 if (s < s1) c->step_first(s + 1);
             }
         }
@@ -2153,7 +2157,7 @@ int sm_adjoint(sm_ctx *c, int32_t type_a, int32_t type_b, int32_t nsteps, int32_
         c->pair_force();
         c->bonded(KICK_INIT, nullptr);
         for (int seg = 0; seg < nseg; seg++) {
-            if (seg + 1 < nseg && grad) run.save(run.checkpoint[seg]);
+            if (seg + 1 < nseg) run.save(run.checkpoint[seg]);
             run.steps(seg * k, std::min(S, seg * k + k), true);
             if (seg + 1 < nseg) HIPCHK(hipMemcpyAsync(run.x[0], c->beads, sizeof(Bead) * n, hipMemcpyDeviceToDevice, st));
             if (seg + 1 < nseg) c->beads = run.x[0];
