@@ -37,7 +37,11 @@ T *dalloc(size_t count)
 {
     void *p = nullptr;
     if (count == 0) count = 1;
-    HIPCHK(hipMalloc(&p, count * sizeof(T)));
+    const hipError_t e = hipMalloc(&p, count * sizeof(T));
+    if (e != hipSuccess) {
+        (void)hipGetLastError();   // reported here, not by the next launch's check
+        HIPCHK(e);
+    }
     return static_cast<T *>(p);
 }
 
@@ -179,32 +183,38 @@ struct sm_ctx {
     uint32_t *k2 = nullptr, *v2 = nullptr, *wdesc = nullptr, *counts[2] = {}, *counted[2] = {}, *bucket = nullptr;
     size_t count_cells = 0;   // cells that counts and bucket hold
     bool counters_ready = false;   // the last build was a counting build with these buffers
-    bool win_now() const { return sort_mode == 2 && win_ok && sort_bits >= 17 && sort_bits <= 24; }
+    bool win_now() const { return sort_mode == 2 && win_ok && bucket && sort_bits >= 17 && sort_bits <= 24; }
     bool dense_now() const
     {
         return !win_now() && sort_mode != 1 && bucket && capacity <= kWinCells && sortw_fits(n);
     }
     bool count_now() const { return dense_now() || win_now(); }
-    // room to count in windows, or in the whole table while that is small
+    // room to count in windows, or in the whole table while that is small; without the memory for
+    // it the builds sort
     void alloc_counts()
     {
         if (!sortw_fits(n)) return;
         size_t cells = win_ok ? count_limit(n) : 0;
         if (capacity <= kWinCells) cells = std::max(cells, ((size_t)capacity + kCoarseCells - 1) / kCoarseCells * kCoarseCells);
         if (cells <= count_cells) return;
-        dfree(bucket);
-        bucket = dalloc<uint32_t>(cells * kBucket);
-        if (!k2) k2 = dalloc<uint32_t>(n);
-        if (!v2) v2 = dalloc<uint32_t>(n);
-        for (int p = 0; p < 2; p++) {
-            dfree(counts[p]);
-            counts[p] = dalloc<uint32_t>(cells);
-            if (counted[p]) continue;
-            counted[p] = dalloc<uint32_t>(n);
-            HIPCHK(hipMemsetAsync(counted[p], 0, sizeof(uint32_t) * n, st));
-        }
-        count_cells = cells;
         counters_ready = false;
+        count_cells = 0;
+        dfree(bucket);
+        for (uint32_t *&p : counts) dfree(p);
+        try {
+            if (!k2) k2 = dalloc<uint32_t>(n);
+            if (!v2) v2 = dalloc<uint32_t>(n);
+            for (int p = 0; p < 2; p++) {
+                counts[p] = dalloc<uint32_t>(cells);
+                if (counted[p]) continue;
+                counted[p] = dalloc<uint32_t>(n);
+                HIPCHK(hipMemsetAsync(counted[p], 0, sizeof(uint32_t) * n, st));
+            }
+            bucket = dalloc<uint32_t>(cells * kBucket);
+            count_cells = cells;
+        } catch (const ApiError &) {
+            for (uint32_t *&p : counts) dfree(p);
+        }
     }
     int *cstart = nullptr, *cend = nullptr;
     long long capacity = 0;   // cells in the dense table, all replicas
@@ -475,7 +485,8 @@ struct sm_ctx {
 
     // Dense cell table sized for every box the next `moves` MC moves can reach, in every
     // replica; a replica that outgrows its reservation moves every cell base (keys are
-    // recomputed each step, so only the table is reallocated).
+    // recomputed each step, so only the table is reallocated).  A table that cannot be had
+    // leaves the context as it was.
     void ensure_capacity(long long moves)
     {
         auto grows = [&](int r) {
@@ -490,25 +501,35 @@ struct sm_ctx {
         for (int r = 0; r < nrep && !relayout; r++) relayout = grows(r);
         if (!relayout) return;
         std::vector<DevRep> hr = read_reps();
+        std::vector<RepHost> laid = rh;
         long long base = 0;
         for (int r = 0; r < nrep; r++) {
             if (grows(r)) {
                 const long long need = cells_needed(r, moves);
-                rh[r].capacity = need + need / 8;
+                laid[r].capacity = need + need / 8;
             }
-            rh[r].cellbase = base;
-            if (rh[r].capacity > 0xFFFFFFFFll || (base += rh[r].capacity) > 0xFFFFFFFFll)
+            laid[r].cellbase = base;
+            if (laid[r].capacity > 0xFFFFFFFFll || (base += laid[r].capacity) > 0xFFFFFFFFll)
                 unsupported("cell tables of all replicas exceed 2^32 cells");
-            hr[r].cellbase = rh[r].cellbase;
-            hr[r].capacity = rh[r].capacity;
+            hr[r].cellbase = laid[r].cellbase;
+            hr[r].capacity = laid[r].capacity;
+        }
+        int *start = dalloc<int>((size_t)base), *end = nullptr;
+        try {
+            end = dalloc<int>((size_t)base);
+            HIPCHK(hipMemsetAsync(start, 0xFF, sizeof(int) * (size_t)base, st));
+            HIPCHK(hipMemsetAsync(end, 0xFF, sizeof(int) * (size_t)base, st));
+        } catch (...) {
+            dfree(start);
+            dfree(end);
+            throw;
         }
         drop_graph();
         dfree(cstart);
         dfree(cend);
-        cstart = dalloc<int>((size_t)base);
-        cend = dalloc<int>((size_t)base);
-        HIPCHK(hipMemsetAsync(cstart, 0xFF, sizeof(int) * (size_t)base, st));
-        HIPCHK(hipMemsetAsync(cend, 0xFF, sizeof(int) * (size_t)base, st));
+        cstart = start;
+        cend = end;
+        rh = std::move(laid);
         capacity = base;
         write_reps(hr);
         int bits = 1;
@@ -1300,8 +1321,23 @@ int sm_upload_state(sm_ctx *c, const double *pos, const double *vel, const doubl
                         if (!(p >= 0 && p <= L[3 * (size_t)r + d]))
                             invalid("particle " + std::to_string(i) + " position is out of bounds");
                     }
-            c->link.send_positions(c->st, n, pos, c->beads);
         }
+        if (box) {   // the cells that it needs, before anything changes
+            struct Tried {
+                sm_ctx *c;
+                std::vector<double> was;
+                long long since;
+                ~Tried()
+                {
+                    c->boxL.swap(was);
+                    c->moves_since = since;
+                }
+            } tried{c, c->boxL, c->moves_since};
+            c->boxL = L;
+            c->moves_since = 0;
+            c->ensure_capacity(0);
+        }
+        if (pos) c->link.send_positions(c->st, n, pos, c->beads);
         auto up3 = [&](float4 *dst, const double *src) {
             std::vector<float4> h(n);
             for (int i = 0; i < n; i++)
@@ -1322,7 +1358,6 @@ int sm_upload_state(sm_ctx *c, const double *pos, const double *vel, const doubl
             c->write_reps(hr);
             c->boxL = L;
             c->moves_since = 0;
-            c->ensure_capacity(0);
         }
     });
 }
