@@ -273,6 +273,7 @@ struct sm_ctx {
     long long pairs_cap = 0;
     unsigned long long *dnp = nullptr;
     int chunk = 8, echunk = 8;   // sorted slots per wave: the force and the counts; the FP64 energy traversals
+    bool chunk_set = false;      // by sm_tune or the autotuner
     int pair_variant = 0;
     // box-move steps: the pair dU in the same traversal as the step's pair force (1) or in
     // a gather of its own after the kick (0, as the adjoint uses)
@@ -536,6 +537,31 @@ struct sm_ctx {
         while ((1ll << bits) < base) bits++;
         sort_bits = bits;
         alloc_counts();
+    }
+
+    // The launch shapes that follow from the box: at creation and when one is uploaded (box moves
+    // change it by percents).  Chunks that were set or tuned stay.
+    void launch_rules()
+    {
+        const int flat = nrep == 1 && boxL[2] / P.cutoff < 64.0 ? 1 : 0;
+        if (flat != P.flat) drop_graph();   // captured launches hold it, and the chunks that it sets
+        P.flat = flat;
+        if (chunk_set) return;
+        // sorted slots per wave in the pair kernels: short chunks keep small systems filling the
+        // chip and even out flat ones, longer ones cut the overhead per wave (every chunk gives
+        // the same forces).  Whole steps in us at 2, 4, 8, 16 slots: 1.5k vesicle 27.1, 28 at 4;
+        // 18k bilayer 48.0, 46.7; 90k vesicle 63.7, 62.3, 61.7; 120k 74.5, 72.5, 71.7; 300k
+        // bilayer 148 at 4, 158, 178; 990k bilayer 450 at 4, 451, 468; 3M bilayer 1216 at 4,
+        // 1188, 1191; 1.35M vesicle 530 at 8, 522; 3M vesicle 1123 at 8, 1098; 1.5M beads in 64
+        // bilayers 648 at 8, 658.
+        const int many = P.flat ? 1000000 : 100000;
+        chunk = n < 10000 ? 2 : (n < many ? 4 : (n < 2000000 || P.flat ? 8 : 16));
+        // The energy traversals do more per candidate.  Force with dU and U in us: 1.5k vesicle
+        // 24 and 15.0 at 2, 31 and 19.4 at 8; 12k bilayer 57 and 29.4 at 2, 46 and 25.4 at 8; 37k
+        // vesicle 54 and 29.2 at 2, 51 and 27.1 at 4, 49 and 29.6 at 8; 90k bilayer 84 and 44.2
+        // at 4, 82 and 43.0 at 8; 1.2M vesicle 687 and 325 at 8, 677 and 317 at 16; 1.2M bilayer
+        // 653 and 311 at 8, 667 and 317 at 16.
+        echunk = n < 10000 ? 2 : (P.flat ? 8 : (n < 50000 ? 4 : (n < 1000000 ? 8 : 16)));
     }
 
     // keys (optionally after Verlet::first) with the next sort's digit histograms, sort,
@@ -965,7 +991,6 @@ sm_ctx *create(const sm_system *s, int nrep)
         c->P.nT = s[0].n_types;
         c->P.cutoff = s[0].cutoff;
         c->P.dt = s[0].dt;
-        c->P.flat = nrep == 1 && s[0].box[2] / s[0].cutoff < 64.0 ? 1 : 0;
         HIPCHK(hipStreamCreate(&c->st));
         // the device's fixed scratch for the entry points that allocate nothing, looked up
         // once per device while it is current
@@ -1198,21 +1223,7 @@ sm_ctx *create(const sm_system *s, int nrep)
             HIPCHK(hipMemcpyAsync(c->chainList, list.data(), sizeof(int2) * list.size(), hipMemcpyHostToDevice, st));
             HIPCHK(hipMemcpyAsync(c->cconstD, ccD.data(), sizeof(double4) * ccD.size(), hipMemcpyHostToDevice, st));
         }
-        // sorted slots per wave in the pair kernels: short chunks keep small systems filling the
-        // chip and even out flat ones, longer ones cut the overhead per wave (every chunk gives
-        // the same forces).  Whole steps in us at 2, 4, 8, 16 slots: 1.5k vesicle 27.1, 28 at 4;
-        // 18k bilayer 48.0, 46.7; 90k vesicle 63.7, 62.3, 61.7; 120k 74.5, 72.5, 71.7; 300k
-        // bilayer 148 at 4, 158, 178; 990k bilayer 450 at 4, 451, 468; 3M bilayer 1216 at 4,
-        // 1188, 1191; 1.35M vesicle 530 at 8, 522; 3M vesicle 1123 at 8, 1098; 1.5M beads in 64
-        // bilayers 648 at 8, 658.
-        const int many = c->P.flat ? 1000000 : 100000;
-        c->chunk = n < 10000 ? 2 : (n < many ? 4 : (n < 2000000 || c->P.flat ? 8 : 16));
-        // The energy traversals do more per candidate.  Force with dU and U in us: 1.5k vesicle
-        // 24 and 15.0 at 2, 31 and 19.4 at 8; 12k bilayer 57 and 29.4 at 2, 46 and 25.4 at 8; 37k
-        // vesicle 54 and 29.2 at 2, 51 and 27.1 at 4, 49 and 29.6 at 8; 90k bilayer 84 and 44.2
-        // at 4, 82 and 43.0 at 8; 1.2M vesicle 687 and 325 at 8, 677 and 317 at 16; 1.2M bilayer
-        // 653 and 311 at 8, 667 and 317 at 16.
-        c->echunk = n < 10000 ? 2 : (c->P.flat ? 8 : (n < 50000 ? 4 : (n < 1000000 ? 8 : 16)));
+        c->launch_rules();
         c->ensure_capacity(0);
         HIPCHK(hipStreamSynchronize(st));
     } catch (...) {
@@ -1358,6 +1369,7 @@ int sm_upload_state(sm_ctx *c, const double *pos, const double *vel, const doubl
             c->write_reps(hr);
             c->boxL = L;
             c->moves_since = 0;
+            c->launch_rules();
         }
     });
 }
@@ -1668,6 +1680,7 @@ int sm_tune(sm_ctx *c, const char *knob, int32_t value)
         if (std::strcmp(knob, "pair_chunk") == 0) {
             if (value < 1 || value > 4096) invalid("pair_chunk must be in [1, 4096]");
             c->chunk = c->echunk = value;
+            c->chunk_set = true;
         } else if (std::strcmp(knob, "pair_variant") == 0) {
             if (value < 0 || value > 1) invalid("pair_variant must be 0 or 1");
             c->pair_variant = value;
@@ -1788,6 +1801,7 @@ int sm_autotune(sm_ctx *c, int32_t steps, double *best_ms_per_step)
                 if (m != b0.sort && (m != 2 || c->win_ok)) trial({b0.chunk, b0.variant, 1, m});
             trial({bestc.chunk, bestc.variant, 0, bestc.sort});       // is the graph worth it here
             c->chunk = c->echunk = bestc.chunk;
+            c->chunk_set = true;
             c->pair_variant = bestc.variant;
             c->use_graph = bestc.graph != 0;
             if (c->sort_mode != bestc.sort) {

@@ -215,12 +215,39 @@ int growth_fails()
     return 0;
 }
 
+// The launch shapes of a context whose box was uploaded are those of one created with it; a
+// chunk that was set stays.
+int box_and_shapes()
+{
+    const auto knob = [](sm_ctx *c, const char *k) {
+        int32_t v = -1;
+        EXPECT(sm_tune_get(c, k, &v) == SM_OK);
+        return v;
+    };
+    for (const double from : {24.0, 200.0}) {
+        const double to = 224.0 - from;
+        System a(20000, from), b(20000, to);
+        sm_ctx *c = nullptr, *d = nullptr;
+        EXPECT(sm_create(&a.s, &c) == SM_OK && sm_create(&b.s, &d) == SM_OK);
+        EXPECT(knob(c, "energy_chunk") != knob(d, "energy_chunk"));
+        const double L[3] = {to, to, to};
+        EXPECT(sm_upload_state(c, nullptr, nullptr, nullptr, L) == SM_OK);
+        for (const char *k : {"pair_chunk", "energy_chunk"}) EXPECT(knob(c, k) == knob(d, k));
+        EXPECT(sm_tune(c, "pair_chunk", 32) == SM_OK);
+        const double back[3] = {from, from, from};
+        EXPECT(sm_upload_state(c, nullptr, nullptr, nullptr, back) == SM_OK && knob(c, "pair_chunk") == 32);
+        EXPECT(sm_destroy(c) == SM_OK && sm_destroy(d) == SM_OK);
+    }
+    return 0;
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
 {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "growth_fails") return growth_fails();
+    if (what == "box_and_shapes") return box_and_shapes();
     std::fprintf(stderr, "unknown scenario\n");
     return 2;
 }

@@ -4,6 +4,7 @@ sanitizer.
 
 - growth_fails: an upload of a larger box whose allocations fail one after another leaves a
   context that reports an error or works, with every buffer that a kernel would use in place.
+- box_and_shapes: an uploaded box sets the launch shapes that follow from the box.
 """
 import os
 import shutil
@@ -29,7 +30,7 @@ def harness(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("scenario", ["growth_fails"])
+@pytest.mark.parametrize("scenario", ["growth_fails", "box_and_shapes"])
 def test_context(harness, scenario):
     env = dict(os.environ, ASAN_OPTIONS="verify_asan_link_order=0:detect_leaks=0")
     r = subprocess.run([harness, scenario], env=env, capture_output=True, text=True, timeout=60)
