@@ -327,10 +327,16 @@ struct sm_ctx {
         launch_fill_u32(st, win_scratch(gh, n), kWinKeyWords, 0u);
         if (counts[0]) launch_fill_u32(st, counts[sort_parity], count_cells, 0u);
     }
+    // keys that no build has taken, made for another sort mode, table or state: gone
+    void forget_keys()
+    {
+        if (hist_pending) restart_hist(hist[sort_parity]);
+        hist_pending = false;
+    }
     // before a key kernel: its scratch holds nothing yet
     void begin_keys()
     {
-        if (hist_pending) restart_hist(hist[sort_parity]);   // keys computed twice before a sort: start over
+        forget_keys();   // keys computed twice before a sort: start over
         hist_pending = true;
         // a counting build clears the counters of the one right before it only
         if (count_now() && !counters_ready)
@@ -526,6 +532,7 @@ struct sm_ctx {
             throw;
         }
         drop_graph();
+        forget_keys();
         dfree(cstart);
         dfree(cend);
         cstart = start;
@@ -584,6 +591,9 @@ struct sm_ctx {
     }
     void sort_and_reorder()
     {
+        // a step's rest without its first half, or with something in between that the keys do not
+        // fit: the keys of the positions there are
+        if (!hist_pending) first_and_keys(0, kStepKeep);
         const int p = sort_parity;
         const bool count = count_now();
         win_last = count && win_now();
@@ -793,12 +803,6 @@ struct sm_ctx {
         if (measure) measure_device();
         if (mc) mc_finish();
     }
-    void eager_step(long long step)
-    {
-        step_first(step);
-        step_finish(false, mc_step(step));
-    }
-
     // Steps s .. s+7 with s % 8 == 1 as one graph: the step counter advances on the
     // device, so the same graph serves every such block; the MC move (if any replica
     // has one) falls on the block's last step.  The kernels are run()'s: seven fused kicks, and
@@ -813,10 +817,7 @@ struct sm_ctx {
             eager(s, s + 8);
             return;
         }
-        if (hist_pending) {   // keys computed but not sorted: the graph's are the first
-            restart_hist(hist[sort_parity]);
-            hist_pending = false;
-        }
+        forget_keys();   // the graph's are the first
         const int p = sort_parity, q = 2 * p + (beads != beads_home ? 1 : 0);
         if (!gexec[q]) {
             HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
@@ -1348,6 +1349,7 @@ int sm_upload_state(sm_ctx *c, const double *pos, const double *vel, const doubl
             c->moves_since = 0;
             c->ensure_capacity(0);
         }
+        if (pos || box) c->forget_keys();
         if (pos) c->link.send_positions(c->st, n, pos, c->beads);
         auto up3 = [&](float4 *dst, const double *src) {
             std::vector<float4> h(n);
@@ -1690,6 +1692,7 @@ int sm_tune(sm_ctx *c, const char *knob, int32_t value)
         } else if (std::strcmp(knob, "sort_mode") == 0) {
             if (value < 0 || value > 2) invalid("sort_mode must be 0, 1 or 2");
             if (value == 2 && !c->win_ok) invalid("sort_mode 2 needs a single replica of at most 524288 beads");
+            c->forget_keys();
             c->sort_mode = value;
             c->order_valid = false;
         } else if (std::strcmp(knob, "mc_fused") == 0) {

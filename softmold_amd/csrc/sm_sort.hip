@@ -687,7 +687,8 @@ __device__ void build_slots(BLds &L, int n, const BuildArgs &a, const WinDesc &w
     __syncthreads();
     for (int q = 0; q < wave; q++) head = max(head, (int)L.scan[q]);
     if (s >= n) return;
-    const uint32_t wk = min(L.cell[head] - 1u, a.wb.limit - 1u);
+    // in bounds, here and below, also for counts that are not this build's
+    const uint32_t wk = min(L.cell[head] - 1u, (dense ? a.wb.cells : w.wx * w.wy * w.wz) - 1u);
     const uint32_t start = L.start[head], count = min(L.count[head], (uint32_t)kBucket);
     const uint32_t *row = a.wb.bucket + (size_t)wk * kBucket;
     const uint32_t i = min(row[min((uint32_t)s - start, (uint32_t)kBucket - 1u)], (uint32_t)n - 1u);
@@ -699,7 +700,7 @@ __device__ void build_slots(BLds &L, int n, const BuildArgs &a, const WinDesc &w
         pos += (e.x < i ? 1u : 0u) + (q + 1 < count && e.y < i ? 1u : 0u) + (q + 2 < count && e.z < i ? 1u : 0u) +
                (q + 3 < count && e.w < i ? 1u : 0u);
     }
-    pos = min(pos, (uint32_t)n - 1u);   // in bounds also for counts that are not this build's
+    pos = min(pos, (uint32_t)n - 1u);
     uint32_t full = wk;
     if (!dense) {
         const uint32_t nx = (uint32_t)a.reps[0].nc[0], ny = (uint32_t)a.reps[0].nc[1];
@@ -712,7 +713,7 @@ __device__ void build_slots(BLds &L, int n, const BuildArgs &a, const WinDesc &w
     a.cells_now[s] = wk;
     if (pos == start) {
         a.cstart[full] = (int)start;
-        a.cend[full] = (int)(start + count);
+        a.cend[full] = (int)min(start + count, (uint32_t)n);
     }
 }
 

@@ -20,6 +20,15 @@ int g_bad_malloc = -1;      // the device allocation that fails, counted down
 bool g_failed = false;      // one did
 hipError_t g_last = hipSuccess;
 size_t g_cells = 0;         // cells of the table that the replicas were given
+// The keys that the last key kernel left for a build, as far as a build must agree with it.
+struct Keys {
+    bool there;
+    const void *counts, *desc;
+    unsigned cells;
+    const void *moved;
+    size_t table;
+};
+Keys g_keys{};
 
 #define EXPECT(cond)                                                       \
     do {                                                                   \
@@ -92,6 +101,13 @@ WinBook win_book(uint32_t *s, int n, const uint32_t *desc, uint32_t *counts, uin
 }
 hipError_t noalloc_scratch_init(int) { return hipSuccess; }
 
+static void made_keys(const WinBook &wb, const MoveBook &mb) { g_keys = Keys{true, wb.counts, wb.desc, wb.cells, mb.cnt_b, g_cells}; }
+static void take_keys(const WinBook &wb, bool moved)
+{
+    EXPECT(g_keys.there && g_keys.counts == wb.counts && g_keys.desc == wb.desc && g_keys.cells == wb.cells);
+    EXPECT((g_keys.moved != nullptr) == moved && g_keys.table == g_cells);
+    g_keys.there = false;
+}
 static void touch_book(const WinBook &wb)
 {
     if (!wb.desc && wb.cells == 0) return;   // no counting build
@@ -104,7 +120,7 @@ static void touch_book(const WinBook &wb)
 void launch_fill_u32(hipStream_t, uint32_t *p, size_t count, uint32_t v) { std::fill(p, p + count, v); }
 void launch_set_step(hipStream_t, DevGlobal *g, long long step) { g->step = g->base = step; }
 void launch_first(hipStream_t, const Params &P, const Bead *beads, Bead *out, float4 *, const float4 *, const DevRep *reps,
-                  DevGlobal *, uint32_t *key, uint32_t *idx, int, long long, uint32_t *, int, const MoveBook &, const WinBook &wb)
+                  DevGlobal *, uint32_t *key, uint32_t *idx, int, long long, uint32_t *, int, const MoveBook &mb, const WinBook &wb)
 {
     touch(beads, P.n);
     touch(out, P.n);
@@ -115,24 +131,29 @@ void launch_first(hipStream_t, const Params &P, const Bead *beads, Bead *out, fl
     for (int r = 0; r < P.nrep; r++) g_cells = std::max(g_cells, (size_t)(reps[r].cellbase + reps[r].capacity));
     for (int r = 0; r < P.nrep; r++)
         EXPECT((long long)reps[r].nc[0] * reps[r].nc[1] * reps[r].nc[2] <= reps[r].capacity);
+    made_keys(wb, mb);
 }
 void launch_kick_first(hipStream_t, const Params &P, const Bead *beads, Bead *out, const int2 *, const double4 *, const GenTables &,
                        const float4 *, float4 *, const DevRep *, DevGlobal *, long long, bool, uint32_t *key, uint32_t *,
-                       uint32_t *, int, const MoveBook &, const WinBook &wb)
+                       uint32_t *, int, const MoveBook &mb, const WinBook &wb)
 {
     touch(beads, P.n);
     touch(out, P.n);
     touch(key, P.n);
     touch_book(wb);
+    made_keys(wb, mb);
 }
 int radix_sort(hipStream_t, SortBuffers &b, int, int)
 {
     touch(b.k1, b.n);
+    take_keys(WinBook{}, false);
     return 0;
 }
+void sort_moved(hipStream_t, SortBuffers &, const MoveSort &, int, int) { take_keys(WinBook{}, true); }
 void launch_build(hipStream_t, int n, const BuildArgs &a)
 {
     touch_book(a.wb);
+    take_keys(a.wb, false);
     for (const uint32_t *p : {a.k2, a.v0, a.v2, (uint32_t *)a.cells_old, a.cells_now}) touch(p, n);
     touch(a.counts_old, a.wb.limit);
     touch(a.cstart, g_cells);
@@ -241,6 +262,31 @@ int box_and_shapes()
     return 0;
 }
 
+// The rest of a step without its first half right before it: another mode, another table or other
+// positions in between, or no first half at all.  Every build has the keys that it expects.
+int step_phases()
+{
+    for (const double box : {24.0, 90.0})
+        for (int from = 0; from < 3; from++) {
+            System a(200, box);
+            sm_ctx *c = nullptr;
+            EXPECT(sm_create(&a.s, &c) == SM_OK);
+            EXPECT(sm_tune(c, "sort_mode", from) == SM_OK && sm_init_forces(c) == SM_OK);
+            for (int to = 0; to < 3; to++) {
+                EXPECT(sm_step_first(c, 1) == SM_OK && sm_tune(c, "sort_mode", to) == SM_OK);
+                EXPECT(sm_step_finish(c, 1, nullptr) == SM_OK);
+                EXPECT(sm_step_finish(c, 1, nullptr) == SM_OK);
+                EXPECT(sm_step_first(c, 2) == SM_OK && sm_step_first(c, 2) == SM_OK && sm_step_finish(c, 2, nullptr) == SM_OK);
+            }
+            const double L[3] = {box * 1.5, box * 1.5, box * 1.5};
+            EXPECT(sm_tune(c, "sort_mode", from) == SM_OK && sm_step_first(c, 3) == SM_OK);
+            EXPECT(sm_upload_state(c, nullptr, nullptr, nullptr, L) == SM_OK && sm_step_finish(c, 3, nullptr) == SM_OK);
+            EXPECT(sm_run(c, 4, 9) == SM_OK && sm_step_finish(c, 12, nullptr) == SM_OK);
+            EXPECT(sm_destroy(c) == SM_OK);
+        }
+    return 0;
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
@@ -248,6 +294,7 @@ int main(int argc, char **argv)
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "growth_fails") return growth_fails();
     if (what == "box_and_shapes") return box_and_shapes();
+    if (what == "step_phases") return step_phases();
     std::fprintf(stderr, "unknown scenario\n");
     return 2;
 }

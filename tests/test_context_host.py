@@ -5,6 +5,8 @@ sanitizer.
 - growth_fails: an upload of a larger box whose allocations fail one after another leaves a
   context that reports an error or works, with every buffer that a kernel would use in place.
 - box_and_shapes: an uploaded box sets the launch shapes that follow from the box.
+- step_phases: whatever comes between the two halves of a step (another sort mode, another
+  table, or no first half at all), a build is launched on keys that were made for it.
 """
 import os
 import shutil
@@ -30,7 +32,7 @@ def harness(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("scenario", ["growth_fails", "box_and_shapes"])
+@pytest.mark.parametrize("scenario", ["growth_fails", "box_and_shapes", "step_phases"])
 def test_context(harness, scenario):
     env = dict(os.environ, ASAN_OPTIONS="verify_asan_link_order=0:detect_leaks=0")
     r = subprocess.run([harness, scenario], env=env, capture_output=True, text=True, timeout=60)
