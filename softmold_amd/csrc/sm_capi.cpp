@@ -183,10 +183,45 @@ struct sm_ctx {
     uint32_t *k2 = nullptr, *v2 = nullptr, *wdesc = nullptr, *counts[2] = {}, *counted[2] = {}, *bucket = nullptr;
     size_t count_cells = 0;   // cells that counts and bucket hold
     bool counters_ready = false;   // the last build was a counting build with these buffers
-    bool win_now() const { return sort_mode == 2 && win_ok && bucket && sort_bits >= 17 && sort_bits <= 24; }
+    // Builds that keep falling back -- a cell of more beads than a bucket that stays, a vesicle
+    // whose window never fits -- count for nothing and then sort in one launch what the radix sort
+    // orders faster: per step 165 against 121 us at 192k beads in 16 bilayers, 334 against 224 for
+    // a vesicle of 480k.  The device's count of fallbacks comes with every result; where more than
+    // half of the builds since the last result fell back, the context stops counting, until its
+    // sort mode is set or a box uploaded.  counts_known: a result has told about this context's
+    // builds; a first long run asks for one after 8 steps (run()).
+    bool count_off = false, counts_known = false;
+    uint32_t fallbacks_seen = 0;
+    long long counted_builds = 0;   // launched since
+    void learn()
+    {
+        constexpr int kEnough = 4;   // the first build of a window always falls back
+        if (counted_builds < kEnough) return;
+        const uint32_t now = link.fallbacks();
+        counts_known = true;
+        if (2ll * (uint32_t)(now - fallbacks_seen) > counted_builds && !count_off) {
+            drop_graph();
+            forget_keys();
+            count_off = true;
+        }
+        fallbacks_seen = now;
+        counted_builds = 0;
+    }
+    void count_again()
+    {
+        if (count_off) {
+            drop_graph();
+            forget_keys();
+        }
+        count_off = counts_known = false;
+    }
+    bool win_now() const
+    {
+        return sort_mode == 2 && win_ok && bucket && !count_off && sort_bits >= 17 && sort_bits <= 24;
+    }
     bool dense_now() const
     {
-        return !win_now() && sort_mode != 1 && bucket && capacity <= kWinCells && sortw_fits(n);
+        return !win_now() && sort_mode != 1 && bucket && !count_off && capacity <= kWinCells && sortw_fits(n);
     }
     bool count_now() const { return dense_now() || win_now(); }
     // room to count in windows, or in the whole table while that is small; without the memory for
@@ -446,8 +481,10 @@ struct sm_ctx {
     }
 
     void check_flags() { check_bits(link.fetch(st, glob, nullptr, 0, nullptr)); }
-    static void check_bits(int flags)
+    // the flags of a result, and what its count of fallbacks says
+    void check_bits(int flags)
     {
+        learn();
         if (flags & FLAG_BAD_POSITION)
             throw ApiError(SM_ERR_STATE, "a particle position left the box or became non-finite");
         if (flags & FLAG_SORT_TIMEOUT)
@@ -599,11 +636,12 @@ struct sm_ctx {
         win_last = count && win_now();
         cnt_last = counters_ready = count;
         if (count) {
+            counted_builds++;
             timed(K_REORDER, [&] {
                 launch_build(st, n, BuildArgs{k0, v0, k1, v1, k2, v2, win_keys(p), counts[1 - p], counted[1 - p],
                                               counted[p], wdesc ? wdesc + 8 * (1 - p) : nullptr, beads, sbeads, cstart,
                                               cend, hist[1 - p], hist_words, reps, hist[p],
-                                              win_scratch(hist[p], n) + kWinKeyWords, &glob->flags, build_tiles(n)});
+                                              win_scratch(hist[p], n) + kWinKeyWords, &glob->flags, &glob->fallbacks, build_tiles(n)});
             });
             order_valid = false;
             sort_parity = 1 - p;
@@ -839,10 +877,12 @@ struct sm_ctx {
                 HIPCHK(e);
             }
             HIPCHK(hipGraphInstantiate(&gexec[q], graph[q], nullptr, nullptr, 0));
-            if (any_mc) moves_since--;   // capture only recorded the move
+            if (any_mc) moves_since--;   // capture only recorded the move, and the builds
+            if (cnt_last) counted_builds -= 8;
         }
         sort_parity = p;   // and the toggles
         if (any_mc) moves_since++;
+        if (cnt_last) counted_builds += 8;
         // the block advances from step s - 1
         launch_set_step(st, glob, s - 1);
         HIPCHK(hipGraphLaunch(gexec[q], st));
@@ -876,6 +916,12 @@ struct sm_ctx {
         if (moves) ensure_capacity(moves);
         long long s = first;
         const long long end = first + nsteps;
+        if (nsteps >= 64 && count_now() && !counts_known) {
+            eager(s, s + 8);
+            s += 8;
+            (void)link.fetch(st, glob, nullptr, 0, nullptr);
+            learn();
+        }
         if (use_graph && !prof) {
             const long long lead = std::min(end, s + (9 - s % 8) % 8);   // up to the next s % 8 == 1
             eager(s, lead);
@@ -1372,6 +1418,7 @@ int sm_upload_state(sm_ctx *c, const double *pos, const double *vel, const doubl
             c->boxL = L;
             c->moves_since = 0;
             c->launch_rules();
+            c->count_again();
         }
     });
 }
@@ -1693,6 +1740,7 @@ int sm_tune(sm_ctx *c, const char *knob, int32_t value)
             if (value < 0 || value > 2) invalid("sort_mode must be 0, 1 or 2");
             if (value == 2 && !c->win_ok) invalid("sort_mode 2 needs a single replica of at most 524288 beads");
             c->forget_keys();
+            c->count_again();
             c->sort_mode = value;
             c->order_valid = false;
         } else if (std::strcmp(knob, "mc_fused") == 0) {
@@ -1727,7 +1775,8 @@ int sm_autotune(sm_ctx *c, int32_t steps, double *best_ms_per_step)
         if (!c) invalid("null context");
         if (steps < 8 || steps > 100000) invalid("steps per trial must be in [8, 100000]");
         if (c->prof) invalid("profiling is on");
-        const long long s0 = c->read_glob().step + 1;
+        const DevGlobal entry = c->read_glob();
+        const long long s0 = entry.step + 1;
         // every trial starts from the same state; reserve cells for the trials' moves
         // first so that no trial moves the cell bases
         long long moves = 0;
@@ -1760,6 +1809,8 @@ int sm_autotune(sm_ctx *c, int32_t steps, double *best_ms_per_step)
                 copy(c->beads, b0, sizeof(Bead) * n); copy(c->vel, v0, sizeof(float4) * n);
                 copy(c->acc, a0, sizeof(float4) * n); copy(c->reps, r0, sizeof(DevRep) * c->nrep);
                 copy(c->glob, g0, sizeof(DevGlobal));
+                c->fallbacks_seen = entry.fallbacks;
+                c->counted_builds = 0;
             };
             HIPCHK(hipEventCreate(&e0));
             HIPCHK(hipEventCreate(&e1));
@@ -1780,11 +1831,18 @@ int sm_autotune(sm_ctx *c, int32_t steps, double *best_ms_per_step)
                 if (c->sort_mode != k.sort) {
                     c->sort_mode = k.sort;
                     c->order_valid = false;
+                    c->count_again();
                 }
                 c->drop_graph();
                 restore();
                 c->run(s0, 8);          // warm: first launches, graph capture
+                const bool counted = c->count_now();
+                c->check_flags();
                 restore();
+                if (counted != c->count_now()) {   // it stopped counting: warm again
+                    c->run(s0, 8);
+                    restore();
+                }
                 HIPCHK(hipEventRecord(e0, st));
                 c->run(s0, steps);
                 HIPCHK(hipEventRecord(e1, st));
@@ -1810,6 +1868,7 @@ int sm_autotune(sm_ctx *c, int32_t steps, double *best_ms_per_step)
             if (c->sort_mode != bestc.sort) {
                 c->sort_mode = bestc.sort;
                 c->order_valid = false;
+                c->count_again();
             }
             c->drop_graph();
             restore();
@@ -1989,6 +2048,8 @@ struct AdjointRun {
     State own;                        // the context's
     Bead *own_alt;
     bool own_fused;
+    uint32_t own_fallbacks;           // with the counts of builds in the context's step counter
+    long long own_builds;
     // x[t]: a segment's positions after its t-th step, before that step's box move.  An
     // objective alone needs the step before only: two buffers in turns (at), and no segments.
     std::vector<Bead *> x;
@@ -2008,6 +2069,8 @@ struct AdjointRun {
         own = State{c->beads, c->vel, c->acc, c->reps, c->glob};
         own_alt = c->beads_alt;
         own_fused = c->mc_fused;
+        own_fallbacks = c->fallbacks_seen;
+        own_builds = c->counted_builds;
         // two passes over one list: the workspace's size, then its addresses
         State cur{};
         for (int pass = 0; pass < 2; pass++) {
@@ -2065,6 +2128,8 @@ struct AdjointRun {
         c->reps = own.reps;
         c->glob = own.glob;
         c->mc_fused = own_fused;
+        c->fallbacks_seen = own_fallbacks;
+        c->counted_builds = own_builds;
         c->forget_boxes();
         if (c->adj_ws_bytes > kIdleBytes) c->free_adj_workspace();
     }

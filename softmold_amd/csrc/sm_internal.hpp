@@ -69,7 +69,7 @@ struct __align__(16) GenEnt {
 // Context-wide device state.
 struct DevGlobal {
     int flags;
-    int pad;
+    uint32_t fallbacks;        // counting builds that sorted instead; read with the flags in one word
     long long step;            // step index of the step in progress (Philox counter)
     long long base;            // the step before the captured block in progress
 };
@@ -260,7 +260,7 @@ void launch_mc_propose(hipStream_t st, int nrep, DevRep *reps, const DevGlobal *
 void launch_mc_decide(hipStream_t st, const Params &P, DevRep *reps, DevGlobal *glob, const double *du);
 void launch_rescale(hipStream_t st, int n, Bead *beads, const DevRep *reps);
 // Result packing (sm_transfer.hpp), into pinned host memory.  launch_post: head[0] = the state
-// flags as a 64-bit integer, head[1 ..] = src[0 .. count).  launch_pack: `count` beads from
+// flags and the fallbacks as a 64-bit integer, head[1 ..] = src[0 .. count).  launch_pack: `count` beads from
 // `first` on, the positions as doubles, then each float4 array's x, y, z as floats (a NULL
 // source is left out); where head is given, the flags and the nrep boxes go to it.
 struct PackSrc {
@@ -347,6 +347,7 @@ struct BuildArgs {
     uint32_t *ghist;        // the cell indices' digit histograms [copies][4][256]
     uint32_t *status;       // look-back words of the fallback's three passes, tiles x 256 each
     int *errflag;
+    uint32_t *fallbacks;    // counts the builds that fall back
     int tiles;              // the fallback's tiles
 };
 void launch_build(hipStream_t st, int n, const BuildArgs &a);

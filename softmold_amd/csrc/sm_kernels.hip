@@ -854,7 +854,7 @@ __global__ __launch_bounds__(kBlock) void k_post(const double *__restrict__ src,
                                                  const DevGlobal *__restrict__ glob, double *__restrict__ head)
 {
     const size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x;
-    if (i == 0) *reinterpret_cast<long long *>(head) = glob->flags;
+    if (i == 0) *reinterpret_cast<long long *>(head) = *reinterpret_cast<const long long *>(glob);
     if (i < count) head[1 + i] = src[i];
 }
 
@@ -870,7 +870,7 @@ __global__ __launch_bounds__(kBlock) void k_pack(int first, int count, PackSrc s
                                                  const DevGlobal *__restrict__ glob, double *__restrict__ head)
 {
     if (head && blockIdx.x == 0) {
-        if (threadIdx.x == 0) *reinterpret_cast<long long *>(head) = glob->flags;
+        if (threadIdx.x == 0) *reinterpret_cast<long long *>(head) = *reinterpret_cast<const long long *>(glob);
         for (int i = threadIdx.x; i < 3 * nrep; i += kBlock) head[1 + i] = reps[i / 3].L[i % 3];
     }
     const int e = blockIdx.x * kBlock + threadIdx.x;

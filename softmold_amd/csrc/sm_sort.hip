@@ -864,6 +864,7 @@ __device__ void build_sorted(WLds<kRounds> &L, int n, const BuildArgs &a, const 
                            v[p + 1u], a.status + (size_t)p * tiles * 256u, a.errflag);
         } else {
             if (!dense && tile == 0 && threadIdx.x < kWave) next_window(a, w, true);
+            if (tile == 0 && threadIdx.x == 0) atomicAdd(a.fallbacks, 1u);
             build_reorder<kRounds>(n, tile, a);
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");

@@ -186,6 +186,9 @@ public:
         return flags();
     }
 
+    // the count of fallbacks (DevGlobal) that came with the last result
+    uint32_t fallbacks() const { return (uint32_t)((unsigned long long)word() >> 32); }
+
     // reps[r].scale = scale[3r ..]; the caller's array is free again on return, the buffer after
     // the next fetch
     void send_scale(hipStream_t st, DevRep *reps, int nrep, const double *scale)
@@ -214,7 +217,7 @@ public:
 private:
     void *buf_[kBuffers] = {};
     size_t beads_[kBuffers] = {};
-    double *head_ = nullptr;      // flags, then room_ doubles
+    double *head_ = nullptr;      // flags and fallbacks, then room_ doubles
     size_t room_ = 0;
     int device_ = 0;              // the context's
     hipEvent_t ev_[kBuffers] = {};
@@ -257,12 +260,13 @@ private:
         check(hipEventRecord(ev_[e], st), "event");
         check(hipEventSynchronize(ev_[e]), "event");
     }
-    int flags() const
+    long long word() const
     {
         long long f;
         std::memcpy(&f, head_, sizeof f);
-        return (int)f;
+        return f;
     }
+    int flags() const { return (int)word(); }
 };
 
 }  // namespace smdev

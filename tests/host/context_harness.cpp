@@ -29,6 +29,8 @@ struct Keys {
     size_t table;
 };
 Keys g_keys{};
+bool g_crowded = false;              // counting builds fall back
+int g_builds = 0, g_sorts = 0;       // counting builds, radix sorts
 
 #define EXPECT(cond)                                                       \
     do {                                                                   \
@@ -60,6 +62,12 @@ hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
 hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
 hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) { *ms = 1.f; return hipSuccess; }
+hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipSuccess; }
+hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t *g) { *g = reinterpret_cast<hipGraph_t>(1); return hipSuccess; }
+hipError_t hipGraphInstantiate(hipGraphExec_t *e, hipGraph_t, hipGraphNode_t *, char *, size_t) { *e = reinterpret_cast<hipGraphExec_t>(1); return hipSuccess; }
+hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return hipSuccess; }
+hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
+hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
 hipError_t hipStreamCreate(hipStream_t *st) { *st = nullptr; return hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
@@ -147,6 +155,7 @@ int radix_sort(hipStream_t, SortBuffers &b, int, int)
 {
     touch(b.k1, b.n);
     take_keys(WinBook{}, false);
+    g_sorts++;
     return 0;
 }
 void sort_moved(hipStream_t, SortBuffers &, const MoveSort &, int, int) { take_keys(WinBook{}, true); }
@@ -154,6 +163,8 @@ void launch_build(hipStream_t, int n, const BuildArgs &a)
 {
     touch_book(a.wb);
     take_keys(a.wb, false);
+    g_builds++;
+    if (g_crowded) ++*a.fallbacks;
     for (const uint32_t *p : {a.k2, a.v0, a.v2, (uint32_t *)a.cells_old, a.cells_now}) touch(p, n);
     touch(a.counts_old, a.wb.limit);
     touch(a.cstart, g_cells);
@@ -183,10 +194,10 @@ void launch_pair_gather(hipStream_t, const Params &, int, int, const Bead *, con
 void launch_sums(hipStream_t, SumKind, const SumArgs &) {}
 void launch_pack(hipStream_t, int, int, const PackSrc &, double *, const DevRep *reps, int nrep, const DevGlobal *g, double *head)
 {
-    *reinterpret_cast<long long *>(head) = g->flags;
+    std::memcpy(head, (const void *)g, sizeof(long long));
     for (int i = 0; i < 3 * nrep; i++) head[1 + i] = reps[i / 3].L[i % 3];
 }
-void launch_post(hipStream_t, const double *, size_t, const DevGlobal *g, double *head) { *reinterpret_cast<long long *>(head) = g->flags; }
+void launch_post(hipStream_t, const double *, size_t, const DevGlobal *g, double *head) { std::memcpy(head, (const void *)g, sizeof(long long)); }
 }  // namespace smdev
 
 namespace {
@@ -287,6 +298,53 @@ int step_phases()
     return 0;
 }
 
+// Builds that keep falling back are left to the sort: in a first long run, and from results; a
+// context whose builds count goes on counting, and one that stopped does again when it is told
+// to or has another box.
+int crowded_cells()
+{
+    for (const int graph : {0, 1})
+        for (const int mode : {0, 2}) {
+            System a(200, 24);
+            sm_ctx *c = nullptr;
+            double e[3];
+            const auto runs = [&](int steps, bool counted) {
+                g_builds = g_sorts = 0;
+                EXPECT(sm_run(c, 1, steps) == SM_OK);
+                EXPECT(counted ? g_builds > 0 && g_sorts == 0 : g_builds == 0 && g_sorts > 0);
+            };
+            g_crowded = false;
+            EXPECT(sm_create(&a.s, &c) == SM_OK && sm_tune(c, "sort_mode", mode) == SM_OK);
+            EXPECT(sm_init_forces(c) == SM_OK);
+            for (int k = 0; k < 3; k++) {
+                runs(100, true);
+                EXPECT(sm_measure(c, e) == SM_OK);
+            }
+            // the box gets crowded: seen by the next result
+            g_crowded = true;
+            runs(100, true);
+            EXPECT(sm_sync(c) == SM_OK);
+            runs(100, false);
+            EXPECT(sm_tune(c, "graph", graph) == SM_OK);
+            runs(100, false);
+            // told to count again: a first long run finds out after 8 steps
+            EXPECT(sm_tune(c, "sort_mode", mode) == SM_OK);
+            g_builds = g_sorts = 0;
+            EXPECT(sm_run(c, 1, 100) == SM_OK && g_builds == 8 && g_sorts > 0);
+            runs(100, false);
+            // another box: counted again, and that stays
+            const double L[3] = {26, 26, 26};
+            g_crowded = false;
+            EXPECT(sm_upload_state(c, nullptr, nullptr, nullptr, L) == SM_OK);
+            for (int k = 0; k < 3; k++) {
+                runs(100, true);
+                EXPECT(sm_measure(c, e) == SM_OK);
+            }
+            EXPECT(sm_destroy(c) == SM_OK);
+        }
+    return 0;
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
@@ -295,6 +353,7 @@ int main(int argc, char **argv)
     if (what == "growth_fails") return growth_fails();
     if (what == "box_and_shapes") return box_and_shapes();
     if (what == "step_phases") return step_phases();
+    if (what == "crowded_cells") return crowded_cells();
     std::fprintf(stderr, "unknown scenario\n");
     return 2;
 }

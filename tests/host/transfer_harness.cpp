@@ -79,14 +79,14 @@ hipError_t hipHostFree(void *p) { std::free(p); return hipSuccess; }
 namespace smdev {
 void launch_post(hipStream_t, const double *src, size_t count, const DevGlobal *glob, double *head)
 {
-    *reinterpret_cast<long long *>(head) = glob->flags;
+    std::memcpy(head, (const void *)glob, sizeof(long long));
     for (size_t i = 0; i < count; i++) head[1 + i] = src[i];
 }
 void launch_pack(hipStream_t, int first, int count, const PackSrc &src, double *out, const DevRep *reps, int nrep,
                  const DevGlobal *glob, double *head)
 {
     if (head) {
-        *reinterpret_cast<long long *>(head) = glob->flags;
+        std::memcpy(head, (const void *)glob, sizeof(long long));
         for (int i = 0; i < 3 * nrep; i++) head[1 + i] = reps[i / 3].L[i % 3];
     }
     float *f = reinterpret_cast<float *>(out + (src.beads ? 3 * (size_t)count : 0));
@@ -127,7 +127,7 @@ struct State {
         }
         for (int r = 0; r < R; r++)
             for (int d = 0; d < 3; d++) reps[r].L[d] = 10.0 * r + d;
-        glob.flags = 5;
+        glob.flags = 5, glob.fallbacks = 9;
     }
     hipStream_t st() { return reinterpret_cast<hipStream_t>(&stream); }
     PackSrc src() { return PackSrc{beads.data(), vel.data(), nullptr}; }
@@ -143,6 +143,7 @@ void check_download(State &s, HostLink &link)
             EXPECT(vel[3 * (size_t)i + c] == (&s.vel[i].x)[c]);
         }
     for (int i = 0; i < 3 * s.R; i++) EXPECT(box[i] == s.reps[i / 3].L[i % 3]);
+    EXPECT(link.fallbacks() == 9);
 }
 
 // Calls made while another device is current than the context's.
