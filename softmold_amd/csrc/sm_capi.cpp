@@ -151,6 +151,7 @@ struct sm_ctx {
     uint32_t *k0 = nullptr, *v0 = nullptr, *k1 = nullptr, *v1 = nullptr;
     uint32_t *hist[2] = {nullptr, nullptr};   // sort scratch, double-buffered
     size_t hist_words = 0;
+    uint32_t *zeros = nullptr;                // holds hist, wdesc, counted and the sums' tickets
     int sort_parity = 0;                      // scratch the next sort uses
     bool hist_pending = false;                // its histograms hold keys not sorted yet
     // Incremental re-sort (sort_mode 1; 0: every build sorts all keys from index order): the
@@ -229,8 +230,9 @@ struct sm_ctx {
     void alloc_counts()
     {
         if (!sortw_fits(n)) return;
+        // a window is a part of the table, so a small table's cells are enough for either
         size_t cells = win_ok ? count_limit(n) : 0;
-        if (capacity <= kWinCells) cells = std::max(cells, ((size_t)capacity + kCoarseCells - 1) / kCoarseCells * kCoarseCells);
+        if (capacity <= kWinCells) cells = ((size_t)capacity + kCoarseCells - 1) / kCoarseCells * kCoarseCells;
         if (cells <= count_cells) return;
         counters_ready = false;
         count_cells = 0;
@@ -239,12 +241,7 @@ struct sm_ctx {
         try {
             if (!k2) k2 = dalloc<uint32_t>(n);
             if (!v2) v2 = dalloc<uint32_t>(n);
-            for (int p = 0; p < 2; p++) {
-                counts[p] = dalloc<uint32_t>(cells);
-                if (counted[p]) continue;
-                counted[p] = dalloc<uint32_t>(n);
-                HIPCHK(hipMemsetAsync(counted[p], 0, sizeof(uint32_t) * n, st));
-            }
+            for (uint32_t *&p : counts) p = dalloc<uint32_t>(cells);
             bucket = dalloc<uint32_t>(cells * kBucket);
             count_cells = cells;
         } catch (const ApiError &) {
@@ -393,9 +390,8 @@ struct sm_ctx {
         for (auto &r : recs) { (void)hipEventDestroy(r.a); (void)hipEventDestroy(r.b); }
         for (auto e : pool) (void)hipEventDestroy(e);
         dfree(beads); dfree(sbeads); dfree(beads_alt); dfree(vel); dfree(acc); dfree(fpair); dfree(fscratch);
-        dfree(k0); dfree(v0); dfree(k1); dfree(v1); dfree(hist[0]); dfree(hist[1]); dfree(cstart); dfree(cend);
-        dfree(k2); dfree(v2); dfree(wdesc); dfree(bucket);
-        for (int p = 0; p < 2; p++) { dfree(counts[p]); dfree(counted[p]); }
+        dfree(k0); dfree(v0); dfree(k1); dfree(v1); dfree(zeros); dfree(cstart); dfree(cend);
+        dfree(k2); dfree(v2); dfree(bucket); dfree(counts[0]); dfree(counts[1]);
         for (int p = 0; p < 2; p++) { dfree(kidx[p]); dfree(sk[p]); dfree(sv[p]); }
         dfree(mbefore); dfree(cnt_b); dfree(cnt_i); dfree(cnt_s); dfree(mflags); dfree(mcount);
         dfree(reps); dfree(glob); dfree(fconstF); dfree(uconstD); dfree(fconstD); dfree(chainPerBead); dfree(chainList);
@@ -403,8 +399,8 @@ struct sm_ctx {
         dfree(cconstD); dfree(ebead); dfree(edelta); dfree(dres); dfree(dcounts); dfree(dpairs); dfree(dnp);
         free_adj_workspace();
         dfree(adjF); dfree(adjDF); dfree(adjDU); dfree(pdU); dfree(pdTab); dfree(pdC);
-        dfree(segB.tile); dfree(segB.rep_first); dfree(segB.tilesum); dfree(segB.ticket);
-        dfree(segC.tile); dfree(segC.rep_first); dfree(segC.tilesum); dfree(segC.ticket);
+        dfree(segB.tile); dfree(segB.rep_first); dfree(segB.tilesum);
+        dfree(segC.tile); dfree(segC.rep_first); dfree(segC.tilesum);
         if (st) (void)hipStreamDestroy(st);
     }
 
@@ -1203,8 +1199,6 @@ sm_ctx *create(const sm_system *s, int nrep)
         if (c->win_ok) {
             c->k2 = dalloc<uint32_t>(n);
             c->v2 = dalloc<uint32_t>(n);
-            c->wdesc = dalloc<uint32_t>(16);
-            HIPCHK(hipMemsetAsync(c->wdesc, 0, sizeof(uint32_t) * 16, c->st));
         }
         c->mbefore = dalloc<uint32_t>(n);
         c->cnt_b = dalloc<uint32_t>(move_blocks(n));
@@ -1213,9 +1207,27 @@ sm_ctx *create(const sm_system *s, int nrep)
         c->mflags = dalloc<unsigned long long>(((size_t)n + 63) / 64);
         c->mcount = dalloc<int>(1);
         c->hist_words = sort_scratch_words(n, 4) + sortw_words(n, sortw_fits(n));
-        for (int p = 0; p < 2; p++) {
-            c->hist[p] = dalloc<uint32_t>(c->hist_words);
-            HIPCHK(hipMemsetAsync(c->hist[p], 0, sizeof(uint32_t) * c->hist_words, c->st));
+        // what starts as zeros, in one buffer with one clear: six of them took a new 12k-bead
+        // context 80 us longer to make
+        {
+            size_t words = 0;
+            const auto room = [&](size_t count) {
+                const size_t at = words;
+                words += (count + 63) / 64 * 64;
+                return at;
+            };
+            const size_t tickets = (size_t)kTicketWords * nrep;
+            const size_t h[2] = {room(c->hist_words), room(c->hist_words)}, w = room(16), tb = room(tickets),
+                         tc = room(tickets), cells[2] = {room(sortw_fits(n) ? n : 0), room(sortw_fits(n) ? n : 0)};
+            c->zeros = dalloc<uint32_t>(words);
+            HIPCHK(hipMemsetAsync(c->zeros, 0, sizeof(uint32_t) * words, c->st));
+            for (int p = 0; p < 2; p++) {
+                c->hist[p] = c->zeros + h[p];
+                c->counted[p] = c->zeros + cells[p];
+            }
+            if (c->win_ok) c->wdesc = c->zeros + w;
+            c->segB.ticket = c->zeros + tb;
+            c->segC.ticket = c->zeros + tc;
         }
         c->reps = dalloc<DevRep>(nrep);
         c->glob = dalloc<DevGlobal>(1);
@@ -1235,8 +1247,6 @@ sm_ctx *create(const sm_system *s, int nrep)
             S.tile = dalloc<int4>(h.tile.size());
             S.rep_first = dalloc<int>(h.rep_first.size());
             S.tilesum = dalloc<double>(kSumCols * h.tile.size());
-            S.ticket = dalloc<uint32_t>((size_t)kTicketWords * nrep);
-            HIPCHK(hipMemsetAsync(S.ticket, 0, sizeof(uint32_t) * kTicketWords * nrep, c->st));
             if (!h.tile.empty())
                 HIPCHK(hipMemcpyAsync(S.tile, h.tile.data(), sizeof(int4) * h.tile.size(), hipMemcpyHostToDevice, c->st));
             HIPCHK(hipMemcpyAsync(S.rep_first, h.rep_first.data(), sizeof(int) * h.rep_first.size(),

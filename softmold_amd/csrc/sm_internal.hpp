@@ -151,10 +151,12 @@ struct MoveBook {
 //  - window (sort_mode 2: one replica, every key sorted, keys of 17 to 24 bits, at most
 //    kWinMaxTiles tiles of keys): each build has a window of cells, the previous measured
 //    occupied cell range widened by one cell on each side, used when it holds at most
-//    count_limit(n) cells: four a bead, 2^14 to 2^18, so that a small context's buckets are
-//    small too (a vesicle's window has half a cell a bead at most).  A key whose cell lies in
-//    it is stored as kWinTag | the cell's index in the window's own (z, y, x) order, which
-//    orders keys as the cell index does.
+//    count_limit(n) cells: two a bead, 2^14 to 2^18, so that a small context's buckets are
+//    small too (with four a bead, a 90k-bead context took 1.1 ms to make and 1.2 to destroy,
+//    0.9 and 0.2 now).  A vesicle's window, the cube around its shell, has 0.52 cells a bead at
+//    240k beads and 0.67 at 510k; past 420k beads it holds more than 2^18 cells, and the context
+//    stops counting.  A key whose cell lies in the window is stored as kWinTag | the cell's
+//    index in the window's own (z, y, x) order, which orders keys as the cell index does.
 //  - dense (sort_mode 0 or 2, any context of at most kWinMaxTiles tiles of keys, 524288 beads,
 //    whose cell table holds at most kWinCells cells): the cell index itself.  The counters take
 //    25 atomics a ns, a radix pass 5 us at least: per step 119 us counted against 144

@@ -1000,7 +1000,7 @@ uint32_t *win_scratch(uint32_t *sort_scratch, int n) { return sort_scratch + sor
 
 size_t count_limit(int n)
 {
-    const long long want = std::min<long long>(std::max<long long>(4ll * n, 1 << 14), kWinCells);
+    const long long want = std::min<long long>(std::max<long long>(2ll * n, 1 << 14), kWinCells);
     return (size_t)((want + kCoarseCells - 1) / kCoarseCells * kCoarseCells);
 }
 

@@ -19,6 +19,8 @@ namespace {
 int g_bad_malloc = -1;      // the device allocation that fails, counted down
 bool g_failed = false;      // one did
 hipError_t g_last = hipSuccess;
+size_t g_bytes = 0;         // device memory allocated so far
+int g_clears = 0;           // and clears
 size_t g_cells = 0;         // cells of the table that the replicas were given
 // The keys that the last key kernel left for a build, as far as a build must agree with it.
 struct Keys {
@@ -80,11 +82,12 @@ hipError_t hipMalloc(void **p, size_t bytes)
         return g_last = hipErrorOutOfMemory;
     }
     *p = std::calloc(1, bytes);
+    g_bytes += bytes;
     return hipSuccess;
 }
 hipError_t hipFree(void *p) { std::free(p); return hipSuccess; }
 hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t) { std::memcpy(d, s, n); return hipSuccess; }
-hipError_t hipMemsetAsync(void *d, int v, size_t n, hipStream_t) { std::memset(d, v, n); return hipSuccess; }
+hipError_t hipMemsetAsync(void *d, int v, size_t n, hipStream_t) { std::memset(d, v, n); g_clears++; return hipSuccess; }
 }
 
 namespace smdev {
@@ -99,7 +102,7 @@ size_t sortw_words(int n, bool counting) { return kWinKeyWords + (counting ? (si
 uint32_t *win_scratch(uint32_t *s, int n) { return s + sort_scratch_words(n, 4); }
 size_t count_limit(int n)
 {
-    const long long want = std::min<long long>(std::max<long long>(4ll * n, 1 << 14), kWinCells);
+    const long long want = std::min<long long>(std::max<long long>(2ll * n, 1 << 14), kWinCells);
     return (size_t)((want + kCoarseCells - 1) / kCoarseCells * kCoarseCells);
 }
 WinBook win_book(uint32_t *s, int n, const uint32_t *desc, uint32_t *counts, uint32_t *bucket, uint32_t cells, uint32_t limit)
@@ -345,6 +348,26 @@ int crowded_cells()
     return 0;
 }
 
+// What making a context takes from the device: the counting builds' buckets follow the cells of
+// a small table, and the beads of a small context in a large one; and few clears.
+int creation()
+{
+    struct { int n; double box; size_t mib; } cases[] = {
+        {90000, 92, 60},       // 46^3 cells, 107k in the table: 26 MiB of buckets, not 64
+        {20000, 200, 36},      // a million cells (8 MiB of table), 40k counted: 10 MiB, not 20
+    };
+    for (const auto &k : cases) {
+        System a(k.n, k.box);
+        sm_ctx *c = nullptr;
+        g_bytes = 0, g_clears = 0;
+        EXPECT(sm_create(&a.s, &c) == SM_OK);
+        std::fprintf(stderr, "%d beads: %zu MiB, %d clears\n", k.n, g_bytes >> 20, g_clears);
+        EXPECT(g_bytes >> 20 < k.mib && g_clears <= 4);
+        EXPECT(sm_destroy(c) == SM_OK);
+    }
+    return 0;
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
@@ -354,6 +377,7 @@ int main(int argc, char **argv)
     if (what == "box_and_shapes") return box_and_shapes();
     if (what == "step_phases") return step_phases();
     if (what == "crowded_cells") return crowded_cells();
+    if (what == "creation") return creation();
     std::fprintf(stderr, "unknown scenario\n");
     return 2;
 }

@@ -8,6 +8,7 @@ sanitizer.
 - step_phases: whatever comes between the two halves of a step (another sort mode, another
   table, or no first half at all), a build is launched on keys that were made for it.
 - crowded_cells: counting builds that keep falling back are left to the sort.
+- creation: the device memory and the clears that making a context takes.
 """
 import os
 import shutil
@@ -33,7 +34,7 @@ def harness(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("scenario", ["growth_fails", "box_and_shapes", "step_phases", "crowded_cells"])
+@pytest.mark.parametrize("scenario", ["growth_fails", "box_and_shapes", "step_phases", "crowded_cells", "creation"])
 def test_context(harness, scenario):
     env = dict(os.environ, ASAN_OPTIONS="verify_asan_link_order=0:detect_leaks=0")
     r = subprocess.run([harness, scenario], env=env, capture_output=True, text=True, timeout=60)
