@@ -13,6 +13,8 @@
 #include <cmath>
 #include <cstring>
 #include <string>
+#include <type_traits>
+#include <utility>
 #include <vector>
 
 using namespace smdev;
@@ -113,8 +115,8 @@ struct RepHost {
     long long capacity = 0, cellbase = 0;
 };
 
-// Tiles of a segment set: ranges [begin_r, begin_r + len_r) cut into kSegTile pieces that
-// start at each range's start.
+// Tiles of a segment set: ranges [begin_r, begin_r + len_r) cut into tiles that start at each
+// range's start, of kSumTile elements or, in a range of more than kSumTiles of those, a multiple.
 struct SegHost {
     std::vector<int4> tile;
     std::vector<int> rep_first;
@@ -144,14 +146,17 @@ struct sm_ctx {
     int nchains = 0;
     bool any_mc = false;   // some replica has delta_lxy != 0
     std::vector<RepHost> rh;
-    // device state
+    // device state: `slab` holds every buffer whose size stays, `table` cstart and cend, `counting`
+    // counts and bucket
+    char *slab = nullptr;
+    int *table = nullptr;
+    uint32_t *counting = nullptr;
     Bead *beads = nullptr, *sbeads = nullptr;
     Bead *beads_alt = nullptr;   // the fused kick + next first half writes positions here, then swaps
     float4 *vel = nullptr, *acc = nullptr, *fpair = nullptr, *fscratch = nullptr;
     uint32_t *k0 = nullptr, *v0 = nullptr, *k1 = nullptr, *v1 = nullptr;
     uint32_t *hist[2] = {nullptr, nullptr};   // sort scratch, double-buffered
     size_t hist_words = 0;
-    uint32_t *zeros = nullptr;                // holds hist, wdesc, counted and the sums' tickets
     int sort_parity = 0;                      // scratch the next sort uses
     bool hist_pending = false;                // its histograms hold keys not sorted yet
     // Incremental re-sort (sort_mode 1; 0: every build sorts all keys from index order): the
@@ -236,17 +241,17 @@ struct sm_ctx {
         if (cells <= count_cells) return;
         counters_ready = false;
         count_cells = 0;
-        dfree(bucket);
-        for (uint32_t *&p : counts) dfree(p);
+        bucket = nullptr;
+        counts[0] = counts[1] = nullptr;
+        dfree(counting);
         try {
-            if (!k2) k2 = dalloc<uint32_t>(n);
-            if (!v2) v2 = dalloc<uint32_t>(n);
-            for (uint32_t *&p : counts) p = dalloc<uint32_t>(cells);
-            bucket = dalloc<uint32_t>(cells * kBucket);
-            count_cells = cells;
+            counting = dalloc<uint32_t>(cells * (kBucket + 2));
         } catch (const ApiError &) {
-            for (uint32_t *&p : counts) dfree(p);
+            return;
         }
+        bucket = counting;
+        for (int p = 0; p < 2; p++) counts[p] = counting + cells * (kBucket + p);
+        count_cells = cells;
     }
     int *cstart = nullptr, *cend = nullptr;
     long long capacity = 0;   // cells in the dense table, all replicas
@@ -389,18 +394,9 @@ struct sm_ctx {
         link.destroy();
         for (auto &r : recs) { (void)hipEventDestroy(r.a); (void)hipEventDestroy(r.b); }
         for (auto e : pool) (void)hipEventDestroy(e);
-        dfree(beads); dfree(sbeads); dfree(beads_alt); dfree(vel); dfree(acc); dfree(fpair); dfree(fscratch);
-        dfree(k0); dfree(v0); dfree(k1); dfree(v1); dfree(zeros); dfree(cstart); dfree(cend);
-        dfree(k2); dfree(v2); dfree(bucket); dfree(counts[0]); dfree(counts[1]);
-        for (int p = 0; p < 2; p++) { dfree(kidx[p]); dfree(sk[p]); dfree(sv[p]); }
-        dfree(mbefore); dfree(cnt_b); dfree(cnt_i); dfree(cnt_s); dfree(mflags); dfree(mcount);
-        dfree(reps); dfree(glob); dfree(fconstF); dfree(uconstD); dfree(fconstD); dfree(chainPerBead); dfree(chainList);
-        dfree(gptr); dfree(gent); dfree(gconstD);
-        dfree(cconstD); dfree(ebead); dfree(edelta); dfree(dres); dfree(dcounts); dfree(dpairs); dfree(dnp);
+        dfree(slab); dfree(table); dfree(counting); dfree(dpairs);
         free_adj_workspace();
         dfree(adjF); dfree(adjDF); dfree(adjDU); dfree(pdU); dfree(pdTab); dfree(pdC);
-        dfree(segB.tile); dfree(segB.rep_first); dfree(segB.tilesum);
-        dfree(segC.tile); dfree(segC.rep_first); dfree(segC.tilesum);
         if (st) (void)hipStreamDestroy(st);
     }
 
@@ -554,22 +550,19 @@ struct sm_ctx {
             hr[r].cellbase = laid[r].cellbase;
             hr[r].capacity = laid[r].capacity;
         }
-        int *start = dalloc<int>((size_t)base), *end = nullptr;
+        int *grown = dalloc<int>(2 * (size_t)base);
         try {
-            end = dalloc<int>((size_t)base);
-            HIPCHK(hipMemsetAsync(start, 0xFF, sizeof(int) * (size_t)base, st));
-            HIPCHK(hipMemsetAsync(end, 0xFF, sizeof(int) * (size_t)base, st));
+            HIPCHK(hipMemsetAsync(grown, 0xFF, 2 * sizeof(int) * (size_t)base, st));
         } catch (...) {
-            dfree(start);
-            dfree(end);
+            dfree(grown);
             throw;
         }
         drop_graph();
         forget_keys();
-        dfree(cstart);
-        dfree(cend);
-        cstart = start;
-        cend = end;
+        dfree(table);
+        table = grown;
+        cstart = table;
+        cend = table + base;
         rh = std::move(laid);
         capacity = base;
         write_reps(hr);
@@ -1177,76 +1170,69 @@ sm_ctx *create(const sm_system *s, int nrep)
         }
         const SegHost tb = make_tiles(bb, bl), tc = make_tiles(cb, cl);
 
-        c->beads = dalloc<Bead>(n);
-        c->sbeads = dalloc<Bead>(n);
-        c->beads_alt = dalloc<Bead>(n);
-        c->beads_home = c->beads;
-        c->vel = dalloc<float4>(n);
-        c->acc = dalloc<float4>(n);
-        c->fpair = dalloc<float4>(n);
-        c->fscratch = dalloc<float4>(n);
-        c->k0 = dalloc<uint32_t>(n);
-        c->v0 = dalloc<uint32_t>(n);
-        c->k1 = dalloc<uint32_t>(n);
-        c->v1 = dalloc<uint32_t>(n);
-        for (int p = 0; p < 2; p++) {
-            c->kidx[p] = dalloc<uint32_t>(n);
-            c->sk[p] = dalloc<uint32_t>(n);
-            c->sv[p] = dalloc<uint32_t>(n);
-        }
         c->win_ok = nrep == 1 && sortw_fits(n);
         c->sort_mode = n >= 1000000 ? 1 : (c->win_ok ? 2 : 0);
-        if (c->win_ok) {
-            c->k2 = dalloc<uint32_t>(n);
-            c->v2 = dalloc<uint32_t>(n);
-        }
-        c->mbefore = dalloc<uint32_t>(n);
-        c->cnt_b = dalloc<uint32_t>(move_blocks(n));
-        c->cnt_i = dalloc<uint32_t>(move_tiles(n));
-        c->cnt_s = dalloc<uint32_t>(move_tiles(n));
-        c->mflags = dalloc<unsigned long long>(((size_t)n + 63) / 64);
-        c->mcount = dalloc<int>(1);
         c->hist_words = sort_scratch_words(n, 4) + sortw_words(n, sortw_fits(n));
-        // what starts as zeros, in one buffer with one clear: six of them took a new 12k-bead
-        // context 80 us longer to make
-        {
-            size_t words = 0;
-            const auto room = [&](size_t count) {
-                const size_t at = words;
-                words += (count + 63) / 64 * 64;
-                return at;
+        // Every buffer whose size stays, in one allocation: each of some 50 cost 10 us and, past the
+        // runtime's cache of freed memory, 250 us more to free.  Twice over one list: its size, then
+        // the addresses; what starts as zeros comes last and has one clear.
+        size_t zeros_at = 0, bytes = 0;
+        for (int pass = 0; pass < 2; pass++) {
+            if (pass) c->slab = dalloc<char>(bytes);
+            size_t at = 0;
+            const auto take = [&](auto *&p, size_t count) {
+                using T = std::remove_reference_t<decltype(*p)>;
+                if (pass) p = reinterpret_cast<T *>(c->slab + at);
+                at += (sizeof(T) * std::max<size_t>(count, 1) + 255) / 256 * 256;
             };
-            const size_t tickets = (size_t)kTicketWords * nrep;
-            const size_t h[2] = {room(c->hist_words), room(c->hist_words)}, w = room(16), tb = room(tickets),
-                         tc = room(tickets), cells[2] = {room(sortw_fits(n) ? n : 0), room(sortw_fits(n) ? n : 0)};
-            c->zeros = dalloc<uint32_t>(words);
-            HIPCHK(hipMemsetAsync(c->zeros, 0, sizeof(uint32_t) * words, c->st));
-            for (int p = 0; p < 2; p++) {
-                c->hist[p] = c->zeros + h[p];
-                c->counted[p] = c->zeros + cells[p];
+            for (Bead **p : {&c->beads, &c->sbeads, &c->beads_alt}) take(*p, n);
+            for (float4 **p : {&c->vel, &c->acc, &c->fscratch}) take(*p, n);
+            for (uint32_t **p : {&c->k0, &c->v0, &c->k1, &c->v1, &c->kidx[0], &c->kidx[1], &c->sk[0], &c->sk[1], &c->sv[0],
+                                 &c->sv[1], &c->mbefore})
+                take(*p, n);
+            if (sortw_fits(n))
+                for (uint32_t **p : {&c->k2, &c->v2}) take(*p, n);
+            take(c->cnt_b, move_blocks(n));
+            take(c->cnt_i, move_tiles(n));
+            take(c->cnt_s, move_tiles(n));
+            take(c->mflags, ((size_t)n + 63) / 64);
+            take(c->mcount, 1);
+            take(c->reps, nrep);
+            take(c->glob, 1);
+            take(c->fconstF, fF.size());
+            take(c->uconstD, nconst);
+            take(c->fconstD, nconst);
+            take(c->chainPerBead, n);
+            take(c->chainList, list.size());
+            take(c->cconstD, ccD.size());
+            take(c->ebead, n);
+            take(c->edelta, n);
+            take(c->dres, 8 * (size_t)nrep);
+            take(c->dcounts, n);
+            take(c->dnp, 1);
+            if (!gentH.empty()) {
+                take(c->gptr, gptrH.size());
+                take(c->gent, gentH.size());
+                take(c->gconstD, gcstH.size());
             }
-            if (c->win_ok) c->wdesc = c->zeros + w;
-            c->segB.ticket = c->zeros + tb;
-            c->segC.ticket = c->zeros + tc;
+            for (auto [S, h] : {std::make_pair(&c->segB, &tb), std::make_pair(&c->segC, &tc)}) {
+                take(S->tile, h->tile.size());
+                take(S->rep_first, h->rep_first.size());
+                take(S->tilesum, kSumCols * h->tile.size());
+            }
+            zeros_at = at;
+            take(c->fpair, n);
+            for (uint32_t **p : {&c->hist[0], &c->hist[1]}) take(*p, c->hist_words);
+            if (c->win_ok) take(c->wdesc, 16);
+            if (sortw_fits(n))
+                for (uint32_t **p : {&c->counted[0], &c->counted[1]}) take(*p, n);
+            for (SegTiles *S : {&c->segB, &c->segC}) take(S->ticket, (size_t)kTicketWords * nrep);
+            bytes = at;
         }
-        c->reps = dalloc<DevRep>(nrep);
-        c->glob = dalloc<DevGlobal>(1);
-        c->fconstF = dalloc<float>(fF.size());
-        c->uconstD = dalloc<double>(nconst);
-        c->fconstD = dalloc<double>(nconst);
-        c->chainPerBead = dalloc<int2>(n);
-        c->chainList = dalloc<int2>(list.size());
-        c->cconstD = dalloc<double4>(ccD.size());
-        c->ebead = dalloc<double>(n);
-        c->edelta = dalloc<double>(n);
-        c->dres = dalloc<double>(8 * (size_t)nrep);
-        c->dcounts = dalloc<int>(n);
-        c->dnp = dalloc<unsigned long long>(1);
+        c->beads_home = c->beads;
+        HIPCHK(hipMemsetAsync(c->slab + zeros_at, 0, bytes - zeros_at, c->st));
         auto upseg = [&](SegTiles &S, const SegHost &h) {
             S.ntiles = (int)h.tile.size();
-            S.tile = dalloc<int4>(h.tile.size());
-            S.rep_first = dalloc<int>(h.rep_first.size());
-            S.tilesum = dalloc<double>(kSumCols * h.tile.size());
             if (!h.tile.empty())
                 HIPCHK(hipMemcpyAsync(S.tile, h.tile.data(), sizeof(int4) * h.tile.size(), hipMemcpyHostToDevice, c->st));
             HIPCHK(hipMemcpyAsync(S.rep_first, h.rep_first.data(), sizeof(int) * h.rep_first.size(),
@@ -1260,7 +1246,6 @@ sm_ctx *create(const sm_system *s, int nrep)
         HIPCHK(hipMemcpyAsync(c->beads, hb.data(), sizeof(Bead) * n, hipMemcpyHostToDevice, st));
         HIPCHK(hipMemcpyAsync(c->vel, hv.data(), sizeof(float4) * n, hipMemcpyHostToDevice, st));
         HIPCHK(hipMemcpyAsync(c->acc, ha.data(), sizeof(float4) * n, hipMemcpyHostToDevice, st));
-        HIPCHK(hipMemsetAsync(c->fpair, 0, sizeof(float4) * n, st));
         HIPCHK(hipMemcpyAsync(c->reps, hr.data(), sizeof(DevRep) * nrep, hipMemcpyHostToDevice, st));
         HIPCHK(hipMemcpyAsync(c->glob, &g, sizeof g, hipMemcpyHostToDevice, st));
         HIPCHK(hipMemcpyAsync(c->fconstF, fF.data(), sizeof(float) * fF.size(), hipMemcpyHostToDevice, st));
@@ -1268,9 +1253,6 @@ sm_ctx *create(const sm_system *s, int nrep)
         HIPCHK(hipMemcpyAsync(c->fconstD, s[0].fconst, sizeof(double) * nconst, hipMemcpyHostToDevice, st));
         HIPCHK(hipMemcpyAsync(c->chainPerBead, perBead.data(), sizeof(int2) * n, hipMemcpyHostToDevice, st));
         if (!gentH.empty()) {
-            c->gptr = dalloc<int>(gptrH.size());
-            c->gent = dalloc<GenEnt>(gentH.size());
-            c->gconstD = dalloc<double2>(gcstH.size());
             HIPCHK(hipMemcpyAsync(c->gptr, gptrH.data(), sizeof(int) * gptrH.size(), hipMemcpyHostToDevice, st));
             HIPCHK(hipMemcpyAsync(c->gent, gentH.data(), sizeof(GenEnt) * gentH.size(), hipMemcpyHostToDevice, st));
             HIPCHK(hipMemcpyAsync(c->gconstD, gcstH.data(), sizeof(double2) * gcstH.size(), hipMemcpyHostToDevice,

@@ -153,7 +153,7 @@ struct MoveBook {
 //    occupied cell range widened by one cell on each side, used when it holds at most
 //    count_limit(n) cells: two a bead, 2^14 to 2^18, so that a small context's buckets are
 //    small too (with four a bead, a 90k-bead context took 1.1 ms to make and 1.2 to destroy,
-//    0.9 and 0.2 now).  A vesicle's window, the cube around its shell, has 0.52 cells a bead at
+//    0.9 and 0.2 with two).  A vesicle's window, the cube around its shell, has 0.52 cells a bead at
 //    240k beads and 0.67 at 510k; past 420k beads it holds more than 2^18 cells, and the context
 //    stops counting.  A key whose cell lies in the window is stored as kWinTag | the cell's
 //    index in the window's own (z, y, x) order, which orders keys as the cell index does.

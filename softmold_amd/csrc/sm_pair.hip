@@ -15,7 +15,7 @@
 //      per-cell LDS tables), so all global loads of a pass are in flight together; a
 //      pass holds kMaxC candidates and runs only the 64-slot rounds it fills;
 //   3. tpp = 64/H lanes serve each of the H home particles, each lane walking every
-//      tpp-th candidate; a home's partial results are combined by a fixed-shape tree of
+//      tpp-th candidate of the cell, through all its passes; a home's partial results are combined by a fixed-shape tree of
 //      shuffles (at step s, lane sub adds lane sub + s when sub is a multiple of 2s).
 // Force, one phase (M_FORCE1, the default): candidates are staged as FP64 imaged
 // positions, and each staged candidate is entered into the list of each quarter of the home
@@ -31,8 +31,10 @@
 // the exact FP64 test and the force law on the hits only.  Gathers: FP64 throughout, each pair's
 // difference taken in the reference's direction -- the particle of the cell that owns
 // the pair in the 13-cell half shell (cellOpt.h:715) minus the imaged other.  The energy
-// gathers (U, dU) stage only the home cell and its forward half shell and use the same
-// quarter-cell culling, with the reach radius widened by the trial scale for dU.
+// gathers (U, dU) stage only the home cell and its forward half shell.  Every traversal with
+// energies, the force's too (M_FDU, M_FU), culls in the same way against the quarters of the box
+// that the cell's home particles fill instead of the cell's, with the reach radius widened by the
+// trial scale for dU.
 //
 // What bounds it: vector instructions.  At 240k beads and 16 waves a CU the force issues 2270
 // of them per occupied cell, 78 % of the issue slots (92 us); with 12 waves a CU it takes 113.
