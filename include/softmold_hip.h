@@ -117,7 +117,9 @@ int sm_step_first(sm_ctx *ctx, int64_t step);
  * 0 gives the separate dU gather. */
 int sm_step_finish(sm_ctx *ctx, int64_t step, double *measure);
 /* Whole steps first_step .. first_step+nsteps-1 with no measurement, all on the device.
- * With the "graph" knob on, aligned blocks of 8 steps replay one captured hipGraph. */
+ * With the "graph" knob on, aligned blocks of 8 steps replay one captured hipGraph.  Returns
+ * with the steps queued; a context's first run of 64 steps or more waits for its first 8, which
+ * tell whether to count its beads per cell ("sort_mode"). */
 int sm_run(sm_ctx *ctx, int64_t first_step, int32_t nsteps);
 /* MC statistics so far, per replica (MD.cpp:713-720,748). */
 int sm_mc_stats(sm_ctx *ctx, int64_t *trials, int64_t *accepted);
@@ -188,7 +190,8 @@ int sm_potential_delta(sm_ctx *ctx, const double *scale, double *du_pair, double
  * occupied cells: counted per cell when every key lies in it, else sorted by the cell
  * indices' 8-bit passes, decided on the device.  0 and 2 count per cell without a window
  * where the whole cell table holds at most 2^18 cells and there are at most 524288 beads.
- * All give the same order, so none changes a result.
+ * A context most of whose counting builds had to sort goes over to sorting, until sort_mode
+ * is set again or a box uploaded.  All give the same order, so none changes a result.
  * "mc_fused" = 1 (default) to take a box-move step's pair dU in the traversal of
  * that step's pair force, 0 in a gather of its own after the kick (sm_potential_delta
  * follows the same knob); the two sum the same FP64 terms in different orders.

@@ -908,8 +908,12 @@ struct sm_ctx {
         if (nsteps >= 64 && count_now() && !counts_known) {
             eager(s, s + 8);
             s += 8;
-            (void)link.fetch(st, glob, nullptr, 0, nullptr);
-            learn();
+            try {
+                (void)link.fetch(st, glob, nullptr, 0, nullptr);
+                learn();
+            } catch (const ApiError &) {   // a wait that is refused where it is called: the next result tells
+                counts_known = true;
+            }
         }
         if (use_graph && !prof) {
             const long long lead = std::min(end, s + (9 - s % 8) % 8);   // up to the next s % 8 == 1
