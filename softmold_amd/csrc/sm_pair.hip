@@ -36,10 +36,10 @@
 // that the cell's home particles fill instead of the cell's, with the reach radius widened by the
 // trial scale for dU.
 //
-// What bounds it: vector instructions.  At 240k beads and 16 waves a CU the force issues 2270
-// of them per occupied cell, 78 % of the issue slots (92 us); with 12 waves a CU it takes 113.
-// So instructions are what counts outside the candidate loop (40 a candidate): the quarters
-// are taken from the comparisons' lane masks, the lists hold byte offsets, scans run in DPP
+// What bounds it: vector instructions.  At 240k beads and 16 waves a CU the force issued 2270
+// of them per occupied cell, 78 % of the issue slots, in 92 us (87 with a fifth wave a SIMD and
+// the box loaded with the keys); with 12 waves a CU it took 113.  So instructions are what
+// counts outside the candidate loop (40 a candidate): the quarters are taken from the comparisons' lane masks, the lists hold byte offsets, scans run in DPP
 // steps, the small divisions by reciprocals, a chunk without a cell leaves at once, and the
 // tables take the LDS of the types there are.  Together 95.7 -> 92 us for that force, the
 // force with dU 195 -> 178, U 87.6 -> 84.4; 3M-bead bilayer 955 -> 931 and 1705 -> 1555.
